@@ -145,6 +145,113 @@ def run(state):
     return (out,) + torch.autograd.grad(out, (a, b), g)
 
 
+def exact(case, seed):
+    """What `run` returns for these inputs, by plain torch in float64.  A maximum compares sums (products)
+    rounded once to float32, as its definition has it, and takes the lowest index that attains it; the
+    gradients of a drawn path have no such value."""
+    state = prepare(case, seed)
+    op = case["op"]
+    a, b = (state[x].detach().double().requires_grad_() for x in "ab")
+    g = state["g"].detach().double()
+    if op == "second":
+        g.requires_grad_()
+        out = _log_product(a, b)
+        first = torch.autograd.grad(out, (a, b), g, create_graph=True)
+        return (out,) + first + torch.autograd.grad(first, (a, b, g), [u.double() for u in state["u"]])
+    if op in ("max", "prodmax"):
+        return _best_product(a.detach(), b.detach(), g, op == "prodmax")
+    if op in _BAND_OPS:
+        wa, wb = case["a_lu"] + case["a_ld"] + 1, case["b_lu"] + case["b_ld"] + 1
+        rows = _band_rows(b, case["b_ld"], wb)
+        if op == "band_max":
+            return _best_band(a.detach(), rows.detach(), g, case)
+        # inputs within [-1, 1): exponentials need no shift
+        x, y = (a, rows) if op == "band_mul" else (a.exp(), torch.where(_band_cells(rows, case), rows.exp(), 0))
+        out = torch.zeros(*a.shape[:2], wa + wb - 1, dtype=torch.float64, device=a.device)
+        for i, cols, pos in _band_terms(case):
+            out[:, cols, i : i + wb] += x[:, cols, i : i + 1] * y[:, pos]
+        if op == "band_log":        # cells without a term hold 0
+            out = torch.where(out > 0, torch.where(out > 0, out, 1).log(), 0)
+    else:
+        out = _log_product(a, b)
+    if op == "sample":
+        return out.detach(), None, None
+    return (out.detach(),) + torch.autograd.grad(out, (a, b), g)
+
+
+def _log_product(a, b):
+    ma, mb = a.detach().amax(2, keepdim=True), b.detach().amax(1, keepdim=True)
+    return torch.bmm((a - ma).exp(), (b - mb).exp()).log() + ma + mb
+
+
+def _best_product(a, b, g, prod):
+    out, ga, gb = torch.empty_like(g), torch.zeros_like(a), torch.zeros_like(b)
+    K = a.shape[2]
+    step = max(1, 2**28 // (a.shape[1] * K * b.shape[2]))
+    ks = torch.arange(K, device=a.device).view(1, 1, K, 1)
+    for i in range(0, a.shape[0], step):
+        x, y, s = a[i : i + step].unsqueeze(3), b[i : i + step].unsqueeze(1), slice(i, i + step)
+        terms = (x * y if prod else x + y).float()
+        best = terms.amax(2, keepdim=True)
+        idx = torch.where(terms == best, ks, K).amin(2)
+        out[s] = best.squeeze(2)
+        gs = g[s]
+        if prod:
+            ga[s].scatter_add_(2, idx, gs * b[s].gather(1, idx))
+            gb[s].scatter_add_(1, idx, gs * a[s].gather(2, idx))
+        else:
+            ga[s].scatter_add_(2, idx, gs)
+            gb[s].scatter_add_(1, idx, gs)
+    return out, ga, gb
+
+
+def _band_rows(b, ld, width):
+    """rows[:, p, j]: the band's cell of dense row p and column p - ld + j (0 where there is none)."""
+    n = b.shape[1]
+    j = torch.arange(width, device=b.device)
+    col = torch.arange(n, device=b.device).unsqueeze(1) - ld + j
+    ok = (col >= 0) & (col < n)
+    return torch.where(ok, b[:, col.clamp(0, n - 1), (width - 1 - j).expand_as(col)], 0)
+
+
+def _band_cells(rows, case):
+    """Which cells of _band_rows are cells of the matrix."""
+    col = torch.arange(case["n"], device=rows.device).unsqueeze(1) - case["b_ld"] + torch.arange(rows.shape[2], device=rows.device)
+    return (col >= 0) & (col < case["n"])
+
+
+def _band_terms(case):
+    """(diagonal i of a, its columns, the dense rows they meet b in): out[c, i + j] takes a[c, i] and rows[c + i - a_lu, j]."""
+    n = case["n"]
+    for i in range(case["a_lu"] + case["a_ld"] + 1):
+        shift = i - case["a_lu"]
+        low, high = max(0, -shift), min(n, n - shift)
+        if low < high:
+            yield i, slice(low, high), slice(low + shift, high + shift)
+
+
+def _best_band(a, rows, g, case):
+    wb, cells = rows.shape[2], _band_cells(rows, case)
+    best, at = torch.full_like(g, -1e9), torch.zeros_like(g, dtype=torch.int64)
+    for i, cols, pos in _band_terms(case):
+        terms = torch.where(cells[pos], a[:, cols, i : i + 1] + rows[:, pos], -2e9).float().double()
+        old = best[:, cols, i : i + wb]
+        at[:, cols, i : i + wb] = torch.where(terms > old, i, at[:, cols, i : i + wb])
+        best[:, cols, i : i + wb] = torch.maximum(terms, old)
+    ga, grows = torch.zeros_like(a), torch.zeros_like(rows)
+    for i, cols, pos in _band_terms(case):
+        won = torch.where((at[:, cols, i : i + wb] == i) & cells[pos], g[:, cols, i : i + wb], 0)
+        ga[:, cols, i] = won.sum(2)
+        grows[:, pos] += won
+    # back from rows to columns: cell (c, k) of b lies in dense row c + k - b_lu
+    n = case["n"]
+    k = torch.arange(wb, device=a.device)
+    row = torch.arange(n, device=a.device).unsqueeze(1) + k - case["b_lu"]
+    ok = (row >= 0) & (row < n)
+    gb = torch.where(ok, grows[:, row.clamp(0, n - 1), (wb - 1 - k).expand_as(row)], 0)
+    return torch.where(best > -1e9, best, 0), ga, gb
+
+
 def work(case):
     """Operations: a multiply-add (a compare and an add) per term and result for every sum a pass
     needs - log products: one forward, two backward, eight in the second order; max products:
