@@ -375,7 +375,7 @@ template <class CX, int FBR, int FBC, bool GRAD_A>
 __global__ __launch_bounds__(CX::NT) void k_log_bwd_fixup(const LogBwdArgs p,
                                                           const int* __restrict__ hdr,
                                                           const int* __restrict__ fwd_flags,
-                                                          int need_factors, int total_tiles) {
+                                                          int need, int total_tiles) {
   static_assert(FBR % CX::BR == 0 && FBC % CX::BC == 0, "");
   __shared__ __attribute__((aligned(16))) float smem[LogBwdLds<CX, GRAD_A>::FLOATS];
   const int per = p.tiles_r * p.tiles_c;  // of the factored launch
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(CX::NT) void k_log_bwd_fixup(const LogBwdArgs p,
   for (int t = blockIdx.x; t < total_tiles; t += gridDim.x) {
     const int batch = t / per, r = t - batch * per;
     const int r0 = (r / p.tiles_c) * FBR, c0 = (r % p.tiles_c) * FBC;
-    if (!bwd_tile_flagged(hdr, fwd_flags, need_factors, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? FBR : FBC,
+    if (!bwd_tile_flagged(hdr, fwd_flags, need, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? FBR : FBC,
                           batch, p.M, p.N, threadIdx.x, CX::NT))
       continue;
     for (int h = 0; h < FBR / CX::BR; ++h)
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(CX::NT) void k_log_bwd_fixup_both(const LogBwdArgs 
                                                                const LogBwdArgs pb,
                                                                const int* __restrict__ hdr,
                                                                const int* __restrict__ fwd_flags,
-                                                               int tiles_a, int tiles_b, int need_factors) {
+                                                               int tiles_a, int tiles_b, int need) {
   constexpr int kFa = LogBwdLds<CX, true>::FLOATS, kFb = LogBwdLds<CX, false>::FLOATS;
   __shared__ __attribute__((aligned(16))) float smem[kFa > kFb ? kFa : kFb];
   for (int t = blockIdx.x; t < tiles_a + tiles_b; t += gridDim.x) {
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(CX::NT) void k_log_bwd_fixup_both(const LogBwdArgs 
     const int FR = is_a ? AR : BR, FC = is_a ? AC : BC;
     const int R = is_a ? p.M : p.K, Cc = is_a ? p.K : p.N;
     const int r0 = (r / p.tiles_c) * FR, c0 = (r % p.tiles_c) * FC;
-    if (!bwd_tile_flagged(hdr, fwd_flags, need_factors, is_a, is_a ? r0 : c0, is_a ? FR : FC, batch, p.M, p.N,
+    if (!bwd_tile_flagged(hdr, fwd_flags, need, is_a, is_a ? r0 : c0, is_a ? FR : FC, batch, p.M, p.N,
                           threadIdx.x, CX::NT))
       continue;
     for (int h = 0; h < FR / CX::BR; ++h)
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(C::NT, 2) void k_log_bwd_fast(const LogBwdArgs p,
   // Every cell this tile reduces over must come from a forward tile that passed the
   // factoring guard (S >= 2^-40, finite shifts): H = g * exp(alpha + beta - out) is then
   // at most |g| * 2^40.  Otherwise the fix-up launch recomputes this tile.
-  if (bwd_tile_flagged(hdr, fwd_flags, false, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? C::BR : C::BC, batch, M,
+  if (bwd_tile_flagged(hdr, fwd_flags, kKeepNone, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? C::BR : C::BC, batch, M,
                        N, tid, C::NT))
     return;
 
@@ -629,14 +629,15 @@ constexpr int kFixupGrid = 1024;
 
 inline bool valid_path(int path) {
   return path == GENBMM_PATH_AUTO || path == GENBMM_PATH_EXACT || path == GENBMM_PATH_VALU ||
-         path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_MFMA32;
+         path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_MFMA32 || path == GENBMM_PATH_RECIP;
 }
 inline bool auto_path(int path) {
-  return path == GENBMM_PATH_AUTO || path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_MFMA32;
+  return path == GENBMM_PATH_AUTO || path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_MFMA32 ||
+         path == GENBMM_PATH_RECIP;
 }
 // MFMA32: as AUTO, but the tiled matrix-core kernels always use the fp32 matrix instruction; under
 // AUTO, full-tile shapes run on the bf16 instruction with every factor in three parts (logbmm_split.h).
-inline bool split_path(int path) { return path == GENBMM_PATH_AUTO; }
+inline bool split_path(int path) { return path == GENBMM_PATH_AUTO || path == GENBMM_PATH_RECIP; }
 // dynamic LDS beyond 64 KB must be asked for
 template <class Kern>
 inline void allow_lds(Kern kern, int bytes) {
@@ -839,7 +840,7 @@ int launch_bwd_mfma(LogBwdArgs p, const float* stats, int B, hipStream_t s, bool
                        p.grad, p.M, p.K, p.N, p.tiles_r, p.tiles_c);
   };
   auto go_lean = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(total), dim3(T::NT), 0, s, p.g, LeanSrc{p.a, p.b, p.out, stats}, ws.hdr, ff, p.grad,
+    hipLaunchKernelGGL(kern, dim3(total), dim3(T::NT), 0, s, p.g, LeanSrc{p.a, p.b, p.out, stats, nullptr}, ws.hdr, ff, p.grad,
                        p.M, p.K, p.N, p.tiles_r, p.tiles_c);
   };
   const bool ragged = R % T::TR != 0 || Cc % T::TC != 0 || Q % kMS != 0;
@@ -852,7 +853,7 @@ int launch_bwd_mfma(LogBwdArgs p, const float* stats, int B, hipStream_t s, bool
   }
   if (int e = launch_status()) return e;
   hipLaunchKernelGGL((k_log_bwd_fixup<BCfgWide, T::TR, T::TC, GRAD_A>),
-                     dim3(min(total, kFixupGrid)), dim3(BCfgWide::NT), 0, s, p, ws.hdr, ff, lean ? 0 : 1, total);
+                     dim3(min(total, kFixupGrid)), dim3(BCfgWide::NT), 0, s, p, ws.hdr, ff, lean ? kKeepNone : kKeepFactors, total);
   return launch_status();
 }
 
@@ -874,7 +875,7 @@ int launch_bwd_mfma_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int B
   const bool ragged = M % TA::TR != 0 || K % TA::TC != 0 || N % kMS != 0 || K % TB::TR != 0 ||
                       N % TB::TC != 0 || M % kMS != 0;
   auto go_lean = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)(ta + tb)), dim3(TA::NT), 0, s, pa.g, LeanSrc{pa.a, pa.b, pa.out, stats},
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ta + tb)), dim3(TA::NT), 0, s, pa.g, LeanSrc{pa.a, pa.b, pa.out, stats, nullptr},
                        ws.hdr, ff, pa.grad, pb.grad, M, K, N, (int)ta, pa.tiles_r, pa.tiles_c, pb.tiles_r,
                        pb.tiles_c);
   };
@@ -888,7 +889,7 @@ int launch_bwd_mfma_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int B
   if (int e = launch_status()) return e;
   hipLaunchKernelGGL((k_log_bwd_fixup_both<BCfgWide, TA::TR, TA::TC, TB::TR, TB::TC>),
                      dim3((unsigned)std::min<int64_t>(ta + tb, kFixupGrid)), dim3(BCfgWide::NT), 0,
-                     s, pa, pb, ws.hdr, ff, (int)ta, (int)tb, lean ? 0 : 1);
+                     s, pa, pb, ws.hdr, ff, (int)ta, (int)tb, lean ? kKeepNone : kKeepFactors);
   return launch_status();
 }
 
@@ -900,8 +901,18 @@ inline bool pads_to_256(int x) { return ceil_div(x, 256) * 2 == ceil_div(x, 128)
 inline bool split_big_fits(int B, int out_r, int out_c) {
   return pads_to_256(out_r) && pads_to_256(out_c) && (int64_t)B * ceil_div(out_r, 256) * ceil_div(out_c, 256) >= 192;
 }
+// GENBMM_PATH_RECIP: 1 / S lies right behind the header (no EA, EB in front of it).
+inline float* recip_of(const float* stats, int B, int M, int N) {
+  return const_cast<float*>(stats) + header_offset(B, M, N) + 4;
+}
+// A batch item's matrices are addressed by 32-bit offsets in the three-part backward, which takes any M,
+// and K and N in whole pieces of four.
+inline bool bwd_split_sizes(int M, int K, int N) {
+  return N % 4 == 0 && K % 4 == 0 && (int64_t)M * N < (1ll << 31) && (int64_t)K * N < (1ll << 31) &&
+         (int64_t)M * K < (1ll << 31);
+}
 template <class T>
-int launch_fwd_split(DenseArgs p, float* stats, int B, int M, int K, int N, bool keep, hipStream_t s) {
+int launch_fwd_split(DenseArgs p, float* stats, int B, int M, int K, int N, int keep, hipStream_t s) {
   p.M = M; p.K = K; p.N = N;
   p.tiles_m = ceil_div(M, T::TR);
   p.tiles_n = ceil_div(N, T::TC);
@@ -916,22 +927,25 @@ int launch_fwd_split(DenseArgs p, float* stats, int B, int M, int K, int N, bool
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
   auto go = [&](auto kern) {
     allow_lds(kern, lds);
-    hipLaunchKernelGGL(kern, dim3(total), dim3(T::NT), lds, s, p.a, p.b, p.out, stats, flags, ws.ea, ws.eb, ws.r,
-                       ws.hdr, M, K, N, p.tiles_m, p.tiles_n, 1);
+    hipLaunchKernelGGL(kern, dim3(total), dim3(T::NT), lds, s, p.a, p.b, p.out, stats, flags, ws.ea, ws.eb,
+                       keep == kKeepRecip ? recip_of(stats, B, M, N) : ws.r, ws.hdr, M, K, N, p.tiles_m, p.tiles_n, 1);
   };
   const bool ragged = M % T::TR != 0 || N % T::TC != 0 || K % kMS != 0;
-  if (keep) {
-    if (ragged) go(k_log_fwd_split<T, true, true>);
-    else go(k_log_fwd_split<T, false, true>);
+  if (keep == kKeepFactors) {
+    if (ragged) go(k_log_fwd_split<T, true, kKeepFactors>);
+    else go(k_log_fwd_split<T, false, kKeepFactors>);
+  } else if (keep == kKeepRecip) {
+    if (ragged) go(k_log_fwd_split<T, true, kKeepRecip>);
+    else go(k_log_fwd_split<T, false, kKeepRecip>);
   } else {
-    if (ragged) go(k_log_fwd_split<T, true, false>);
-    else go(k_log_fwd_split<T, false, false>);
+    if (ragged) go(k_log_fwd_split<T, true, kKeepNone>);
+    else go(k_log_fwd_split<T, false, kKeepNone>);
   }
   if (int e = launch_status()) return e;
   return launch_fwd_fixup<CfgWide, T::TR, T::TC>(p, flags, total, s);
 }
 template <class TA, class TB>
-int launch_bwd_split_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int B, hipStream_t s) {
+int launch_bwd_split_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int B, bool recip, hipStream_t s) {
   const int M = pa.M, K = pa.K, N = pa.N;
   pa.tiles_r = ceil_div(M, TA::TR); pa.tiles_c = ceil_div(K, TA::TC);
   pb.tiles_r = ceil_div(K, TB::TR); pb.tiles_c = ceil_div(N, TB::TC);
@@ -942,17 +956,22 @@ int launch_bwd_split_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int 
   constexpr int lds = split_bwd_lds_bytes<TA, TB>();
   auto go = [&](auto kern) {
     allow_lds(kern, lds);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(ta + tb)), dim3(TA::NT), lds, s, pa.g, LeanSrc{pa.a, pa.b, pa.out, stats},
-                       hdr, ff, pa.grad, pb.grad, M, K, N, pa.tiles_r, pa.tiles_c, pb.tiles_r, pb.tiles_c);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ta + tb)), dim3(TA::NT), lds, s, pa.g,
+                       LeanSrc{pa.a, pa.b, pa.out, stats, recip_of(stats, B, M, N)}, hdr, ff, pa.grad, pb.grad, M, K, N, pa.tiles_r, pa.tiles_c, pb.tiles_r, pb.tiles_c);
   };
   const bool ragged = M % TA::TR != 0 || K % TA::TC != 0 || K % TB::TR != 0 || N % TB::TC != 0 || N % kMS != 0 ||
                       M % kMS != 0;
-  if (ragged) go(k_log_bwd_split_both<TA, TB, true>);
-  else go(k_log_bwd_split_both<TA, TB, false>);
+  if (recip) {
+    if (ragged) go(k_log_bwd_split_both<TA, TB, true, true>);
+    else go(k_log_bwd_split_both<TA, TB, false, true>);
+  } else {
+    if (ragged) go(k_log_bwd_split_both<TA, TB, true, false>);
+    else go(k_log_bwd_split_both<TA, TB, false, false>);
+  }
   if (int e = launch_status()) return e;
   hipLaunchKernelGGL((k_log_bwd_fixup_both<BCfgWide, TA::TR, TA::TC, TB::TR, TB::TC>),
                      dim3((unsigned)std::min<int64_t>(ta + tb, kFixupGrid)), dim3(BCfgWide::NT), 0, s, pa, pb, hdr, ff,
-                     (int)ta, (int)tb, 0);
+                     (int)ta, (int)tb, recip ? kKeepRecip : kKeepNone);
   return launch_status();
 }
 
@@ -968,6 +987,14 @@ inline int mfma_kind(int path, int B, int out_r, int out_c, int red, bool long_c
   const int L = long_cols ? out_c : out_r;
   if (ceil_div(L, 256) * 2 == ceil_div(L, 128) && t128 >= 512) return 2;
   return 1;
+}
+
+// Shapes whose forward under GENBMM_PATH_RECIP keeps 1 / S alone, because both gradients run on the
+// three-part kernels, which form EA and EB again; other matrix-core shapes keep EA, EB and 1 / S under
+// that path and their backward is GENBMM_PATH_FACTORS's.
+inline bool recip_shape(int B, int M, int K, int N) {
+  const int ka = mfma_kind(GENBMM_PATH_RECIP, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_RECIP, B, K, N, M, false);
+  return fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N) && ka == kb && ka != 0 && bwd_split_sizes(M, K, N);
 }
 
 using MT128 = MTile<128, 128>;
@@ -1052,7 +1079,7 @@ int launch_fwd_pieces(DenseArgs p, float* stats, int B, int M, int K, int N, int
   constexpr int lds = 4 * split_lds_words<SplitT<T::TR, T::NT>, SplitS<T::TC, T::NT>>();
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
   float* parts = ws.ea;
-  auto kern = k_log_fwd_split<T, true, false, true>;
+  auto kern = k_log_fwd_split<T, true, kKeepNone, true>;
   allow_lds(kern, lds);
   hipLaunchKernelGGL(kern, dim3(total * pieces), dim3(T::NT), lds, s, p.a, p.b, p.out, stats, flags, nullptr, nullptr,
                      parts, ws.hdr, M, K, N, p.tiles_m, p.tiles_n, pieces);
@@ -1064,12 +1091,13 @@ int launch_fwd_pieces(DenseArgs p, float* stats, int B, int M, int K, int N, int
 }
 // pieces_ok: the workspace has room for the sums of a forward in pieces (fwd_pieces)
 int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, int M, int K, int N,
-            int path, bool keep, hipStream_t s, bool factors = false, bool pieces_ok = true) {
+            int path, bool keep_factors, hipStream_t s, bool factors = false, bool pieces_ok = true) {
   if (int e = check_dense_dims(B, M, K, N)) return e;
   if (!valid_path(path)) return GENBMM_E_MODE;
   const int64_t mk = (int64_t)B * M * K, kn = (int64_t)B * K * N, mn = (int64_t)B * M * N;
   if (missing(a, mk) || missing(b, kn) || missing(out, mn)) return GENBMM_E_NULLPTR;
-  if (path != GENBMM_PATH_FACTORS && !factors) keep = false;
+  int keep = keep_factors && (path == GENBMM_PATH_FACTORS || factors) ? kKeepFactors : kKeepNone;
+  if (path == GENBMM_PATH_RECIP) keep = recip_shape(B, M, K, N) ? kKeepRecip : kKeepFactors;
   if (stats && B > 0 && item_shape(M, K, N) && auto_path(path)) {  // whole items per workgroup
     int* hdr = prepared_of(stats, B, M, K, N).hdr;
     if (M == 32 && K == 32 && N == 32)  // one wave per item on the matrix cores
@@ -1087,7 +1115,7 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
     if (int e = launch_stats(a, b, stats, B, M, K, N, s)) return e;
   }
   if (mn == 0) return GENBMM_OK;
-  if (stats && split_path(path) && !keep && pieces_ok) {
+  if (stats && path == GENBMM_PATH_AUTO && keep == kKeepNone && pieces_ok) {
     const int pieces = fwd_pieces(B, M, K, N);
     if (pieces > 1) return launch_fwd_pieces(p, stats, B, M, K, N, pieces, s);
   }
@@ -1099,10 +1127,10 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
           if (split_big_fits(B, M, N)) return launch_fwd_split<MTBig>(p, stats, B, M, K, N, keep, s);
           return launch_fwd_split<MTTall>(p, stats, B, M, K, N, keep, s);
         }
-        return launch_fwd_mfma<MTTall>(p, stats, B, M, K, N, keep, s);
+        return launch_fwd_mfma<MTTall>(p, stats, B, M, K, N, keep == kKeepFactors, s);
       case 1:
         if (split_path(path)) return launch_fwd_split<MT128S>(p, stats, B, M, K, N, keep, s);
-        return launch_fwd_mfma<MT128>(p, stats, B, M, K, N, keep, s);
+        return launch_fwd_mfma<MT128>(p, stats, B, M, K, N, keep == kKeepFactors, s);
       default: break;
     }
     if (M <= 32 && N <= 32) return launch_fwd_fast<CfgSmall, CfgSmall>(p, stats, B, M, K, N, s);
@@ -1160,6 +1188,7 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
     }
     return launch_status();
   }
+  if (path == GENBMM_PATH_RECIP && !recip_shape(B, M, K, N)) path = GENBMM_PATH_FACTORS;  // what its forward kept
   if (st && grad_a && grad_b && mk > 0 && kn > 0 && fwd_mfma_shape(B, M, K, N)) {
     const int ka = mfma_kind(path, B, M, K, N, true), kb = mfma_kind(path, B, K, N, M, false);
     if (ka == kb && ka != 0) {
@@ -1167,14 +1196,12 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
       pa.grad = grad_a;
       pb.grad = grad_b;
       const bool lean = path != GENBMM_PATH_FACTORS;
-      // (the three-part backward takes any M, and K and N in whole pieces of four - the forward any
-      //  sizes -; it addresses a batch item's matrices by 32-bit offsets)
-      const bool small_items = (int64_t)M * N < (1ll << 31) && (int64_t)K * N < (1ll << 31) && (int64_t)M * K < (1ll << 31);
-      if (lean && split_path(path) && N % 4 == 0 && K % 4 == 0 && small_items) {
-        if (ka == 1) return launch_bwd_split_both<MT128S, MT128S>(pa, pb, st, B, s);
+      if (lean && split_path(path) && bwd_split_sizes(M, K, N)) {
+        const bool recip = path == GENBMM_PATH_RECIP;
+        if (ka == 1) return launch_bwd_split_both<MT128S, MT128S>(pa, pb, st, B, recip, s);
         if (split_big_fits(B, M, K) && split_big_fits(B, K, N))
-          return launch_bwd_split_both<MTBig, MTBig>(pa, pb, st, B, s);
-        return launch_bwd_split_both<MTWide, MTTall>(pa, pb, st, B, s);
+          return launch_bwd_split_both<MTBig, MTBig>(pa, pb, st, B, recip, s);
+        return launch_bwd_split_both<MTWide, MTTall>(pa, pb, st, B, recip, s);
       }
       return ka == 2 ? launch_bwd_mfma_both<MTWide, MTTall>(pa, pb, st, B, s, lean)
                      : launch_bwd_mfma_both<MT128, MT128>(pa, pb, st, B, s, lean);
@@ -1386,7 +1413,8 @@ size_t genbmm_logbmm_stats_size_path(int B, int M, int K, int N, int path) {
   if (check_dense_dims(B, M, K, N)) return 0;
   int64_t n = header_offset(B, M, N) + 4;  // maxima, flags and the header
   // the by-products of the matrix-core forward (the one-tile kernels keep the maxima only)
-  if (path == GENBMM_PATH_FACTORS && fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N))
+  if (path == GENBMM_PATH_RECIP && recip_shape(B, M, K, N)) n += (int64_t)B * M * N;
+  else if ((path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_RECIP) && fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N))
     n += (int64_t)B * ((int64_t)M * K + (int64_t)K * N + (int64_t)M * N);
   // the sums of a forward that cuts a long reduction into pieces
   if (path == GENBMM_PATH_AUTO) {

@@ -171,8 +171,8 @@ struct LogPrepared {
 };
 
 // Must a backward tile be left to the exact routine?  Yes if the workspace does not
-// hold what the tile's kernel reads (need_factors: EA, EB, 1/S of the matrix-core
-// forward; otherwise the flags of any factored forward), or if the forward flagged a
+// hold what the tile's kernel reads (`need` - kKeepFactors: EA, EB, 1/S of the
+// matrix-core forward; kKeepRecip: 1/S; kKeepNone: the flags of any factored forward), or if the forward flagged a
 // tile among the cells this tile reduces over - rows [lo, lo + extent) of out and
 // every column (by_rows: a grad_a tile), or columns [lo, lo + extent) and every row (a
 // grad_b tile).  A pure function of what the forward left, so the backward kernel and
@@ -180,11 +180,14 @@ struct LogPrepared {
 // Every thread of the workgroup must call it (one barrier inside).
 __device__ __forceinline__ int bwd_tile_flagged(const int* __restrict__ hdr,
                                                 const int* __restrict__ fwd_flags,
-                                                bool need_factors, bool by_rows, int lo, int extent,
+                                                int need, bool by_rows, int lo, int extent,
                                                 int batch, int M, int N, int tid, int nt) {
   const int tag = hdr[0], ftr = hdr[1], ftc = hdr[2];
   // flag words exist per 32 x 32 cells at the densest
-  int bad = !(need_factors ? tag == kWsMfma : (tag == kWsMfma || tag == kWsFast)) || ftr < 32 || ftc < 32;
+  int bad = !(need == kKeepFactors  ? tag == kWsMfma
+              : need == kKeepRecip ? tag == kWsRecip
+                                   : (tag == kWsMfma || tag == kWsFast || tag == kWsRecip)) ||
+            ftr < 32 || ftc < 32;
   if (!bad) {
     const int fm = (M + ftr - 1) / ftr, fn = (N + ftc - 1) / ftc;
     const int mlo = by_rows ? lo / ftr : 0, mhi = by_rows ? min((lo + extent - 1) / ftr, fm - 1) : fm - 1;
@@ -563,7 +566,7 @@ __device__ __forceinline__ void log_bwd_mfma_tile(
   // Forward flags over the cells this tile reduces over: the fix-up launch takes a flagged tile.
   // Asked while the first slab's loads are in flight (the workspace is allocated whatever it
   // holds, so the loads are harmless for a tile that then leaves).
-  if (bwd_tile_flagged(ws_hdr, fwd_flags, true, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? T::TR : T::TC, batch,
+  if (bwd_tile_flagged(ws_hdr, fwd_flags, kKeepFactors, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? T::TR : T::TC, batch,
                        M, N, tid, NT))
     return;
   stage(0);
@@ -664,6 +667,7 @@ struct LeanSrc {
   const elem_t* b;
   const elem_t* out;
   const float* stats;  // alpha (M) then beta (N) per batch item
+  const float* r;      // 1 / S of the forward (the three-part backward with RECIP), else unused
 };
 __device__ __forceinline__ float4 mul_exp4(float4 g, float4 sh, float4 o) {  // g * exp(sh - o)
   return make_float4(g.x * exp_st(sh.x - o.x), g.y * exp_st(sh.y - o.y), g.z * exp_st(sh.z - o.z),
@@ -804,7 +808,7 @@ __device__ __forceinline__ void log_bwd_mfma_tile_lean(
   };
 
   load(slabs == 1 && qtail != 0);
-  if (bwd_tile_flagged(ws_hdr, fwd_flags, false, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? T::TR : T::TC, batch,
+  if (bwd_tile_flagged(ws_hdr, fwd_flags, kKeepNone, GRAD_A, GRAD_A ? r0 : c0, GRAD_A ? T::TR : T::TC, batch,
                        M, N, tid, NT))
     return;
   stage(0);

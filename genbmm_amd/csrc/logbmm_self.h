@@ -347,7 +347,7 @@ __device__ __forceinline__ void log_self_bwd_tile(float* __restrict__ smem, floa
 
   // the shifts the forward left (any forward that writes them will do)
   const int tag = hdr[0];
-  int bad = !(tag == kWsSelf || tag == kWsMfma || tag == kWsFast);
+  int bad = !(tag == kWsSelf || tag == kWsMfma || tag == kWsFast || tag == kWsRecip);
   float my_shift;
   {
     const bool row = tid < kSelfMax;

@@ -104,13 +104,13 @@ struct SplitS {
 };
 
 // LW consecutive elements as floats
-template <int LW>
-__device__ __forceinline__ void ldw(const elem_t* p, float (&v)[LW]) {
+template <int LW, class E>
+__device__ __forceinline__ void ldw(const E* p, float (&v)[LW]) {
   if constexpr (LW == 4) {
     const float4 t = ld4(p);
     v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
   } else {
-    typedef elem_t e2u __attribute__((ext_vector_type(2), aligned(sizeof(elem_t))));
+    typedef E e2u __attribute__((ext_vector_type(2), aligned(sizeof(E))));
     const e2u t = *reinterpret_cast<const e2u*>(p);
     v[0] = (float)t.x; v[1] = (float)t.y;
   }
@@ -231,13 +231,14 @@ __device__ __forceinline__ bool split_early(int wave) { return wave >= NT / 128;
 // ([piece][batch][M][N]) and k_log_fwd_join adds them, tests the guard and takes the logarithm.
 // For problems with few output tiles and a long reduction, which would otherwise run on a few
 // compute units.
-template <class T, bool RAGGED, bool KEEP, bool PIECES = false>
+template <class T, bool RAGGED, int KEEPS, bool PIECES = false>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WPE, T::WPE)))
 void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b, elem_t* __restrict__ out,
                      const float* __restrict__ stats, int* __restrict__ flags, float* __restrict__ ws_ea,
                      float* __restrict__ ws_eb, float* __restrict__ ws_r, int* __restrict__ ws_hdr, int M, int K,
                      int N, int tiles_m, int tiles_n, int pieces = 1) {
-  static_assert(!PIECES || (RAGGED && !KEEP), "");
+  static_assert(!PIECES || (RAGGED && KEEPS == kKeepNone), "");
+  constexpr bool KEEP = KEEPS == kKeepFactors;
   constexpr int NT = T::NT;
   using SA = SplitT<T::TR, NT>;
   using SB = SplitS<T::TC, NT>;
@@ -286,7 +287,7 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
   if (!PIECES && tile == 0 && tid == 0) {
     ws_hdr[1] = T::TR;
     ws_hdr[2] = T::TC;
-    ws_hdr[0] = KEEP ? kWsMfma : kWsFast;
+    ws_hdr[0] = KEEP ? kWsMfma : KEEPS == kKeepRecip ? kWsRecip : kWsFast;
   }
 
   floatx16 acc[2][2];
@@ -433,7 +434,7 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
                                            __builtin_fmaf(fast_log2(sv.w), kLn2, alr + be4.w));
              if (RAGGED) st4m(out + ubase + (long)ru * N + voff, cc, ov);
              else st4(out + ubase + (long)ru * N + voff, ov);
-             if constexpr (KEEP) {
+             if constexpr (KEEPS != kKeepNone) {
                const float4 rv = make_float4(__builtin_amdgcn_rcpf(sv.x), __builtin_amdgcn_rcpf(sv.y),
                                              __builtin_amdgcn_rcpf(sv.z), __builtin_amdgcn_rcpf(sv.w));
                if (RAGGED) st4m(ws_r + ubase + (long)ru * N + voff, cc, rv);
@@ -691,7 +692,11 @@ struct SplitBwd {
   static constexpr int WORDS = split_lds_words<SR, SC>();
 };
 
-template <class T, bool GRAD_A, bool RAGGED>
+//
+// RECIP: H = g R with the forward's R = 1 / S (fp32, in the workspace) in the place of out and an
+// exponential - for float16 / bfloat16 tensors, whose `out` is stored rounded.  The header is read before
+// anything else: a workspace of another forward need not hold R.
+template <class T, bool GRAD_A, bool RAGGED, bool RECIP>
 __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, int tile, const elem_t* __restrict__ g,
                                                    const LeanSrc src, const int* __restrict__ ws_hdr,
                                                    const int* __restrict__ fwd_flags, elem_t* __restrict__ grad, int M,
@@ -713,6 +718,11 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
   const int R = GRAD_A ? M : K, Cc = GRAD_A ? K : N;
   const float* al = src.stats + (long)batch * (M + N);
   const float* be = al + M;
+  using W_t = std::conditional_t<RECIP, float, elem_t>;
+  const W_t* wsrc;  // what H is formed from beside g: R, or out
+  if constexpr (RECIP) wsrc = src.r;
+  else wsrc = src.out;
+  constexpr int kNeed = RECIP ? kKeepRecip : kKeepNone;
   floatx16 acc[2][2];
 #pragma unroll
   for (int x = 0; x < 4; ++x)
@@ -732,7 +742,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
     // rows: H pieces (line m, four n); columns: EB pieces (line k, four n); beta of the slab's four
     // columns is the same for every piece of a thread (all share their quad).  Lines beyond the
     // matrix re-read the last line: they only feed results that are not stored.
-    const elem_t* ob = src.out + (long)batch * M * N;
+    const W_t* ob = wsrc + (long)batch * M * N;
     const elem_t* gb = g + (long)batch * M * N;
     const elem_t* bb = src.b + (long)batch * K * N;
     const float* beb = be;
@@ -767,12 +777,17 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
       for (int l = 0; l < SC::PER; ++l) SC::put(Cs(buf), tid, l, exp4(ry[l], bslab));
 #pragma unroll
       for (int l = 0; l < SR::PER; ++l) {
-        const float4 sh = make_float4(alh[l] + bslab.x, alh[l] + bslab.y, alh[l] + bslab.z, alh[l] + bslab.w);
-        SR::put(Rs(buf), tid, l, mul_exp4(rg[l], sh, ro[l]));
+        if constexpr (RECIP) {
+          SR::put(Rs(buf), tid, l, make_float4(rg[l].x * ro[l].x, rg[l].y * ro[l].y, rg[l].z * ro[l].z, rg[l].w * ro[l].w));
+        } else {
+          const float4 sh = make_float4(alh[l] + bslab.x, alh[l] + bslab.y, alh[l] + bslab.z, alh[l] + bslab.w);
+          SR::put(Rs(buf), tid, l, mul_exp4(rg[l], sh, ro[l]));
+        }
       }
     };
+    if (RECIP && ws_hdr[0] != kWsRecip) return;  // uniform
     load();
-    if (bwd_tile_flagged(ws_hdr, fwd_flags, false, true, r0, T::TR, batch, M, N, tid, NT)) return;
+    if (bwd_tile_flagged(ws_hdr, fwd_flags, kNeed, true, r0, T::TR, batch, M, N, tid, NT)) return;
     stage(0);
     split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
       split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
@@ -783,7 +798,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
       for (int l = 0; l < SC::PER; ++l) ry[l] = ld4m(bb + yo[l], left, -INFINITY);
 #pragma unroll
       for (int l = 0; l < SR::PER; ++l) {
-        ro[l] = ld4m(ob + oo[l], left, INFINITY);
+        ro[l] = ld4m(ob + oo[l], left, RECIP ? 0.f : INFINITY);
         rg[l] = ld4m(gb + oo[l], left, 0.f);
       }
       bslab = ld4m(beb + beo, left, 0.f);
@@ -800,7 +815,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
     static_assert(SR::Q == SC::Q, "");
     const int m2 = 2 * SR::pair(tid);
     const elem_t* ab = src.a + (long)batch * M * K;
-    const elem_t* ob = src.out + (long)batch * M * N;
+    const W_t* ob = wsrc + (long)batch * M * N;
     const elem_t* gb = g + (long)batch * M * N;
     const float* alb = al;
     const int kc = RAGGED ? min(r0 + SR::line0(tid), K - LR) : r0 + SR::line0(tid);
@@ -834,14 +849,15 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
       }
 #pragma unroll
       for (int j = 0; j < LC; ++j) {
-        h0[j] = ge[j] * exp_st(a0 + bec[j] - oe[j]);
-        h1[j] = gd[j] * exp_st(a1 + bec[j] - od[j]);
+        h0[j] = ge[j] * (RECIP ? oe[j] : exp_st(a0 + bec[j] - oe[j]));
+        h1[j] = gd[j] * (RECIP ? od[j] : exp_st(a1 + bec[j] - od[j]));
       }
       SR::put(Rs(buf), tid, e0, e1);
       SC::put(Cs(buf), tid, h0, h1);
     };
+    if (RECIP && ws_hdr[0] != kWsRecip) return;  // uniform
     load();
-    if (bwd_tile_flagged(ws_hdr, fwd_flags, false, false, c0, T::TC, batch, M, N, tid, NT)) return;
+    if (bwd_tile_flagged(ws_hdr, fwd_flags, kNeed, false, c0, T::TC, batch, M, N, tid, NT)) return;
     stage(0);
     split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
       split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
@@ -913,7 +929,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
 }
 
 // Both gradients in one launch, item by item, a tile of each in turn (see k_log_bwd_mfma_both).
-template <class TA, class TB, bool RAGGED>
+template <class TA, class TB, bool RAGGED, bool RECIP>
 __global__ __launch_bounds__(TA::NT) __attribute__((amdgpu_waves_per_eu(TA::WPE, TA::WPE)))
 void k_log_bwd_split_both(const elem_t* __restrict__ g, const LeanSrc src, const int* __restrict__ ws_hdr,
                           const int* __restrict__ fwd_flags, elem_t* __restrict__ grad_a,
@@ -927,9 +943,9 @@ void k_log_bwd_split_both(const elem_t* __restrict__ g, const LeanSrc src, const
   const bool is_a = alt ? (r & 1) == 0 : r < per_a;
   const int idx = alt ? r >> 1 : (r < per_a ? r : r - per_a);
   if (is_a)
-    log_bwd_split_tile<TA, true, RAGGED>(split_smem, item * per_a + idx, g, src, ws_hdr, fwd_flags, grad_a, M, K, N, ar, ac);
+    log_bwd_split_tile<TA, true, RAGGED, RECIP>(split_smem, item * per_a + idx, g, src, ws_hdr, fwd_flags, grad_a, M, K, N, ar, ac);
   else
-    log_bwd_split_tile<TB, false, RAGGED>(split_smem, item * per_b + idx, g, src, ws_hdr, fwd_flags, grad_b, M, K, N, br, bc);
+    log_bwd_split_tile<TB, false, RAGGED, RECIP>(split_smem, item * per_b + idx, g, src, ws_hdr, fwd_flags, grad_b, M, K, N, br, bc);
 }
 
 template <class TA, class TB>

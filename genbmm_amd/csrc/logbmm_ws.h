@@ -11,6 +11,10 @@ constexpr int kWsNone = 0;  // one that leaves no per-tile flags (exact and whol
 constexpr int kWsMfma = 1;  // the matrix-core forward: flags, EA, EB and 1/S
 constexpr int kWsFast = 2;  // the factored vector-ALU forward: flags only
 constexpr int kWsSelf = 3;  // the one-tile-per-item forward: the maxima only
+constexpr int kWsRecip = 4; // the three-part matrix-core forward: flags and 1/S, right behind the header
+
+// What a tiled forward keeps for its backward beside maxima and flags, and what a backward needs.
+constexpr int kKeepNone = 0, kKeepFactors = 1, kKeepRecip = 2;
 
 struct LogFactors {
   const float* ea;   // exp(a - row maximum), (B, M, K)

@@ -53,7 +53,7 @@ def _sfx(t):
     return _lib.HALF_SUFFIX.get(t.dtype, "")
 
 
-PATH_AUTO, PATH_EXACT, PATH_VALU, PATH_FACTORS, PATH_MFMA32 = 0, 1, 2, 3, 4  # GENBMM_PATH_* of the C header
+PATH_AUTO, PATH_EXACT, PATH_VALU, PATH_FACTORS, PATH_MFMA32, PATH_RECIP = 0, 1, 2, 3, 4, 5  # GENBMM_PATH_* of the C header
 
 
 def _prep(a, b):
@@ -384,16 +384,17 @@ def logbmm(a, b):
         b_s = (b.float() if b.dtype in _lib.HALF_SUFFIX else b).view(B * S, K // S, N)
         parts = LogMatMul.apply(a_s, b_s, PATH_AUTO).view(B, S, M, N)
         return restore(torch.logsumexp(parts, dim=1).to(a.dtype))
-    # float16 / bfloat16 tensors keep 1 / sum in float32 for the backward (PATH_FACTORS): with the
+    # float16 / bfloat16 tensors keep 1 / sum in float32 for the backward (PATH_RECIP): with the
     # maxima alone it would be rebuilt from `out` as stored, i.e. rounded to 11 or 8 bits
-    return restore(LogMatMul.apply(a, b, PATH_FACTORS if a.dtype in _lib.HALF_SUFFIX else PATH_AUTO))
+    return restore(LogMatMul.apply(a, b, PATH_RECIP if a.dtype in _lib.HALF_SUFFIX else PATH_AUTO))
 
 
 def logbmm_on_path(a, b, path):
     """logbmm with the library's kernel family named (PATH_AUTO / PATH_EXACT / PATH_VALU / PATH_FACTORS:
     as PATH_AUTO, but autograd saves exp(a - max), exp(b - max) and 1 / sum beside the maxima - three
     more tensors than the reference saves - and the matrix-core backward takes no exponential /
-    PATH_MFMA32: as PATH_AUTO with the fp32 matrix instruction for every tiled shape);
+    PATH_MFMA32: as PATH_AUTO with the fp32 matrix instruction for every tiled shape / PATH_RECIP: as
+    PATH_AUTO with 1 / sum kept for the backward, what half tensors use by default);
     forward and backward both use it.  For tests and measurements."""
     a, b, restore = _canonical(a, b)
     return restore(LogMatMul.apply(a, b, path))

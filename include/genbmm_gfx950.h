@@ -154,6 +154,13 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *                      at 2.7 times less matrix-pipe time (the forward for any
  *                      sizes; the backward where K and N are multiples of 4,
  *                      else it stays on the fp32 instruction).
+ *   GENBMM_PATH_RECIP  as AUTO, with 1 / sum kept in fp32 for the backward, which
+ *                      then weighs g by it instead of by exp(max - out): what
+ *                      float16 / bfloat16 tensors want, whose `out` is stored
+ *                      rounded (4 bytes per result cell; shapes whose backward
+ *                      does not run on the bf16 instruction keep all three
+ *                      factors and take FACTORS's).  One gradient alone (the
+ *                      other pointer NULL) is formed from `out`.
  * Any other value: GENBMM_E_MODE.  Forward and backward of one problem need not
  * name the same path (see genbmm_logbmm_bwd).  No counterpart in the reference.
  */
@@ -162,6 +169,7 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
 #define GENBMM_PATH_VALU 2
 #define GENBMM_PATH_FACTORS 3
 #define GENBMM_PATH_MFMA32 4
+#define GENBMM_PATH_RECIP 5
 /* Number of fp32 elements of `stats` for a forward / backward pair on `path`
  * (genbmm_logbmm_stats_size is this for GENBMM_PATH_AUTO). */
 size_t genbmm_logbmm_stats_size_path(int B, int M, int K, int N, int path);

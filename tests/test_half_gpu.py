@@ -316,3 +316,61 @@ def test_logbmm_second_order_half_equals_float_kernels_rounded(gpu, dt, suffix, 
     # the workspace is required for the half types
     assert getattr(lib, "genbmm_logbmm_bwdbwd_ws" + suffix)(P(a), P(b), P(out), P(g), P(ua), P(ub), P(ga), P(gb), P(gg),
                                                            P(None), B, M, K, N, s) == -1
+
+
+# tiled matrix-core shapes whose backward runs on the three-part kernels (any M; K, N multiples of four):
+# full 256-, 128-wide and mixed tiles, ragged edges and a partial last slab; then shapes that keep all
+# factors instead (odd K or N, a gradient too narrow for a tile), one tile per item, a small item
+RECIP_SHAPES = [(48, 512, 512, 512), (32, 256, 512, 256), (128, 256, 128, 512), (2, 130, 140, 132), (2, 257, 100, 260),
+                (3, 300, 516, 200), (2, 200, 177, 131), (2, 160, 48, 160), (3, 128, 128, 128), (2, 64, 64, 64)]
+
+
+@pytest.mark.parametrize("dt,suffix,eps", TYPES)
+@pytest.mark.parametrize("B,M,K,N", RECIP_SHAPES)
+def test_logbmm_half_on_kept_reciprocals(gpu, dt, suffix, eps, B, M, K, N):
+    """PATH_RECIP, the default of half tensors: bit for bit the float kernels on the widened tensors,
+    rounded once; on tiled shapes the gradients carry the rounding of their own store and fp32 sums of
+    products only (|error| <= eps |w| + 2^-18 of the largest: up to 512 terms of relative error 2^-22,
+    weights below one), not that of `out` (eps |out|).  A workspace that another forward filled
+    is recognised: every tile then takes the exact routine."""
+    lib = _lib.load()
+    path, other = genbmm.genmul.PATH_RECIP, genbmm.genmul.PATH_VALU
+    torch.manual_seed(5)
+    a, b, g = _operands(gpu, dt, B, M, K, N, 1.0)
+    a32, b32, g32 = a.float(), b.float(), g.float()
+    n = lib.genbmm_logbmm_stats_size_path(B, M, K, N, path)
+    st, st32 = torch.full((n,), float("nan"), device=gpu), torch.empty(n, device=gpu)
+    out, out32 = torch.empty(B, M, N, device=gpu, dtype=dt), torch.empty(B, M, N, device=gpu)
+    s = _lib.stream_of(a)
+    fwd, bwd = (getattr(lib, "genbmm_logbmm_%s_path%s" % (x, suffix)) for x in ("fwd", "bwd"))
+
+    def backward(fn, x, y, o, gr, ws, p):
+        ga, gb = torch.empty_like(x), torch.empty_like(y)
+        assert fn(P(x), P(y), P(o), P(gr), P(ws), P(ga), P(gb), B, M, K, N, p, s) == 0
+        return ga, gb
+
+    assert fwd(P(a), P(b), P(out), P(st), B, M, K, N, path, s) == 0
+    assert lib.genbmm_logbmm_fwd_path(P(a32), P(b32), P(out32), P(st32), B, M, K, N, path, s) == 0
+    assert torch.equal(out, out32.to(dt))
+    oh = out.float()
+    ga, gb = backward(bwd, a, b, out, g, st, path)
+    ga32, gb32 = backward(lib.genbmm_logbmm_bwd_path, a32, b32, oh, g32, st32, path)
+    assert torch.equal(ga, ga32.to(dt)) and torch.equal(gb, gb32.to(dt))
+    if min(M, K, N) >= 96 and max(M, K, N) > 128:     # both gradients tiled (a narrower one reads `out`)
+        x, y = (t[:2].double().cpu().requires_grad_() for t in (a32, b32))
+        wa, wb = torch.autograd.grad(oracle.logbmm_broadcast(x, y), (x, y), g32[:2].double().cpu())
+        for got, want in ((ga, wa), (gb, wb)):
+            err = (got[:2].double().cpu() - want).abs()
+            assert bool((err <= eps * want.abs() + 2.0 ** -18 * max(1.0, float(want.abs().max()))).all())
+    # a workspace of this size that the vector-ALU forward filled
+    st.fill_(float("nan"))
+    assert fwd(P(a), P(b), P(out), P(st), B, M, K, N, other, s) == 0
+    xa, xb = backward(bwd, a, b, out, g, st, path)
+    ea, eb = backward(bwd, a, b, out, g, st, genbmm.genmul.PATH_EXACT)
+    for got, want in ((xa, ea), (xb, eb)):
+        assert float((got.double() - want.double()).norm() / want.double().norm()) <= 4 * eps
+    # one gradient alone is formed from `out`: its weights carry the rounding of `out`
+    only = torch.empty_like(a)
+    assert fwd(P(a), P(b), P(out), P(st), B, M, K, N, path, s) == 0
+    assert bwd(P(a), P(b), P(out), P(g), P(st), P(only), P(None), B, M, K, N, path, s) == 0
+    assert float((only.double() - ea.double()).norm() / ea.double().norm()) <= 4 * eps
