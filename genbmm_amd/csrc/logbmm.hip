@@ -905,11 +905,9 @@ inline bool split_big_fits(int B, int out_r, int out_c) {
 inline float* recip_of(const float* stats, int B, int M, int N) {
   return const_cast<float*>(stats) + header_offset(B, M, N) + 4;
 }
-// A batch item's matrices are addressed by 32-bit offsets in the three-part backward, which takes any M,
-// and K and N in whole pieces of four.
+// A batch item's matrices are addressed by 32-bit offsets in the three-part backward.
 inline bool bwd_split_sizes(int M, int K, int N) {
-  return N % 4 == 0 && K % 4 == 0 && (int64_t)M * N < (1ll << 31) && (int64_t)K * N < (1ll << 31) &&
-         (int64_t)M * K < (1ll << 31);
+  return (int64_t)M * N < (1ll << 31) && (int64_t)K * N < (1ll << 31) && (int64_t)M * K < (1ll << 31);
 }
 template <class T>
 int launch_fwd_split(DenseArgs p, float* stats, int B, int M, int K, int N, int keep, hipStream_t s) {

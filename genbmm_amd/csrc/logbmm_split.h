@@ -15,10 +15,11 @@
 // the staged form and the inner loop.  Ragged edges are a second instantiation of each
 // kernel (RAGGED), handled as in logbmm_mfma.h: lines of a tile beyond the matrix re-read
 // the last line (under a shift that makes the factor vanish where the line feeds stored
-// results), stores are masked.  The forward takes any sizes: pieces that straddle the right
-// edge are read element by element, the reduction tail is filled by the loader of the last
-// slab.  The backward takes any M but K and N in multiples of four (no piece straddles an
-// edge), and its partial last slab is a step of its own behind the loop.
+// results), stores are masked.  Any sizes: pieces that straddle the right edge are read element
+// by element and the reduction tail is filled by the loader of the last slab in the forward; the
+// backward reads a straddling piece from the last lines and moves its values down when they are
+// staged, and its partial last slab is a step of its own behind the loop.  (Backward of
+// (64, 511, 509, 510): 368 us on the fp32 instruction, 256 here.)
 //
 // LDS layouts, three planes (h, m, l) per operand, words of two bf16:
 //  * an operand whose source is [line][reduction] (reduction contiguous): plane[line][8
@@ -125,6 +126,18 @@ __device__ __forceinline__ void ldwm(const elem_t* p, int cnt, float fill, float
   }
 #pragma unroll
   for (int j = 0; j < LW; ++j) v[j] = j < cnt ? (float)p[j] : fill;
+}
+// v[j] <- v[j + by] for 0 < by < LW (the places behind keep what they hold); other `by`: nothing
+template <int LW>
+__device__ __forceinline__ void shift_down(float (&v)[LW], int by) {
+  if constexpr (LW == 4) {
+    if (by == 1) { v[0] = v[1]; v[1] = v[2]; v[2] = v[3]; }
+    if (by == 2) { v[0] = v[2]; v[1] = v[3]; }
+    if (by == 3) v[0] = v[3];
+  } else {
+    static_assert(LW == 2, "");
+    if (by == 1) v[0] = v[1];
+  }
 }
 __device__ __forceinline__ int clampw(int x, int w) { return min(max(x, 0), w); }
 
@@ -735,9 +748,8 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
 
   // Addresses are a base per workgroup (scalar registers, stepped slab by slab) plus a fixed
   // 32-bit offset per thread: the vector registers go to operands and accumulators.
-  // RAGGED: any M; K and N multiples of four, so that no piece straddles the right edge of its
-  // matrix (other shapes run their backward on the fp32 instruction).  Fills of the partial last
-  // slab make a factor vanish: -inf for a and b, +inf for out, 0 for g.
+  // RAGGED: any sizes (every extent at least a piece).  Fills of the partial last slab make a factor
+  // vanish: -inf for a and b, +inf for out, 0 for g.
   if constexpr (GRAD_A) {
     // rows: H pieces (line m, four n); columns: EB pieces (line k, four n); beta of the slab's four
     // columns is the same for every piece of a thread (all share their quad).  Lines beyond the
@@ -810,7 +822,10 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
   } else {
     // rows: EA pieces (steps m, m + 1; LW lines k); columns: H pieces (steps m, m + 1; LW lines n);
     // both operands' pieces of a thread are on the same pair of steps.  RAGGED: lines beyond the
-    // matrix re-read the last LW lines - they only feed results that are not stored.
+    // matrix re-read the last LW lines - they only feed results that are not stored -, and a piece that
+    // straddles the right edge reads the last LW lines too: the staged values then move down to the
+    // lines they belong to (a few lanes of the last tile; the branch costs the others nothing, where a
+    // loader that reads such a piece element by element would hold back every load behind it).
     constexpr int LR = SR::LW, LC = SC::LW;
     static_assert(SR::Q == SC::Q, "");
     const int m2 = 2 * SR::pair(tid);
@@ -821,6 +836,8 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
     const int kc = RAGGED ? min(r0 + SR::line0(tid), K - LR) : r0 + SR::line0(tid);
     const int nc = RAGGED ? min(c0 + SC::line0(tid), N - LC) : c0 + SC::line0(tid);
     const int yo = m2 * K + kc, oo = m2 * N + nc;
+    const int sr = RAGGED ? r0 + SR::line0(tid) - kc : 0, sc = RAGGED ? c0 + SC::line0(tid) - nc : 0;
+    const bool straddle = RAGGED && ((sr > 0 && sr < LR) || (sc > 0 && sc < LC));
     float bec[LC];
 #pragma unroll
     for (int j = 0; j < LC; ++j) bec[j] = be[nc + j];
@@ -851,6 +868,12 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
       for (int j = 0; j < LC; ++j) {
         h0[j] = ge[j] * (RECIP ? oe[j] : exp_st(a0 + bec[j] - oe[j]));
         h1[j] = gd[j] * (RECIP ? od[j] : exp_st(a1 + bec[j] - od[j]));
+      }
+      if (straddle) {
+        shift_down<LR>(e0, sr);
+        shift_down<LR>(e1, sr);
+        shift_down<LC>(h0, sc);
+        shift_down<LC>(h1, sc);
       }
       SR::put(Rs(buf), tid, e0, e1);
       SC::put(Cs(buf), tid, h0, h1);

@@ -151,9 +151,7 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *                      parts that add up to it exactly and six partial
  *                      products per product, accumulated in fp32 - what is
  *                      dropped is below 2^-23 of a product, one fp32 rounding -
- *                      at 2.7 times less matrix-pipe time (the forward for any
- *                      sizes; the backward where K and N are multiples of 4,
- *                      else it stays on the fp32 instruction).
+ *                      at 2.7 times less matrix-pipe time.
  *   GENBMM_PATH_RECIP  as AUTO, with 1 / sum kept in fp32 for the backward, which
  *                      then weighs g by it instead of by exp(max - out): what
  *                      float16 / bfloat16 tensors want, whose `out` is stored

@@ -331,8 +331,7 @@ def test_three_part_products_are_as_accurate_as_fp32_products(gpu, B, M, K, N, s
 
 def test_logbmm_matrix_core_shape_sweep(gpu):
     """A seeded sweep of 48 shapes around the switching points of the matrix-core kernels (tile forms
-    256 x 256 / 256 x 128 / 128 x 128, full and ragged, extents in multiples of 16, of 4 and odd -
-    the backward takes the bf16 instruction for K and N in multiples of four, else the fp32 one):
+    256 x 256 / 256 x 128 / 128 x 128, full and ragged, extents in multiples of 16, of 4 and odd):
     the default path against float64 on the device, and against GENBMM_PATH_MFMA32."""
     rng = np.random.RandomState(7)
     shapes = []
@@ -358,6 +357,29 @@ def test_logbmm_matrix_core_shape_sweep(gpu):
             close_on_device(x[pick], w, "%s of %s" % (what, (B, M, K, N)))
             close_on_device(x, y.double(), "%s of %s against the fp32 matrix instruction" % (what, (B, M, K, N)),
                             rtol=2e-5, atol=2e-5)
+
+
+# K and N of every remainder of four on each tile of the three-part backward: 256 x 256 (both extents in
+# 256s, enough tiles), 128 x 256 / 256 x 128, 128 x 128; a last line that is a lone straddling piece
+@pytest.mark.parametrize("B,M,K,N", [(64, 511, 509, 510), (100, 250, 507, 509), (64, 512, 385, 387), (300, 130, 131, 253),
+                                     (150, 255, 254, 197), (3, 99, 97, 129), (2, 133, 101, 103), (2, 96, 259, 130),
+                                     (2, 97, 130, 98), (1, 257, 513, 385)])
+def test_logbmm_three_part_backward_on_any_size(gpu, B, M, K, N):
+    """Gradients of odd sizes against float64 (first and last batch item), and every batch item against the
+    fp32 instruction's kernels: both form H = g exp(max - out) from an `out` rounded to 2^-24 of itself
+    (|out| < 16: a relative 2^-20 of a weight), so at the tolerance of the other path tests."""
+    torch.manual_seed(B + M + K + N)
+    a, b, g = torch.randn(B, M, K, device=gpu), torch.randn(B, K, N, device=gpu), torch.randn(B, M, N, device=gpu)
+    got = {}
+    for path in (genmul.PATH_AUTO, genmul.PATH_MFMA32):
+        x, y = a.clone().requires_grad_(), b.clone().requires_grad_()
+        out = genmul.logbmm_on_path(x, y, path)
+        got[path] = torch.autograd.grad(out, (x, y), g)
+    pick = torch.tensor([0, B - 1], device=gpu)
+    _, wa, wb = oracle.logbmm_grads64(a[pick].cpu(), b[pick].cpu(), g[pick].cpu())
+    for u, v, w in zip(got[genmul.PATH_AUTO], got[genmul.PATH_MFMA32], (wa, wb)):
+        close(u[pick], w)
+        close(u, v, rtol=2e-5, atol=2e-5)
 
 
 @pytest.mark.parametrize("B,M,K,N", [(20, 128, 128, 128), (17, 100, 70, 128), (12, 64, 128, 65), (9, 127, 99, 101)])
