@@ -24,11 +24,105 @@ constexpr int kKC = 128;  // cells of the reduction axis per lane
 // covers every k of its lines (up to 64 * kKC; longer K: further workgroups) and idx
 // and g are read from memory once - the lanes of a line read the same addresses.
 // Each lane walks its whole line and adds the terms whose k falls into its part.
+//
+// A lane's cells are its own and lie at [k][lane]: whatever k each lane adds to, the 64 lanes
+// stay in 64 different banks, and nothing is exchanged between lanes (no barrier).  33 KB per
+// wave leave four waves on a compute unit, one per SIMD, so nothing but a lane's own loads
+// hides the latency of memory: the walk is double-buffered in registers, the next chunk of the
+// line is in flight while one is added.  Bound by the chains of ordered additions, one LDS round
+// trip per four cells.  Measured (both gradients, max product; before: loads waited for 16 cells at a
+// time, cells of a row side by side so that the lanes' additions met in banks, rows of unaligned
+// length one cell at a time): (256, 256^3) 104 -> 87 us, (64, 512^3) 141 -> 123, (8192, 32^3) 79 -> 54,
+// (40, 251, 173, 301) 111 -> 37.
+static_assert(kKC == 128, "the shifts of the write-out");
+constexpr int kArgAcc = 64 * kKC + 64;  // floats of LDS: the cells, one spare cell per lane
+constexpr int kChA = 32, kChB = 16;     // cells per chunk (a column's cells are single loads, and at most
+                                        // 63 loads can be in flight)
 
-// grad_a: line = row m.  The row is read 16 cells at a time (int4 / float4 when the
-// rows are 16-byte aligned), then the 16 additions are made in order.
-constexpr int kArgAccA = 64 * kKC + 64 + 64, kArgAccB = kKC * 64 + 64;  // floats of LDS
-// (blk: the workgroup's number among those of grad_a; accs: kArgAccA floats of LDS)
+// Chunks of a line as they come from memory - indices, gradients and for PROD == 2 the other factor;
+// nothing is converted before it is added, which would wait for the load - of a row (pieces of four
+// cells, any alignment) and of a column (single cells).
+typedef int argmax_i4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float argmax_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef elem_t argmax_e4 __attribute__((ext_vector_type(4), aligned(sizeof(elem_t))));
+template <int PROD>
+struct ArgRow {
+  static constexpr int CH = kChA;
+  argmax_i4 i4[CH / 4];
+  argmax_e4 g4[CH / 4];
+  argmax_f4 f4[PROD == 2 ? CH / 4 : 1];
+  __device__ __forceinline__ int iv(int q) const { return i4[q >> 2][q & 3]; }
+  __device__ __forceinline__ float gv(int q) const { return (float)g4[q >> 2][q & 3]; }
+  __device__ __forceinline__ float fv(int q) const { return f4[q >> 2][q & 3]; }
+};
+template <int PROD>
+struct ArgCol {
+  static constexpr int CH = kChB;
+  int i[CH];
+  elem_t g[CH];
+  float f[PROD == 2 ? CH : 1];
+  __device__ __forceinline__ int iv(int q) const { return i[q]; }
+  __device__ __forceinline__ float gv(int q) const { return (float)g[q]; }
+  __device__ __forceinline__ float fv(int q) const { return f[q]; }
+};
+// Compiler-level ordering point for a wave's own LDS traffic (one wave's LDS instructions execute in order).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The lane's cells cleared; then the line's `cells` cells through load(chunk, number), tail(chunk, number)
+// (the cells of a partial last chunk, index -1 behind them) and add(chunk, number).  No load stands
+// under a branch in the loop - the last chunk is asked for again instead -: behind a branch the compiler
+// can no longer tell which loads are younger than the chunk it waits for, and waits for all of them.
+template <class Chunk, class Load, class Tail, class Add>
+__device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int cells, int kcap, Load load, Tail tail, Add add) {
+  const int lane = threadIdx.x, full = cells / Chunk::CH;
+  Chunk x, y;
+  if (full > 0) load(x, 0);
+#pragma unroll 16
+  for (int kk = 0; kk < kcap; ++kk) accs[kk * 64 + lane] = 0.f;
+  accs[kKC * 64 + lane] = 0.f;
+  int c = 0;
+  for (; c + 1 < full; c += 2) {
+    load(y, c + 1);
+    add(x, c);
+    load(x, min(c + 2, full - 1));
+    add(y, c + 1);
+  }
+  if (c < full) add(x, c);
+  if (full * Chunk::CH < cells) {
+    tail(y, full);
+    add(y, full);
+  }
+}
+// The chunk's terms (g, times the other factor for the product semiring) in order.  other(cell, k):
+// that factor read from its matrix (PROD == 1), only when the index falls into the lane's part.
+template <int PROD, class Chunk, class Other>
+__device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk& x, int c0, int kc, Other other) {
+  constexpr int CH = Chunk::CH;
+  const int lane = threadIdx.x;
+  int sl[CH];
+  float tv[CH];
+#pragma unroll
+  for (int q = 0; q < CH; ++q) {
+    const int k = x.iv(q) - c0;
+    const bool mine = k >= 0 && k < kc;
+    sl[q] = (mine ? k : kKC) * 64 + lane;  // [kKC]: the spare cells
+    tv[q] = x.gv(q);
+    if (PROD == 2) tv[q] = __fmul_rn(x.fv(q), tv[q]);
+    if (PROD == 1 && mine) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < CH; q += 4) {
+    const int s4[4] = {sl[q], sl[q + 1], sl[q + 2], sl[q + 3]};
+    const float t4[4] = {tv[q], tv[q + 1], tv[q + 2], tv[q + 3]};
+    add4_ordered(accs, s4, t4);
+  }
+}
+
+// grad_a: line = row m, read in pieces of four cells (any alignment).
+// (blk: the workgroup's number among those of grad_a; accs: kArgAcc floats of LDS)
 template <int PROD>
 __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int blk,
                                                    const elem_t* __restrict__ bmat,
@@ -36,93 +130,76 @@ __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int
                                                    const int32_t* __restrict__ idx,
                                                    const elem_t* __restrict__ g,
                                                    elem_t* __restrict__ grad_a, int M, int K,
-                                                   int N, int row_tiles, int k_chunks, int ps,
-                                                   int vec) {
+                                                   int N, int row_tiles, int k_chunks, int ps) {
   const int lane = threadIdx.x, parts = 1 << ps, lines = 64 >> ps;
   const int part = lane & (parts - 1), line = lane >> ps;
-  const int spare = 64 * kKC + 64 + lane;
   const int kc_id = blk % k_chunks, rt = blk / k_chunks;
   const int batch = rt / row_tiles;
-  const int m0 = (rt - batch * row_tiles) * lines;
-  const int kw = parts * kKC;                       // k covered by the workgroup
-  const int w0 = kc_id * kw, c0 = w0 + part * kKC;  // first k of the workgroup / of this lane
-  const int kc = min(kKC, K - c0);                  // <= 0: the part lies beyond K
-  const int m = m0 + line;
-  const bool live = m < M;
-  const int32_t* irow = idx + ((long)batch * M + (live ? m : 0)) * N;
-  const elem_t* grow = g + ((long)batch * M + (live ? m : 0)) * N;
+  const int m = (rt - batch * row_tiles) * lines + line;
+  const int c0 = kc_id * (parts * kKC) + part * kKC;  // first k of this lane
+  const int kc = min(kKC, K - c0);                    // <= 0: the part lies beyond K
+  const long row = (long)batch * M + min(m, M - 1);   // lanes beyond the matrix walk the last row
+  const int32_t* irow = idx + row * N;
+  const elem_t* grow = g + row * N;
   const elem_t* bb = PROD == 1 ? bmat + (long)batch * K * N : nullptr;
-  const float* frow = PROD == 2 ? fac + ((long)batch * M + (live ? m : 0)) * N : nullptr;
-  const int base = line * (kw + 1) + part * kKC;
-  float* mine = accs + base;
-  for (int kk = 0; kk < kKC; ++kk) mine[kk] = 0.f;
-  accs[spare] = 0.f;
-  auto slot = [&](int ki) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    return (k >= 0 && k < kc) ? base + k : spare;
-  };
-  // the term of cell n: g, times b[idx, n] for the product semiring (read only when
-  // the index falls into this lane's k range)
-  auto term = [&](int n, int ki, float gv) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    if (PROD == 1 && k >= 0 && k < kc) return __fmul_rn(bb[(long)ki * N + n], gv);
-    return gv;
-  };
-  auto add = [&](int ki, float v) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    if (k >= 0 && k < kc) mine[k] = __fadd_rn(mine[k], v);
-  };
-  if (live) {
-    int n = 0;
-    if (vec) {
-      for (; n + 16 <= N; n += 16) {
-        int4 iv[4];
-        float4 gv[4];
+  const float* frow = PROD == 2 ? fac + row * N : nullptr;
+  const int kcap = min(kKC, K);  // no lane has more cells
+  using Chunk = ArgRow<PROD>;
+  auto load = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int n0 = c * kChA;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          iv[q] = *reinterpret_cast<const int4*>(irow + n + 4 * q);
-          gv[q] = ld4a(grow + n + 4 * q);
-        }
-        if (PROD == 2) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float4 f = *reinterpret_cast<const float4*>(frow + n + 4 * q);
-            gv[q].x = __fmul_rn(f.x, gv[q].x);
-            gv[q].y = __fmul_rn(f.y, gv[q].y);
-            gv[q].z = __fmul_rn(f.z, gv[q].z);
-            gv[q].w = __fmul_rn(f.w, gv[q].w);
-          }
-        }
-        // all sixteen factors are requested before the first (ordered) addition
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          gv[q].x = term(n + 4 * q, iv[q].x, gv[q].x);
-          gv[q].y = term(n + 4 * q + 1, iv[q].y, gv[q].y);
-          gv[q].z = term(n + 4 * q + 2, iv[q].z, gv[q].z);
-          gv[q].w = term(n + 4 * q + 3, iv[q].w, gv[q].w);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int sl[4] = {slot(iv[q].x), slot(iv[q].y), slot(iv[q].z), slot(iv[q].w)};
-          const float tv[4] = {gv[q].x, gv[q].y, gv[q].z, gv[q].w};
-          add4_ordered(accs, sl, tv);
-        }
-      }
+    for (int q = 0; q < kChA / 4; ++q) {
+      x.i4[q] = *reinterpret_cast<const argmax_i4*>(irow + n0 + 4 * q);
+      x.g4[q] = *reinterpret_cast<const argmax_e4*>(grow + n0 + 4 * q);
+      if constexpr (PROD == 2) x.f4[q] = *reinterpret_cast<const argmax_f4*>(frow + n0 + 4 * q);
     }
-    for (; n < N; ++n)
-      add(irow[n], PROD == 2 ? __fmul_rn(frow[n], grow[n]) : term(n, irow[n], grow[n]));
+  };
+  auto tail = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int n0 = c * kChA;
+#pragma unroll
+    for (int q = 0; q < kChA; ++q) {
+      const bool in = n0 + q < N;
+      x.i4[q >> 2][q & 3] = in ? irow[n0 + q] : -1;
+      x.g4[q >> 2][q & 3] = in ? grow[n0 + q] : (elem_t)0.f;
+      if constexpr (PROD == 2) x.f4[q >> 2][q & 3] = in ? frow[n0 + q] : 0.f;
+    }
+  };
+  argmax_walk<Chunk>(accs, N, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
+    argmax_add<PROD>(accs, x, c0, kc, [&](int q, int k) { return (float)bb[(long)k * N + c * kChA + q]; });
+  });
+  // The cells change places, through registers, to [lane][kKC + 1] - a row's parts one after the other -
+  // so that the rows leave in runs (a lane storing its own cells, 16 bytes at a time and 512 apart, took
+  // longer than the walk).
+  wave_lds_sync();
+  {
+    float cell[kKC];
+#pragma unroll
+    for (int k0 = 0; k0 < kKC; k0 += 32)
+      if (k0 < kcap) {  // uniform
+#pragma unroll
+        for (int kk = k0; kk < k0 + 32; ++kk) cell[kk] = accs[kk * 64 + lane];
+      }
+    wave_lds_sync();
+#pragma unroll
+    for (int k0 = 0; k0 < kKC; k0 += 32)
+      if (k0 < kcap) {
+#pragma unroll
+        for (int kk = k0; kk < k0 + 32; ++kk) accs[lane * (kKC + 1) + kk] = cell[kk];
+      }
   }
-  __syncthreads();
-  const int rows = min(lines, M - m0), kn = min(kw, K - w0);
-  for (int r = 0; r < rows; ++r) {
-    elem_t* dst = grad_a + ((long)batch * M + m0 + r) * K + w0;
-    for (int kk = lane; kk < kn; kk += 64) dst[kk] = to_elem<elem_t>(accs[r * (kw + 1) + kk]);
+  wave_lds_sync();
+  const int kw = parts * kKC, w0 = kc_id * kw, kn = min(kw, K - w0);
+  const int m0 = (rt - batch * row_tiles) * lines, rows = min(lines, M - m0);
+  elem_t* dst = grad_a + ((long)batch * M + m0) * K + w0;
+  for (int kk = lane; kk < kn; kk += 64) {
+    const float* src = accs + (kk >> 7) * (kKC + 1) + (kk & (kKC - 1));
+#pragma unroll 8
+    for (int r = 0; r < rows; ++r) dst[(long)r * K + kk] = to_elem<elem_t>(src[r * parts * (kKC + 1)]);
   }
 }
 
-// grad_b: line = column n; the column is read 16 rows at a time, then added in order.
-// Accumulators are [k][line].
-// (blk: the workgroup's number among those of grad_b; accs: kArgAccB floats of LDS)
+// grad_b: line = column n.
+// (blk: the workgroup's number among those of grad_b; accs: kArgAcc floats of LDS)
 template <int PROD>
 __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int blk,
                                                    const elem_t* __restrict__ amat,
@@ -132,66 +209,44 @@ __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int
                                                    elem_t* __restrict__ grad_b, int M, int K,
                                                    int N, int col_tiles, int k_chunks, int ps) {
   const int lane = threadIdx.x, parts = 1 << ps, lines = 64 >> ps;
-  const int part = lane & (parts - 1), line = lane >> ps;
-  const int spare = kKC * 64 + lane;
+  const int part = lane / lines, line = lane & (lines - 1);  // the lanes of a part: adjacent columns
   const int kc_id = blk % k_chunks, ct = blk / k_chunks;
   const int batch = ct / col_tiles;
-  const int n0 = (ct - batch * col_tiles) * lines, n = n0 + line;
-  const int kw = parts * kKC;
-  const int w0 = kc_id * kw, c0 = w0 + part * kKC;
+  const int n = (ct - batch * col_tiles) * lines + line, nn = min(n, N - 1);
+  const int c0 = kc_id * (parts * kKC) + part * kKC;
   const int kc = min(kKC, K - c0);
-  const bool live = n < N;
-  const int nn = live ? n : N - 1;
   const int32_t* icol = idx + (long)batch * M * N + nn;
   const elem_t* gcol = g + (long)batch * M * N + nn;
   const elem_t* ab = PROD == 1 ? amat + (long)batch * M * K : nullptr;
   const float* fcol = PROD == 2 ? fac + (long)batch * M * N + nn : nullptr;
-  const int base = (part * kKC) * lines + line;  // cell k of this lane: accs[base + k * lines]
-  float* mine = accs + base;
-  for (int kk = 0; kk < kKC; ++kk) mine[kk * lines] = 0.f;
-  accs[spare] = 0.f;
-  auto slot = [&](int ki) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    return (k >= 0 && k < kc) ? base + k * lines : spare;
-  };
-  auto term = [&](int m, int ki, float gv) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    if (PROD == 1 && k >= 0 && k < kc) return __fmul_rn(ab[(long)m * K + ki], gv);
-    if (PROD == 2) return __fmul_rn(fcol[(long)m * N], gv);
-    return gv;
-  };
-  auto add = [&](int ki, float v) __attribute__((always_inline)) {
-    const int k = ki - c0;
-    if (k >= 0 && k < kc) mine[k * lines] = __fadd_rn(mine[k * lines], v);
-  };
-  if (live) {
-    int m = 0;
-    for (; m + 16 <= M; m += 16) {
-      int iv[16];
-      float gv[16];
+  const int kcap = min(kKC, K);  // no lane has more cells
+  using Chunk = ArgCol<PROD>;
+  auto load = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int m0 = c * kChB;
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        iv[q] = icol[(long)(m + q) * N];
-        gv[q] = gcol[(long)(m + q) * N];
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) gv[q] = term(m + q, iv[q], gv[q]);
-#pragma unroll
-      for (int q = 0; q < 16; q += 4) {
-        const int sl[4] = {slot(iv[q]), slot(iv[q + 1]), slot(iv[q + 2]), slot(iv[q + 3])};
-        const float tv[4] = {gv[q], gv[q + 1], gv[q + 2], gv[q + 3]};
-        add4_ordered(accs, sl, tv);
-      }
+    for (int q = 0; q < kChB; ++q) {
+      x.i[q] = icol[(long)(m0 + q) * N];
+      x.g[q] = gcol[(long)(m0 + q) * N];
+      if constexpr (PROD == 2) x.f[q] = fcol[(long)(m0 + q) * N];
     }
-    for (; m < M; ++m) add(icol[(long)m * N], term(m, icol[(long)m * N], gcol[(long)m * N]));
-  }
-  __syncthreads();
-  // rows k of the result: `lines` consecutive columns each
-  const int cols = min(lines, N - n0), kn = min(kw, K - w0);
-  const int lc = lane & (lines - 1), lk = lane / lines;
-  if (lc < cols)
-    for (int kk = lk; kk < kn; kk += parts)
-      grad_b[((long)batch * K + w0 + kk) * N + n0 + lc] = to_elem<elem_t>(accs[kk * lines + lc]);
+  };
+  auto tail = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int m0 = c * kChB;
+#pragma unroll
+    for (int q = 0; q < kChB; ++q) {
+      const bool in = m0 + q < M;
+      x.i[q] = in ? icol[(long)(m0 + q) * N] : -1;
+      x.g[q] = in ? gcol[(long)(m0 + q) * N] : (elem_t)0.f;
+      if constexpr (PROD == 2) x.f[q] = in ? fcol[(long)(m0 + q) * N] : 0.f;
+    }
+  };
+  argmax_walk<Chunk>(accs, M, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
+    argmax_add<PROD>(accs, x, c0, kc, [&](int q, int k) { return (float)ab[(long)(c * kChB + q) * K + k]; });
+  });
+  if (n < N)
+#pragma unroll 16
+    for (int kk = 0; kk < kc; ++kk)
+      grad_b[((long)batch * K + c0 + kk) * N + n] = to_elem<elem_t>(accs[kk * 64 + lane]);
 }
 
 // Both gradients in one launch, batch item by batch item (ta workgroups of grad_a, then tb of
@@ -206,14 +261,14 @@ __global__ __launch_bounds__(64) void k_argmax_bwd_both(const elem_t* __restrict
                                                        const elem_t* __restrict__ g,
                                                        elem_t* __restrict__ grad_a,
                                                        elem_t* __restrict__ grad_b, int M, int K, int N,
-                                                       int row_tiles, int kc_a, int ps_a, int vec,
+                                                       int row_tiles, int kc_a, int ps_a,
                                                        int col_tiles, int kc_b, int ps_b) {
-  __shared__ float accs[kArgAccA > kArgAccB ? kArgAccA : kArgAccB];
+  __shared__ float accs[kArgAcc];
   const int ta = row_tiles * kc_a, tb = col_tiles * kc_b;
   const int v = xcd_renumber(blockIdx.x, gridDim.x);
   const int item = v / (ta + tb), r = v - item * (ta + tb);
   if (r < ta)
-    argmax_bwd_a_block<PROD>(accs, item * ta + r, bmat, fac_a, idx, g, grad_a, M, K, N, row_tiles, kc_a, ps_a, vec);
+    argmax_bwd_a_block<PROD>(accs, item * ta + r, bmat, fac_a, idx, g, grad_a, M, K, N, row_tiles, kc_a, ps_a);
   else
     argmax_bwd_b_block<PROD>(accs, item * tb + r - ta, amat, fac_b, idx, g, grad_b, M, K, N, col_tiles, kc_b, ps_b);
 }
@@ -248,15 +303,14 @@ int run_argmax_bwd(const elem_t* a, const elem_t* b, const int32_t* idx, const f
   const int col_tiles = ceil_div(N, 64 >> ps_b), kc_b = ceil_div(K, kKC << ps_b);
   const int64_t total = (int64_t)B * ((int64_t)row_tiles * kc_a + (int64_t)col_tiles * kc_b);
   if (total > 0x7fffffffLL) return GENBMM_E_SHAPE;
-  const int vec = (N % 4 == 0) && aligned16(idx) && aligned16(g);
   if (PROD && factors)
     hipLaunchKernelGGL((k_argmax_bwd_both<2>), dim3((unsigned)total), dim3(64), 0, s, a, b, factors + mn, factors,
-                       idx, g, grad_a, grad_b, M, K, N, row_tiles, kc_a, ps_a, vec && aligned16(factors + mn),
+                       idx, g, grad_a, grad_b, M, K, N, row_tiles, kc_a, ps_a,
                        col_tiles, kc_b, ps_b);
   else
     hipLaunchKernelGGL((k_argmax_bwd_both<kGather>), dim3((unsigned)total), dim3(64), 0, s, a, b,
                        (const float*)nullptr, (const float*)nullptr, idx, g, grad_a, grad_b, M, K, N, row_tiles,
-                       kc_a, ps_a, vec, col_tiles, kc_b, ps_b);
+                       kc_a, ps_a, col_tiles, kc_b, ps_b);
   if (int e = launch_status()) return e;
   return GENBMM_OK;
 }
