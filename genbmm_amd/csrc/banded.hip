@@ -418,27 +418,17 @@ static int banded_bwd(const elem_t* a, int a_lu, int a_ld, const elem_t* b, int 
       return launch_status();
     }
   }
-  if (mode == GENBMM_BAND_MAX &&
-      max(argmax_bwd_a_bytes(p.Wa), argmax_bwd_b_bytes(p.Wb)) <= kDirLdsLimit) {  // a compute unit's LDS
-    const int strips = ceil_div(n, kAT);
-    const dim3 grid((unsigned)((long)B * strips));
-    const size_t na = argmax_bwd_a_bytes(p.Wa), nb = argmax_bwd_b_bytes(p.Wb);
-    if (na > kStripLdsLimit)
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_argmax_bwd_a),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)na);
-    if (nb > kStripLdsLimit)
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_argmax_bwd_b),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)nb);
-    hipLaunchKernelGGL(k_band_argmax_bwd_a, grid, dim3(256), na, s, p, strips);
-    hipLaunchKernelGGL(k_band_argmax_bwd_b, grid, dim3(256), nb, s, p, strips);
+  if (mode == GENBMM_BAND_MAX) {
+    const int strips = ceil_div(n, kArgRows), pa = argmax_parts(p.Wa), pb = argmax_parts(p.Wb);
+    const int64_t total = (int64_t)B * strips * (pa + pb);
+    if (total > 0x7fffffffLL) return GENBMM_E_SHAPE;
+    hipLaunchKernelGGL(k_band_argmax_bwd, dim3((unsigned)total), dim3(64), argmax_bwd_bytes(p.Wa, p.Wb), s, p, strips,
+                       pa, pb);
     return launch_status();
   }
   if (mode == GENBMM_BAND_LOG) {
     hipLaunchKernelGGL((k_band_bwd_a<GENBMM_BAND_LOG, elem_t>), blocks_for(ta), dim3(256), 0, s, p, ta);
     hipLaunchKernelGGL((k_band_bwd_b<GENBMM_BAND_LOG, elem_t>), blocks_for(tb), dim3(256), 0, s, p, tb);
-  } else if (mode == GENBMM_BAND_MAX) {
-    hipLaunchKernelGGL((k_band_bwd_a<GENBMM_BAND_MAX, elem_t>), blocks_for(ta), dim3(256), 0, s, p, ta);
-    hipLaunchKernelGGL((k_band_bwd_b<GENBMM_BAND_MAX, elem_t>), blocks_for(tb), dim3(256), 0, s, p, tb);
   } else {
     hipLaunchKernelGGL((k_band_bwd_a<GENBMM_BAND_MUL, elem_t>), blocks_for(ta), dim3(256), 0, s, p, ta);
     hipLaunchKernelGGL((k_band_bwd_b<GENBMM_BAND_MUL, elem_t>), blocks_for(tb), dim3(256), 0, s, p, tb);

@@ -439,3 +439,25 @@ def test_backward_with_separate_scratch_leaves_the_workspace_alone(gpu, n, a_lu,
     assert lib.genbmm_banded_bwd(p(ad), a_lu, a_ld, p(bd), b_lu, b_ld, p(None), p(None), p(None), p(g), p(wa), p(wb),
                                  B, n, 3, s) == 0
     assert torch.equal(ga, wa) and torch.equal(gb, wb)
+
+
+# rows shorter than a piece of four, one strip and its remainders, bands of whole and partial groups of 32
+# diagonals, bands of more than one workgroup's 128, one-sided bands, bands wider than the matrix
+@pytest.mark.parametrize("n,a_lu,a_ld,b_lu,b_ld", [
+    (1, 0, 0, 0, 0), (3, 0, 1, 0, 0), (65, 1, 0, 0, 1), (64, 0, 0, 2, 1), (63, 1, 1, 1, 1), (130, 15, 16, 16, 14),
+    (129, 16, 16, 7, 9), (200, 32, 32, 32, 32), (70, 0, 63, 40, 0), (190, 64, 63, 64, 64), (150, 70, 60, 0, 3),
+    (260, 100, 160, 3, 130), (20, 30, 35, 25, 33)])
+def test_banded_argmax_backward_sums_in_order(gpu, n, a_lu, a_ld, b_lu, b_ld):
+    """Gradients of the band max product bit for bit: float32 sums of any numbers in the reference's order
+    (the sequential oracle's), and for half bands the float sums rounded once."""
+    torch.manual_seed(n + a_lu)
+    a, b = pair(n, a_lu, a_ld, b_lu, b_ld, mk=grid)      # ties
+    g = torch.randn(a.shape[0], n, a.shape[2] + b.shape[2] - 1)
+    for dt in (torch.float32, torch.bfloat16):
+        gd = g.to(dt)
+        X = BandedMatrix(a.to(gpu, dt).requires_grad_(True), a_lu, a_ld)
+        Y = BandedMatrix(b.to(gpu, dt).requires_grad_(True), b_lu, b_ld)
+        ga, gb = torch.autograd.grad(X.multiply_max(Y).data, (X.data, Y.data), gd.to(gpu))
+        wa, wb = oracle.seq_band_bwd(X.data.detach().float().cpu(), a_lu, a_ld, Y.data.detach().float().cpu(), b_lu, b_ld,
+                                     gd.float(), 1, dtype=np.float32)
+        assert torch.equal(ga.cpu(), wa.to(dt)) and torch.equal(gb.cpu(), wb.to(dt)), dt
