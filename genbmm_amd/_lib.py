@@ -76,6 +76,7 @@ for _name in HALF_VARIANTS:
 for _suffix in ("_f16", "_bf16"):  # one more buffer than the float function: t_scratch (B * n * Wo floats)
     SIGNATURES["genbmm_banded_bwdbwd" + _suffix] = _BAND + [_c_float_p] * 8 + [_i, _i, _vp]
 HALF_SUFFIX = {torch.float16: "_f16", torch.bfloat16: "_bf16"}
+_ELEMENTS = (torch.float32, torch.float64) + tuple(HALF_SUFFIX)
 STRING_FUNCS = {"genbmm_version": [], "genbmm_error_string": [_i]}
 INT_FUNCS = {"genbmm_logbmm_fwd_pieces": [_i, _i, _i, _i], "genbmm_maxbmm_fwd_pieces": [_i, _i, _i, _i],
              "genbmm_banded_on_matrix_cores": [_i, _i, _i, _i, _i, _i]}
@@ -141,6 +142,27 @@ def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+def addr(t):
+    """`ptr` as a plain integer (None: NULL), which the declared argument types take as well."""
+    return t.data_ptr() if t is not None else None
+
+
+def call(name, t, *args):
+    """The library function `name` on t's device and that device's current stream.  The device is
+    switched only where it is another one, and the stream's handle is read without a Stream object
+    around it: 10 us of host time per call were 5.5 of those two, of 70 us that a small product's
+    forward and backward take in all (the rest is autograd's)."""
+    fn = getattr(_lib or load(), name)
+    index = t.get_device()
+    if index == torch.cuda.current_device():
+        code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(index):
+            code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    if code != 0:
+        check(code, name)
+
+
 def require(t, name, dtype=torch.float32, ndim=3, device=None):
     """Device / layout / dtype checks (reference CHECK_INPUT, matmul_cuda.cpp:65-67)."""
     if not isinstance(t, torch.Tensor):
@@ -161,27 +183,18 @@ def require(t, name, dtype=torch.float32, ndim=3, device=None):
 def dense_dims(a, b):
     """(B, M, K, N) of a (B,M,K) x (B,K,N) product, with agreement checks; a's element
     type (float32, float64, float16 or bfloat16) is the one both must have."""
-    dtype = torch.float32
-    if isinstance(a, torch.Tensor) and (a.dtype == torch.float64 or a.dtype in HALF_SUFFIX):
-        dtype = a.dtype
-    require(a, "a", dtype=dtype)
-    require(b, "b", dtype=dtype, device=a.device)
+    if not (isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor) and a.is_cuda and b.is_cuda
+            and a.dtype == b.dtype and a.dtype in _ELEMENTS and a.dim() == 3 and b.dim() == 3
+            and a.is_contiguous() and b.is_contiguous() and a.get_device() == b.get_device()):
+        # one check after the other, for the message
+        dtype = torch.float32
+        if isinstance(a, torch.Tensor) and (a.dtype == torch.float64 or a.dtype in HALF_SUFFIX):
+            dtype = a.dtype
+        require(a, "a", dtype=dtype)
+        require(b, "b", dtype=dtype, device=a.device)
     B, M, K = a.shape
     if b.shape[0] != B or b.shape[1] != K:
         raise RuntimeError(
             "shape mismatch: a is %s, b is %s" % (tuple(a.shape), tuple(b.shape))
         )
     return B, M, K, b.shape[2]
-
-
-class device_of:
-    """Make the tensors' device current around a library call (the reference has no guard)."""
-
-    def __init__(self, t):
-        self.guard = torch.cuda.device(t.device)
-
-    def __enter__(self):
-        self.guard.__enter__()
-
-    def __exit__(self, *exc):
-        return self.guard.__exit__(*exc)

@@ -106,10 +106,7 @@ def _canonical(a, b):
     return a, b, restore
 
 
-def _call(name, t, *args):
-    lib = _lib.load()
-    with _lib.device_of(t):
-        _lib.check(getattr(lib, name)(*args, _lib.stream_of(t)), name)
+_call = _lib.call
 
 
 # --------------------------------------------------------------------- logbmm
@@ -126,11 +123,11 @@ class _LogBmmGrad(torch.autograd.Function):
         grad_a = torch.empty_like(a)
         grad_b = torch.empty_like(b)
         if _f64(a):
-            _call("genbmm_logbmm_bwd_f64", a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g),
-                  _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+            _call("genbmm_logbmm_bwd_f64", a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g),
+                  _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
         else:
-            _call("genbmm_logbmm_bwd_path" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g),
-                  _lib.ptr(stats), _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N, path)
+            _call("genbmm_logbmm_bwd_path" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g),
+                  _lib.addr(stats), _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N, path)
         ctx.save_for_backward(a, b, g, out)
         ctx.set_materialize_grads(False)
         return grad_a, grad_b
@@ -147,14 +144,14 @@ class _LogBmmGrad(torch.autograd.Function):
         gb = torch.empty_like(b)
         gg = torch.empty_like(g)
         if _f64(a):
-            _call("genbmm_logbmm_bwdbwd_f64", a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g),
-                  _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(ga), _lib.ptr(gb), _lib.ptr(gg), B, M, K, N)
+            _call("genbmm_logbmm_bwdbwd_f64", a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g),
+                  _lib.addr(u_a), _lib.addr(u_b), _lib.addr(ga), _lib.addr(gb), _lib.addr(gg), B, M, K, N)
         else:
             # scratch for the factored form on the matrix cores (and, for float16 / bfloat16 tensors, where
             # the gradient with respect to g stays unrounded for the other two gradients)
             ws = torch.empty(_lib.load().genbmm_logbmm_bwdbwd_ws_size(B, M, K, N), dtype=_COMPUTE, device=a.device)
-            _call("genbmm_logbmm_bwdbwd_ws" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g),
-                  _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(ga), _lib.ptr(gb), _lib.ptr(gg), _lib.ptr(ws), B, M, K, N)
+            _call("genbmm_logbmm_bwdbwd_ws" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g),
+                  _lib.addr(u_a), _lib.addr(u_b), _lib.addr(ga), _lib.addr(gb), _lib.addr(gg), _lib.addr(ws), B, M, K, N)
         return ga, gb, gg, None, None, None
 
 
@@ -168,13 +165,13 @@ class LogMatMul(torch.autograd.Function):
         out = torch.empty(B, M, N, dtype=a.dtype, device=a.device)
         if _f64(a):
             stats = a.new_empty(0)
-            _call("genbmm_logbmm_fwd_f64", a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), B, M, K, N)
+            _call("genbmm_logbmm_fwd_f64", a, _lib.addr(a), _lib.addr(b), _lib.addr(out), B, M, K, N)
         else:
             # the library's workspace: what the reference's `maxes` becomes
             stats = torch.empty(_lib.load().genbmm_logbmm_stats_size_path(B, M, K, N, path), dtype=_COMPUTE,
                                 device=a.device)
-            _call("genbmm_logbmm_fwd_path" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out),
-                  _lib.ptr(stats), B, M, K, N, path)
+            _call("genbmm_logbmm_fwd_path" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out),
+                  _lib.addr(stats), B, M, K, N, path)
         ctx.save_for_backward(a, b, out, stats)
         ctx.path = path
         return out
@@ -199,18 +196,18 @@ def _argmax_backward(ctx, grad_output, prod):
     grad_b = torch.empty(B, K, N, dtype=ct, device=g.device)
     if ct == torch.float64:
         if prod:
-            _call("genbmm_prodmax_bwd_f64", g, _lib.ptr(a), _lib.ptr(b), _lib.ptr(idx), _lib.ptr(g),
-                  _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+            _call("genbmm_prodmax_bwd_f64", g, _lib.addr(a), _lib.addr(b), _lib.addr(idx), _lib.addr(g),
+                  _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
         else:
-            _call("genbmm_argmax_bwd_f64", g, _lib.ptr(idx), _lib.ptr(g), _lib.ptr(grad_a),
-                  _lib.ptr(grad_b), B, M, K, N)
+            _call("genbmm_argmax_bwd_f64", g, _lib.addr(idx), _lib.addr(g), _lib.addr(grad_a),
+                  _lib.addr(grad_b), B, M, K, N)
     elif prod:
         # the factors a[m, idx], b[idx, n] were stored by the forward: a and b are not read
-        _call("genbmm_prodmax_bwd" + _sfx(g), g, _lib.ptr(None), _lib.ptr(None), _lib.ptr(idx),
-              _lib.ptr(factors), _lib.ptr(g), _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+        _call("genbmm_prodmax_bwd" + _sfx(g), g, _lib.addr(None), _lib.addr(None), _lib.addr(idx),
+              _lib.addr(factors), _lib.addr(g), _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
     else:
-        _call("genbmm_argmax_bwd" + _sfx(g), g, _lib.ptr(idx), _lib.ptr(g), _lib.ptr(grad_a),
-              _lib.ptr(grad_b), B, M, K, N)
+        _call("genbmm_argmax_bwd" + _sfx(g), g, _lib.addr(idx), _lib.addr(g), _lib.addr(grad_a),
+              _lib.addr(grad_b), B, M, K, N)
     return grad_a, grad_b
 
 
@@ -230,11 +227,11 @@ def _max_forward(a, b, prod, factors=None):
         out = torch.empty(B, M, N, dtype=a.dtype, device=a.device)
         idx = torch.empty(B, M, N, dtype=torch.int32, device=a.device)
         if _f64(a):
-            _call(name + "_f64", a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), B, M, K, N)
+            _call(name + "_f64", a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), B, M, K, N)
         elif prod:
-            _call(name + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), _lib.ptr(factors), B, M, K, N)
+            _call(name + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), _lib.addr(factors), B, M, K, N)
         else:
-            _call(name + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), B, M, K, N)
+            _call(name + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), B, M, K, N)
         return out, idx
     Ks = K // S
     # (float16 / bfloat16 operands: the pieces are compared unrounded, in float32 - two pieces whose
@@ -247,9 +244,9 @@ def _max_forward(a, b, prod, factors=None):
     idxs = torch.empty(B * S, M, N, dtype=torch.int32, device=a.device)
     if prod:
         fac_s = torch.empty(2, B * S, M, N, dtype=_COMPUTE, device=a.device)
-        _call(name, a, _lib.ptr(a_s), _lib.ptr(b_s), _lib.ptr(vals), _lib.ptr(idxs), _lib.ptr(fac_s), B * S, M, Ks, N)
+        _call(name, a, _lib.addr(a_s), _lib.addr(b_s), _lib.addr(vals), _lib.addr(idxs), _lib.addr(fac_s), B * S, M, Ks, N)
     else:
-        _call(name, a, _lib.ptr(a_s), _lib.ptr(b_s), _lib.ptr(vals), _lib.ptr(idxs), B * S, M, Ks, N)
+        _call(name, a, _lib.addr(a_s), _lib.addr(b_s), _lib.addr(vals), _lib.addr(idxs), B * S, M, Ks, N)
     vals, idxs = vals.view(B, S, M, N), idxs.view(B, S, M, N)
     # a piece without a term above the -1e9 floor reports the floor and index -1: it never wins
     # against a piece with one, and if no piece has one the result is the floor and -1 as well
@@ -332,13 +329,13 @@ class SampleMatMul(torch.autograd.Function):
         idx = torch.empty(B, M, N, dtype=torch.int32, device=a.device)
         seed, offset = int(seed) & 0xFFFFFFFFFFFFFFFF, int(offset) & 0xFFFFFFFFFFFFFFFF
         if _f64(a):
-            _call("genbmm_samplebmm_fwd_f64", a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out),
-                  _lib.ptr(idx), seed, offset, B, M, K, N)
+            _call("genbmm_samplebmm_fwd_f64", a, _lib.addr(a), _lib.addr(b), _lib.addr(out),
+                  _lib.addr(idx), seed, offset, B, M, K, N)
         else:
             stats = torch.empty(_lib.load().genbmm_samplebmm_stats_size(B, M, K, N), dtype=_COMPUTE,
                                 device=a.device)
-            _call("genbmm_samplebmm_fwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx),
-                  _lib.ptr(stats), seed, offset, B, M, K, N)
+            _call("genbmm_samplebmm_fwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx),
+                  _lib.addr(stats), seed, offset, B, M, K, N)
         ctx.save_for_backward(idx)
         ctx.dims, ctx.compute = dims, a.dtype
         return out

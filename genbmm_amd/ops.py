@@ -43,10 +43,7 @@ def _sfx(t: Tensor):
     return _lib.HALF_SUFFIX.get(t.dtype, "")
 
 
-def _call(name, t, *args):
-    lib = _lib.load()
-    with _lib.device_of(t):
-        _lib.check(getattr(lib, name)(*args, _lib.stream_of(t)), name)
+_call = _lib.call
 
 
 def _stats_size(B, M, K, N):
@@ -60,7 +57,7 @@ def logbmm_fwd(a: Tensor, b: Tensor) -> Tuple[Tensor, Tensor]:
     B, M, K, N = _check(a, b)
     out = torch.empty(B, M, N, dtype=a.dtype, device=a.device)
     stats = torch.empty(_stats_size(B, M, K, N), dtype=_F32, device=a.device)
-    _call("genbmm_logbmm_fwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(stats), B, M, K, N)
+    _call("genbmm_logbmm_fwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(stats), B, M, K, N)
     return out, stats
 
 
@@ -75,8 +72,8 @@ def logbmm_bwd(a: Tensor, b: Tensor, out: Tensor, g: Tensor, stats: Tensor) -> T
     B, M, K, N = _check(a, b)
     g = g.to(a.dtype).contiguous()
     grad_a, grad_b = torch.empty_like(a), torch.empty_like(b)
-    _call("genbmm_logbmm_bwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g), _lib.ptr(stats),
-          _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+    _call("genbmm_logbmm_bwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g), _lib.addr(stats),
+          _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
     return grad_a, grad_b
 
 
@@ -93,8 +90,8 @@ def logbmm_bwdbwd(a: Tensor, b: Tensor, out: Tensor, g: Tensor, u_a: Tensor,
     g, u_a, u_b = g.to(a.dtype).contiguous(), u_a.to(a.dtype).contiguous(), u_b.to(a.dtype).contiguous()
     ga, gb, gg = torch.empty_like(a), torch.empty_like(b), torch.empty_like(g)
     ws = torch.empty(_lib.load().genbmm_logbmm_bwdbwd_ws_size(B, M, K, N), dtype=torch.float32, device=a.device)
-    _call("genbmm_logbmm_bwdbwd_ws" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(g), _lib.ptr(u_a),
-          _lib.ptr(u_b), _lib.ptr(ga), _lib.ptr(gb), _lib.ptr(gg), _lib.ptr(ws), B, M, K, N)
+    _call("genbmm_logbmm_bwdbwd_ws" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(g), _lib.addr(u_a),
+          _lib.addr(u_b), _lib.addr(ga), _lib.addr(gb), _lib.addr(gg), _lib.addr(ws), B, M, K, N)
     return ga, gb, gg
 
 
@@ -141,7 +138,7 @@ def maxbmm_fwd(a: Tensor, b: Tensor) -> Tuple[Tensor, Tensor]:
     B, M, K, N = _check(a, b)
     out = torch.empty(B, M, N, dtype=a.dtype, device=a.device)
     idx = torch.empty(B, M, N, dtype=torch.int32, device=a.device)
-    _call("genbmm_maxbmm_fwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), B, M, K, N)
+    _call("genbmm_maxbmm_fwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), B, M, K, N)
     return out, idx
 
 
@@ -158,7 +155,7 @@ def samplebmm_fwd(a: Tensor, b: Tensor, seed: int, offset: int) -> Tuple[Tensor,
     idx = torch.empty(B, M, N, dtype=torch.int32, device=a.device)
     stats = torch.empty(int(_lib.load().genbmm_samplebmm_stats_size(int(B), int(M), int(K), int(N))),
                         dtype=_F32, device=a.device)
-    _call("genbmm_samplebmm_fwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), _lib.ptr(stats),
+    _call("genbmm_samplebmm_fwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), _lib.addr(stats),
           seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, B, M, K, N)
     return out, idx
 
@@ -176,7 +173,7 @@ def argmax_bwd(idx: Tensor, g: Tensor, K: int) -> Tuple[Tensor, Tensor]:
     g = g.contiguous()
     grad_a = torch.empty(B, M, K, dtype=g.dtype, device=g.device)
     grad_b = torch.empty(B, K, N, dtype=g.dtype, device=g.device)
-    _call("genbmm_argmax_bwd" + _sfx(g), g, _lib.ptr(idx), _lib.ptr(g), _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+    _call("genbmm_argmax_bwd" + _sfx(g), g, _lib.addr(idx), _lib.addr(g), _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
     return grad_a, grad_b
 
 
@@ -209,7 +206,7 @@ def prodmaxbmm_fwd(a: Tensor, b: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
     out = torch.empty(B, M, N, dtype=a.dtype, device=a.device)
     idx = torch.empty(B, M, N, dtype=torch.int32, device=a.device)
     factors = torch.empty(2, B, M, N, dtype=_F32, device=a.device)
-    _call("genbmm_prodmaxbmm_fwd" + _sfx(a), a, _lib.ptr(a), _lib.ptr(b), _lib.ptr(out), _lib.ptr(idx), _lib.ptr(factors),
+    _call("genbmm_prodmaxbmm_fwd" + _sfx(a), a, _lib.addr(a), _lib.addr(b), _lib.addr(out), _lib.addr(idx), _lib.addr(factors),
           B, M, K, N)
     return out, idx, factors
 
@@ -226,8 +223,8 @@ def prodmax_bwd(idx: Tensor, factors: Tensor, g: Tensor, K: int) -> Tuple[Tensor
     g = g.contiguous()
     grad_a = torch.empty(B, M, K, dtype=g.dtype, device=g.device)
     grad_b = torch.empty(B, K, N, dtype=g.dtype, device=g.device)
-    _call("genbmm_prodmax_bwd" + _sfx(g), g, _lib.ptr(None), _lib.ptr(None), _lib.ptr(idx), _lib.ptr(factors), _lib.ptr(g),
-          _lib.ptr(grad_a), _lib.ptr(grad_b), B, M, K, N)
+    _call("genbmm_prodmax_bwd" + _sfx(g), g, _lib.addr(None), _lib.addr(None), _lib.addr(idx), _lib.addr(factors), _lib.addr(g),
+          _lib.addr(grad_a), _lib.addr(grad_b), B, M, K, N)
     return grad_a, grad_b
 
 
@@ -302,8 +299,8 @@ def banded_fwd(a: Tensor, b: Tensor, a_lu: int, a_ld: int, b_lu: int, b_ld: int,
     else:
         aux = torch.empty(0, dtype=_F32, device=a.device)
         idx, ws = None, None
-    _call("genbmm_banded_fwd", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld, _lib.ptr(out), _lib.ptr(idx),
-          _lib.ptr(ws), B, n, mode)
+    _call("genbmm_banded_fwd", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld, _lib.addr(out), _lib.addr(idx),
+          _lib.addr(ws), B, n, mode)
     return out, aux
 
 
@@ -334,8 +331,8 @@ def banded_bwd(a: Tensor, b: Tensor, out: Tensor, aux: Tensor, g: Tensor, a_lu: 
     if mode == _BAND_LOG:
         need = int(_lib.load().genbmm_banded_scratch_size(int(a_lu), int(a_ld), int(b_lu), int(b_ld), int(B), int(n)))
         scratch = torch.empty(need, dtype=_F32, device=a.device) if need else None
-    _call("genbmm_banded_bwd_scratch", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld, _lib.ptr(o),
-          _lib.ptr(idx), _lib.ptr(ws), _lib.ptr(scratch), _lib.ptr(g), _lib.ptr(grad_a), _lib.ptr(grad_b), B, n, mode)
+    _call("genbmm_banded_bwd_scratch", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld, _lib.addr(o),
+          _lib.addr(idx), _lib.addr(ws), _lib.addr(scratch), _lib.addr(g), _lib.addr(grad_a), _lib.addr(grad_b), B, n, mode)
     return grad_a, grad_b
 
 
@@ -351,8 +348,8 @@ def banded_bwdbwd(a: Tensor, b: Tensor, out: Tensor, g: Tensor, u_a: Tensor, u_b
     B, n, _ = _band_dims(a, b, a_lu, a_ld, b_lu, b_ld)
     a, b, g, u_a, u_b = a.contiguous(), b.contiguous(), g.contiguous(), u_a.contiguous(), u_b.contiguous()
     ga, gb, gg = torch.empty_like(a), torch.empty_like(b), torch.empty_like(g)
-    _call("genbmm_banded_bwdbwd", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld, _lib.ptr(out), _lib.ptr(g),
-          _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(ga), _lib.ptr(gb), _lib.ptr(gg), B, n)
+    _call("genbmm_banded_bwdbwd", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld, _lib.addr(out), _lib.addr(g),
+          _lib.addr(u_a), _lib.addr(u_b), _lib.addr(ga), _lib.addr(gb), _lib.addr(gg), B, n)
     return ga, gb, gg
 
 

@@ -29,6 +29,8 @@ from . import _lib
 
 MODE_LOG, MODE_MAX, MODE_SAMPLE, MODE_MUL = 0, 1, 2, 3
 
+_call = _lib.call
+
 # The reference sets this when its extension imports (sparse.py:3-9); here: the HIP
 # library has been built.  (It selects nothing: there is no other path to fall back to.)
 has_cuda = os.path.exists(_lib.LIB_PATH)
@@ -47,12 +49,6 @@ def _native(t):
     return t.is_cuda and t.dtype == torch.float32
 
 
-def _struct_call(name, t, *args):
-    lib = _lib.load()
-    with _lib.device_of(t):
-        _lib.check(getattr(lib, name)(*args, _lib.stream_of(t)), name)
-
-
 class _BandShift(torch.autograd.Function):
     """out[b, c, k] = data[b, c + dcol, k + dband] or fill (genbmm_band_shift)."""
 
@@ -61,8 +57,8 @@ class _BandShift(torch.autograd.Function):
         data = data.contiguous()
         B, n, w_in = data.shape
         out = torch.empty(B, n, w_out, dtype=data.dtype, device=data.device)
-        _struct_call("genbmm_band_shift", data, _lib.ptr(data), _lib.ptr(out), B, n, w_in, w_out,
-                     dcol, dband, float(fill))
+        _call("genbmm_band_shift", data, _lib.addr(data), _lib.addr(out), B, n, w_in, w_out,
+              dcol, dband, float(fill))
         ctx.args = (w_in, dcol, dband)
         return out
 
@@ -81,7 +77,7 @@ class _BandTranspose(torch.autograd.Function):
         data = data.contiguous()
         B, n, _ = data.shape
         out = torch.empty_like(data)
-        _struct_call("genbmm_band_transpose", data, _lib.ptr(data), _lib.ptr(out), B, n, lu, ld)
+        _call("genbmm_band_transpose", data, _lib.addr(data), _lib.addr(out), B, n, lu, ld)
         ctx.bands = (lu, ld)
         return out
 
@@ -97,8 +93,8 @@ class _BandToDense(torch.autograd.Function):
         data = data.contiguous()
         B, n, _ = data.shape
         out = torch.empty(B, n, n, dtype=data.dtype, device=data.device)
-        _struct_call("genbmm_band_to_dense", data, _lib.ptr(data), _lib.ptr(out), B, n, lu, ld,
-                     float(fill))
+        _call("genbmm_band_to_dense", data, _lib.addr(data), _lib.addr(out), B, n, lu, ld,
+              float(fill))
         ctx.bands = (lu, ld)
         return out
 
@@ -116,8 +112,8 @@ class _BandFromDense(torch.autograd.Function):
         dense = dense.contiguous()
         B, n_rows, n = dense.shape
         out = torch.empty(B, n, lu + ld + 1, dtype=dense.dtype, device=dense.device)
-        _struct_call("genbmm_band_from_dense", dense, _lib.ptr(dense), _lib.ptr(out), B, n_rows, n,
-                     lu, ld)
+        _call("genbmm_band_from_dense", dense, _lib.addr(dense), _lib.addr(out), B, n_rows, n,
+              lu, ld)
         ctx.bands = (lu, ld)
         return out
 
@@ -290,8 +286,8 @@ class BandedMatrix:
             a, b = self.data.contiguous(), other.data.contiguous()
             batch, n, _ = a.shape
             data = torch.empty(batch, n, lu + ld + 1, dtype=a.dtype, device=a.device)
-            _struct_call("genbmm_band_op", a, _lib.ptr(a), self.lu, self.ld, _lib.ptr(b), other.lu,
-                         other.ld, _lib.ptr(data), batch, n, code, float(zero))
+            _call("genbmm_band_op", a, _lib.addr(a), self.lu, self.ld, _lib.addr(b), other.lu,
+                  other.ld, _lib.addr(data), batch, n, code, float(zero))
             return BandedMatrix(data, lu, ld, self.fill)
         data = self._new(lu, ld).fill_(zero)
         s1 = lu - self.lu
@@ -408,12 +404,6 @@ def _check_pair(a, b):
     return a.shape[0], a.shape[1]
 
 
-def _call(name, t, *args):
-    lib = _lib.load()
-    with _lib.device_of(t):
-        _lib.check(getattr(lib, name)(*args, _lib.stream_of(t)), name)
-
-
 def _forward(a, a_lu, a_ld, b, b_lu, b_ld, mode):
     a = a.contiguous()
     b = b.contiguous()
@@ -424,8 +414,8 @@ def _forward(a, a_lu, a_ld, b, b_lu, b_ld, mode):
     out = torch.empty(B, n, wo, dtype=a.dtype, device=a.device)
     idx = torch.empty(B, n, wo, dtype=torch.int32, device=a.device) if mode == MODE_MAX else None
     if _f64(a):  # the double-precision entry points take no workspace
-        _call("genbmm_banded_fwd_f64", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-              _lib.ptr(out), _lib.ptr(idx), B, n, mode)
+        _call("genbmm_banded_fwd_f64", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+              _lib.addr(out), _lib.addr(idx), B, n, mode)
         return a, b, out, (None if mode == MODE_LOG else idx)
     # log product: the library's workspace (exp(a - max), exp(b - max), maxima, 1/sum),
     # which stands where the reference's `maxes` stands
@@ -433,8 +423,8 @@ def _forward(a, a_lu, a_ld, b, b_lu, b_ld, mode):
     if mode == MODE_LOG:
         size = _lib.load().genbmm_banded_workspace_size(a_lu, a_ld, b_lu, b_ld, B, n)
         ws = torch.empty(size, dtype=torch.float32, device=a.device)
-    _call("genbmm_banded_fwd" + _sfx(a), a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-          _lib.ptr(out), _lib.ptr(idx), _lib.ptr(ws), B, n, mode)
+    _call("genbmm_banded_fwd" + _sfx(a), a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+          _lib.addr(out), _lib.addr(idx), _lib.addr(ws), B, n, mode)
     return a, b, out, (ws if mode == MODE_LOG else idx)
 
 
@@ -445,8 +435,8 @@ def _backward(a, b, bands, out, idx, g, mode, ws=None):
     grad_a = torch.empty_like(a)
     grad_b = torch.empty_like(b)
     if _f64(a):
-        _call("genbmm_banded_bwd_f64", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-              _lib.ptr(out), _lib.ptr(idx), _lib.ptr(g), _lib.ptr(grad_a), _lib.ptr(grad_b), B, n, mode)
+        _call("genbmm_banded_bwd_f64", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+              _lib.addr(out), _lib.addr(idx), _lib.addr(g), _lib.addr(grad_a), _lib.addr(grad_b), B, n, mode)
         return grad_a, grad_b
     # g / sum per output cell, which both gradients of the log product share, goes to a
     # buffer of this call's own: the forward's workspace stays as the forward left it, so
@@ -455,9 +445,9 @@ def _backward(a, b, bands, out, idx, g, mode, ws=None):
     if mode == MODE_LOG and ws is not None:
         need = _lib.load().genbmm_banded_scratch_size(a_lu, a_ld, b_lu, b_ld, B, n)
         scratch = torch.empty(need, dtype=torch.float32, device=a.device) if need else None
-    _call("genbmm_banded_bwd_scratch" + _sfx(a), a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-          _lib.ptr(out), _lib.ptr(idx), _lib.ptr(ws), _lib.ptr(scratch), _lib.ptr(g), _lib.ptr(grad_a),
-          _lib.ptr(grad_b), B, n, mode)
+    _call("genbmm_banded_bwd_scratch" + _sfx(a), a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+          _lib.addr(out), _lib.addr(idx), _lib.addr(ws), _lib.addr(scratch), _lib.addr(g), _lib.addr(grad_a),
+          _lib.addr(grad_b), B, n, mode)
     return grad_a, grad_b
 
 
@@ -507,13 +497,13 @@ class _BandedLogGrad(torch.autograd.Function):
         if a.dtype in _lib.HALF_SUFFIX:
             # the gradient with respect to g is read back by the other two: a float copy of it
             t = torch.empty(g.shape, dtype=torch.float32, device=g.device)
-            _call("genbmm_banded_bwdbwd" + _sfx(a), a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-                  _lib.ptr(out), _lib.ptr(g), _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(ga), _lib.ptr(gb),
-                  _lib.ptr(gg), _lib.ptr(t), a.shape[0], a.shape[1])
+            _call("genbmm_banded_bwdbwd" + _sfx(a), a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+                  _lib.addr(out), _lib.addr(g), _lib.addr(u_a), _lib.addr(u_b), _lib.addr(ga), _lib.addr(gb),
+                  _lib.addr(gg), _lib.addr(t), a.shape[0], a.shape[1])
             return ga, gb, gg, None, None, None
-        _call("genbmm_banded_bwdbwd_f64" if _f64(a) else "genbmm_banded_bwdbwd", a, _lib.ptr(a),
-              a_lu, a_ld, _lib.ptr(b), b_lu, b_ld, _lib.ptr(out), _lib.ptr(g), _lib.ptr(u_a), _lib.ptr(u_b),
-              _lib.ptr(ga), _lib.ptr(gb), _lib.ptr(gg), a.shape[0], a.shape[1])
+        _call("genbmm_banded_bwdbwd_f64" if _f64(a) else "genbmm_banded_bwdbwd", a, _lib.addr(a),
+              a_lu, a_ld, _lib.addr(b), b_lu, b_ld, _lib.addr(out), _lib.addr(g), _lib.addr(u_a), _lib.addr(u_b),
+              _lib.addr(ga), _lib.addr(gb), _lib.addr(gg), a.shape[0], a.shape[1])
         return ga, gb, gg, None, None, None
 
 
@@ -578,13 +568,13 @@ class BandedSampleMul(torch.autograd.Function):
         out = torch.empty(B, n, wo, dtype=a.dtype, device=a.device)
         idx = torch.empty(B, n, wo, dtype=torch.int32, device=a.device)
         if _f64(a):
-            _call("genbmm_banded_sample_fwd_f64", a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-                  _lib.ptr(out), _lib.ptr(idx), seed, offset, B, n)
+            _call("genbmm_banded_sample_fwd_f64", a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+                  _lib.addr(out), _lib.addr(idx), seed, offset, B, n)
         else:
             size = _lib.load().genbmm_banded_workspace_size(a_lu, a_ld, b_lu, b_ld, B, n)
             ws = torch.empty(size, dtype=torch.float32, device=a.device)
-            _call("genbmm_banded_sample_fwd" + _sfx(a), a, _lib.ptr(a), a_lu, a_ld, _lib.ptr(b), b_lu, b_ld,
-                  _lib.ptr(out), _lib.ptr(idx), _lib.ptr(ws), seed, offset, B, n)
+            _call("genbmm_banded_sample_fwd" + _sfx(a), a, _lib.addr(a), a_lu, a_ld, _lib.addr(b), b_lu, b_ld,
+                  _lib.addr(out), _lib.addr(idx), _lib.addr(ws), seed, offset, B, n)
         ctx.save_for_backward(a, b, idx)
         ctx.bands = (a_lu, a_ld, b_lu, b_ld)
         return out
