@@ -525,7 +525,8 @@ class BandedLogMul(torch.autograd.Function):
         a, b, out, ws = ctx.saved_tensors
         a, b = a.contiguous(), b.contiguous()
         g = grad_output.to(a.dtype).contiguous()
-        grad_a, grad_b = _BandedLogGrad.apply(a, b, g, out, ws, ctx.bands)
+        # (`out` as a value, as in LogMatMul.backward)
+        grad_a, grad_b = _BandedLogGrad.apply(a, b, g, out.detach(), ws, ctx.bands)
         return (grad_a, None, None, grad_b) + (None,) * 4
 
 

@@ -1440,3 +1440,28 @@ def test_maxbmm_and_banded_in_a_graph(gpu):
         torch.cuda.synchronize()
         assert torch.equal(out, ref[0]) and torch.equal(idx, ref[1]) and torch.equal(bo, ref[2]), rep
         (a + 1).sum().item()
+
+
+@pytest.mark.parametrize("banded", [False, True])
+def test_second_order_is_one_library_call(gpu, monkeypatch, banded):
+    """The gradients of a log product's gradients are one call of the double backward: the first backward
+    is not run again (its share through `out` is part of the double backward)."""
+    from genbmm_amd import sparse
+
+    torch.manual_seed(2)
+    shapes = ((2, 40, 7), (2, 40, 9), (2, 40, 15)) if banded else ((2, 40, 24), (2, 24, 36), (2, 40, 36))
+    a, b, g = (torch.randn(*s, device=gpu, requires_grad=True) for s in shapes)
+    out = sparse.BandedMatrix(a, 3, 3).multiply_log(sparse.BandedMatrix(b, 4, 4)).data if banded else genbmm.logbmm(a, b)
+    first = torch.autograd.grad(out, (a, b), g, create_graph=True)
+    names = []
+    real = _lib.call
+
+    def call(name, *args):
+        names.append(name)
+        real(name, *args)
+
+    monkeypatch.setattr(genmul, "_call", call)
+    monkeypatch.setattr(sparse, "_call", call)
+    second = torch.autograd.grad(first, (a, b, g), (torch.randn_like(a), torch.randn_like(b)))
+    assert names == ["genbmm_banded_bwdbwd" if banded else "genbmm_logbmm_bwdbwd_ws"]
+    assert all(bool(torch.isfinite(t).all()) for t in second)
