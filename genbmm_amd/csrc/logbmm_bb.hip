@@ -14,7 +14,7 @@
 //  * Exact, on the vector ALU: three passes (t, grad_a, grad_b), one exponential per (m,k,n)
 //    in each.  Any shape; the whole computation for small problems, and the recompute of
 //    batch items that the factored form cannot take.
-//  * Factored, on the fp32 matrix cores (needs the caller's workspace): with the row maxima
+//  * Factored, on the matrix cores (needs the caller's workspace): with the row maxima
 //    alpha of a and column maxima beta of b, EA = exp(a - alpha), EB = exp(b - beta),
 //    R = exp(alpha + beta - out), H = g R, X = EA u_a, Y = EB u_b:
 //      t      = R (X EB + EA Y)
@@ -22,16 +22,17 @@
 //      grad_b = Y (EA^T H) + EB (X^T H - EA^T (H t))
 //    eight products (five when u_b is absent) of batched GEMM shape.  The operands are laid out
 //    once, zero-padded to multiples of 128 in every extent, by three elementwise passes; one
-//    GEMM kernel (128 x 128 tiles of v_mfma_f32_32x32x2_f32, 16-deep slabs through two LDS
-//    buffers) then runs without any edge handling in its loop, sums up to two products into one
+//    GEMM kernel (128 x 128 tiles, three-part operands on v_mfma_f32_32x32x16_bf16, 16-deep slabs
+//    through two LDS buffers) then runs without any edge handling in its loop, sums up to two products into one
 //    accumulator and applies the epilogue of its role.  A batch item with a cell whose
 //    alpha + beta - out is beyond 40 ln 2 or not finite (a factor could underflow against a
-//    term that matters) is flagged by the pass that forms H and redone by the exact kernels,
+//    term that matters), or with an X, Y or H beyond the largest bfloat16 (an infinite operand has
+//    no three parts), is flagged by the passes that form them and redone by the exact kernels,
 //    which run behind the factored ones on the flagged items only.
 #include <algorithm>
 #include <type_traits>
 
-#include "logbmm_mfma.h"
+#include "logbmm_split.h"
 
 namespace GENBMM_NS {
 namespace {
@@ -242,8 +243,6 @@ struct BBWs {
   float *ea, *x;   // (B, Mp, Kp): exp(a - alpha), ea * u_a
   float *eb, *y;   // (B, Kp, Np)
   float *r, *h, *nht;  // (B, Mp, Np): exp(alpha + beta - out), g r, -h t
-  float *ga0;      // (B, Mp, Kp): H EB^T
-  float *gb0;      // (B, Kp, Np): EA^T H
 };
 inline size_t bb_ws_floats(int B, int M, int K, int N, BBWs* w, float* base) {
   size_t off = 0;
@@ -262,8 +261,6 @@ inline size_t bb_ws_floats(int B, int M, int K, int N, BBWs* w, float* base) {
     t.ea = take(B * Mp * Kp); t.x = take(B * Mp * Kp);
     t.eb = take(B * Kp * Np); t.y = take(B * Kp * Np);
     t.r = take(B * Mp * Np); t.h = take(B * Mp * Np); t.nht = take(B * Mp * Np);
-    t.ga0 = take(B * Mp * Kp);
-    t.gb0 = take(B * Kp * Np);
   }
   if (w) *w = t;
   return off;
@@ -276,6 +273,10 @@ __device__ __forceinline__ float4 exp4_st(float4 v, float m) {
 }
 __device__ __forceinline__ float4 mul4(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
 __device__ __forceinline__ float max4(float m, float4 v) { return fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w)); }
+
+// every value has three bfloat16 parts (NaN, infinities and what rounds to one do not)
+__device__ __forceinline__ bool splits(float v) { return fabsf(v) <= 0x1.fep127f; }
+__device__ __forceinline__ bool splits4(float4 v) { return splits(v.x) && splits(v.y) && splits(v.z) && splits(v.w); }
 
 // alpha, EA, X: a wave per padded row (b, mp) - half a wave where a row is 128 cells, 32 lanes' worth;
 // rows and columns of the padding hold zeros.
@@ -307,21 +308,30 @@ __global__ __launch_bounds__(256) void k_bb_prep_a(const elem_t* __restrict__ a,
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     if (off < lpr) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  if (lane == 0) alpha[row] = mx;
+  bool bad = false;
   for (int k = lane * 4; k < Kp; k += step) {
     // (the fill -inf gives exp = 0 in the padding; a row of -inf has mx = -inf and NaN here, and is
     //  flagged by the pass that forms H)
     const float4 e = k < K ? exp4_st(ld4m(ar + k, K - k, -INFINITY), mx) : zero;
+    const float4 xv = (ur && k < K) ? mul4(e, ld4m(ur + k, K - k, 0.f)) : zero;
+    bad = bad || !splits4(xv);
     st4(er + k, e);
-    st4(xr + k, (ur && k < K) ? mul4(e, ld4m(ur + k, K - k, 0.f)) : zero);
+    st4(xr + k, xv);
   }
+  // (the flags are being cleared here: a row that does not split has no maximum, and the pass that
+  //  forms H flags its item)
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    if (off < lpr) bad = bad | (bool)__shfl_xor((int)bad, off, 64);
+  if (lane == 0) alpha[row] = bad ? NAN : mx;
 }
 
 // beta, EB, Y: a workgroup per (batch item, 64 columns): 16 lanes x 4 columns across, the 16 lane
 // groups of the four waves split the rows of b.
 __global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b, const elem_t* __restrict__ ub,
                                                    float* __restrict__ beta, float* __restrict__ eb,
-                                                   float* __restrict__ y, int K, int N, int Kp, int Np) {
+                                                   float* __restrict__ y, int* __restrict__ flags, int K, int N,
+                                                   int Kp, int Np) {
   __shared__ float part[16][64];
   const int cq = threadIdx.x & 15, rg = threadIdx.x >> 4;
   const int cblocks = Np / 64;
@@ -348,6 +358,7 @@ __global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b,
   float* ec = eb + batch * Kp * Np + n;
   float* yc = y + batch * Kp * Np + n;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  bool bad = false;
   for (int k = rg; k < Kp; k += 16) {
     const bool in = cnt > 0 && k < K;
     float4 e = zero;
@@ -356,9 +367,12 @@ __global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b,
       e = make_float4(exp_st(v.x - mx.x), cnt > 1 ? exp_st(v.y - mx.y) : 0.f, cnt > 2 ? exp_st(v.z - mx.z) : 0.f,
                       cnt > 3 ? exp_st(v.w - mx.w) : 0.f);
     }
+    const float4 yv = (uc && in) ? mul4(e, ld4m(uc + (long)k * N, cnt, 0.f)) : zero;
+    bad = bad || !splits4(yv);
     st4(ec + (long)k * Np, e);
-    st4(yc + (long)k * Np, (uc && in) ? mul4(e, ld4m(uc + (long)k * N, cnt, 0.f)) : zero);
+    st4(yc + (long)k * Np, yv);
   }
+  if (bad) flags[batch] = 1;
 }
 
 // R = exp(alpha + beta - out), H = g R over the padded (Mp, Np) grid (zeros in the padding), four
@@ -392,6 +406,7 @@ __global__ __launch_bounds__(256) void k_bb_prep_h(const elem_t* __restrict__ ou
         bad = bad || !(ex <= lim) || !(be[i] > -INFINITY);
         rv[i] = exp_st(ex);
         hv[i] = gv[i] * rv[i];
+        bad = bad || !splits(hv[i]);
       }
     if (bad) flags[batch] = 1;
   }
@@ -399,20 +414,20 @@ __global__ __launch_bounds__(256) void k_bb_prep_h(const elem_t* __restrict__ ou
   st4(h + bm * Np + n, make_float4(hv[0], hv[1], hv[2], hv[3]));
 }
 
-// One tile of C = P1 Q1 (+ P2 Q2) and its epilogue.  Operands are padded workspace arrays:
+// One tile of C = P1 Q1 (+ P2 Q2) and its epilogue; for a gradient also of C0 = P3 Q3.  Operands are padded workspace arrays:
 //   RT: the rows operand is stored [row][red] (staged transposed), else [red][row];
 //   CT: the columns operand is stored [col][red], else [red][col].
-constexpr int kEpiRaw = 0, kEpiT = 1, kEpiGrad = 2;
+constexpr int kEpiT = 0, kEpiGrad = 1;
 struct BBMM {
   const float* rows[2];
   const float* cols[2];
   int pairs;
+  const float* rows0;   // kEpiGrad: C0's operands, or NULL
+  const float* cols0;
   int Rp, Cp, Qp;       // padded extents: output rows, output columns, reduction
   // epilogue
-  float* raw;           // kEpiRaw: (B, Rp, Cp)
   const float* f_acc;   // kEpiT: R; kEpiGrad: EA / EB - the factor of the accumulator
-  const float* f1;      // kEpiGrad: X / Y or NULL ...
-  const float* f2;      //           ... times Ga0 / Gb0, added
+  const float* f0;      // kEpiGrad: X / Y, the factor of C0
   const float* h;       // kEpiT: H
   float* nht;           // kEpiT: -H t
   float* tt;            // kEpiT: t unrounded, (B, R, C) unpadded
@@ -420,16 +435,25 @@ struct BBMM {
   int R, C;             // true extents of the output
 };
 
+// The products run on the bf16 matrix instruction, every operand cut into three parts while it is staged
+// (split_bf16.h; logbmm_split.h has the staging and the inner loop): on the fp32 instruction, which does a
+// sixteenth of the reduction steps in the same time, the five launches of (512, 128^3) took 245 us; three-part
+// 240, and 205 with H EB^T and EA^T H formed in the launches that use them (a second set of accumulators)
+// instead of written out and read back.
+// Bound by what the workspace arrays move (two or four in, one to three more in the epilogue).
+using BBTile = MTile<128, 128, 2>;
 template <bool RT, bool CT, int EPI>
-__global__ __launch_bounds__(256) void k_bb_mm(const BBMM p) {
-  using T = MTile<128, 128>;
-  constexpr int NT = T::NT, LDR = T::LDR, LDC = T::LDC;
-  using SR = std::conditional_t<RT, StageT<T::TR, NT, LDR>, StageS<T::TR, NT, LDR>>;
-  using SC = std::conditional_t<CT, StageT<T::TC, NT, LDC>, StageS<T::TC, NT, LDC>>;
-  __shared__ __attribute__((aligned(16))) float smem[2 * kMS * (LDR + LDC)];
-  static_assert(2 * kMS * (LDR + LDC) >= (NT / 64) * kStripFloats, "");
-  float(*Rs)[kMS * LDR] = reinterpret_cast<float(*)[kMS * LDR]>(smem);
-  float(*Cs)[kMS * LDC] = reinterpret_cast<float(*)[kMS * LDC]>(smem + 2 * kMS * LDR);
+__global__ __launch_bounds__(BBTile::NT) __attribute__((amdgpu_waves_per_eu(BBTile::WPE, BBTile::WPE)))
+void k_bb_mm(const BBMM p) {
+  using T = BBTile;
+  constexpr int NT = T::NT;
+  using SR = std::conditional_t<RT, SplitT<T::TR, NT>, SplitS<T::TR, NT>>;
+  using SC = std::conditional_t<CT, SplitT<T::TC, NT>, SplitS<T::TC, NT>>;
+  constexpr int PER = 2;  // a thread's pieces of either operand: four steps of two lines, or two steps of four
+  __shared__ __attribute__((aligned(16))) unsigned smem[split_lds_words<SR, SC>()];
+  static_assert(split_lds_words<SR, SC>() >= (NT / 64) * kStripFloats, "");
+  auto Rs = [&](int buf) __attribute__((always_inline)) { return smem + buf * SR::BUF; };
+  auto Cs = [&](int buf) __attribute__((always_inline)) { return smem + 2 * SR::BUF + buf * SC::BUF; };
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr0 = (wave / T::WC) * 64, wc0 = (wave % T::WC) * 64;
@@ -439,56 +463,66 @@ __global__ __launch_bounds__(256) void k_bb_mm(const BBMM p) {
   const int r0 = (rem / tiles_c) * T::TR, c0 = (rem % tiles_c) * T::TC;
   const int Qp = p.Qp, slabs = Qp / kMS;
 
-  floatx16 acc[2][2];
+  floatx16 acc[2][2], acc0[2][2];
 #pragma unroll
   for (int x = 0; x < 4; ++x)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[x >> 1][x & 1][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[x >> 1][x & 1][i] = acc0[x >> 1][x & 1][i] = 0.f;
 
-  for (int pair = 0; pair < p.pairs; ++pair) {
-    const float* pr[SR::PER];
-    const float* pc[SC::PER];
-    const float* rbase = p.rows[pair] + (long)batch * p.Rp * Qp;
-    const float* cbase = p.cols[pair] + (long)batch * p.Cp * Qp;
+  // where this thread's pieces of the first slab lie in an operand of either layout
+  long ro[PER], co[PER];
 #pragma unroll
-    for (int l = 0; l < SR::PER; ++l) {
-      if constexpr (RT) pr[l] = rbase + (long)(r0 + SR::line(tid, l)) * Qp + SR::quad(tid) * 4;
-      else pr[l] = rbase + (long)SR::red(tid, l) * p.Rp + r0 + SR::quad(tid) * 4;
+  for (int l = 0; l < PER; ++l) {
+    if constexpr (RT) ro[l] = ((long)batch * p.Rp + r0 + SR::line(tid, l)) * Qp + SR::quad(tid) * 4;
+    else ro[l] = ((long)batch * Qp + 2 * SR::pair(tid) + l) * p.Rp + r0 + SR::line0(tid);
+    if constexpr (CT) co[l] = ((long)batch * p.Cp + c0 + SC::line(tid, l)) * Qp + SC::quad(tid) * 4;
+    else co[l] = ((long)batch * Qp + 2 * SC::pair(tid) + l) * p.Cp + c0 + SC::line0(tid);
+  }
+  // the slabs of both products are one loop: the second's first slab is in flight under the first's last
+  const float *rb = p.rows[0], *cb = p.cols[0];
+  const long rstep = RT ? (long)kMS : (long)kMS * p.Rp, cstep = CT ? (long)kMS : (long)kMS * p.Cp;
+  int s_load = 0;
+  float4 rr[PER], rc[PER];
+  auto load = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int l = 0; l < PER; ++l) {
+      rr[l] = ld4a(rb + ro[l]);
+      rc[l] = ld4a(cb + co[l]);
     }
-#pragma unroll
-    for (int l = 0; l < SC::PER; ++l) {
-      if constexpr (CT) pc[l] = cbase + (long)(c0 + SC::line(tid, l)) * Qp + SC::quad(tid) * 4;
-      else pc[l] = cbase + (long)SC::red(tid, l) * p.Cp + c0 + SC::quad(tid) * 4;
+    rb += rstep;
+    cb += cstep;
+    if (++s_load == slabs) {  // uniform
+      rb = p.rows[1];
+      cb = p.cols[1];
     }
-    float4 rr[SR::PER], rc[SC::PER];
-    auto load = [&]() __attribute__((always_inline)) {
+  };
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+    if constexpr (RT) {
 #pragma unroll
-      for (int l = 0; l < SR::PER; ++l) {
-        rr[l] = ld4a(pr[l]);
-        pr[l] += RT ? (long)kMS : (long)kMS * p.Rp;
-      }
+      for (int l = 0; l < PER; ++l) SR::put(Rs(buf), tid, l, rr[l]);
+    } else {
+      SR::put(Rs(buf), tid, rr[0], rr[1]);
+    }
+    if constexpr (CT) {
 #pragma unroll
-      for (int l = 0; l < SC::PER; ++l) {
-        rc[l] = ld4a(pc[l]);
-        pc[l] += CT ? (long)kMS : (long)kMS * p.Cp;
-      }
-    };
-    auto stage = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-      for (int l = 0; l < SR::PER; ++l) SR::put(Rs[buf], tid, l, rr[l]);
-#pragma unroll
-      for (int l = 0; l < SC::PER; ++l) SC::put(Cs[buf], tid, l, rc[l]);
-    };
+      for (int l = 0; l < PER; ++l) SC::put(Cs(buf), tid, l, rc[l]);
+    } else {
+      SC::put(Cs(buf), tid, rc[0], rc[1]);
+    }
+  };
+  load();
+  stage(0);
+  split_loop(slabs * p.pairs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
+    split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
+  });
+  if (EPI == kEpiGrad && p.rows0) {  // uniform
+    rb = p.rows0;
+    cb = p.cols0;
     load();
     stage(0);
-    __syncthreads();
-    for (int s = 0; s < slabs; ++s) {
-      const bool more = s + 1 < slabs;
-      if (more) load();
-      mfma_slab<LDR, LDC>(Rs[s & 1], Cs[s & 1], wr0, wc0, lane, acc);
-      if (more) stage((s + 1) & 1);
-      __syncthreads();
-    }
+    split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
+      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc0);
+    });
   }
 
   // epilogue, row-wise: f(q, t, v) = four columns lc .. lc + 3 of block row 16 q + 4 t + lr
@@ -496,33 +530,41 @@ __global__ __launch_bounds__(256) void k_bb_mm(const BBMM p) {
   const int row0 = r0 + wr0 + lr, col = c0 + wc0 + lc;
   const long pbase = ((long)batch * p.Rp + row0) * p.Cp + col;   // padded arrays
   const int cc = clamp4(p.C - col);                              // columns of the piece that exist
-  acc_rows(acc, smem + wave * kStripFloats, lane, [](int) {},
-           [&](int q, int t, float4 v) __attribute__((always_inline)) {
-             const int ru = 16 * q + 4 * t;
-             const long pu = pbase + (long)ru * p.Cp;
-             const bool live = row0 + ru < p.R && cc > 0;
-             const long du = ((long)batch * p.R + row0 + ru) * p.C + col;  // unpadded arrays
-             if constexpr (EPI == kEpiRaw) {
-               st4a(p.raw + pu, v);
-             } else if constexpr (EPI == kEpiT) {
+  float* strip = reinterpret_cast<float*>(smem) + wave * kStripFloats;
+  if constexpr (EPI == kEpiT) {
+    acc_rows(acc, strip, lane, [](int) {},
+             [&](int q, int t, float4 v) __attribute__((always_inline)) {
+               const int ru = 16 * q + 4 * t;
+               const long pu = pbase + (long)ru * p.Cp;
+               const long du = ((long)batch * p.R + row0 + ru) * p.C + col;  // unpadded arrays
                const float4 rv = ld4a(p.f_acc + pu), hv = ld4a(p.h + pu);
                const float4 tv = make_float4(rv.x * v.x, rv.y * v.y, rv.z * v.z, rv.w * v.w);
                st4a(p.nht + pu, make_float4(-hv.x * tv.x, -hv.y * tv.y, -hv.z * tv.z, -hv.w * tv.w));
-               if (live) {
+               if (row0 + ru < p.R && cc > 0) {
                  st4m(p.tt + du, cc, tv);
                  if constexpr (!kElemF32) st4m(p.dst + du, cc, tv);
                }
-             } else {
-               const float4 fa = ld4a(p.f_acc + pu);
-               float4 o = make_float4(fa.x * v.x, fa.y * v.y, fa.z * v.z, fa.w * v.w);
-               if (p.f1) {
-                 const float4 x1 = ld4a(p.f1 + pu), x2 = ld4a(p.f2 + pu);
-                 o = make_float4(__builtin_fmaf(x1.x, x2.x, o.x), __builtin_fmaf(x1.y, x2.y, o.y),
-                                 __builtin_fmaf(x1.z, x2.z, o.z), __builtin_fmaf(x1.w, x2.w, o.w));
-               }
-               if (live) st4m(p.dst + du, cc, o);
-             }
-           });
+             });
+  } else {
+    // C0 scaled by its factor first, kept in registers as rows; then the other product joins it
+    float4 o[16];
+    if (p.rows0)
+      acc_rows(acc0, strip, lane, [](int) {}, [&](int q, int t, float4 v) __attribute__((always_inline)) {
+        const float4 x = ld4a(p.f0 + pbase + (long)(16 * q + 4 * t) * p.Cp);
+        o[4 * q + t] = make_float4(x.x * v.x, x.y * v.y, x.z * v.z, x.w * v.w);
+      });
+    else
+#pragma unroll
+      for (int x = 0; x < 16; ++x) o[x] = make_float4(0.f, 0.f, 0.f, 0.f);
+    acc_rows(acc, strip, lane, [](int) {}, [&](int q, int t, float4 v) __attribute__((always_inline)) {
+      const int ru = 16 * q + 4 * t;
+      const float4 fa = ld4a(p.f_acc + pbase + (long)ru * p.Cp), c0v = o[4 * q + t];
+      if (row0 + ru < p.R && cc > 0)
+        st4m(p.dst + ((long)batch * p.R + row0 + ru) * p.C + col, cc,
+             make_float4(__builtin_fmaf(fa.x, v.x, c0v.x), __builtin_fmaf(fa.y, v.y, c0v.y),
+                         __builtin_fmaf(fa.z, v.z, c0v.z), __builtin_fmaf(fa.w, v.w, c0v.w)));
+    });
+  }
 }
 
 template <bool RT, bool CT, int EPI>
@@ -541,7 +583,7 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
     hipLaunchKernelGGL(k_bb_prep_a, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3(256), 0, s, p.a, p.ua, w.alpha, w.ea,
                        w.x, w.flags, M, K, Mp, Kp, rows);
     hipLaunchKernelGGL(k_bb_prep_b, dim3((unsigned)(B * (Np / 64))), dim3(256), 0, s, p.b, p.ub, w.beta, w.eb, w.y,
-                       K, N, Kp, Np);
+                       w.flags, K, N, Kp, Np);
     const long quads = (long)B * Mp * (Np / 4);
     hipLaunchKernelGGL(k_bb_prep_h, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, p.out, p.g, w.alpha,
                        w.beta, w.r, w.h, w.flags, M, N, Mp, Np, quads);
@@ -557,34 +599,24 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
     q.f_acc = w.r; q.h = w.h; q.nht = w.nht; q.tt = p.tt; q.dst = p.gg;
     if (int e = launch_mm<true, false, kEpiT>(q, B, s)) return e;
   }
-  if (has_a) {  // Ga0 = H EB^T
-    BBMM q{};
-    q.rows[0] = w.h; q.cols[0] = w.eb; q.pairs = 1;
-    q.Rp = Mp; q.Cp = Kp; q.Qp = Np; q.R = M; q.C = K; q.raw = w.ga0;
-    if (int e = launch_mm<true, true, kEpiRaw>(q, B, s)) return e;
-  }
-  {  // grad_a = X Ga0 + EA (H Y^T - (H t) EB^T)
+  {  // grad_a = X (H EB^T) + EA (H Y^T - (H t) EB^T)
     BBMM q{};
     int n = 0;
     if (has_b) { q.rows[n] = w.h; q.cols[n] = w.y; ++n; }
     q.rows[n] = w.nht; q.cols[n] = w.eb; ++n;
     q.pairs = n; q.Rp = Mp; q.Cp = Kp; q.Qp = Np; q.R = M; q.C = K;
-    q.f_acc = w.ea; q.f1 = has_a ? w.x : nullptr; q.f2 = w.ga0; q.dst = p.ga;
+    q.f_acc = w.ea; q.dst = p.ga;
+    if (has_a) { q.rows0 = w.h; q.cols0 = w.eb; q.f0 = w.x; }
     if (int e = launch_mm<true, true, kEpiGrad>(q, B, s)) return e;
   }
-  if (has_b) {  // Gb0 = EA^T H
-    BBMM q{};
-    q.rows[0] = w.ea; q.cols[0] = w.h; q.pairs = 1;
-    q.Rp = Kp; q.Cp = Np; q.Qp = Mp; q.R = K; q.C = N; q.raw = w.gb0;
-    if (int e = launch_mm<false, false, kEpiRaw>(q, B, s)) return e;
-  }
-  {  // grad_b = Y Gb0 + EB (X^T H - EA^T (H t))
+  {  // grad_b = Y (EA^T H) + EB (X^T H - EA^T (H t))
     BBMM q{};
     int n = 0;
     if (has_a) { q.rows[n] = w.x; q.cols[n] = w.h; ++n; }
     q.rows[n] = w.ea; q.cols[n] = w.nht; ++n;
     q.pairs = n; q.Rp = Kp; q.Cp = Np; q.Qp = Mp; q.R = K; q.C = N;
-    q.f_acc = w.eb; q.f1 = has_b ? w.y : nullptr; q.f2 = w.gb0; q.dst = p.gb;
+    q.f_acc = w.eb; q.dst = p.gb;
+    if (has_b) { q.rows0 = w.ea; q.cols0 = w.h; q.f0 = w.y; }
     if (int e = launch_mm<false, false, kEpiGrad>(q, B, s)) return e;
   }
   // items beyond the guard: the exact passes, on those items only

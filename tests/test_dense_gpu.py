@@ -1465,3 +1465,28 @@ def test_second_order_is_one_library_call(gpu, monkeypatch, banded):
     second = torch.autograd.grad(first, (a, b, g), (torch.randn_like(a), torch.randn_like(b)))
     assert names == ["genbmm_banded_bwdbwd" if banded else "genbmm_logbmm_bwdbwd_ws"]
     assert all(bool(torch.isfinite(t).all()) for t in second)
+
+
+# an infinite and a huge cotangent, an infinite incoming gradient: such an item has no three-part factors
+@pytest.mark.parametrize("B,M,K,N", [(5, 128, 128, 128), (4, 130, 129, 200), (6, 64, 150, 101)])
+def test_logbmm_double_backward_of_infinite_operands(gpu, B, M, K, N):
+    """The factored double backward (three-part products) against the exact passes (no workspace): items
+    with a cotangent or gradient that has no three bfloat16 parts take the exact passes bit for bit, the
+    others agree to fp32 sums of at most 256 products (1e-5 of the largest)."""
+    lib = _lib.load()
+    torch.manual_seed(N)
+    a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
+    ua, ub = torch.randn(B, M, K), torch.randn(B, K, N)
+    # (3.4e38 rounds to an infinite bfloat16; the column's largest b has the factor 1)
+    ua[0, 3, 5], ub[1, :, 2], g[2, 11, 13] = float("inf"), 3.4e38, -float("inf")
+    special = 3
+    out = genbmm.logbmm(a.to(gpu), b.to(gpu))
+    x = [t.to(gpu).contiguous() for t in (a, b)] + [out] + [t.to(gpu).contiguous() for t in (g, ua, ub)]
+    p, s = _lib.ptr, _lib.stream_of(out)
+    ws = torch.full((lib.genbmm_logbmm_bwdbwd_ws_size(B, M, K, N),), float("nan"), device=gpu)
+    got, want = ([torch.empty_like(t) for t in (x[0], x[1], x[3])] for _ in range(2))
+    assert lib.genbmm_logbmm_bwdbwd_ws(*(p(t) for t in x), *(p(t) for t in got), p(ws), B, M, K, N, s) == 0
+    assert lib.genbmm_logbmm_bwdbwd(*(p(t) for t in x), *(p(t) for t in want), B, M, K, N, s) == 0
+    for u, w in zip(got, want):
+        assert torch.equal(u[:special].nan_to_num(7.0), w[:special].nan_to_num(7.0))   # (bits of a NaN apart)
+        assert float((u[special:] - w[special:]).abs().max()) <= 1e-5 * max(1.0, float(w[special:].abs().max()))
