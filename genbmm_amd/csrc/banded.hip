@@ -107,12 +107,18 @@ inline void launch_max_fwd(const BandArgs& p, int B, hipStream_t s) {
   const int Wseg = max_fwd_segment(p), nseg = ceil_div(p.Wo, Wseg);
   const MaxDims d = max_dims(p.Wa, p.Wb, Wseg);
   const int strips = ceil_div(p.n, kMaxRows);
-  if (d.bytes > kStripLdsLimit)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_max_fwd),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)d.bytes);
   const long rows = (long)B * p.n;
-  hipLaunchKernelGGL(k_band_max_fwd, dim3((unsigned)((long)B * strips * nseg)), dim3(256), d.bytes, s, p, strips, d,
-                     rows * p.Wa, rows * p.Wb, nseg, Wseg);
+  auto go = [&](auto kernel) {
+    if (d.bytes > kStripLdsLimit)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)d.bytes);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((long)B * strips * nseg)), dim3(256), d.bytes, s, p, strips, d,
+                       rows * p.Wa, rows * p.Wb, nseg, Wseg);
+  };
+  // The pairs' end costs a cell about eleven instructions: 33 diagonals each (64 x 4096) 87.4 -> 83-85.5 us in
+  // pairs, 17 diagonals each 45.1 -> 46.0
+  if (min(p.Wa, p.Wb) >= 24) go(k_band_max_fwd<true>);
+  else go(k_band_max_fwd<false>);
 }
 
 inline void launch_prep(const BandArgs& p, const elem_t* a, int a_lu, const elem_t* b, int b_lu, int B,

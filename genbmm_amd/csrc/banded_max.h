@@ -47,6 +47,13 @@ inline MaxDims max_dims(int Wa, int Wb, int Wo) {
   return d;
 }
 
+// PAIRS: the walk takes two k at a time - their sums and the running maximum meet in one three-operand
+// maximum, and one compare and one select keep the pair that raised it last: 2.5 instructions per term
+// instead of 4 - and which k of its pair it was is found behind the walk, by forming the first one's sum
+// again.  The first pair that attains the maximum and the first k inside it are what the walk with a
+// strict comparison keeps.  What is left is bound by the LDS reads (nine values per eight terms): 64 x 4096,
+// 65 diagonals each 281 -> 273 us, 16 x 4096, 129 diagonals each 536 -> 499.
+template <bool PAIRS>
 __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int strips, const MaxDims d,
                                                          long cells_a, long cells_b, int nseg, int Wseg) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -127,6 +134,11 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
         // all 8 cells walk the union of their k ranges: where a cell has no such k it reads
         // -inf from between the rows
         const int klo = max(0, j0 - (Wb - 1)), khi = min(Wa - 1, j0 + 7);
+        auto fold2 = [&](int t, float a0, float a1, float b0, float b1, int k) __attribute__((always_inline)) {
+          const float m = __builtin_fmaxf(__builtin_fmaxf(val[s][t], a0 + b0), a1 + b1);
+          if (m > val[s][t]) ind[s][t] = k;
+          val[s][t] = m;
+        };
         int k = klo;
         for (; k + 3 <= khi; k += 4) {
           float av[4], bv[4][8];
@@ -137,14 +149,36 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
             for (int t = 0; t < 8; ++t) bv[u][t] = bp[t * dt + k + u];
           }
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
+          for (int u = 0; u < 4; u += 2)
 #pragma unroll
-            for (int t = 0; t < 8; ++t) fold(t, av[u], bv[u][t], k + u);
+            for (int t = 0; t < 8; ++t) {
+              if (PAIRS) {
+                fold2(t, av[u], av[u + 1], bv[u][t], bv[u + 1][t], k + u);
+              } else {
+                fold(t, av[u], bv[u][t], k + u);
+                fold(t, av[u + 1], bv[u + 1][t], k + u + 1);
+              }
+            }
         }
         for (; k <= khi; ++k) {
           const float av = ap[k];
 #pragma unroll
           for (int t = 0; t < 8; ++t) fold(t, av, bp[t * dt + k], k);
+        }
+        if (PAIRS) {  // which k of its pair: the first whose sum is the maximum
+          bool zero = false;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            const int at = max(ind[s][t], klo);  // (no term: any cell)
+            const bool second = ap[at] + bp[t * dt + at] != val[s][t];
+            ind[s][t] += ind[s][t] >= 0 && second;
+            zero |= val[s][t] == 0.f;
+          }
+          if (zero) {  // +0 and -0 compare equal: the value is the term's
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              if (val[s][t] == 0.f) val[s][t] = ap[ind[s][t]] + bp[t * dt + ind[s][t]];
+          }
         }
       } else if (x < n) {
         // the reference's k range per cell (k2 in [0, Wb), dense row i + k - lu_a in [0, n))

@@ -6,7 +6,8 @@ import torch
 import oracle
 import genbmm_amd as genbmm
 from genbmm_amd import _lib
-from genbmm_amd.sparse import BandedMatrix, banddiag
+from genbmm_amd.sparse import MODE_MAX, BandedMatrix, banddiag
+from genbmm_amd.sparse import _forward as band_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -461,3 +462,30 @@ def test_banded_argmax_backward_sums_in_order(gpu, n, a_lu, a_ld, b_lu, b_ld):
         wa, wb = oracle.seq_band_bwd(X.data.detach().float().cpu(), a_lu, a_ld, Y.data.detach().float().cpu(), b_lu, b_ld,
                                      gd.float(), 1, dtype=np.float32)
         assert torch.equal(ga.cpu(), wa.to(dt)) and torch.equal(gb.cpu(), wb.to(dt)), dt
+
+
+# min(Wa, Wb) 23 and 24 are either side of the walk in pairs; odd numbers of terms, bands of two segments
+@pytest.mark.parametrize("n,a_lu,a_ld,b_lu,b_ld", [
+    (200, 11, 11, 12, 12), (200, 12, 11, 11, 12), (260, 12, 12, 20, 13), (259, 32, 32, 32, 32), (330, 45, 40, 41, 44)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_banded_max_of_special_values(gpu, n, a_lu, a_ld, b_lu, b_ld, dt):
+    """Values (bit patterns) and indices of the band max product beside the sequential oracle's: ties, zeros of
+    both signs, infinities, NaN and sums at and below the floor."""
+    torch.manual_seed(n + a_lu)
+    a, b = pair(n, a_lu, a_ld, b_lu, b_ld, mk=grid)
+    a, b = (torch.where(torch.rand(t.shape) < 0.3, -0.0, t).clamp(max=0) for t in (a, b))   # -0 ties +0 at the top
+    for t in (a, b):
+        r = torch.rand(t.shape)
+        t[r < 0.02] = 0.0
+        t[(r >= 0.02) & (r < 0.03)] = float("nan")
+        t[(r >= 0.03) & (r < 0.04)] = -float("inf")
+        t[(r >= 0.04) & (r < 0.0405)] = float("inf")
+        t[(r >= 0.05) & (r < 0.06)] = -1e9
+    a[:, 70:90] = -2e9                       # rows without a term above the floor
+    a, b = a.to(dt), b.to(dt)
+    X, Y = BandedMatrix(a.to(gpu), a_lu, a_ld), BandedMatrix(b.to(gpu), b_lu, b_ld)
+    _, _, out, idx = band_forward(X.data, a_lu, a_ld, Y.data, b_lu, b_ld, MODE_MAX)
+    want, widx, _ = oracle.seq_band_fwd(a.float(), a_lu, a_ld, b.float(), b_lu, b_ld, 1, dtype=np.float32)
+    bits = torch.int32 if dt == torch.float32 else torch.int16
+    assert torch.equal(out.cpu().view(bits), want.to(dt).view(bits))
+    assert torch.equal(idx.cpu().long(), widx.long())
