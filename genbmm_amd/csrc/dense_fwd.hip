@@ -136,16 +136,26 @@ __global__ __launch_bounds__(C::NT) void k_max_fwd(const DenseArgs p) {
 // ahead are requested before the current rows are finished and stored.
 //
 // Op supplies what differs: Extra load(e) (read together with the code of cell e),
-// none(e) (a cell whose code is -1) and cell(e, kb, av, br, stride, valid, extra) with
-// av[j] = first operand at k = kb + j, br[j * stride] = second operand, valid = number
-// of terms of the group that lie inside K.
+// none(e) (a cell whose code is -1) and cell<TAIL>(e, kb, av, br, stride, low, valid, extra) with
+// av[j] = first operand at k = kb + j, br[j * stride] = second operand; the group's terms are
+// low <= j < valid.
+//
+// TAIL: kWhole - K is a multiple of the group; kRagged - the last group is cut at K and its terms are taken
+// from the last G of K, those of the group before left out; kShort - K is less than a group, read term by
+// term.  Only kShort knows the number of terms at run time: elsewhere the G values of the second operand
+// are at fixed distances, which the LDS reads carry as immediates.  Bound by the gathers of the first
+// operand: a ragged K's values read one by one (before) against four at a time, forward and draw of
+// (100,500,300,510) 1015 -> 705 us, maxbmm forward (512,127,129,131) 223 -> 185, (64,500,301,510) 394 -> 338;
+// the immediates alone, (256,256^3) 280 -> 273.
 constexpr int kResGroup = 8, kResWaves = 8, kResRows = 4, kResStage = 8;
 constexpr int kResFloats = 16384;  // 64 KB of LDS
 static_assert(kMaxGroup == kResGroup, "");
+enum ResTail { kWhole, kRagged, kShort };
+inline ResTail resolve_tail(int K, int group) { return K % group == 0 ? kWhole : K > group ? kRagged : kShort; }
 
 // E: element type of the two operands (the caller's for max / prod-max, fp32 for the
 // factors the sampling sweep runs on).
-template <int COLS, bool TAIL, int G, int R, class E, class Op>
+template <int COLS, ResTail TAIL, int G, int R, class E, class Op>
 __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const E* __restrict__ second,
                                              int32_t* __restrict__ idx, Op& op, int M, int K, int N,
                                              int panels, int row_chunks, int rows_per, float* Bs) {
@@ -192,9 +202,9 @@ __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const 
       const int k = (-2 - code[r]) * G;
       const bool act = code[r] <= -2 && k >= kc && k < kc + KSTAGE;
       kb[r] = act ? k : -1;
-      const int ks = act ? k : kc;
+      const int ks = TAIL == kRagged ? min(act ? k : kc, K - G) : act ? k : kc;
       const E* ar = ab + (long)min(row_of(mb, r), M - 1) * K + ks;
-      if (!TAIL) {
+      if (TAIL != kShort) {
 #pragma unroll
         for (int q = 0; q < G / 4; ++q) {
           const float4 x = ld4(ar + 4 * q);
@@ -206,23 +216,22 @@ __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const 
       }
     }
   };
-  auto finish = [&](int mb, int kc, int rows, const int (&code)[R], const Extra (&ex)[R],
+  auto finish = [&](int mb, int kc, int kb_staged, const int (&code)[R], const Extra (&ex)[R],
                     const int (&kb)[R], const float (&av)[R][G]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const long e = cell0 + (long)row_of(mb, r) * N + n;
       if (code[r] == -1 && kc == 0) op.none(e);
       if (kb[r] < 0) continue;
-      const int rel = kb[r] - kc;
-      // the last group of a ragged K: its rows past K are not staged; point at row rows - 1
-      const float* br = Bs + rel * COLS + col;
-      const int valid = TAIL ? min(G, K - kb[r]) : G;
-      op.cell(e, kb[r], av[r], br, COLS, valid, min(G, rows - rel), ex[r]);
+      const int k0 = TAIL == kRagged ? min(kb[r], K - G) : kb[r];
+      op.template cell<TAIL>(e, k0, av[r], Bs + (k0 - kb_staged) * COLS + col, COLS, kb[r] - k0,
+                             TAIL == kShort ? K : G, ex[r]);
     }
   };
 
   for (int kc = 0; kc < K; kc += KSTAGE) {
-    const int rows = min(KSTAGE, K - kc);
+    // (the last of a ragged K: KSTAGE rows where there are that many, its last group reaches back)
+    const int ks = TAIL == kRagged ? min(kc, max(0, K - KSTAGE)) : kc, rows = min(KSTAGE, K - ks);
     int mb = m_beg + wave * R * RPW;
     int c0[R], c1[R], kb0[R];
     Extra e0[R], e1[R];
@@ -233,7 +242,7 @@ __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const 
       float x[kResStage];
 #pragma unroll
       for (int u = 0; u < kResStage; ++u)
-        x[u] = bb[(long)(kc + min(r0 + u * kResWaves * RPW, rows - 1)) * N + nc];
+        x[u] = bb[(long)(ks + min(r0 + u * kResWaves * RPW, rows - 1)) * N + nc];
 #pragma unroll
       for (int u = 0; u < kResStage; ++u)
         if (r0 + u * kResWaves * RPW < rows) Bs[(r0 + u * kResWaves * RPW) * COLS + col] = x[u];
@@ -247,7 +256,7 @@ __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const 
       float a1[R][G];
       gather(mb + STEP, kc, c1, kb1, a1);
       load_codes(mb + 2 * STEP, c2, e2);
-      finish(mb, kc, rows, c0, e0, kb0, a0);
+      finish(mb, kc, ks, c0, e0, kb0, a0);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         c0[r] = c1[r]; c1[r] = c2[r];
@@ -293,15 +302,16 @@ struct MaxResolve {
       fb[e] = 0.f;
     }
   }
+  template <ResTail TAIL>
   __device__ __forceinline__ void cell(long e, int kb, const float (&av)[kResGroup], const float* br,
-                                       int stride, int valid, int staged, Extra) const {
+                                       int stride, int low, int valid, Extra) const {
     constexpr int G = kResGroup;
     float t[G], bv[G];
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      bv[j] = br[min(j, staged - 1) * stride];
+      bv[j] = br[(TAIL == kShort ? min(j, valid - 1) : j) * stride];
       t[j] = PROD ? av[j] * bv[j] : av[j] + bv[j];
-      if (j >= valid) t[j] = -INFINITY;
+      if ((TAIL == kRagged && j < low) || (TAIL == kShort && j >= valid)) t[j] = -INFINITY;
     }
     float v = __builtin_fmaxf(__builtin_fmaxf(t[0], t[1]), t[2]);
     v = __builtin_fmaxf(__builtin_fmaxf(v, t[3]), t[4]);
@@ -331,8 +341,7 @@ struct MaxResolve {
   }
 };
 
-// TAIL: K is not a multiple of the group, the last group is cut at K.
-template <bool PROD, int COLS, bool TAIL>
+template <bool PROD, int COLS, ResTail TAIL>
 __global__ __launch_bounds__(kResWaves * 64, 4) void k_max_resolve(
     const elem_t* __restrict__ a, const elem_t* __restrict__ b, elem_t* __restrict__ out,
     int32_t* __restrict__ idx, float* __restrict__ fac_a, float* __restrict__ fac_b, int M, int K,
@@ -577,20 +586,22 @@ struct SampleResolve {
   int K;
   __device__ __forceinline__ float load(long e) const { return rem[e]; }
   __device__ __forceinline__ void none(long) const {}
+  template <ResTail TAIL>
   __device__ __forceinline__ void cell(long e, int kb, const float (&av)[G], const float* br, int stride,
-                                       int valid, int staged, float r) const {
+                                       int low, int valid, float r) const {
     uint32_t past = 0u;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      const float ea = j < valid ? av[j] : 0.f;
-      r = __builtin_fmaf(-ea, br[min(j, staged - 1) * stride], r);
+      const bool out = (TAIL == kRagged && j < low) || (TAIL == kShort && j >= valid);
+      const float ea = out ? 0.f : av[j];
+      r = __builtin_fmaf(-ea, br[(TAIL == kShort ? min(j, valid - 1) : j) * stride], r);
       past = __builtin_amdgcn_alignbit(past, __float_as_uint(r), 31);
     }
     idx[e] = min(kb + G - __builtin_popcount(past), K - 1);
   }
 };
 
-template <int COLS, bool TAIL, int G>
+template <int COLS, ResTail TAIL, int G>
 __global__ __launch_bounds__(kResWaves * 64, 4) void k_sample_resolve(
     const float* __restrict__ ea, const float* __restrict__ eb, const float* __restrict__ remw,
     int32_t* __restrict__ idx, int* __restrict__ valid, int M, int K, int N, int panels,
@@ -621,13 +632,14 @@ int launch_max(DenseArgs p, float* factors, int B, int M, int K, int N, hipStrea
     hipLaunchKernelGGL(kernel, dim3(rgrid), dim3(kResWaves * 64), 0, s, p.a, p.b, p.out, p.idx, fa, fb,
                        M, K, N, panels, row_chunks, rows_per);
   };
-  const bool tail = K % kMaxGroup != 0;
+  const ResTail tail = resolve_tail(K, kMaxGroup);
   if (cols == 64) {
-    if (tail) go(k_max_resolve<PROD, 64, true>);
-    else go(k_max_resolve<PROD, 64, false>);
+    if (tail == kWhole) go(k_max_resolve<PROD, 64, kWhole>);
+    else if (tail == kRagged) go(k_max_resolve<PROD, 64, kRagged>);
+    else go(k_max_resolve<PROD, 64, kShort>);
   } else {
-    if (tail) go(k_max_resolve<PROD, 32, true>);
-    else go(k_max_resolve<PROD, 32, false>);
+    if (tail == kWhole) go(k_max_resolve<PROD, 32, kWhole>);
+    else go(k_max_resolve<PROD, 32, kRagged>);  // K > 256
   }
   return launch_status();
 }
@@ -860,13 +872,14 @@ int launch_sample_resolve(DenseArgs p, const LogFactors& f, int B, int M, int K,
     hipLaunchKernelGGL(kernel, dim3(rgrid), dim3(kResWaves * 64), 0, s, f.ea, f.eb, f.scratch, p.idx,
                        f.valid, M, K, N, panels, row_chunks, rows_per);
   };
-  const bool tail = K % G != 0;
+  const ResTail tail = resolve_tail(K, G);
   if (cols == 64) {
-    if (tail) go(k_sample_resolve<64, true, G>);
-    else go(k_sample_resolve<64, false, G>);
+    if (tail == kWhole) go(k_sample_resolve<64, kWhole, G>);
+    else if (tail == kRagged) go(k_sample_resolve<64, kRagged, G>);
+    else go(k_sample_resolve<64, kShort, G>);
   } else {
-    if (tail) go(k_sample_resolve<32, true, G>);
-    else go(k_sample_resolve<32, false, G>);
+    if (tail == kWhole) go(k_sample_resolve<32, kWhole, G>);
+    else go(k_sample_resolve<32, kRagged, G>);  // K > 256
   }
   return launch_status();
 }

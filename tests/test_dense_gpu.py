@@ -1490,3 +1490,39 @@ def test_logbmm_double_backward_of_infinite_operands(gpu, B, M, K, N):
     for u, w in zip(got, want):
         assert torch.equal(u[:special].nan_to_num(7.0), w[:special].nan_to_num(7.0))   # (bits of a NaN apart)
         assert float((u[special:] - w[special:]).abs().max()) <= 1e-5 * max(1.0, float(w[special:].abs().max()))
+
+
+# the group that ends a ragged K (8 terms of a maximum, 16 of a draw), one row past it, one short of it, a K
+# below one group, and K past the rows staged at a time (256 rows of 64 columns, 512 of 32)
+@pytest.mark.parametrize("K", [1, 7, 9, 15, 23, 173, 249, 257, 259, 511, 513, 519, 530, 1025])
+@pytest.mark.parametrize("name,dt", [("maxbmm", torch.float32), ("prodmaxbmm", torch.float32), ("maxbmm", torch.bfloat16)])
+def test_max_products_of_ragged_reductions(gpu, K, name, dt):
+    """Value and index of the largest term, bit for bit: ties, zeros of both signs, NaN and -inf."""
+    torch.manual_seed(K)
+    a, b = (torch.round(torch.randn(*s) * 4) / 4 for s in ((3, 70, K), (3, K, 67)))
+    for t in (a, b):
+        r = torch.rand(t.shape)
+        t[r < 0.01], t[(r > 0.02) & (r < 0.03)], t[(r > 0.04) & (r < 0.2)] = float("nan"), -float("inf"), -0.0
+    a, b = a.to(dt), b.to(dt)
+    out, idx = genmul._max_forward(a.to(gpu), b.to(gpu), name == "prodmaxbmm",
+                                   torch.empty(2, 3, 70, 67, device=gpu) if name == "prodmaxbmm" else None)
+    want, widx = oracle.seq_maxbmm_fwd(a.float(), b.float(), name == "prodmaxbmm")
+    bits = torch.int32 if dt == torch.float32 else torch.int16
+    assert torch.equal(out.cpu().view(bits), want.to(dt).view(bits))
+    assert torch.equal(idx.cpu(), widx)
+
+
+@pytest.mark.parametrize("B,M,K,N", [(2, 130, 17, 140), (4, 256, 300, 260), (3, 200, 515, 130), (8, 130, 700, 300)])
+def test_draws_of_ragged_reductions(gpu, B, M, K, N):
+    """A reduction whose last 16 terms are not whole draws what the same reduction draws with terms of no mass
+    behind it: the sums of every group, and so the crossings, are the same numbers."""
+    torch.manual_seed(K)
+    a, b = 2 * torch.randn(B, M, K, device=gpu), 2 * torch.randn(B, K, N, device=gpu)
+    pad = -K % 16
+    a2 = torch.cat((a, torch.full((B, M, pad), -1e4, device=gpu)), 2)
+    b2 = torch.cat((b, torch.full((B, pad, N), -50.0, device=gpu)), 1)
+    grads = []
+    for x, y in ((a, b), (a2, b2)):
+        x, y = x.requires_grad_(), y.requires_grad_()
+        grads.append(torch.autograd.grad(genbmm.samplebmm(x, y, stream=(7, 0)).sum(), (x, y)))
+    assert torch.equal(grads[0][0], grads[1][0][:, :, :K]) and torch.equal(grads[0][1], grads[1][1][:, :K])
