@@ -705,10 +705,35 @@ struct SplitBwd {
   static constexpr int WORDS = split_lds_words<SR, SC>();
 };
 
-//
+// One cell of a gradient on plain fp32 products, a lane by itself: (r, c) = (m, k) of grad_a, (k, n) of grad_b.
+// The sum ends where it is NaN for good.
+template <bool GRAD_A, bool RECIP, class W_t>
+__device__ __forceinline__ float log_bwd_cell(const elem_t* __restrict__ ab, const elem_t* __restrict__ bb,
+                                              const W_t* __restrict__ wb, const elem_t* __restrict__ gb,
+                                              const float* __restrict__ al, const float* __restrict__ be, int M, int K,
+                                              int N, int r, int c) {
+  const int Q = GRAD_A ? N : M;
+  float s = 0.f;
+  for (int q0 = 0; q0 < Q && s == s; q0 += 16) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int q = min(q0 + u, Q - 1), m = GRAD_A ? r : q, n = GRAD_A ? q : c;
+      const long at = (long)m * N + n;
+      const float w = (float)wb[at], h = (float)gb[at] * (RECIP ? w : exp_st(al[m] + be[n] - w));
+      const float y = GRAD_A ? exp_st((float)bb[(long)c * N + n] - be[n]) : exp_st((float)ab[(long)m * K + r] - al[m]);
+      s = q0 + u < Q ? __builtin_fmaf(h, y, s) : s;
+    }
+  }
+  return s * (GRAD_A ? exp_st((float)ab[(long)r * K + c] - al[r]) : exp_st((float)bb[(long)r * N + c] - be[c]));
+}
+
 // RECIP: H = g R with the forward's R = 1 / S (fp32, in the workspace) in the place of out and an
 // exponential - for float16 / bfloat16 tensors, whose `out` is stored rounded.  The header is read before
 // anything else: a workspace of another forward need not hold R.
+//
+// An infinite H, or one that rounds to an infinite bfloat16 (beyond 0x1.fep127), has no three parts: inf - inf
+// makes every sum of its line NaN.  A wave that stores a NaN sum forms such cells again on fp32 products
+// (log_bwd_cell), which leaves infinities where they belong and every other cell alone.
 template <class T, bool GRAD_A, bool RAGGED, bool RECIP>
 __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, int tile, const elem_t* __restrict__ g,
                                                    const LeanSrc src, const int* __restrict__ ws_hdr,
@@ -938,10 +963,13 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
     }
   };
   fetch(0);
+  bool lost = false;  // a NaN among the sums (or, without harm, two infinities side by side)
   acc_rows(acc, reinterpret_cast<float*>(smem) + wave * kStripFloats, lane,
            [&](int q) __attribute__((always_inline)) { if (q + 1 < 4) fetch(q + 1); },
            [&](int q, int t, float4 v) __attribute__((always_inline)) {
              if (RAGGED && !(cok && 16 * q + 4 * t < rows_left)) return;
+             const float any = (v.x + v.y) + (v.z + v.w);
+             lost = lost || any != any;
              float4 x;
              if constexpr (GRAD_A) x = exp4(xq[q & 1][t], xa[q & 1][t]);
              else x = exp4(xq[q & 1][t], becol);
@@ -949,6 +977,36 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
              if (RAGGED) st4m(gp + (long)(16 * q + 4 * t) * Cc, cc, r);
              else st4(gp + (long)(16 * q + 4 * t) * Cc, r);
            });
+  if (!__any(lost)) return;
+  // The wave's NaN cells are listed in its strip of LDS, half a block at a time, and shared out to the lanes: a
+  // line's worth would otherwise fall to four of them.  (Where the cells lie is worked out anew: kept from above
+  // it cost the largest tile spilled registers.)
+  unsigned short* list = reinterpret_cast<unsigned short*>(smem + wave * kStripFloats);
+  static_assert(sizeof(float) * kStripFloats >= 2 * 32 * 64, "");
+  const int me = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  elem_t* block = grad + ((long)batch * R + r0 + wr0) * Cc + c0 + wc0;
+  const int rows = R - r0 - wr0, cols = Cc - c0 - wc0;
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    int count = 0;
+    wave_lds_sync();
+#pragma unroll 1
+    for (int e = 32 * half; e < 32 * half + 32; ++e) {  // the cells this lane has stored: four of every fourth row
+      const int r = (me >> 4) + (e & ~3), c = (me & 15) * 4 + (e & 3);
+      const float was = r < rows && c < cols ? (float)block[(long)r * Cc + c] : 0.f;
+      const unsigned long long hits = __ballot(was != was);
+      if (was != was) list[count + __builtin_popcountll(hits & ((1ull << me) - 1))] = (unsigned short)(r * 64 + c);
+      count += __builtin_popcountll(hits);
+    }
+    wave_lds_sync();
+#pragma unroll 1
+    for (int i = me; i < count; i += 64) {
+      const int r = list[i] >> 6, c = list[i] & 63;
+      block[(long)r * Cc + c] = to_elem<elem_t>(
+          log_bwd_cell<GRAD_A, RECIP>(src.a + (long)batch * M * K, src.b + (long)batch * K * N, wsrc + (long)batch * M * N,
+                                      g + (long)batch * M * N, al, be, M, K, N, r0 + wr0 + r, c0 + wc0 + c));
+    }
+  }
 }
 
 // Both gradients in one launch, item by item, a tile of each in turn (see k_log_bwd_mfma_both).

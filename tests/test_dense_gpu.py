@@ -1526,3 +1526,48 @@ def test_draws_of_ragged_reductions(gpu, B, M, K, N):
         x, y = x.requires_grad_(), y.requires_grad_()
         grads.append(torch.autograd.grad(genbmm.samplebmm(x, y, stream=(7, 0)).sum(), (x, y)))
     assert torch.equal(grads[0][0], grads[1][0][:, :, :K]) and torch.equal(grads[0][1], grads[1][1][:, :K])
+
+
+# one tile per item; 128 x 128, 128 x 256 / 256 x 128 and 256 x 256 tiles, each whole and with ragged edges (the
+# infinities in the first slab, the last line and the last, partial slab)
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,M,K,N", [(3, 128, 128, 128), (3, 100, 70, 128), (3, 256, 256, 128), (3, 130, 131, 133),
+                                     (32, 512, 512, 256), (40, 509, 512, 511), (64, 512, 512, 512), (64, 500, 509, 510)])
+def test_logbmm_backward_of_infinite_gradients(gpu, dt, B, M, K, N):
+    """An infinite incoming gradient is infinite in its row of grad_a and its column of grad_b and nowhere else
+    (every weight of these operands is positive), a NaN is NaN there: three bfloat16 parts cannot hold either.  On
+    the tiled kernels every other cell has the bits it has without them; an item of one tile is redone whole, with
+    the exact routine's bits.  A finite gradient beyond the largest bfloat16 stays finite and accurate."""
+    torch.manual_seed(M + K)
+    a, b = (torch.randn(*s, device=gpu).to(dt).requires_grad_() for s in ((B, M, K), (B, K, N)))
+    g = torch.randn(B, M, N, device=gpu).to(dt)
+    inf = float("inf")
+    cells = [(0, 3, 5, inf), (1, M - 1, N - 1, -inf), (2, M // 2, N // 2, float("nan"))]
+    clean, lines_a, lines_b = g.clone(), torch.zeros(B, M, dtype=torch.bool), torch.zeros(B, N, dtype=torch.bool)
+    for i, m, n, v in cells:
+        g[i, m, n], clean[i, m, n], lines_a[i, m], lines_b[i, n] = v, 0, True, True
+    ga, gb = torch.autograd.grad(genbmm.logbmm(a, b), (a, b), g)
+    for i, m, n, v in cells:
+        for line in (ga[i, m], gb[i, :, n]):
+            assert torch.equal(line.float().nan_to_num(7.0, 8.0, 9.0), torch.full_like(line, v).float().nan_to_num(7.0, 8.0, 9.0))
+    if max(M, K, N) <= 128:
+        out = genmul.logbmm_on_path(a, b, genmul.PATH_AUTO if dt == torch.float32 else genmul.PATH_RECIP).detach()
+        wa, wb = torch.empty_like(a), torch.empty_like(b)
+        bwd = getattr(_lib.load(), "genbmm_logbmm_bwd_path" + genmul._sfx(a))
+        assert bwd(*(_lib.ptr(t.detach()) for t in (a, b, out, g)), _lib.ptr(None), _lib.ptr(wa), _lib.ptr(wb), B, M, K, N,
+                   genmul.PATH_EXACT, _lib.stream_of(a)) == 0
+    else:
+        wa, wb = torch.autograd.grad(genbmm.logbmm(a, b), (a, b), clean)
+    live_a, live_b = ~lines_a.to(gpu), ~lines_b.to(gpu)
+    assert torch.equal(ga[live_a], wa[live_a])
+    assert torch.equal(gb.transpose(1, 2)[live_b], wb.transpose(1, 2)[live_b])
+    if dt == torch.float32:   # one term with all the weight: H is g itself
+        with torch.no_grad():
+            a[0, :, 0], b[0, 0, :] = 40.0, 40.0
+        g = torch.randn(B, M, N, device=gpu)
+        g[0, 3, 5], g[0, M - 1, N - 1] = 3.395e38, -3.395e38
+        ga, gb = torch.autograd.grad(genbmm.logbmm(a, b), (a, b), g)
+        _, wa, wb = oracle.logbmm_grads64(a[:1].cpu(), b[:1].cpu(), g[:1].cpu())
+        for got, want in ((ga[:1].cpu().double(), wa), (gb[:1].cpu().double(), wb)):
+            # (weights formed from an `out` near 80: a relative 2^-24 * 80 = 5e-6)
+            assert bool(((got - want).abs() <= 2e-5 * want.abs() + 1e-5).all())
