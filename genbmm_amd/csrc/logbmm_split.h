@@ -993,7 +993,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
 #pragma unroll 1
     for (int e = 32 * half; e < 32 * half + 32; ++e) {  // the cells this lane has stored: four of every fourth row
       const int r = (me >> 4) + (e & ~3), c = (me & 15) * 4 + (e & 3);
-      const float was = r < rows && c < cols ? (float)block[(long)r * Cc + c] : 0.f;
+      const float was = r < rows && c < cols ? settled((float)block[(long)r * Cc + c]) : 0.f;
       const unsigned long long hits = __ballot(was != was);
       if (was != was) list[count + __builtin_popcountll(hits & ((1ull << me) - 1))] = (unsigned short)(r * 64 + c);
       count += __builtin_popcountll(hits);
