@@ -26,9 +26,9 @@
 //    through two LDS buffers) then runs without any edge handling in its loop, sums up to two products into one
 //    accumulator and applies the epilogue of its role.  A batch item with a cell whose
 //    alpha + beta - out is beyond 40 ln 2 or not finite (a factor could underflow against a
-//    term that matters), or with an X, Y or H beyond the largest bfloat16 (an infinite operand has
-//    no three parts), is flagged by the passes that form them and redone by the exact kernels,
-//    which run behind the factored ones on the flagged items only.
+//    term that matters), or with an X, Y, H or -H t beyond the largest bfloat16 (an infinite operand has
+//    no three parts), is flagged where they are formed and redone by the exact kernels, which run
+//    behind the factored ones on the flagged items only.
 #include <algorithm>
 #include <type_traits>
 
@@ -430,6 +430,7 @@ struct BBMM {
   const float* f0;      // kEpiGrad: X / Y, the factor of C0
   const float* h;       // kEpiT: H
   float* nht;           // kEpiT: -H t
+  int* flags;           // kEpiT: per item, set where -H t does not split
   float* tt;            // kEpiT: t unrounded, (B, R, C) unpadded
   elem_t* dst;          // kEpiT: grad_g; kEpiGrad: grad_a / grad_b; (B, R, C) unpadded
   int R, C;             // true extents of the output
@@ -532,6 +533,7 @@ void k_bb_mm(const BBMM p) {
   const int cc = clamp4(p.C - col);                              // columns of the piece that exist
   float* strip = reinterpret_cast<float*>(smem) + wave * kStripFloats;
   if constexpr (EPI == kEpiT) {
+    bool bad = false;
     acc_rows(acc, strip, lane, [](int) {},
              [&](int q, int t, float4 v) __attribute__((always_inline)) {
                const int ru = 16 * q + 4 * t;
@@ -539,12 +541,15 @@ void k_bb_mm(const BBMM p) {
                const long du = ((long)batch * p.R + row0 + ru) * p.C + col;  // unpadded arrays
                const float4 rv = ld4a(p.f_acc + pu), hv = ld4a(p.h + pu);
                const float4 tv = make_float4(rv.x * v.x, rv.y * v.y, rv.z * v.z, rv.w * v.w);
-               st4a(p.nht + pu, make_float4(-hv.x * tv.x, -hv.y * tv.y, -hv.z * tv.z, -hv.w * tv.w));
+               const float4 nv = make_float4(-hv.x * tv.x, -hv.y * tv.y, -hv.z * tv.z, -hv.w * tv.w);
+               bad = bad || !splits4(nv);
+               st4a(p.nht + pu, nv);
                if (row0 + ru < p.R && cc > 0) {
                  st4m(p.tt + du, cc, tv);
                  if constexpr (!kElemF32) st4m(p.dst + du, cc, tv);
                }
              });
+    if (bad) p.flags[batch] = 1;
   } else {
     // C0 scaled by its factor first, kept in registers as rows; then the other product joins it
     float4 o[16];
@@ -596,7 +601,7 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
     if (has_a) { q.rows[n] = w.x; q.cols[n] = w.eb; ++n; }
     if (has_b) { q.rows[n] = w.ea; q.cols[n] = w.y; ++n; }
     q.pairs = n; q.Rp = Mp; q.Cp = Np; q.Qp = Kp; q.R = M; q.C = N;
-    q.f_acc = w.r; q.h = w.h; q.nht = w.nht; q.tt = p.tt; q.dst = p.gg;
+    q.f_acc = w.r; q.h = w.h; q.nht = w.nht; q.flags = w.flags; q.tt = p.tt; q.dst = p.gg;
     if (int e = launch_mm<true, false, kEpiT>(q, B, s)) return e;
   }
   {  // grad_a = X (H EB^T) + EA (H Y^T - (H t) EB^T)

@@ -1571,3 +1571,27 @@ def test_logbmm_backward_of_infinite_gradients(gpu, dt, B, M, K, N):
         for got, want in ((ga[:1].cpu().double(), wa), (gb[:1].cpu().double(), wb)):
             # (weights formed from an `out` near 80: a relative 2^-24 * 80 = 5e-6)
             assert bool(((got - want).abs() <= 2e-5 * want.abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("B,M,K,N", [(5, 128, 128, 128), (4, 130, 129, 200)])
+def test_logbmm_double_backward_whose_product_of_two_factors_overflows(gpu, B, M, K, N):
+    """Row and column maxima that never meet (S = 2 e^-24: H = g / S) and large cotangents: H, X and Y split into
+    three parts, their product H t (1e30 * 1e10) does not although every result is finite.  Such an item takes
+    the exact passes bit for bit; the others agree to fp32 sums of at most 200 products (1e-5 of the largest)."""
+    lib = _lib.load()
+    torch.manual_seed(N)
+    a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
+    ua, ub = torch.randn(B, M, K), torch.randn(B, K, N)
+    a[0], b[0] = 0, 0
+    a[0, :, 0], b[0, 1, :] = 24, 24
+    g[0], ua[0], ub[0] = 1e20 * (1 + g[0].abs()), 1e10 * (1 + ua[0].abs()), 1e10 * (1 + ub[0].abs())
+    out = genbmm.logbmm(a.to(gpu), b.to(gpu))
+    x = [t.to(gpu) for t in (a, b)] + [out] + [t.to(gpu) for t in (g, ua, ub)]
+    p, s = _lib.ptr, _lib.stream_of(out)
+    ws = torch.full((lib.genbmm_logbmm_bwdbwd_ws_size(B, M, K, N),), float("nan"), device=gpu)
+    got, want = ([torch.empty_like(t) for t in (x[0], x[1], x[3])] for _ in range(2))
+    assert lib.genbmm_logbmm_bwdbwd_ws(*(p(t) for t in x), *(p(t) for t in got), p(ws), B, M, K, N, s) == 0
+    assert lib.genbmm_logbmm_bwdbwd(*(p(t) for t in x), *(p(t) for t in want), B, M, K, N, s) == 0
+    for u, w in zip(got, want):
+        assert bool(torch.isfinite(w).all()) and torch.equal(u[0], w[0])
+        assert float((u[1:] - w[1:]).abs().max()) <= 1e-5 * max(1.0, float(w[1:].abs().max()))
