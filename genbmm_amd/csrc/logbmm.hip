@@ -987,12 +987,20 @@ inline int mfma_kind(int path, int B, int out_r, int out_c, int red, bool long_c
   return 1;
 }
 
+// The tiling of both gradients of a matrix-core shape in one launch of the three-part kernels: 2 or 1 as
+// above, 0 where the gradients are too narrow for tiles (K) or an item too large.  The two gradients count
+// their tiles apart and may land on either side of the 512: both then run on 128 x 128 tiles.
+inline int bwd_split_kind(int B, int M, int K, int N) {
+  if (!fwd_mfma_shape(B, M, K, N) || !bwd_split_sizes(M, K, N)) return 0;
+  const int ka = mfma_kind(GENBMM_PATH_AUTO, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_AUTO, B, K, N, M, false);
+  return ka == 0 || kb == 0 ? 0 : min(ka, kb);
+}
+
 // Shapes whose forward under GENBMM_PATH_RECIP keeps 1 / S alone, because both gradients run on the
 // three-part kernels, which form EA and EB again; other matrix-core shapes keep EA, EB and 1 / S under
 // that path and their backward is GENBMM_PATH_FACTORS's.
 inline bool recip_shape(int B, int M, int K, int N) {
-  const int ka = mfma_kind(GENBMM_PATH_RECIP, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_RECIP, B, K, N, M, false);
-  return fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N) && ka == kb && ka != 0 && bwd_split_sizes(M, K, N);
+  return !self_shape(M, K, N) && bwd_split_kind(B, M, K, N) != 0;
 }
 
 using MT128 = MTile<128, 128>;
@@ -1188,22 +1196,21 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
   }
   if (path == GENBMM_PATH_RECIP && !recip_shape(B, M, K, N)) path = GENBMM_PATH_FACTORS;  // what its forward kept
   if (st && grad_a && grad_b && mk > 0 && kn > 0 && fwd_mfma_shape(B, M, K, N)) {
+    LogBwdArgs pa = p, pb = p;
+    pa.grad = grad_a;
+    pb.grad = grad_b;
+    if (const int kind = split_path(path) ? bwd_split_kind(B, M, K, N) : 0; kind != 0) {
+      const bool recip = path == GENBMM_PATH_RECIP;
+      if (kind == 1) return launch_bwd_split_both<MT128S, MT128S>(pa, pb, st, B, recip, s);
+      if (split_big_fits(B, M, K) && split_big_fits(B, K, N))
+        return launch_bwd_split_both<MTBig, MTBig>(pa, pb, st, B, recip, s);
+      return launch_bwd_split_both<MTWide, MTTall>(pa, pb, st, B, recip, s);
+    }
     const int ka = mfma_kind(path, B, M, K, N, true), kb = mfma_kind(path, B, K, N, M, false);
-    if (ka == kb && ka != 0) {
-      LogBwdArgs pa = p, pb = p;
-      pa.grad = grad_a;
-      pb.grad = grad_b;
-      const bool lean = path != GENBMM_PATH_FACTORS;
-      if (lean && split_path(path) && bwd_split_sizes(M, K, N)) {
-        const bool recip = path == GENBMM_PATH_RECIP;
-        if (ka == 1) return launch_bwd_split_both<MT128S, MT128S>(pa, pb, st, B, recip, s);
-        if (split_big_fits(B, M, K) && split_big_fits(B, K, N))
-          return launch_bwd_split_both<MTBig, MTBig>(pa, pb, st, B, recip, s);
-        return launch_bwd_split_both<MTWide, MTTall>(pa, pb, st, B, recip, s);
-      }
+    const bool lean = path != GENBMM_PATH_FACTORS;
+    if (ka == kb && ka != 0)
       return ka == 2 ? launch_bwd_mfma_both<MTWide, MTTall>(pa, pb, st, B, s, lean)
                      : launch_bwd_mfma_both<MT128, MT128>(pa, pb, st, B, s, lean);
-    }
   }
   if (grad_a) {
     p.grad = grad_a;

@@ -261,9 +261,7 @@ def test_logbmm_three_part_kernels(gpu, B, M, K, N):
     """Shapes which the default path runs on the bf16 matrix instruction with
     every factor cut into three bf16 parts (256 x 256 tiles where they fill the chip, 256 x 128 /
     128 x 256 otherwise; forward and backward switch independently; the last seven with ragged
-    edges - partial tiles, partial slabs, odd row lengths; the backward takes any M, and K and N in
-    multiples of four): every batch item against
-    float64 on the device, among them items whose tiles must take the exact routine (factors that
+    edges - partial tiles, partial slabs, odd row lengths): every batch item against float64 on the device, among them items whose tiles must take the exact routine (factors that
     underflow against live terms: everywhere, and in a single row), an item with rows padded at
     the floor, one with a masked reduction step, one with magnitudes near 1000 - and the whole
     result against the fp32 matrix instruction (GENBMM_PATH_MFMA32) at twice the tolerance."""
@@ -360,10 +358,11 @@ def test_logbmm_matrix_core_shape_sweep(gpu):
 
 
 # K and N of every remainder of four on each tile of the three-part backward: 256 x 256 (both extents in
-# 256s, enough tiles), 128 x 256 / 256 x 128, 128 x 128; a last line that is a lone straddling piece
+# 256s, enough tiles), 128 x 256 / 256 x 128, 128 x 128; a last line that is a lone straddling piece; gradients on
+# either side of the tile count from which on they would be 256 wide
 @pytest.mark.parametrize("B,M,K,N", [(64, 511, 509, 510), (100, 250, 507, 509), (64, 512, 385, 387), (300, 130, 131, 253),
                                      (150, 255, 254, 197), (3, 99, 97, 129), (2, 133, 101, 103), (2, 96, 259, 130),
-                                     (2, 97, 130, 98), (1, 257, 513, 385)])
+                                     (2, 97, 130, 98), (1, 257, 513, 385), (90, 267, 241, 251), (155, 117, 215, 230)])
 def test_logbmm_three_part_backward_on_any_size(gpu, B, M, K, N):
     """Gradients of odd sizes against float64 (first and last batch item), and every batch item against the
     fp32 instruction's kernels: both form H = g exp(max - out) from an `out` rounded to 2^-24 of itself

@@ -187,6 +187,15 @@ def test_launch_grids_beyond_32_bits_are_refused():
     assert lib.genbmm_logbmm_stats_size(64, 512, 512, 512) > 0
 
 
+def test_kept_reciprocals_take_one_float_per_result():
+    """GENBMM_PATH_RECIP: where both gradients run on the three-part kernels the workspace grows by 1 / S alone,
+    also where the two count their tiles on either side of the line between tile sizes.  Host code only."""
+    lib = _lib.load()
+    size = lib.genbmm_logbmm_stats_size_path
+    for B, M, K, N in ((64, 512, 512, 512), (2, 200, 177, 131), (90, 267, 241, 251), (155, 117, 215, 230), (60, 500, 400, 250)):
+        assert size(B, M, K, N, 5) == size(B, M, K, N, 0) + B * M * N, (B, M, K, N)
+
+
 def test_half_builds_compute_in_float():
     """The float16 / bfloat16 builds of the dense sources widen on load and narrow on store
     and do nothing else in the narrow type: their device code (LLVM IR) holds no arithmetic,
