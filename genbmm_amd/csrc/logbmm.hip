@@ -996,11 +996,15 @@ inline int bwd_split_kind(int B, int M, int K, int N) {
   return ka == 0 || kb == 0 ? 0 : min(ka, kb);
 }
 
-// Shapes whose forward under GENBMM_PATH_RECIP keeps 1 / S alone, because both gradients run on the
-// three-part kernels, which form EA and EB again; other matrix-core shapes keep EA, EB and 1 / S under
-// that path and their backward is GENBMM_PATH_FACTORS's.
-inline bool recip_shape(int B, int M, int K, int N) {
-  return !self_shape(M, K, N) && bwd_split_kind(B, M, K, N) != 0;
+// What the forward keeps under GENBMM_PATH_RECIP: 1 / S alone where both gradients run on the three-part
+// kernels, which form EA and EB again; all three factors where they run on the fp32 instruction (an item too
+// large for the former), as under GENBMM_PATH_FACTORS; nothing where no gradient is tiled (K below 96): the
+// vector-ALU kernels read maxima and `out` ((64, 300, 60, 300): 32 MB that the forward wrote and nothing read).
+inline int recip_keeps(int B, int M, int K, int N) {
+  if (!fwd_mfma_shape(B, M, K, N) || self_shape(M, K, N)) return kKeepNone;
+  if (bwd_split_kind(B, M, K, N) != 0) return kKeepRecip;
+  const int ka = mfma_kind(GENBMM_PATH_AUTO, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_AUTO, B, K, N, M, false);
+  return ka != 0 || kb != 0 ? kKeepFactors : kKeepNone;
 }
 
 using MT128 = MTile<128, 128>;
@@ -1103,7 +1107,7 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
   const int64_t mk = (int64_t)B * M * K, kn = (int64_t)B * K * N, mn = (int64_t)B * M * N;
   if (missing(a, mk) || missing(b, kn) || missing(out, mn)) return GENBMM_E_NULLPTR;
   int keep = keep_factors && (path == GENBMM_PATH_FACTORS || factors) ? kKeepFactors : kKeepNone;
-  if (path == GENBMM_PATH_RECIP) keep = recip_shape(B, M, K, N) ? kKeepRecip : kKeepFactors;
+  if (path == GENBMM_PATH_RECIP) keep = recip_keeps(B, M, K, N);
   if (stats && B > 0 && item_shape(M, K, N) && auto_path(path)) {  // whole items per workgroup
     int* hdr = prepared_of(stats, B, M, K, N).hdr;
     if (M == 32 && K == 32 && N == 32)  // one wave per item on the matrix cores
@@ -1194,7 +1198,7 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
     }
     return launch_status();
   }
-  if (path == GENBMM_PATH_RECIP && !recip_shape(B, M, K, N)) path = GENBMM_PATH_FACTORS;  // what its forward kept
+  if (path == GENBMM_PATH_RECIP && recip_keeps(B, M, K, N) != kKeepRecip) path = GENBMM_PATH_FACTORS;
   if (st && grad_a && grad_b && mk > 0 && kn > 0 && fwd_mfma_shape(B, M, K, N)) {
     LogBwdArgs pa = p, pb = p;
     pa.grad = grad_a;
@@ -1418,8 +1422,11 @@ size_t genbmm_logbmm_stats_size_path(int B, int M, int K, int N, int path) {
   if (check_dense_dims(B, M, K, N)) return 0;
   int64_t n = header_offset(B, M, N) + 4;  // maxima, flags and the header
   // the by-products of the matrix-core forward (the one-tile kernels keep the maxima only)
-  if (path == GENBMM_PATH_RECIP && recip_shape(B, M, K, N)) n += (int64_t)B * M * N;
-  else if ((path == GENBMM_PATH_FACTORS || path == GENBMM_PATH_RECIP) && fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N))
+  int keep = kKeepNone;
+  if (path == GENBMM_PATH_RECIP) keep = recip_keeps(B, M, K, N);
+  else if (path == GENBMM_PATH_FACTORS && fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N)) keep = kKeepFactors;
+  if (keep == kKeepRecip) n += (int64_t)B * M * N;
+  else if (keep == kKeepFactors)
     n += (int64_t)B * ((int64_t)M * K + (int64_t)K * N + (int64_t)M * N);
   // the sums of a forward that cuts a long reduction into pieces
   if (path == GENBMM_PATH_AUTO) {

@@ -155,10 +155,12 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *   GENBMM_PATH_RECIP  as AUTO, with 1 / sum kept in fp32 for the backward, which
  *                      then weighs g by it instead of by exp(max - out): what
  *                      float16 / bfloat16 tensors want, whose `out` is stored
- *                      rounded (4 bytes per result cell; shapes whose backward
- *                      does not run on the bf16 instruction keep all three
- *                      factors and take FACTORS's).  One gradient alone (the
- *                      other pointer NULL) is formed from `out`.
+ *                      rounded (4 bytes per result cell).  Items too large for
+ *                      the bf16 instruction's backward keep all three factors
+ *                      and take FACTORS's; problems with an extent below 96 or
+ *                      none above 128 keep nothing and weigh by exp(max - out).
+ *                      One gradient alone (the other pointer NULL) is formed
+ *                      from `out`.
  * Any other value: GENBMM_E_MODE.  Forward and backward of one problem need not
  * name the same path (see genbmm_logbmm_bwd).  No counterpart in the reference.
  */

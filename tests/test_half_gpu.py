@@ -319,8 +319,8 @@ def test_logbmm_second_order_half_equals_float_kernels_rounded(gpu, dt, suffix, 
 
 
 # tiled matrix-core shapes whose backward runs on the three-part kernels: full 256-, 128-wide and mixed tiles,
-# ragged edges, a partial last slab, odd K and N; then a gradient too narrow for a tile, which keeps all factors
-# instead, one tile per item, a small item; gradients that count their tiles on either side of the 512 from
+# ragged edges, a partial last slab, odd K and N; then a gradient too narrow for a tile, whose backward reads
+# `out`, one tile per item, a small item; gradients that count their tiles on either side of the 512 from
 # which on they would be 256 wide
 RECIP_SHAPES = [(48, 512, 512, 512), (32, 256, 512, 256), (128, 256, 128, 512), (2, 130, 140, 132), (2, 257, 100, 260),
                 (3, 300, 516, 200), (2, 200, 177, 131), (2, 160, 48, 160), (3, 128, 128, 128), (2, 64, 64, 64),

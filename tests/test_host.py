@@ -196,6 +196,14 @@ def test_kept_reciprocals_take_one_float_per_result():
         assert size(B, M, K, N, 5) == size(B, M, K, N, 0) + B * M * N, (B, M, K, N)
 
 
+def test_kept_reciprocals_of_narrow_gradients_take_nothing():
+    """GENBMM_PATH_RECIP where no gradient is tiled (K below 96): nothing reads a factor, none is kept.  Host code only."""
+    lib = _lib.load()
+    size = lib.genbmm_logbmm_stats_size_path
+    for B, M, K, N in ((64, 300, 60, 300), (2, 160, 48, 160), (1, 96, 16, 129), (3, 500, 95, 97)):
+        assert size(B, M, K, N, 5) == size(B, M, K, N, 4), (B, M, K, N)
+
+
 def test_half_builds_compute_in_float():
     """The float16 / bfloat16 builds of the dense sources widen on load and narrow on store
     and do nothing else in the narrow type: their device code (LLVM IR) holds no arithmetic,
