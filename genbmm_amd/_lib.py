@@ -157,7 +157,7 @@ def call(name, t, *args):
     if index == torch.cuda.current_device():
         code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
     else:
-        with torch.cuda.device(index):
+        with torch.cuda.device(t.device):  # (refuses tensors that are on no device)
             code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
     if code != 0:
         check(code, name)

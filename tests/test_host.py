@@ -12,7 +12,7 @@ from hypothesis.strategies import integers
 
 import oracle
 import genbmm_amd
-from genbmm_amd import _lib
+from genbmm_amd import _lib, ops
 from genbmm_amd.sparse import BandedMatrix, banddiag
 
 mint = integers(min_value=6, max_value=10)
@@ -243,6 +243,26 @@ def test_no_cpu_fallback():
     for name in ("multiply", "multiply_log", "multiply_max"):
         with pytest.raises(RuntimeError):
             getattr(BandedMatrix(band, 1, 1), name)(BandedMatrix(band, 1, 1))
+
+
+def test_no_host_pointer_reaches_the_library(monkeypatch):
+    """Entry points whose tensors no other check looks at refuse CPU tensors before the library is called."""
+    calls = []
+    monkeypatch.setattr(_lib, "_lib", type("Lib", (), {"__getattr__": lambda self, name: lambda *args: calls.append(name) or 0})())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    band, idx, g = torch.rand(2, 6, 3), torch.zeros(2, 4, 5, dtype=torch.int32), torch.rand(2, 4, 5)
+    wide, fac = torch.rand(2, 6, 5), torch.rand(2, 2, 4, 5)
+    x = BandedMatrix(band, 1, 1)
+    for attempt in (lambda: x.multiply_back(x, None, wide),
+                    lambda: ops.argmax_bwd(idx, g, 3),
+                    lambda: ops.prodmax_bwd(idx, fac, g, 3),
+                    lambda: ops.banded_fwd(band, band, 1, 1, 1, 1, 3),
+                    lambda: ops.banded_bwd(band, band, wide, wide, wide, 1, 1, 1, 1, 3),
+                    lambda: ops.banded_bwdbwd(band, band, wide, wide, band, band, 1, 1, 1, 1)):
+        with pytest.raises(ValueError, match="cuda device"):
+            attempt()
+    assert not calls
 
 
 def test_product_does_not_import_the_oracle():
