@@ -12,9 +12,8 @@ Differences in mechanism (not in results):
   * instead of the (B, M, N) `maxes` tensor the forward saves a workspace sized by
     the library: row maxima of a, column maxima of b and a few per-tile flags,
     which let forward and backward factor exp(a + b) wherever that is exact
-    (csrc/logbmm.hip), and - for shapes that run on the matrix cores - the
-    factors exp(a - max), exp(b - max) and 1/sum, so that the backward takes no
-    exponential at all (csrc/logbmm_mfma.h).
+    (csrc/logbmm.hip); for float16 / bfloat16 tensors of tiled matrix-core
+    shapes also 1/sum in float32 (PATH_RECIP below).
   * the arg-max / sample index stays int32 into the backward; the reference
     converts it (and a, b, g) to float first (genmul.py:62-65).
   * samplebmm draws its uniforms from a counter-based Philox4x32-10 stream
@@ -25,8 +24,7 @@ Element types: float32 takes the kernels above; float64 takes the library's
 double-precision entry points (`*_f64`, no workspaces); float16 / bfloat16 take the
 same kernels compiled for that element type (`*_f16` / `*_bf16`: the loads widen,
 arithmetic and workspaces are float32, the stores round to nearest), the reference's
-AT_DISPATCH_FLOATING_TYPES_AND_HALF (matmul_cuda_kernel.cu:489).  Only logbmm's
-double backward widens half tensors on the host.
+AT_DISPATCH_FLOATING_TYPES_AND_HALF (matmul_cuda_kernel.cu:489).
 
 Beyond the reference's contract the four functions also take operands with any
 number of leading batch dimensions (equal or broadcastable; they are flattened to

@@ -148,7 +148,7 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *   GENBMM_PATH_MFMA32 as AUTO, but the matrix-core kernels use the fp32 matrix
  *                      instruction.  Under AUTO they run on the bf16 matrix
  *                      instruction with every factor cut into three bf16
- *                      parts that add up to it exactly and six partial
+ *                      parts that add up to it exactly (above 2^-100) and six partial
  *                      products per product, accumulated in fp32 - what is
  *                      dropped is below 2^-23 of a product, one fp32 rounding -
  *                      at 2.7 times less matrix-pipe time.

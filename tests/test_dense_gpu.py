@@ -261,10 +261,11 @@ def test_logbmm_three_part_kernels(gpu, B, M, K, N):
     """Shapes which the default path runs on the bf16 matrix instruction with
     every factor cut into three bf16 parts (256 x 256 tiles where they fill the chip, 256 x 128 /
     128 x 256 otherwise; forward and backward switch independently; the last seven with ragged
-    edges - partial tiles, partial slabs, odd row lengths): every batch item against float64 on the device, among them items whose tiles must take the exact routine (factors that
-    underflow against live terms: everywhere, and in a single row), an item with rows padded at
-    the floor, one with a masked reduction step, one with magnitudes near 1000 - and the whole
-    result against the fp32 matrix instruction (GENBMM_PATH_MFMA32) at twice the tolerance."""
+    edges - partial tiles, partial slabs, odd row lengths): every batch item against float64 on
+    the device, among them items whose tiles must take the exact routine (factors that underflow
+    against live terms: everywhere, and in a single row), an item with rows padded at the floor, one
+    with a masked reduction step, one with magnitudes near 1000 - and the whole result against the
+    fp32 matrix instruction (GENBMM_PATH_MFMA32) at twice the tolerance."""
     torch.manual_seed(M + N)
     a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
     a[1, ::2, 0] += 200.0
