@@ -33,7 +33,9 @@ constexpr int kKC = 128;  // cells of the reduction axis per lane
 // trip per four cells.  Measured (both gradients, max product; before: loads waited for 16 cells at a
 // time, cells of a row side by side so that the lanes' additions met in banks, rows of unaligned
 // length one cell at a time): (256, 256^3) 104 -> 87 us, (64, 512^3) 141 -> 123, (8192, 32^3) 79 -> 54,
-// (40, 251, 173, 301) 111 -> 37.
+// (40, 251, 173, 301) 111 -> 37.  A row's partial last chunk too is read in pieces of four, the last one cell by
+// cell (all 32 cell by cell cost forward and backward of float16 draws at (64, 20^3) 32.7 -> 33.5 us, now 32.3;
+// prodmaxbmm (814, 76, 51, 83) 165 -> 153; clamped addresses in the place of the uniform tests: 5 % slower).
 static_assert(kKC == 128, "the shifts of the write-out");
 constexpr int kArgAcc = 64 * kKC + 64;  // floats of LDS: the cells, one spare cell per lane
 constexpr int kChA = 32, kChB = 16;     // cells per chunk (a column's cells are single loads, and at most
@@ -157,11 +159,21 @@ __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int
   auto tail = [&](Chunk& x, int c) __attribute__((always_inline)) {
     const int n0 = c * kChA;
 #pragma unroll
-    for (int q = 0; q < kChA; ++q) {
-      const bool in = n0 + q < N;
-      x.i4[q >> 2][q & 3] = in ? irow[n0 + q] : -1;
-      x.g4[q >> 2][q & 3] = in ? grow[n0 + q] : (elem_t)0.f;
-      if constexpr (PROD == 2) x.f4[q >> 2][q & 3] = in ? frow[n0 + q] : 0.f;
+    for (int q = 0; q < kChA / 4; ++q) {
+      const int nq = n0 + 4 * q;
+      if (nq + 4 <= N) {  // uniform
+        x.i4[q] = *reinterpret_cast<const argmax_i4*>(irow + nq);
+        x.g4[q] = *reinterpret_cast<const argmax_e4*>(grow + nq);
+        if constexpr (PROD == 2) x.f4[q] = *reinterpret_cast<const argmax_f4*>(frow + nq);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool in = nq + j < N;
+          x.i4[q][j] = in ? irow[nq + j] : -1;
+          x.g4[q][j] = in ? grow[nq + j] : (elem_t)0.f;
+          if constexpr (PROD == 2) x.f4[q][j] = in ? frow[nq + j] : 0.f;
+        }
+      }
     }
   };
   argmax_walk<Chunk>(accs, N, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {

@@ -64,6 +64,20 @@ def test_argmax_backward_with_many_k_ranges(gpu):
         assert torch.equal(ga.cpu(), wa) and torch.equal(gb.cpu(), wb), (B, M, K, N)
 
 
+@pytest.mark.parametrize("prod", [False, True])
+def test_argmax_backward_of_every_row_length(gpu, prod):
+    """Rows of 1 to 68 cells: whole chunks of 32, whole pieces of four, single cells, in every combination,
+    rows of odd length (so that pieces start at any cell).  Bit for bit as the ordered sums."""
+    torch.manual_seed(8)
+    for N in range(1, 69):
+        a, b, g = grid(2, 5, 9), grid(2, 9, N), grid(2, 5, N)
+        for dt in (torch.float32, torch.float16):
+            ad, bd = a.to(gpu, dt).requires_grad_(True), b.to(gpu, dt).requires_grad_(True)
+            ga, gb = torch.autograd.grad((genbmm.prodmaxbmm if prod else genbmm.maxbmm)(ad, bd), (ad, bd), g.to(gpu, dt))
+            _, si = oracle.seq_maxbmm_fwd(a, b, prod)
+            wa, wb = oracle.seq_argmax_bwd(a if prod else 9, b, si, g, prod)
+            assert torch.equal(ga.cpu(), wa.to(dt)) and torch.equal(gb.cpu(), wb.to(dt)), (N, dt)
+
 def test_sample_on_many_shapes(gpu):
     """Every index brackets its uniform in the float64 CDF; shapes on both sides of the
     matrix-core limits (M, N >= 96, K >= 16), of the 62 slabs that its six-bit tag counts
