@@ -51,8 +51,11 @@ inline MaxDims max_dims(int Wa, int Wb, int Wo) {
 // maximum, and one compare and one select keep the pair that raised it last: 2.5 instructions per term
 // instead of 4 - and which k of its pair it was is found behind the walk, by forming the first one's sum
 // again.  The first pair that attains the maximum and the first k inside it are what the walk with a
-// strict comparison keeps.  What is left is bound by the LDS reads (nine values per eight terms): 64 x 4096,
-// 65 diagonals each 281 -> 273 us, 16 x 4096, 129 diagonals each 536 -> 499.
+// strict comparison keeps.  64 x 4096, 65 diagonals each 281 -> 273 us, 16 x 4096, 129 diagonals each
+// 536 -> 497.  What is left has no single bound (counters, 64 x 4096): 1.8 waves per SIMD issue vector
+// instructions in 63 % of a busy compute unit's cycles (85 M of them) and keep its LDS reading in 50 %
+// (nine values per eight terms; a quarter of that are bank conflicts), and compute units have no wave for a
+// fifth of the launch.
 template <bool PAIRS>
 __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int strips, const MaxDims d,
                                                          long cells_a, long cells_b, int nseg, int Wseg) {
