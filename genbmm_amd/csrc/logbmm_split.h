@@ -29,6 +29,7 @@
 //  * an operand whose source is [reduction][line]: plane[8 step pairs][lines + 8]; a lane
 //    stages a pair of reduction steps for LW consecutive lines (the pair shares a word;
 //    one store of LW words per plane) and reads its eight steps as four words a row apart.
+//  * the same, staged by a line's own threads (SplitL): plane[half of the slab][line][4 words].
 #pragma once
 
 #include "logbmm_mfma.h"
@@ -101,6 +102,42 @@ struct SplitS {
     uintx4 w;
     w.x = p[0]; w.y = p[LD]; w.z = p[2 * LD]; w.w = p[3 * LD];
     return __builtin_bit_cast(bf16x8, w);
+  }
+};
+
+// source [reduction][line], a thread stages ST consecutive reduction steps of one line: plane[half of the
+// slab][line][4 words].  The loads of a step run along the lines, a wave's steps are its own (uniform row
+// addresses), the staged words leave in one store per plane and an operand is one 16-byte read of
+// neighbouring lanes side by side.
+template <int OUT, int NT>
+struct SplitL {
+  static constexpr int PLANE = 8 * OUT;      // words
+  static constexpr int BUF = 3 * PLANE;
+  static constexpr int ST = 16 * OUT / NT;   // steps per thread
+  static_assert((ST == 4 || ST == 8) && OUT % 64 == 0, "");
+  static __device__ __forceinline__ int line(int tid) { return tid % OUT; }
+  static __device__ __forceinline__ int step0(int tid) { return __builtin_amdgcn_readfirstlane(tid / OUT) * ST; }
+  static __device__ __forceinline__ void put(unsigned* __restrict__ buf, int tid, const float (&v)[ST]) {
+    unsigned h[ST / 2], m[ST / 2], l[ST / 2];
+#pragma unroll
+    for (int j = 0; j < ST / 2; ++j) split2(v[2 * j], v[2 * j + 1], h[j], m[j], l[j]);
+    const int s0 = step0(tid);
+    unsigned* p = buf + (s0 >> 3) * (4 * OUT) + line(tid) * 4 + (ST == 4 ? (s0 & 4) >> 1 : 0);
+    if constexpr (ST == 8) {
+      uintx4 w;
+      w.x = h[0]; w.y = h[1]; w.z = h[2]; w.w = h[3]; *reinterpret_cast<uintx4*>(p) = w;
+      w.x = m[0]; w.y = m[1]; w.z = m[2]; w.w = m[3]; *reinterpret_cast<uintx4*>(p + PLANE) = w;
+      w.x = l[0]; w.y = l[1]; w.z = l[2]; w.w = l[3]; *reinterpret_cast<uintx4*>(p + 2 * PLANE) = w;
+    } else {
+      uintx2 w;
+      w.x = h[0]; w.y = h[1]; *reinterpret_cast<uintx2*>(p) = w;
+      w.x = m[0]; w.y = m[1]; *reinterpret_cast<uintx2*>(p + PLANE) = w;
+      w.x = l[0]; w.y = l[1]; *reinterpret_cast<uintx2*>(p + 2 * PLANE) = w;
+    }
+  }
+  static __device__ __forceinline__ bf16x8 frag(const unsigned* __restrict__ buf, int plane, int line0, int lane) {
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uintx4*>(buf + plane * PLANE + (lane >> 5) * (4 * OUT) +
+                                                                       (line0 + (lane & 31)) * 4));
   }
 };
 
@@ -523,6 +560,55 @@ __global__ __launch_bounds__(256) void k_log_fwd_join(const float* __restrict__ 
 }
 
 // ------------------------------------------------------- sampling sweep
+// split_slab with the four accumulators finished two at a time: block row 0's products, then block row
+// 1's with done(0) - vector work on the finished accumulators, 64 instructions - spread between them.
+// done(1) is left to the caller, beside its staging.  Every accumulator takes its products in
+// split_slab's order.
+template <class SR, class SC, class Done>
+__device__ __forceinline__ void split_slab_rows(const unsigned* __restrict__ R, const unsigned* __restrict__ Cs, int wr0,
+                                                int wc0, int lane, floatx16 (&acc)[2][2], Done&& done) {
+  bf16x8 rh[2], rm[2], rl[2], ch[2], cm[2], cl[2];
+  rh[0] = SR::frag(R, 0, wr0, lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) cl[i] = SC::frag(Cs, 2, wc0 + 32 * i, lane);
+  rl[0] = SR::frag(R, 2, wr0, lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) ch[i] = SC::frag(Cs, 0, wc0 + 32 * i, lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) cm[i] = SC::frag(Cs, 1, wc0 + 32 * i, lane);
+  rm[0] = SR::frag(R, 1, wr0, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_setprio(3);
+  auto products = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rh[r], cl[x], acc[r][x]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rl[r], ch[x], acc[r][x]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rh[r], cm[x], acc[r][x]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rm[r], cm[x], acc[r][x]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rm[r], ch[x], acc[r][x]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) acc[r][x] = mfma_bf16(rh[r], ch[x], acc[r][x]);
+  };
+  products(0);
+  rh[1] = SR::frag(R, 0, wr0 + 32, lane);
+  rl[1] = SR::frag(R, 2, wr0 + 32, lane);
+  rm[1] = SR::frag(R, 1, wr0 + 32, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  products(1);
+  done(0);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // The sampling sweep described in logbmm_mfma.h: the forward's contraction again on its fp32
 // factors EA, EB - cut into their three parts while they are staged, no exponential - with the
 // accumulators started at -t, t = u S the cell's target; after every slab of 16 terms a
@@ -533,8 +619,16 @@ __global__ __launch_bounds__(256) void k_log_fwd_join(const float* __restrict__ 
 // forward's order, so the sums the sweep compares with its targets are the forward's.  A tile
 // with a cell whose S is below 2^-40 or not finite, or that lies in a tile the forward
 // flagged, sets that flag and leaves: the forward's tile is redone exactly.  128 x 128 tiles of
-// four waves with 256 registers (64 accumulators and 64 history registers per lane); always
-// the any-size form of the loaders.
+// four waves with 256 registers (64 accumulators and 64 history registers per lane); any sizes, N >= 4.
+//
+// What bounds it: matrix instructions (24 a slab and wave) and the vector instructions beside them (128 for the
+// history, about 100 to cut and stage) with two waves on a SIMD.  So half of the history is spread between the
+// slab's second twelve matrix instructions, no load stands under a branch of a lane's own (pieces beyond an
+// edge are read from the last lines and feed cells that are not stored), targets and results change
+// places with the accumulator layout in a wave's own LDS strip.  Forward and draw, both gradients of (64, 512^3):
+// 642 -> 537 us against loads, targets and stores under a branch per lane or cell - the loads of a slab were
+// waited for ahead of the products, a tile's targets formed one trip to memory after the other -, operands put
+// together word by word (SplitS) and the history behind all products.
 template <class T>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restrict__ ws_eb,
@@ -542,11 +636,12 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
                           int* __restrict__ flags, float* __restrict__ remw, int32_t* __restrict__ idx,
                           uint64_t seed, uint64_t offset, int M, int K, int N, int tiles_m, int tiles_n, int ftr,
                           int ftc, int ftiles_m, int ftiles_n, int tmask) {
-  constexpr bool RAGGED = true;
   constexpr int NT = T::NT;
   using SA = SplitT<T::TR, NT>;
-  using SB = SplitS<T::TC, NT>;
-  static_assert(SB::LW == 4, "");
+  using SB = SplitL<T::TC, NT>;
+  constexpr int ST = SB::ST;
+  static_assert(T::TR + T::TC == NT, "one shift per thread");
+  static_assert(split_lds_words<SA, SB>() >= (NT / 64) * kStripFloats, "");
   __shared__ __attribute__((aligned(16))) unsigned smem[split_lds_words<SA, SB>()];
   auto As = [&](int buf) __attribute__((always_inline)) { return smem + buf * SA::BUF; };
   auto Bs = [&](int buf) __attribute__((always_inline)) { return smem + 2 * SA::BUF + buf * SB::BUF; };
@@ -558,136 +653,163 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
   const int m0 = (rem / tiles_n) * T::TR, n0 = (rem % tiles_n) * T::TC;
   const float* st = stats + (long)batch * (M + N);
 
-  // ---- targets: -t = -u S per cell into `remw`, row by row, four adjacent cells per lane and
-  // step (they share one Philox block when rows are a multiple of four cells); then the
-  // accumulators pick their cells up in the matrix-core layout.  The flags are the forward's,
-  // one per tile of ITS shape (ftr x ftc).
+  // ---- the guard.  The flags are the forward's, one per tile of ITS shape (ftr x ftc): S >= 2^-40 and finite
+  // wherever a flag is clear.  What `out` adds is its rounding: a cell passes where alpha + beta - out, i.e.
+  // -log S as `out` tells it, is at most 40 ln 2 + 1e-3.  While no shift of the tile exceeds 2048 both roundings
+  // together stay below 2.5e-4 and no cell can fail; otherwise, and for half types, the cells are looked at.
   int* flag = flags + (batch * ftiles_m + m0 / ftr) * ftiles_n + n0 / ftc;
-  const float lim = kMfmaGuardBits * kLn2 + 1e-3f;
   int bad = *flag;
   {
-    constexpr int QR = T::TC / 4;  // quads per tile row
-    const bool blocks = (N & 3) == 0;
-#pragma unroll 4
-    for (int q = tid; q < T::TR * QR; q += NT) {
-      const int r = q / QR, m = m0 + r, n = n0 + (q - r * QR) * 4;
-      if (RAGGED && (m >= M || n >= N)) continue;
-      const long cell = ((long)batch * M + m) * N + n;
-      const int cn = RAGGED ? clamp4(N - n) : 4;
-      float u[4];
-      philox_uniform4((uint64_t)cell, blocks, seed, offset, u);
-      const float alr = st[m];
-      const float4 be4 = ld4m(st + M + n, cn, 0.f), o4 = ld4m(out + cell, cn, 0.f);
-      const float4 r4 = ld4m(remw + cell, cn, 1.f);  // the forward's 1 / S
-      const float bev[4] = {be4.x, be4.y, be4.z, be4.w}, ov[4] = {o4.x, o4.y, o4.z, o4.w};
-      const float rv[4] = {r4.x, r4.y, r4.z, r4.w};
-      float tv[4];
+    const int line = tid < T::TR ? min(m0 + tid, M - 1) : M + min(n0 + tid - T::TR, N - 1);
+    const int look = !kElemF32 || !(__builtin_fabsf(st[line]) <= 2048.f);
+    if (__syncthreads_or(look)) {  // uniform
+      constexpr int QR = T::TC / 4;  // quads per tile row
+      const float lim = kMfmaGuardBits * kLn2 + 1e-3f;
+      for (int q = tid; q < T::TR * QR; q += NT) {
+        const int r = q / QR, m = m0 + r, n = n0 + (q - r * QR) * 4;
+        if (m >= M || n >= N) continue;
+        const int cn = clamp4(N - n);
+        const float alr = st[m];
+        const float4 be4 = ld4m(st + M + n, cn, 0.f), o4 = ld4m(out + ((long)batch * M + m) * N + n, cn, 0.f);
+        const float bev[4] = {be4.x, be4.y, be4.z, be4.w}, ov[4] = {o4.x, o4.y, o4.z, o4.w};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float e = alr + bev[j] - ov[j];  // -log S
-        if (j < cn && (!(e <= lim) || !(e > -INFINITY))) bad = 1;
-        tv[j] = -(u[j] * kSampleShrink) * __builtin_amdgcn_rcpf(rv[j]);
+        for (int j = 0; j < 4; ++j) {
+          const float e = alr + bev[j] - ov[j];  // -log S
+          if (j < cn && (!(e <= lim) || !(e > -INFINITY))) bad = 1;
+        }
       }
-      st4m(remw + cell, cn, make_float4(tv[0], tv[1], tv[2], tv[3]));
     }
   }
-  bad = __syncthreads_or(bad);  // also: the tile's -t are visible to the whole workgroup
-  if (bad) {
+  if (__syncthreads_or(bad)) {
     if (tid == 0) *flag = 1;
     return;
   }
+
+  // ---- targets: -t = -u S for the wave's 64 x 64 cells, a lane four adjacent cells of sixteen rows (they share
+  // one Philox block when rows are a multiple of four cells), and on to the accumulator layout through the
+  // wave's strip.  Pieces beyond an edge are read from the last lines, a piece astride the right one moved down.
   floatx16 acc[2][2];
   int low[2][2][16];
-  const int col = lane & 31;
+  float* strip = reinterpret_cast<float*>(smem) + wave * kStripFloats;
+  const int lr = lane >> 4, lc = (lane & 15) * 4;
+  const long cell0 = (long)batch * M * N;
+  {
+    const int n = n0 + wn0 + lc, nc = min(n, N - 4), by = n - nc;
+    const bool blocks = (N & 3) == 0;
+    float4 r4[16];
 #pragma unroll
-  for (int br = 0; br < 2; ++br)
+    for (int t = 0; t < 16; ++t) r4[t] = ld4(remw + cell0 + (long)min(m0 + wm0 + lr + 4 * t, M - 1) * N + nc);
 #pragma unroll
-    for (int bc = 0; bc < 2; ++bc) {
-      const int n = n0 + wn0 + bc * 32 + col;
+    for (int q = 0; q < 4; ++q) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = m0 + wm0 + br * 32 + mfma_row(i, lane);
-        const bool ok = !RAGGED || (m < M && n < N);
-        const float nt = ok ? remw[((long)batch * M + m) * N + n] : 0.f;
-        acc[br][bc][i] = nt;
-        low[br][bc][i] = __float_as_int(nt) | tmask;  // all tag bits set: no slab has ended below t
+      for (int t = 0; t < 4; ++t) {
+        float u[4], rv[4] = {r4[4 * q + t].x, r4[4 * q + t].y, r4[4 * q + t].z, r4[4 * q + t].w};
+        shift_down<4>(rv, by);
+        philox_uniform4((uint64_t)(cell0 + (long)(m0 + wm0 + 16 * q + 4 * t + lr) * N + n), blocks, seed, offset, u);
+        float tv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tv[j] = -(u[j] * kSampleShrink) * __builtin_amdgcn_rcpf(rv[j]);
+        *reinterpret_cast<float4*>(strip + (lr + 4 * t) * 64 + lc) = make_float4(tv[0], tv[1], tv[2], tv[3]);
       }
+      wave_lds_sync();
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float nt = strip[(mfma_row_u(i) + mfma_row_l(lane)) * 64 + c * 32 + (lane & 31)];
+          acc[q >> 1][c][(q & 1) * 8 + i] = nt;
+          low[q >> 1][c][(q & 1) * 8 + i] = __float_as_int(nt) | tmask;  // all tag bits: no slab has ended below t
+        }
+      wave_lds_sync();
     }
+  }
+  __syncthreads();  // the strips make way for the staged slabs
 
-  // ---- staging of EA ([line][reduction]) and EB (pairs of reduction steps), zeros beyond the matrix
-  const int bcol = n0 + SB::line0(tid);
-  const int cb = clamp4(N - bcol);
-  const int brow = 2 * SB::pair(tid);
-  bool va[SA::PER];
+  // ---- staging of EA ([line][reduction]) and EB ([reduction][line]).  A slab's loads are the same whatever it
+  // meets - behind a branch the compiler waits for them ahead of the products they should hide behind - so the
+  // last slab of a ragged K reads on past the end of its rows (into the workspace array that follows, at the very
+  // end) and what lies beyond K is zeroed when it is staged.
   const float* pa[SA::PER];
 #pragma unroll
-  for (int l = 0; l < SA::PER; ++l) {
-    const int line = m0 + SA::line(tid, l);
-    va[l] = line < M;
-    pa[l] = ws_ea + ((long)batch * M + (va[l] ? line : M - 1)) * K + SA::quad(tid) * 4;
-  }
-  const float* pb = ws_eb + ((long)batch * K + brow) * N + (cb > 0 ? bcol : 0);
-  const int ktail = K % kMS;
-  const int slabs = (K + kMS - 1) / kMS;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 ra[SA::PER], rbe, rbo;
-  int s_load = 0, s_mma = 0;
+  for (int l = 0; l < SA::PER; ++l)
+    pa[l] = ws_ea + ((long)batch * M + min(m0 + SA::line(tid, l), M - 1)) * K + SA::quad(tid) * 4;
+  const int brow = SB::step0(tid), bcol = min(n0 + SB::line(tid), N - 1);
+  const float* pb = ws_eb + ((long)batch * K + brow) * N;  // uniform
+  const int ktail = K % kMS, slabs = (K + kMS - 1) / kMS;
+  float4 ra[SA::PER];
+  float rb[ST];
   auto load = [&]() __attribute__((always_inline)) {
-    if (ktail != 0 && s_load == slabs - 1) {
-      const int ca = clamp4(ktail - SA::quad(tid) * 4);
 #pragma unroll
-      for (int l = 0; l < SA::PER; ++l) ra[l] = va[l] ? ld4m(pa[l], ca, 0.f) : zero;
-      rbe = brow < ktail ? ld4m(pb, cb, 0.f) : zero;
-      rbo = brow + 1 < ktail ? ld4m(pb + N, cb, 0.f) : zero;
-    } else {
-#pragma unroll
-      for (int l = 0; l < SA::PER; ++l) ra[l] = va[l] ? ld4(pa[l]) : zero;
-      rbe = ld4m(pb, cb, 0.f);
-      rbo = ld4m(pb + N, cb, 0.f);
+    for (int l = 0; l < SA::PER; ++l) {
+      ra[l] = ld4(pa[l]);
+      pa[l] += kMS;
     }
 #pragma unroll
-    for (int l = 0; l < SA::PER; ++l) pa[l] += kMS;
+    for (int j = 0; j < ST; ++j) rb[j] = pb[(long)j * N + bcol];
     pb += (long)kMS * N;
-    ++s_load;
   };
-  auto stage = [&](int buf) __attribute__((always_inline)) {
+  auto stage = [&](int slab) __attribute__((always_inline)) {
+    if (ktail != 0 && slab == slabs - 1) {  // uniform
+      const int ca = ktail - SA::quad(tid) * 4;
 #pragma unroll
-    for (int l = 0; l < SA::PER; ++l) SA::put(As(buf), tid, l, ra[l]);
-    SB::put(Bs(buf), tid, rbe, rbo);
+      for (int l = 0; l < SA::PER; ++l)
+        ra[l] = make_float4(ca > 0 ? ra[l].x : 0.f, ca > 1 ? ra[l].y : 0.f, ca > 2 ? ra[l].z : 0.f, ca > 3 ? ra[l].w : 0.f);
+#pragma unroll
+      for (int j = 0; j < ST; ++j) rb[j] = brow + j < ktail ? rb[j] : 0.f;
+    }
+#pragma unroll
+    for (int l = 0; l < SA::PER; ++l) SA::put(As(slab & 1), tid, l, ra[l]);
+    SB::put(Bs(slab & 1), tid, rb);
+  };
+  int keep = ~tmask;
+  asm("" : "+v"(keep));  // a vector register: with the tag one v_and_or_b32 per cell (one scalar operand at most)
+  auto multiply = [&](int slab) __attribute__((always_inline)) {
+    const int tag = (tmask - 1 - slab) & tmask;
+    auto history = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          low[r][x][i] = min(low[r][x][i], (__float_as_int(acc[r][x][i]) & keep) | tag);
+          asm volatile("" : "+v"(low[r][x][i]));  // here, not sunk behind the staging
+        }
+    };
+    split_slab_rows<SA, SB>(As(slab & 1), Bs(slab & 1), wm0, wn0, lane, acc, history);
+    history(1);
   };
   load();
   stage(0);
-  split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-    split_slab<SA, SB>(As(buf), Bs(buf), wm0, wn0, wave, lane, acc);
-    const int tag = tmask - 1 - s_mma;
-    ++s_mma;
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int v = (__float_as_int(acc[x >> 1][x & 1][i]) & ~tmask) | (tag & tmask);  // one v_bfi_b32
-        low[x >> 1][x & 1][i] = min(low[x >> 1][x & 1][i], v);
-      }
-  });
+  __syncthreads();
+  for (int s = 0; s + 1 < slabs; ++s) {
+    load();
+    multiply(s);
+    stage(s + 1);
+    __syncthreads();
+  }
+  multiply(slabs - 1);
+  __syncthreads();  // every wave is done with the staged slabs
 
-  // ---- slab in which the prefix passes t, and rem at its start
+  // ---- slab in which the prefix passes t, and rem at its start, row by row
+  const int cc = clamp4(N - (n0 + wn0 + lc)), rows_left = M - (m0 + wm0) - lr;
+  const long ubase = cell0 + (long)(m0 + wm0) * N + n0 + wn0 + lr * N + lc;
+  floatx16 code[2][2];
 #pragma unroll
-  for (int br = 0; br < 2; ++br)
+  for (int x = 0; x < 4; ++x)
 #pragma unroll
-    for (int bc = 0; bc < 2; ++bc) {
-      const int n = n0 + wn0 + bc * 32 + col;
-      if (RAGGED && n >= N) continue;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = m0 + wm0 + br * 32 + mfma_row(i, lane);
-        if (RAGGED && m >= M) continue;
-        const long cell = ((long)batch * M + m) * N + n;
-        const int below = tmask - (low[br][bc][i] & tmask);
-        // a target that the sums never reach lies within their rounding of the total: the last term
-        idx[cell] = below >= slabs ? K - 1 : -2 - below;
-        remw[cell] = -__int_as_float(low[br][bc][i] & ~tmask);
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int v = low[x >> 1][x & 1][i], below = tmask - (v & tmask);
+      // a target that the sums never reach lies within their rounding of the total: the last term
+      code[x >> 1][x & 1][i] = __int_as_float(below >= slabs ? K - 1 : -2 - below);
+      acc[x >> 1][x & 1][i] = -__int_as_float(v & ~tmask);
     }
+  auto rows_to = [&](const floatx16 (&src)[2][2], float* dst) __attribute__((always_inline)) {
+    acc_rows(src, strip, lane, [](int) {}, [&](int q, int t, float4 v) __attribute__((always_inline)) {
+      const int ru = 16 * q + 4 * t;
+      if (cc > 0 && ru < rows_left) st4m(dst + ubase + (long)ru * N, cc, v);
+    });
+  };
+  rows_to(code, reinterpret_cast<float*>(idx));  // bit patterns
+  rows_to(acc, remw);
 }
 
 // ---------------------------------------------------------------- backward

@@ -862,6 +862,34 @@ def test_sample_index_brackets_cdf(gpu, use_stats, B, M, K, N):
     assert not torch.equal(idx, idx2)
 
 
+@pytest.mark.parametrize("shift", [0.0, 3000.0])
+@pytest.mark.parametrize("B,M,K,N", [(1, 96, 16, 96), (2, 129, 17, 97), (1, 97, 31, 99), (2, 191, 33, 130), (1, 257, 96, 129),
+                                     (1, 100, 993, 101)])
+def test_sample_sweep_at_tile_edges(gpu, shift, B, M, K, N):
+    """The matrix-core sweep where its 128 x 128 tiles, pieces of four columns and slabs of 16 terms end inside the
+    matrix, one slab alone, and more slabs than a six-bit tag numbers; with shifts beyond 2048 the guard reads `out`
+    as well.  Every index brackets its uniform: the sums carry one rounding per slab and part, 993 / 16 * 2^-24 * 6 =
+    2.2e-5 of the total at the longest; a seven-bit tag leaves rem 1.5e-5 short."""
+    torch.manual_seed(M + K)
+    a, b = 2 * torch.randn(B, M, K), 2 * torch.randn(B, K, N)
+    a[:, 1::3] += shift
+    lib = _lib.load()
+    ad, bd = a.to(gpu), b.to(gpu)
+    out = torch.empty(B, M, N, device=gpu)
+    idx = torch.empty(B, M, N, dtype=torch.int32, device=gpu)
+    stats = torch.empty(lib.genbmm_samplebmm_stats_size(B, M, K, N), device=gpu)
+    assert lib.genbmm_samplebmm_fwd(_lib.ptr(ad), _lib.ptr(bd), _lib.ptr(out), _lib.ptr(idx), _lib.ptr(stats),
+                                    31, 4, B, M, K, N, _lib.stream_of(ad)) == 0
+    close(out, lse64(a, b))
+    u = oracle.philox_uniform(0, B * M * N, 31, 4).view(B, M, N).double()
+    cdf = oracle.sample_cdf64(a, b)
+    got = idx.cpu().long()
+    assert int(got.min()) >= 0 and int(got.max()) < K
+    hi = torch.gather(cdf, 2, got.unsqueeze(2)).squeeze(2)
+    lo = torch.where(got > 0, torch.gather(cdf, 2, (got - 1).clamp(min=0).unsqueeze(2)).squeeze(2), torch.zeros_like(hi))
+    assert bool(((lo - 4e-5 <= u) & (u <= hi + 4e-5)).all())
+
+
 @pytest.mark.parametrize("B,M,K,N", [(2, 40, 4096, 30), (1, 16, 6000, 16), (2, 100, 2101, 97), (1, 7, 8192, 5)])
 def test_sample_on_long_reductions_with_few_tiles(gpu, B, M, K, N):
     """samplebmm on a problem whose forward cuts the reduction axis into pieces: the draw picks the
