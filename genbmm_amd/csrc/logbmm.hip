@@ -921,7 +921,7 @@ int launch_fwd_split(DenseArgs p, float* stats, int B, int M, int K, int N, int 
   if (total64 > 0x7fffffffLL) return GENBMM_E_SHAPE;
   const int total = (int)total64;
   int* flags = fwd_flags_of(stats, B, M, N);
-  constexpr int lds = 4 * split_lds_words<SplitT<T::TR, T::NT>, SplitS<T::TC, T::NT>>();
+  constexpr int lds = 4 * split_lds_words<SplitT<T::TR, T::NT>, SplitL<T::TC, T::NT>>();
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
   auto go = [&](auto kern) {
     allow_lds(kern, lds);
@@ -1086,7 +1086,7 @@ int launch_fwd_pieces(DenseArgs p, float* stats, int B, int M, int K, int N, int
   p.vec_o = (N % 4 == 0) && aligned16(p.out);
   const int total = B * p.tiles_m * p.tiles_n;  // below 128
   int* flags = fwd_flags_of(stats, B, M, N);
-  constexpr int lds = 4 * split_lds_words<SplitT<T::TR, T::NT>, SplitS<T::TC, T::NT>>();
+  constexpr int lds = 4 * split_lds_words<SplitT<T::TR, T::NT>, SplitL<T::TC, T::NT>>();
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
   float* parts = ws.ea;
   auto kern = k_log_fwd_split<T, true, kKeepNone, true>;

@@ -29,7 +29,11 @@
 //  * an operand whose source is [reduction][line]: plane[8 step pairs][lines + 8]; a lane
 //    stages a pair of reduction steps for LW consecutive lines (the pair shares a word;
 //    one store of LW words per plane) and reads its eight steps as four words a row apart.
-//  * the same, staged by a line's own threads (SplitL): plane[half of the slab][line][4 words].
+//  * the same, staged by a line's own threads (SplitL, what forward, backward and sweep use): plane[half of the
+//    slab][line][4 words], an operand one 16-byte read.  The form above takes four reads an operand, which the
+//    compiler pairs across operands and then moves apart (24 moves and a wait for each pair per slab, ahead of the
+//    products): (64, 512^3) forward 108 -> 102 us, both gradients 229 -> 210; (48, 251, 173, 301) 33.8 -> 28.8
+//    and 49.8 -> 46.6, results bit for bit.
 #pragma once
 
 #include "logbmm_mfma.h"
@@ -291,8 +295,8 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
   constexpr bool KEEP = KEEPS == kKeepFactors;
   constexpr int NT = T::NT;
   using SA = SplitT<T::TR, NT>;
-  using SB = SplitS<T::TC, NT>;
-  constexpr int LW = SB::LW;
+  using SB = SplitL<T::TC, NT>;
+  constexpr int ST = SB::ST;
   extern __shared__ __attribute__((aligned(16))) unsigned split_smem[];
   static_assert(split_lds_words<SA, SB>() >= (NT / 64) * kStripFloats, "");
   auto As = [&](int buf) __attribute__((always_inline)) { return split_smem + buf * SA::BUF; };
@@ -310,8 +314,7 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
   const int slabs_piece = PIECES ? (slabs_all + pieces - 1) / pieces : slabs_all;
   const int slab0 = piece * slabs_piece;
 
-  // a pieces: line m0 + line(l), four k from quad * 4;  the b piece: rows 2 pair, 2 pair + 1 of the
-  // slab, LW columns from bcol
+  // a pieces: line m0 + line(l), four k from quad * 4;  b: ST steps of one column
   const elem_t* pa[SA::PER];
   float al[SA::PER];
   bool va[SA::PER];
@@ -326,14 +329,12 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
   // ahead of what is being staged, whichever side of its products a wave stages on)
   const int nblk = rem % tiles_n, mblk = rem / tiles_n;
   const long da = KEEP ? ws_distance(ws_ea, a) - 4l * kMS : 0, db = KEEP ? ws_distance(ws_eb, b) - 4l * kMS * N : 0;
-  int s_stage = 0, sa = 0, sb = 0;  // the slab the next stage() forms; s_stage mod tiles_n, mod tiles_m
-  const int bcol = n0 + SB::line0(tid);
-  const int cb = RAGGED ? clampw(N - bcol, LW) : LW;  // columns of the b piece inside the matrix
-  const int brow = 2 * SB::pair(tid);
-  const elem_t* pb = b + ((long)batch * K + brow + (long)slab0 * kMS) * N + (cb > 0 ? bcol : 0);
-  float be[LW];
-#pragma unroll
-  for (int j = 0; j < LW; ++j) be[j] = j < cb ? st[M + bcol + j] : INFINITY;
+  int sa = 0, sb = 0;  // the slab the next stage() forms, mod tiles_n and mod tiles_m
+  const int brow = SB::step0(tid);  // uniform
+  const bool vb = !RAGGED || n0 + SB::line(tid) < N;
+  const unsigned bcol = vb ? n0 + SB::line(tid) : N - 1;
+  const elem_t* pb = b + ((long)batch * K + brow + (long)slab0 * kMS) * N;
+  const float be = vb ? st[M + bcol] : INFINITY;
   if (!PIECES && tile == 0 && tid == 0) {
     ws_hdr[1] = T::TR;
     ws_hdr[2] = T::TC;
@@ -347,72 +348,69 @@ void k_log_fwd_split(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
     for (int i = 0; i < 16; ++i) acc[x >> 1][x & 1][i] = 0.f;
 
   const int slabs = PIECES ? min(slabs_piece, slabs_all - slab0) : slabs_all;
-  // reduction steps of a partial last slab (of the last piece)
+  // reduction steps of a partial last slab (of the last piece): one more step behind the loop, with a loader of
+  // its own - the loads of the loop stand under no branch, where they would be waited for ahead of the products
   const int ktail = RAGGED && (!PIECES || slab0 + slabs == slabs_all) ? K % kMS : 0;
-  int s_load = 0;                                  // the slab the next load() fetches
+  const int whole = slabs - (RAGGED && ktail != 0 ? 1 : 0);
   float4 ra[SA::PER];
-  float rbe[LW], rbo[LW];
+  elem_t rb[ST];
   auto load = [&]() __attribute__((always_inline)) {
-    if (RAGGED && ktail != 0 && s_load == slabs - 1) {
-      const int ca = clamp4(ktail - SA::quad(tid) * 4);
 #pragma unroll
-      for (int l = 0; l < SA::PER; ++l) ra[l] = ld4m(pa[l], ca, -INFINITY);
-      ldwm<LW>(pb, brow < ktail ? cb : 0, -INFINITY, rbe);
-      ldwm<LW>(pb + N, brow + 1 < ktail ? cb : 0, -INFINITY, rbo);
-    } else {
+    for (int l = 0; l < SA::PER; ++l) ra[l] = ld4(pa[l]);
 #pragma unroll
-      for (int l = 0; l < SA::PER; ++l) ra[l] = ld4(pa[l]);
-      if (RAGGED) {
-        ldwm<LW>(pb, cb, -INFINITY, rbe);
-        ldwm<LW>(pb + N, cb, -INFINITY, rbo);
-      } else {
-        ldw<LW>(pb, rbe);
-        ldw<LW>(pb + N, rbo);
-      }
-    }
+    for (int j = 0; j < ST; ++j) rb[j] = (pb + (long)j * N)[bcol];
 #pragma unroll
     for (int l = 0; l < SA::PER; ++l) pa[l] += kMS;
     pb += (long)kMS * N;
-    ++s_load;
   };
-  auto stage = [&](int buf) __attribute__((always_inline)) {
-    const bool tail = RAGGED && ktail != 0 && s_stage == slabs - 1;
+  auto stage_to = [&](int buf, int steps) __attribute__((always_inline)) {
 #pragma unroll
     for (int l = 0; l < SA::PER; ++l) {
       const float4 e = exp4(ra[l], al[l]);
       SA::put(As(buf), tid, l, e);
       if (KEEP && sa == nblk) {
         if (!RAGGED) st4(ws_twin(pa[l], da), e);
-        else if (va[l]) st4m(ws_twin(pa[l], da), tail ? clamp4(ktail - SA::quad(tid) * 4) : 4, e);
+        else if (va[l]) st4m(ws_twin(pa[l], da), clamp4(steps - SA::quad(tid) * 4), e);
       }
     }
-    float ee[LW], eo[LW];
+    float eb[ST];
 #pragma unroll
-    for (int j = 0; j < LW; ++j) {
-      ee[j] = exp_st(rbe[j] - be[j]);
-      eo[j] = exp_st(rbo[j] - be[j]);
-    }
-    SB::put(Bs(buf), tid, ee, eo);
+    for (int j = 0; j < ST; ++j) eb[j] = exp_st((float)rb[j] - be);
+    SB::put(Bs(buf), tid, eb);
     if (KEEP && sb == mblk) {
       float* we = ws_twin(pb, db);
 #pragma unroll
-      for (int j = 0; j < LW; ++j) {
-        if (j < cb && (!tail || brow < ktail)) we[j] = ee[j];
-        if (j < cb && (!tail || brow + 1 < ktail)) we[N + j] = eo[j];
-      }
+      for (int j = 0; j < ST; ++j)
+        if (vb && brow + j < steps) (we + (long)j * N)[bcol] = eb[j];
     }
     if (KEEP) {
-      ++s_stage;
       sa = sa + 1 == tiles_n ? 0 : sa + 1;
       sb = sb + 1 == tiles_m ? 0 : sb + 1;
     }
   };
+  auto stage = [&](int buf) __attribute__((always_inline)) { stage_to(buf, kMS); };
 
-  load();
-  stage(0);
-  split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-    split_slab<SA, SB>(As(buf), Bs(buf), wm0, wn0, wave, lane, acc);
-  });
+  if (!PIECES || whole > 0) {
+    load();
+    stage(0);
+    split_loop(whole, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
+      split_slab<SA, SB>(As(buf), Bs(buf), wm0, wn0, wave & (NT / 64 - 1), lane, acc);
+    });
+  }
+  if (RAGGED && ktail != 0) {  // uniform
+#pragma unroll
+    for (int l = 0; l < SA::PER; ++l) {
+      ra[l] = ld4m(pa[l], clamp4(ktail - SA::quad(tid) * 4), -INFINITY);
+      pa[l] += kMS;
+    }
+#pragma unroll
+    for (int j = 0; j < ST; ++j) rb[j] = brow + j < ktail ? (pb + (long)j * N)[bcol] : (elem_t)-INFINITY;
+    pb += (long)kMS * N;
+    stage_to(0, ktail);
+    __syncthreads();
+    split_slab<SA, SB>(As(0), Bs(0), wm0, wn0, wave & (NT / 64 - 1), lane, acc);
+    __syncthreads();
+  }
 
   if constexpr (PIECES) {  // the piece's sums, row-wise; the guard is k_log_fwd_join's
     __syncthreads();       // every wave is done with the staging buffers
@@ -822,8 +820,8 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
 template <class T, bool GRAD_A>
 struct SplitBwd {
   static constexpr int NT = T::NT;
-  using SR = std::conditional_t<GRAD_A, SplitT<T::TR, NT>, SplitS<T::TR, NT>>;
-  using SC = std::conditional_t<GRAD_A, SplitT<T::TC, NT>, SplitS<T::TC, NT>>;
+  using SR = std::conditional_t<GRAD_A, SplitT<T::TR, NT>, SplitL<T::TR, NT>>;
+  using SC = std::conditional_t<GRAD_A, SplitT<T::TC, NT>, SplitL<T::TC, NT>>;
   static constexpr int WORDS = split_lds_words<SR, SC>();
 };
 
@@ -949,7 +947,7 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
     if (bwd_tile_flagged(ws_hdr, fwd_flags, kNeed, true, r0, T::TR, batch, M, N, tid, NT)) return;
     stage(0);
     split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
+      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave & (NT / 64 - 1), lane, acc);
     });
     if (RAGGED && qtail != 0) {  // uniform
       const int left = qtail - beo;  // all pieces of a thread share their quad
@@ -963,99 +961,77 @@ __device__ __forceinline__ void log_bwd_split_tile(unsigned* __restrict__ smem, 
       bslab = ld4m(beb + beo, left, 0.f);
       stage(0);
       __syncthreads();
-      split_slab<SR, SC>(Rs(0), Cs(0), wr0, wc0, wave, lane, acc);
+      split_slab<SR, SC>(Rs(0), Cs(0), wr0, wc0, wave & (NT / 64 - 1), lane, acc);
       __syncthreads();
     }
   } else {
-    // rows: EA pieces (steps m, m + 1; LW lines k); columns: H pieces (steps m, m + 1; LW lines n);
-    // both operands' pieces of a thread are on the same pair of steps.  RAGGED: lines beyond the
-    // matrix re-read the last LW lines - they only feed results that are not stored -, and a piece that
-    // straddles the right edge reads the last LW lines too: the staged values then move down to the
-    // lines they belong to (a few lanes of the last tile; the branch costs the others nothing, where a
-    // loader that reads such a piece element by element would hold back every load behind it).
-    constexpr int LR = SR::LW, LC = SC::LW;
-    static_assert(SR::Q == SC::Q, "");
-    const int m2 = 2 * SR::pair(tid);
+    // rows: EA, SR::ST steps m of one line k; columns: H, SC::ST steps m of one line n.  Lines beyond the matrix
+    // re-read the last one: they only feed results that are not stored.  alpha of the slab's sixteen steps is one
+    // load of the wave's, read lane by lane.
+    constexpr int NR = SR::ST, NC = SC::ST;
+    const int r_s = SR::step0(tid), c_s = SC::step0(tid);  // uniform
     const elem_t* ab = src.a + (long)batch * M * K;
     const W_t* ob = wsrc + (long)batch * M * N;
     const elem_t* gb = g + (long)batch * M * N;
     const float* alb = al;
-    const int kc = RAGGED ? min(r0 + SR::line0(tid), K - LR) : r0 + SR::line0(tid);
-    const int nc = RAGGED ? min(c0 + SC::line0(tid), N - LC) : c0 + SC::line0(tid);
-    const int yo = m2 * K + kc, oo = m2 * N + nc;
-    const int sr = RAGGED ? r0 + SR::line0(tid) - kc : 0, sc = RAGGED ? c0 + SC::line0(tid) - nc : 0;
-    const bool straddle = RAGGED && ((sr > 0 && sr < LR) || (sc > 0 && sc < LC));
-    float bec[LC];
-#pragma unroll
-    for (int j = 0; j < LC; ++j) bec[j] = be[nc + j];
-    float ye[LR], yd[LR], oe[LC], od[LC], ge[LC], gd[LC];
-    float a0, a1;
+    const unsigned kc = RAGGED ? min(r0 + SR::line(tid), K - 1) : r0 + SR::line(tid);
+    const unsigned nc = RAGGED ? min(c0 + SC::line(tid), N - 1) : c0 + SC::line(tid);
+    const unsigned step = lane & (kMS - 1);
+    const float bec = be[nc];
+    elem_t ry[NR], rg[NC];
+    W_t ro[NC];
+    float als;
     auto load = [&]() __attribute__((always_inline)) {
-      ldw<LR>(ab + yo, ye);
-      ldw<LR>(ab + yo + K, yd);
-      ldw<LC>(ob + oo, oe);
-      ldw<LC>(ob + oo + N, od);
-      ldw<LC>(gb + oo, ge);
-      ldw<LC>(gb + oo + N, gd);
-      a0 = alb[m2];
-      a1 = alb[m2 + 1];
+#pragma unroll
+      for (int j = 0; j < NR; ++j) ry[j] = (ab + (long)(r_s + j) * K)[kc];
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        ro[j] = (ob + (long)(c_s + j) * N)[nc];
+        rg[j] = (gb + (long)(c_s + j) * N)[nc];
+      }
+      als = alb[step];
       ab += (long)kMS * K;
       ob += (long)kMS * N;
       gb += (long)kMS * N;
       alb += kMS;
     };
+    auto alpha = [&](int m) __attribute__((always_inline)) {
+      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(als), m));
+    };
     auto stage = [&](int buf) __attribute__((always_inline)) {
-      float e0[LR], e1[LR], h0[LC], h1[LC];
+      float e[NR], h[NC];
 #pragma unroll
-      for (int j = 0; j < LR; ++j) {
-        e0[j] = exp_st(ye[j] - a0);
-        e1[j] = exp_st(yd[j] - a1);
-      }
+      for (int j = 0; j < NR; ++j) e[j] = exp_st((float)ry[j] - alpha(r_s + j));
 #pragma unroll
-      for (int j = 0; j < LC; ++j) {
-        h0[j] = ge[j] * (RECIP ? oe[j] : exp_st(a0 + bec[j] - oe[j]));
-        h1[j] = gd[j] * (RECIP ? od[j] : exp_st(a1 + bec[j] - od[j]));
-      }
-      if (straddle) {
-        shift_down<LR>(e0, sr);
-        shift_down<LR>(e1, sr);
-        shift_down<LC>(h0, sc);
-        shift_down<LC>(h1, sc);
-      }
-      SR::put(Rs(buf), tid, e0, e1);
-      SC::put(Cs(buf), tid, h0, h1);
+      for (int j = 0; j < NC; ++j)
+        h[j] = (float)rg[j] * (RECIP ? (float)ro[j] : exp_st(alpha(c_s + j) + bec - (float)ro[j]));
+      SR::put(Rs(buf), tid, e);
+      SC::put(Cs(buf), tid, h);
     };
     if (RECIP && ws_hdr[0] != kWsRecip) return;  // uniform
     load();
     if (bwd_tile_flagged(ws_hdr, fwd_flags, kNeed, false, c0, T::TC, batch, M, N, tid, NT)) return;
     stage(0);
     split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
+      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave & (NT / 64 - 1), lane, acc);
     });
     if (RAGGED && qtail != 0) {  // uniform; steps beyond M re-read row M - 1 and are replaced by the fills
-      const int c0r = min(m2, qtail - 1), c1r = min(m2 + 1, qtail - 1);
-      ldw<LR>(ab + c0r * K + kc, ye);
-      ldw<LR>(ab + c1r * K + kc, yd);
-      ldw<LC>(ob + c0r * N + nc, oe);
-      ldw<LC>(ob + c1r * N + nc, od);
-      ldw<LC>(gb + c0r * N + nc, ge);
-      ldw<LC>(gb + c1r * N + nc, gd);
-      a0 = alb[c0r];
-      a1 = alb[c1r];
-      const bool in0 = m2 < qtail, in1 = m2 + 1 < qtail;
 #pragma unroll
-      for (int j = 0; j < LR; ++j) {
-        ye[j] = in0 ? ye[j] : -INFINITY;
-        yd[j] = in1 ? yd[j] : -INFINITY;
+      for (int j = 0; j < NR; ++j) {
+        ry[j] = (ab + (long)min(r_s + j, qtail - 1) * K)[kc];
+        ry[j] = r_s + j < qtail ? ry[j] : (elem_t)-INFINITY;
       }
 #pragma unroll
-      for (int j = 0; j < LC; ++j) {
-        ge[j] = in0 ? ge[j] : 0.f;
-        gd[j] = in1 ? gd[j] : 0.f;
+      for (int j = 0; j < NC; ++j) {
+        const long at = (long)min(c_s + j, qtail - 1) * N;
+        ro[j] = (ob + at)[nc];
+        rg[j] = (gb + at)[nc];
+        rg[j] = c_s + j < qtail ? rg[j] : (elem_t)0.f;
       }
+      als = alb[min((int)step, qtail - 1)];
       stage(0);
       __syncthreads();
-      split_slab<SR, SC>(Rs(0), Cs(0), wr0, wc0, wave, lane, acc);
+      split_slab<SR, SC>(Rs(0), Cs(0), wr0, wc0, wave & (NT / 64 - 1), lane, acc);
       __syncthreads();
     }
   }
