@@ -448,9 +448,9 @@ __global__ __launch_bounds__(BBTile::NT) __attribute__((amdgpu_waves_per_eu(BBTi
 void k_bb_mm(const BBMM p) {
   using T = BBTile;
   constexpr int NT = T::NT;
-  using SR = std::conditional_t<RT, SplitT<T::TR, NT>, SplitS<T::TR, NT>>;
-  using SC = std::conditional_t<CT, SplitT<T::TC, NT>, SplitS<T::TC, NT>>;
-  constexpr int PER = 2;  // a thread's pieces of either operand: four steps of two lines, or two steps of four
+  using SR = std::conditional_t<RT, SplitT<T::TR, NT>, SplitL<T::TR, NT>>;
+  using SC = std::conditional_t<CT, SplitT<T::TC, NT>, SplitL<T::TC, NT>>;
+  constexpr int PER = 2, ST = 8;  // a thread's pieces of an operand: four steps of two lines, or eight steps of one
   __shared__ __attribute__((aligned(16))) unsigned smem[split_lds_words<SR, SC>()];
   static_assert(split_lds_words<SR, SC>() >= (NT / 64) * kStripFloats, "");
   auto Rs = [&](int buf) __attribute__((always_inline)) { return smem + buf * SR::BUF; };
@@ -470,59 +470,76 @@ void k_bb_mm(const BBMM p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[x >> 1][x & 1][i] = acc0[x >> 1][x & 1][i] = 0.f;
 
-  // where this thread's pieces of the first slab lie in an operand of either layout
-  long ro[PER], co[PER];
+  // where this thread's pieces of the first slab lie in an operand of either layout: uniform base, lane offsets
+  long rbase, cbase;
+  unsigned ro[PER], co[PER];
+  if constexpr (RT) {
+    rbase = ((long)batch * p.Rp + r0) * Qp;
 #pragma unroll
-  for (int l = 0; l < PER; ++l) {
-    if constexpr (RT) ro[l] = ((long)batch * p.Rp + r0 + SR::line(tid, l)) * Qp + SR::quad(tid) * 4;
-    else ro[l] = ((long)batch * Qp + 2 * SR::pair(tid) + l) * p.Rp + r0 + SR::line0(tid);
-    if constexpr (CT) co[l] = ((long)batch * p.Cp + c0 + SC::line(tid, l)) * Qp + SC::quad(tid) * 4;
-    else co[l] = ((long)batch * Qp + 2 * SC::pair(tid) + l) * p.Cp + c0 + SC::line0(tid);
+    for (int l = 0; l < PER; ++l) ro[l] = SR::line(tid, l) * Qp + SR::quad(tid) * 4;
+  } else {
+    rbase = ((long)batch * Qp + SR::step0(tid)) * p.Rp + r0;
+    ro[0] = SR::line(tid);
+  }
+  if constexpr (CT) {
+    cbase = ((long)batch * p.Cp + c0) * Qp;
+#pragma unroll
+    for (int l = 0; l < PER; ++l) co[l] = SC::line(tid, l) * Qp + SC::quad(tid) * 4;
+  } else {
+    cbase = ((long)batch * Qp + SC::step0(tid)) * p.Cp + c0;
+    co[0] = SC::line(tid);
   }
   // the slabs of both products are one loop: the second's first slab is in flight under the first's last
-  const float *rb = p.rows[0], *cb = p.cols[0];
+  const float *rb = p.rows[0] + rbase, *cb = p.cols[0] + cbase;
   const long rstep = RT ? (long)kMS : (long)kMS * p.Rp, cstep = CT ? (long)kMS : (long)kMS * p.Cp;
   int s_load = 0;
-  float4 rr[PER], rc[PER];
+  float4 rr[RT ? PER : 1], rc[CT ? PER : 1];
+  float sr[RT ? 1 : ST], sc[CT ? 1 : ST];
   auto load = [&]() __attribute__((always_inline)) {
+    if constexpr (RT) {
 #pragma unroll
-    for (int l = 0; l < PER; ++l) {
-      rr[l] = ld4a(rb + ro[l]);
-      rc[l] = ld4a(cb + co[l]);
+      for (int l = 0; l < PER; ++l) rr[l] = ld4a(rb + ro[l]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < ST; ++j) sr[j] = (rb + (long)j * p.Rp)[ro[0]];
     }
-    rb += rstep;
-    cb += cstep;
-    if (++s_load == slabs) {  // uniform
-      rb = p.rows[1];
-      cb = p.cols[1];
+    if constexpr (CT) {
+#pragma unroll
+      for (int l = 0; l < PER; ++l) rc[l] = ld4a(cb + co[l]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < ST; ++j) sc[j] = (cb + (long)j * p.Cp)[co[0]];
     }
+    const bool next = ++s_load == slabs;  // uniform
+    rb = next ? p.rows[1] + rbase : rb + rstep;
+    cb = next ? p.cols[1] + cbase : cb + cstep;
   };
   auto stage = [&](int buf) __attribute__((always_inline)) {
     if constexpr (RT) {
 #pragma unroll
       for (int l = 0; l < PER; ++l) SR::put(Rs(buf), tid, l, rr[l]);
     } else {
-      SR::put(Rs(buf), tid, rr[0], rr[1]);
+      SR::put(Rs(buf), tid, sr);
     }
     if constexpr (CT) {
 #pragma unroll
       for (int l = 0; l < PER; ++l) SC::put(Cs(buf), tid, l, rc[l]);
     } else {
-      SC::put(Cs(buf), tid, rc[0], rc[1]);
+      SC::put(Cs(buf), tid, sc);
     }
   };
   load();
   stage(0);
   split_loop(slabs * p.pairs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-    split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc);
+    split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave & (NT / 64 - 1), lane, acc);
   });
   if (EPI == kEpiGrad && p.rows0) {  // uniform
-    rb = p.rows0;
-    cb = p.cols0;
+    rb = p.rows0 + rbase;
+    cb = p.cols0 + cbase;
     load();
     stage(0);
     split_loop(slabs, split_early<NT>(wave), load, stage, [&](int buf) __attribute__((always_inline)) {
-      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave, lane, acc0);
+      split_slab<SR, SC>(Rs(buf), Cs(buf), wr0, wc0, wave & (NT / 64 - 1), lane, acc0);
     });
   }
 

@@ -145,42 +145,12 @@ struct SplitL {
   }
 };
 
-// LW consecutive elements as floats
-template <int LW, class E>
-__device__ __forceinline__ void ldw(const E* p, float (&v)[LW]) {
-  if constexpr (LW == 4) {
-    const float4 t = ld4(p);
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-  } else {
-    typedef E e2u __attribute__((ext_vector_type(2), aligned(sizeof(E))));
-    const e2u t = *reinterpret_cast<const e2u*>(p);
-    v[0] = (float)t.x; v[1] = (float)t.y;
-  }
+// v[j] <- v[j + by] for 0 < by < 4 (the places behind keep what they hold); other `by`: nothing
+__device__ __forceinline__ void shift_down(float (&v)[4], int by) {
+  if (by == 1) { v[0] = v[1]; v[1] = v[2]; v[2] = v[3]; }
+  if (by == 2) { v[0] = v[2]; v[1] = v[3]; }
+  if (by == 3) v[0] = v[3];
 }
-
-// the first cnt of them (<= 0: none), `fill` for the rest
-template <int LW>
-__device__ __forceinline__ void ldwm(const elem_t* p, int cnt, float fill, float (&v)[LW]) {
-  if (cnt >= LW) {
-    ldw<LW>(p, v);
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < LW; ++j) v[j] = j < cnt ? (float)p[j] : fill;
-}
-// v[j] <- v[j + by] for 0 < by < LW (the places behind keep what they hold); other `by`: nothing
-template <int LW>
-__device__ __forceinline__ void shift_down(float (&v)[LW], int by) {
-  if constexpr (LW == 4) {
-    if (by == 1) { v[0] = v[1]; v[1] = v[2]; v[2] = v[3]; }
-    if (by == 2) { v[0] = v[2]; v[1] = v[3]; }
-    if (by == 3) v[0] = v[3];
-  } else {
-    static_assert(LW == 2, "");
-    if (by == 1) v[0] = v[1];
-  }
-}
-__device__ __forceinline__ int clampw(int x, int w) { return min(max(x, 0), w); }
 
 // The waves of a SIMD (waves i, i + 4, ... of the workgroup) run their matrix instructions at
 // different priorities, all above the priority of staging: behind a barrier they would otherwise
@@ -702,7 +672,7 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         float u[4], rv[4] = {r4[4 * q + t].x, r4[4 * q + t].y, r4[4 * q + t].z, r4[4 * q + t].w};
-        shift_down<4>(rv, by);
+        shift_down(rv, by);
         philox_uniform4((uint64_t)(cell0 + (long)(m0 + wm0 + 16 * q + 4 * t + lr) * N + n), blocks, seed, offset, u);
         float tv[4];
 #pragma unroll
