@@ -10,6 +10,7 @@ There is no CPU path: calling any op without the library, or with CPU tensors,
 raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
@@ -122,6 +123,24 @@ def load():
         fn.restype = ctypes.c_size_t
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The extension with the eager products' autograd nodes (once). Raises RuntimeError if it has not been built."""
+    global _host
+    if _host is None:
+        load()      # the library it is linked to
+        path = os.path.join(_HERE, "lib", "_host.so")
+        if not os.path.exists(path):
+            raise RuntimeError("genbmm_amd: %s is missing; build it with `python -m genbmm_amd.build`" % path)
+        spec = importlib.util.spec_from_file_location("genbmm_amd.lib._host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def version():

@@ -3,9 +3,9 @@
     python -m genbmm_amd.build
 
 This takes the place of the reference's setup.py (setup.py:1-27, a
-torch CUDAExtension named `_genbmm`): there is no pybind11 / torch extension
-here, only a plain shared library with a C ABI (include/genbmm_gfx950.h) that
-genbmm_amd/_lib.py loads with ctypes.  hipcc cross-compiles for gfx950 without
+torch CUDAExtension named `_genbmm`): the kernels are a plain shared library with a C ABI
+(include/genbmm_gfx950.h) that genbmm_amd/_lib.py loads with ctypes; beside it a small
+torch extension (csrc/host.cpp, lib/_host.so) holds the eager products' autograd nodes.  hipcc cross-compiles for gfx950 without
 a GPU being present.
 """
 import os
@@ -47,8 +47,38 @@ HIPCC_FLAGS = [
 EXTRA_FLAGS = {"banded.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
+# The eager route's autograd nodes (csrc/host.cpp): a Python extension linked to the library above, built by the
+# host compiler against torch's own headers.
+HOST_NAME = "_host.so"
+
+
 def lib_path():
     return os.path.join(LIBDIR, LIBNAME)
+
+
+def host_path():
+    return os.path.join(LIBDIR, HOST_NAME)
+
+
+def _host_commands(obj):
+    """(compile, link) commands of the host extension."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    cxx = shutil.which("g++") or "c++"
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    include = cpp_extension.include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"],
+                                               os.path.join(os.path.dirname(HERE), "include")]
+    compile_ = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+                "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    compile_ += [x for path in include for x in ("-isystem", path)]
+    compile_ += ["-c", os.path.join(CSRC, "host.cpp"), "-o", obj]
+    link = [cxx, "-shared", obj, "-o", host_path() + ".tmp", "-L" + LIBDIR, "-l:" + LIBNAME, "-L" + torch_lib,
+            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    return compile_, link
 
 
 def hipcc():
@@ -74,18 +104,28 @@ def build(verbose=True):
                 print(" ".join(cmd), flush=True)
             procs.append((src + suffix, obj,
                           subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
+    host_obj = os.path.join(objdir, "host.o")
+    host_compile, host_link = _host_commands(host_obj)
+    if verbose:
+        print(" ".join(host_compile), flush=True)
+    procs.append(("host.cpp", host_obj, subprocess.Popen(host_compile, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
     objs = []
     for src, obj, proc in procs:
         out = proc.communicate()[0].decode()
         if proc.returncode != 0:
-            raise RuntimeError("hipcc failed on %s:\n%s" % (src, out))
-        objs.append(obj)
+            raise RuntimeError("compiler failed on %s:\n%s" % (src, out))
+        if obj != host_obj:
+            objs.append(obj)
     tmp = lib_path() + ".tmp"
     cmd = [cc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc"] + objs + ["-o", tmp]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
     os.replace(tmp, lib_path())
+    if verbose:
+        print(" ".join(host_link), flush=True)
+    subprocess.run(host_link, check=True)
+    os.replace(host_path() + ".tmp", host_path())
     return lib_path()
 
 

@@ -4,8 +4,8 @@
     python setup.py build        # or: pip install --no-build-isolation .
 
 Takes the place of the reference's setup.py (a torch CUDAExtension named `_genbmm`,
-setup.py:1-27); there is no Python extension module here, only libgenbmm_gfx950.so,
-which genbmm_amd/_lib.py loads with ctypes.  The C header is installed next to it.
+setup.py:1-27): libgenbmm_gfx950.so, which genbmm_amd/_lib.py loads with ctypes, and beside it the
+extension with the eager products' autograd nodes.  The C header is installed next to it.
 """
 import os
 import shutil

@@ -1,0 +1,145 @@
+"""The eager route of csrc/host.cpp against the Python Functions it takes the place of: the same results bit for bit
+over types, sizes, layouts and the ways gradients are asked for, and the same calls refused."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+import genbmm_amd as genbmm
+from genbmm_amd import _lib, genmul
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.float16, torch.bfloat16]
+STREAM = (11, 4)
+
+
+def log_python(a, b):
+    return genmul.LogMatMul.apply(a, b, genmul.PATH_AUTO if a.dtype == torch.float32 else genmul.PATH_RECIP)
+
+
+PAIRS = {"log": (genbmm.logbmm, log_python), "max": (genbmm.maxbmm, genmul.MaxMatMul.apply),
+         "prodmax": (genbmm.prodmaxbmm, genmul.ProdMaxMatMul.apply),
+         "sample": (lambda a, b: genbmm.samplebmm(a, b, STREAM), lambda a, b: genmul.SampleMatMul.apply(a, b, STREAM))}
+
+
+def operands(gpu, B, M, K, N, dtype):
+    torch.manual_seed(B + M + K + N)
+    return [torch.randn(*s).to(gpu, dtype) for s in ((B, M, K), (B, K, N), (B, M, N))]
+
+
+def native(a, b):
+    return _lib.host().plain(a, b)
+
+
+@pytest.mark.parametrize("op", list(PAIRS))
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,M,K,N", [(1, 1, 1, 1), (3, 7, 5, 9), (2, 130, 97, 101), (0, 3, 4, 5), (2, 3, 0, 5), (2, 0, 4, 5)])
+def test_results(gpu, op, dtype, B, M, K, N):
+    a, b, g = operands(gpu, B, M, K, N, dtype)
+    new, old = PAIRS[op]
+    assert native(a, b)
+    with torch.no_grad():
+        assert torch.equal(new(a, b), old(a, b))
+    for needs in ("ab", "a", "b"):
+        x, y = a.clone().requires_grad_("a" in needs), b.clone().requires_grad_("b" in needs)
+        wrt = [t for t in (x, y) if t.requires_grad]
+        for grad in (g, g.float(), g.transpose(1, 2).contiguous().transpose(1, 2), g[:1, :1, :1].expand_as(g) if g.numel() else g):
+            if op == "prodmax" and M == 0:      # no factors to read the gradient from: refused
+                for f in (new, old):
+                    with pytest.raises(RuntimeError):
+                        torch.autograd.grad(f(x, y), wrt, grad.to(dtype))
+                continue
+            got = torch.autograd.grad(new(x, y), wrt, grad.to(dtype))
+            want = torch.autograd.grad(old(x, y), wrt, grad.to(dtype))
+            assert all(torch.equal(p, q) for p, q in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("part", ["ab", "a", "b"])
+@pytest.mark.parametrize("B,M,K,N", [(3, 7, 5, 9), (2, 128, 128, 128), (2, 130, 97, 101)])
+def test_second_order(gpu, dtype, part, B, M, K, N):
+    a, b, g = operands(gpu, B, M, K, N, dtype)
+    got = []
+    for f in PAIRS["log"]:
+        x, y, h = (t.clone().requires_grad_() for t in (a, b, g))
+        first = torch.autograd.grad(f(x, y), (x, y), h, create_graph=True)
+        asked = [first["ab".index(c)] for c in part]
+        got.append(torch.autograd.grad(asked, (x, y, h), [torch.cos(t).detach() for t in asked]))
+    assert all(torch.equal(p, q) for p, q in zip(*got))
+
+
+def test_what_takes_the_route(gpu):
+    a, b, _ = operands(gpu, 2, 6, 5, 7, torch.float32)
+    assert native(a, b) and native(torch.nn.Parameter(a), b)
+    wide = operands(gpu, 2, 6, 4096, 7, torch.float32)
+
+    class Sub(torch.Tensor):
+        pass
+
+    for x, y in ((a.cpu(), b.cpu()), (a.double(), b.double()), (a, b.half()), (a[0], b[0]), (a, b[:1]), (a, b[:, :4]),
+                 (a.transpose(1, 2).contiguous().transpose(1, 2), b), (a.as_subclass(Sub), b), (wide[0], wide[1]),
+                 (torch.complex(a, a).conj().imag, b), (a.int(), b.int())):
+        assert not native(x, y)
+
+
+@pytest.mark.parametrize("op", list(PAIRS))
+def test_refused_as_before(gpu, op):
+    a, b, g = operands(gpu, 2, 6, 5, 7, torch.float32)
+    for f in PAIRS[op]:
+        x = a.clone().requires_grad_()
+        with forward_ad.dual_level(), pytest.raises(Exception):       # no forward-mode formula
+            f(forward_ad.make_dual(a, a), b)
+        out = f(x, b)
+        with pytest.raises(RuntimeError):                             # no batching rule
+            torch.autograd.grad(out, x, torch.stack([g, g]), is_grads_batched=True)
+        with pytest.raises(Exception):
+            torch.func.vmap(f)(torch.stack([a, a]), torch.stack([b, b]))
+        with pytest.raises(Exception):
+            torch.func.grad(lambda t: f(t, b).sum())(a)
+        y = a.clone().requires_grad_()
+        out = f(y * 1, b)
+        torch.autograd.grad(out, y, g)
+        with pytest.raises(RuntimeError):                             # the graph is gone
+            torch.autograd.grad(out, y, g)
+    if op == "log":
+        for f in PAIRS[op]:
+            x = (a * 1).requires_grad_()
+            out = f(x, b)
+            with torch.no_grad():
+                x.add_(1)
+            with pytest.raises(RuntimeError):                         # saved for the backward, then changed
+                torch.autograd.grad(out, x, g)
+            x = a.clone().requires_grad_()
+            out = f(x, b)
+            with forward_ad.dual_level(), pytest.raises(Exception):   # a tangent on the incoming gradient
+                torch.autograd.grad(out, x, forward_ad.make_dual(g, g))
+
+
+@pytest.mark.parametrize("op", list(PAIRS))
+def test_hooks_traces_streams_threads(gpu, op):
+    import threading
+
+    a, b, g = operands(gpu, 2, 40, 33, 50, torch.float32)
+    new, old = PAIRS[op]
+    x = a.clone().requires_grad_()
+    want = torch.autograd.grad(old(x, b), x, g)[0]
+    with torch.autograd.graph.save_on_cpu():
+        out = new(x, b)
+    assert torch.equal(torch.autograd.grad(out, x, g)[0], want)
+    traced = torch.jit.trace(new, (a, b), check_trace=False)          # a Python Function records itself; a native one would not
+    assert "^" in str(traced.graph) and torch.equal(traced(a, b), old(a, b))
+    got = {}
+
+    def work(i):
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(s):
+            y = a.clone().requires_grad_()
+            got[i] = torch.autograd.grad(new(y, b), y, g)[0]
+        s.synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert all(torch.equal(got[i], want) for i in range(4))
