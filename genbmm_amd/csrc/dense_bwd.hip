@@ -36,6 +36,11 @@ constexpr int kKC = 128;  // cells of the reduction axis per lane
 // (40, 251, 173, 301) 111 -> 37.  A row's partial last chunk too is read in pieces of four, the last one cell by
 // cell (all 32 cell by cell cost forward and backward of float16 draws at (64, 20^3) 32.7 -> 33.5 us, now 32.3;
 // prodmaxbmm (814, 76, 51, 83) 165 -> 153; clamped addresses in the place of the uniform tests: 5 % slower).
+// One wave on a SIMD issues everything itself, so instructions count: a slot by one unsigned minimum and a column's
+// addresses carried along (two chunks of a column 687 -> 482 instructions, of a row 950 -> 760): max and
+// sample (256, 256^3) 75 -> 66 us, (64, 512^3) 123 -> 99, (40, 251, 173, 301) 21.5 -> 17.8, (100, 500, 300, 510)
+// 197 -> 159, (512, 128^3) 34 either way (memory).  With the product semiring's factors the same took more registers
+// than a wave's 256 ((512, 128^3) 47 -> 51, (64, 512^3) 158 -> 139): it keeps the longer form.
 static_assert(kKC == 128, "the shifts of the write-out");
 constexpr int kArgAcc = 64 * kKC + 64;  // floats of LDS: the cells, one spare cell per lane
 constexpr int kChA = 32, kChB = 16;     // cells per chunk (a column's cells are single loads, and at most
@@ -47,6 +52,10 @@ constexpr int kChA = 32, kChB = 16;     // cells per chunk (a column's cells are
 typedef int argmax_i4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float argmax_f4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef elem_t argmax_e4 __attribute__((ext_vector_type(4), aligned(sizeof(elem_t))));
+// (typed as global memory: a pointer carried around the loop was taken for one of unknown address space, whose
+// loads are flat and drain all others)
+template <class E>
+using argmax_global = const __attribute__((address_space(1))) E*;
 template <int PROD>
 struct ArgRow {
   static constexpr int CH = kChA;
@@ -108,12 +117,17 @@ __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk
   float tv[CH];
 #pragma unroll
   for (int q = 0; q < CH; ++q) {
-    const int k = x.iv(q) - c0;
-    const bool mine = k >= 0 && k < kc;
-    sl[q] = (mine ? k : kKC) * 64 + lane;  // [kKC]: the spare cells
-    tv[q] = x.gv(q);
-    if (PROD == 2) tv[q] = __fmul_rn(x.fv(q), tv[q]);
-    if (PROD == 1 && mine) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
+    if constexpr (PROD == 2) {
+      const int k = x.iv(q) - c0;
+      sl[q] = (k >= 0 && k < kc ? k : kKC) * 64 + lane;  // [kKC]: the spare cells
+      tv[q] = __fmul_rn(x.fv(q), x.gv(q));
+    } else {
+      // the lane's cell, or its spare one: an index below the part wraps around, and none is K or beyond
+      const unsigned k = min((unsigned)(x.iv(q) - c0), (unsigned)kKC);
+      sl[q] = k * 64 + lane;
+      tv[q] = x.gv(q);
+      if (PROD == 1 && k < kKC) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
+    }
   }
 #pragma unroll
   for (int q = 0; q < CH; q += 4) {
@@ -246,13 +260,33 @@ __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int
   const float* fcol = PROD == 2 ? fac + (long)batch * M * N + nn : nullptr;
   const int kcap = min(kKC, K);  // no lane has more cells
   using Chunk = ArgCol<PROD>;
-  auto load = [&](Chunk& x, int c) __attribute__((always_inline)) {
-    const int m0 = c * kChB;
+  // HOLD: where a lane's cells of a chunk lie, one address each, a chunk on at a time.  Formed anew from the row's
+  // number they take three scalar instructions a load, which a lone wave issues in the place of everything else.
+  constexpr bool HOLD = PROD != 2;
+  argmax_global<int32_t> ip[HOLD ? kChB : 1];
+  argmax_global<elem_t> gp[HOLD ? kChB : 1];
+  if constexpr (HOLD) {
 #pragma unroll
     for (int q = 0; q < kChB; ++q) {
-      x.i[q] = icol[(long)(m0 + q) * N];
-      x.g[q] = gcol[(long)(m0 + q) * N];
-      if constexpr (PROD == 2) x.f[q] = fcol[(long)(m0 + q) * N];
+      ip[q] = (argmax_global<int32_t>)(icol + (long)q * N);
+      gp[q] = (argmax_global<elem_t>)(gcol + (long)q * N);
+    }
+  }
+  int reached = 0;  // the chunk they point at
+  auto load = [&](Chunk& x, int c) __attribute__((always_inline)) {
+    const int m0 = c * kChB;
+    const long on = (long)((c - reached) * kChB) * N;  // none where the last chunk is asked for again
+    reached = c;
+#pragma unroll
+    for (int q = 0; q < kChB; ++q) {
+      if constexpr (HOLD) {
+        x.i[q] = *(ip[q] += on);
+        x.g[q] = *(gp[q] += on);
+      } else {
+        x.i[q] = icol[(long)(m0 + q) * N];
+        x.g[q] = gcol[(long)(m0 + q) * N];
+        x.f[q] = fcol[(long)(m0 + q) * N];
+      }
     }
   };
   auto tail = [&](Chunk& x, int c) __attribute__((always_inline)) {
