@@ -54,25 +54,31 @@ struct BB {
 // The blocks of a pass.  A block is `per_block` consecutive units (cells or rows) starting at `base`
 // and ending before `limit`; f(base, limit) works on one.  Without `only`: one block per workgroup
 // over all units (numbered so that an item's workgroups share an XCD).  With it - the pass over
-// flagged items, which usually finds none - a small grid reads the flags 64 at a time; its workgroups
+// flagged items, which usually finds none - a small grid looks all flags over at once (a round trip to
+// memory per 64 of them took 6 to 7 us a launch at 512 items); if there are any, its workgroups
 // form groups of one item's blocks (or one group that strides, for items of more blocks than the
 // grid), and the flagged items go to the groups in turn: tens of thousands of workgroups that look
-// up a flag and exit cost 60 us a launch, this costs 2.
+// up a flag and exit cost 60 us a launch.  blk of nblk: the workgroup's number in its pass.
 constexpr int kBBOnlyGrid = 2048;
 template <bool ONLY, class F>
-__device__ __forceinline__ void bb_blocks(const BB& p, long total, long per_item, int per_block, F&& f) {
+__device__ __forceinline__ void bb_blocks(const BB& p, unsigned blk, unsigned nblk, long total, long per_item,
+                                          int per_block, F&& f) {
   if constexpr (!ONLY) {
-    f((long)xcd_renumber(blockIdx.x, gridDim.x) * per_block, total);
+    f((long)xcd_renumber(blk, nblk) * per_block, total);
     return;
   }
+  int any = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < p.B; i += 256) any |= p.only[i];
+  if (!__syncthreads_or(any)) return;
   const int lane = threadIdx.x & 63;
   const long bpi = (per_item + per_block - 1) / per_block;  // blocks per item
-  const bool fits = bpi <= (long)gridDim.x;
-  const long groups = fits ? (long)gridDim.x / bpi : 1;
-  const long grp = fits ? (long)blockIdx.x / bpi : 0;
+  const bool fits = bpi <= (long)nblk;
+  const long groups = fits ? (long)nblk / bpi : 1;
+  const long grp = fits ? (long)blk / bpi : 0;
   if (grp >= groups) return;
-  const long first = fits ? (long)blockIdx.x - grp * bpi : (long)blockIdx.x;
-  const long stride = fits ? bpi : (long)gridDim.x;
+  const long first = fits ? (long)blk - grp * bpi : (long)blk;
+  const long stride = fits ? bpi : (long)nblk;
   long seen = 0;
   for (int b0 = 0; b0 < p.B; b0 += 64) {
     unsigned long long live = __ballot(b0 + lane < p.B && p.only[b0 + lane] != 0);
@@ -91,7 +97,7 @@ inline dim3 bb_grid(const BB& p, long nblocks) {
 
 template <bool ONLY>
 __global__ __launch_bounds__(256) void k_log_bwdbwd_t(const BB p, long total) {
-  bb_blocks<ONLY>(p, total, (long)p.M * p.N, 256, [&](long base, long limit) __attribute__((always_inline)) {
+  bb_blocks<ONLY>(p, blockIdx.x, gridDim.x, total, (long)p.M * p.N, 256, [&](long base, long limit) __attribute__((always_inline)) {
   const long e = base + threadIdx.x;
   if (e >= limit) return;
   const int n = (int)(e % p.N);
@@ -120,8 +126,8 @@ __global__ __launch_bounds__(256) void k_log_bwdbwd_t(const BB p, long total) {
 // partial sums are added across the wave and 64 finished cells are written at once.
 constexpr int kBBChunks = 4;  // n chunks of 64 a lane keeps in registers
 template <bool ONLY>
-__global__ __launch_bounds__(256) void k_log_bwdbwd_a(const BB p, long rows) {
-  bb_blocks<ONLY>(p, rows, (long)p.M, 4, [&](long base, long limit) __attribute__((always_inline)) {
+__device__ __forceinline__ void bb_grad_a(const BB& p, unsigned blk, unsigned nblk, long rows) {
+  bb_blocks<ONLY>(p, blk, nblk, rows, (long)p.M, 4, [&](long base, long limit) __attribute__((always_inline)) {
   const int lane = threadIdx.x & 63;
   const long bm = base + (threadIdx.x >> 6);
   if (bm >= limit) return;
@@ -180,8 +186,8 @@ __global__ __launch_bounds__(256) void k_log_bwdbwd_a(const BB p, long rows) {
 }
 
 template <bool ONLY>
-__global__ __launch_bounds__(256) void k_log_bwdbwd_b(const BB p, long total) {
-  bb_blocks<ONLY>(p, total, (long)p.K * p.N, 256, [&](long base, long limit) __attribute__((always_inline)) {
+__device__ __forceinline__ void bb_grad_b(const BB& p, unsigned blk, unsigned nblk, long total) {
+  bb_blocks<ONLY>(p, blk, nblk, total, (long)p.K * p.N, 256, [&](long base, long limit) __attribute__((always_inline)) {
   const long e = base + threadIdx.x;
   if (e >= limit) return;
   const int n = (int)(e % p.N);
@@ -207,6 +213,25 @@ __global__ __launch_bounds__(256) void k_log_bwdbwd_b(const BB p, long total) {
   });
 }
 
+// Both gradients in one launch, which need t and not each other: workgroups [0, split) take grad_a.
+template <bool ONLY>
+__global__ __launch_bounds__(256) void k_log_bwdbwd_ab(const BB p, unsigned split, long rows, long total) {
+  if (blockIdx.x < split) bb_grad_a<ONLY>(p, blockIdx.x, split, rows);
+  else bb_grad_b<ONLY>(p, blockIdx.x - split, gridDim.x - split, total);
+}
+
+// Two passes' workgroups in one launch of go(grid, split), the first pass's in front; in two launches where the
+// sum of their work-items is beyond what one may have.
+template <class F>
+void launch_pair(dim3 first, dim3 second, F&& go) {
+  if (((int64_t)first.x + second.x) * 256 <= 0xffffffffLL) {
+    if (first.x + second.x > 0) go(dim3(first.x + second.x), first.x);
+    return;
+  }
+  if (first.x > 0) go(first, first.x);
+  if (second.x > 0) go(second, 0u);
+}
+
 int launch_exact(const BB& p, int B, hipStream_t s) {
   auto blocks = [&](long total) { return bb_grid(p, (total + 255) / 256); };
   const long tmn = (long)B * p.M * p.N, tmk = (long)B * p.M * p.K, tkn = (long)B * p.K * p.N;
@@ -214,17 +239,11 @@ int launch_exact(const BB& p, int B, hipStream_t s) {
     hipLaunchKernelGGL(p.only ? k_log_bwdbwd_t<true> : k_log_bwdbwd_t<false>, blocks(tmn), dim3(256), 0, s, p, tmn);
     if (int e = launch_status()) return e;
   }
-  if (tmk > 0) {
-    const long rows = (long)B * p.M;  // four rows per workgroup
-    hipLaunchKernelGGL(p.only ? k_log_bwdbwd_a<true> : k_log_bwdbwd_a<false>, bb_grid(p, (rows + 3) / 4), dim3(256), 0, s,
-                       p, rows);
-    if (int e = launch_status()) return e;
-  }
-  if (tkn > 0) {
-    hipLaunchKernelGGL(p.only ? k_log_bwdbwd_b<true> : k_log_bwdbwd_b<false>, blocks(tkn), dim3(256), 0, s, p, tkn);
-    if (int e = launch_status()) return e;
-  }
-  return GENBMM_OK;
+  const long rows = tmk > 0 ? (long)B * p.M : 0;  // four rows per workgroup
+  launch_pair(bb_grid(p, (rows + 3) / 4), blocks(tkn), [&](dim3 grid, unsigned split) {
+    hipLaunchKernelGGL(p.only ? k_log_bwdbwd_ab<true> : k_log_bwdbwd_ab<false>, grid, dim3(256), 0, s, p, split, rows, tkn);
+  });
+  return launch_status();
 }
 
 // ------------------------------------------------------------------ factored form
@@ -280,13 +299,12 @@ __device__ __forceinline__ bool splits4(float4 v) { return splits(v.x) && splits
 
 // alpha, EA, X: a wave per padded row (b, mp) - half a wave where a row is 128 cells, 32 lanes' worth;
 // rows and columns of the padding hold zeros.
-__global__ __launch_bounds__(256) void k_bb_prep_a(const elem_t* __restrict__ a, const elem_t* __restrict__ ua,
-                                                   float* __restrict__ alpha, float* __restrict__ ea,
-                                                   float* __restrict__ x, int* __restrict__ flags, int M, int K,
-                                                   int Mp, int Kp, long rows) {
+__device__ __forceinline__ void bb_prep_a(unsigned blk, const elem_t* __restrict__ a, const elem_t* __restrict__ ua,
+                                          float* __restrict__ alpha, float* __restrict__ ea, float* __restrict__ x,
+                                          int* __restrict__ flags, int M, int K, int Mp, int Kp, long rows) {
   const int lpr = Kp == 128 ? 32 : 64;  // lanes per row
   const int lane = threadIdx.x & (lpr - 1);
-  const long row = ((long)blockIdx.x * 256 + threadIdx.x) / lpr;
+  const long row = ((long)blk * 256 + threadIdx.x) / lpr;
   if (row >= rows) return;
   const long batch = row / Mp;
   const int m = (int)(row - batch * Mp);
@@ -328,15 +346,14 @@ __global__ __launch_bounds__(256) void k_bb_prep_a(const elem_t* __restrict__ a,
 
 // beta, EB, Y: a workgroup per (batch item, 64 columns): 16 lanes x 4 columns across, the 16 lane
 // groups of the four waves split the rows of b.
-__global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b, const elem_t* __restrict__ ub,
-                                                   float* __restrict__ beta, float* __restrict__ eb,
-                                                   float* __restrict__ y, int* __restrict__ flags, int K, int N,
-                                                   int Kp, int Np) {
-  __shared__ float part[16][64];
+__device__ __forceinline__ void bb_prep_b(unsigned blk, const elem_t* __restrict__ b, const elem_t* __restrict__ ub,
+                                          float* __restrict__ beta, float* __restrict__ eb, float* __restrict__ y,
+                                          int K, int N, int Kp, int Np) {
+  __shared__ __attribute__((aligned(16))) float part[16][64];
   const int cq = threadIdx.x & 15, rg = threadIdx.x >> 4;
   const int cblocks = Np / 64;
-  const long batch = blockIdx.x / cblocks;
-  const int n = (blockIdx.x - batch * cblocks) * 64 + cq * 4;
+  const long batch = blk / cblocks;
+  const int n = (int)(blk - batch * cblocks) * 64 + cq * 4;
   const int cnt = N - n;  // live columns of this lane's four (<= 0: none)
   const elem_t* bc = b + batch * K * N + (cnt > 0 ? n : 0);
   const elem_t* uc = ub ? ub + batch * K * N + (cnt > 0 ? n : 0) : nullptr;
@@ -352,9 +369,6 @@ __global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b,
     const float4 v = ld4a(&part[r][cq * 4]);
     mx = make_float4(fmaxf(mx.x, v.x), fmaxf(mx.y, v.y), fmaxf(mx.z, v.z), fmaxf(mx.w, v.w));
   }
-  if (rg == 0)
-    st4(beta + batch * Np + n, make_float4(cnt > 0 ? mx.x : 0.f, cnt > 1 ? mx.y : 0.f, cnt > 2 ? mx.z : 0.f,
-                                           cnt > 3 ? mx.w : 0.f));
   float* ec = eb + batch * Kp * Np + n;
   float* yc = y + batch * Kp * Np + n;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -372,7 +386,21 @@ __global__ __launch_bounds__(256) void k_bb_prep_b(const elem_t* __restrict__ b,
     st4(ec + (long)k * Np, e);
     st4(yc + (long)k * Np, yv);
   }
-  if (bad) flags[batch] = 1;
+  // (a column that does not split has no maximum, as a row above)
+  bad = __syncthreads_or(bad);
+  if (rg == 0)
+    st4(beta + batch * Np + n, bad ? make_float4(NAN, NAN, NAN, NAN)
+                                   : make_float4(cnt > 0 ? mx.x : 0.f, cnt > 1 ? mx.y : 0.f, cnt > 2 ? mx.z : 0.f,
+                                                 cnt > 3 ? mx.w : 0.f));
+}
+
+// Both operands' passes in one launch, workgroups [0, split) the columns'.
+__global__ __launch_bounds__(256) void k_bb_prep_ab(const elem_t* __restrict__ a, const elem_t* __restrict__ ua,
+                                                    const elem_t* __restrict__ b, const elem_t* __restrict__ ub,
+                                                    const BBWs w, unsigned split, int M, int K, int N, int Mp, int Kp,
+                                                    int Np, long rows) {
+  if (blockIdx.x < split) bb_prep_b(blockIdx.x, b, ub, w.beta, w.eb, w.y, K, N, Kp, Np);
+  else bb_prep_a(blockIdx.x - split, a, ua, w.alpha, w.ea, w.x, w.flags, M, K, Mp, Kp, rows);
 }
 
 // R = exp(alpha + beta - out), H = g R over the padded (Mp, Np) grid (zeros in the padding), four
@@ -602,10 +630,10 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
   {
     const long rows = (long)B * Mp;
     const long per_wg = Kp == 128 ? 8 : 4;  // rows per workgroup: 32 or 64 lanes each
-    hipLaunchKernelGGL(k_bb_prep_a, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3(256), 0, s, p.a, p.ua, w.alpha, w.ea,
-                       w.x, w.flags, M, K, Mp, Kp, rows);
-    hipLaunchKernelGGL(k_bb_prep_b, dim3((unsigned)(B * (Np / 64))), dim3(256), 0, s, p.b, p.ub, w.beta, w.eb, w.y,
-                       w.flags, K, N, Kp, Np);
+    launch_pair(dim3((unsigned)(B * (Np / 64))), dim3((unsigned)((rows + per_wg - 1) / per_wg)),
+                [&](dim3 grid, unsigned split) {
+      hipLaunchKernelGGL(k_bb_prep_ab, grid, dim3(256), 0, s, p.a, p.ua, p.b, p.ub, w, split, M, K, N, Mp, Kp, Np, rows);
+    });
     const long quads = (long)B * Mp * (Np / 4);
     hipLaunchKernelGGL(k_bb_prep_h, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, p.out, p.g, w.alpha,
                        w.beta, w.r, w.h, w.flags, M, N, Mp, Np, quads);

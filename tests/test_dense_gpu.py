@@ -612,6 +612,30 @@ def test_logbmm_double_backward_flagged_items_walk(gpu, B, M, K, N, flagged):
         close(x[rest], y[rest], rtol=1e-4, atol=2e-4)
 
 
+@pytest.mark.parametrize("B,K,N,flagged", [(1100, 64, 64, [0, 255, 256, 300, 1099]), (3, 70, 130, [1])])
+@pytest.mark.parametrize("cell", ["ua", "ub"])
+def test_logbmm_double_backward_cotangent_beyond_three_parts(gpu, B, K, N, flagged, cell):
+    """One cell of u_a or u_b, at its row's or column's maximum, above the largest bfloat16 flags its item, whichever
+    of the workgroup's looks at the flags it falls to: the exact passes bit for bit; every other
+    item within the factored form's tolerance."""
+    M = 64
+    torch.manual_seed(B + K)
+    a, b = torch.randn(B, M, K, device=gpu), torch.randn(B, K, N, device=gpu)
+    g, ua, ub = torch.randn(B, M, N, device=gpu), torch.randn(B, M, K, device=gpu), torch.randn(B, K, N, device=gpu)
+    for i in flagged:
+        if cell == "ua":
+            a[i, 5, K - 1], ua[i, 5, K - 1] = 9.0, 3.395e38
+        else:
+            b[i, K - 1, N - 1], ub[i, K - 1, N - 1] = 9.0, 3.395e38
+    out = genbmm.logbmm(a, b)
+    got = _bwdbwd_abi(gpu, a, b, out, g, ua, ub, True)
+    exact = _bwdbwd_abi(gpu, a, b, out, g, ua, ub, False)
+    rest = [i for i in range(B) if i not in flagged]
+    for x, y in zip(got, exact):
+        assert torch.equal(x[flagged].nan_to_num(), y[flagged].nan_to_num())
+        close(x[rest], y[rest], rtol=1e-4, atol=2e-4)
+
+
 def test_logbmm_double_backward_at_the_headline_shape(gpu):
     """(64, 512, 512, 512) through autograd with create_graph; three batch items against float64
     second-order autograd evaluated on the device."""
