@@ -21,8 +21,8 @@
 //      grad_a = X (H EB^T) + EA (H Y^T - (H t) EB^T)
 //      grad_b = Y (EA^T H) + EB (X^T H - EA^T (H t))
 //    eight products (five when u_b is absent) of batched GEMM shape.  The operands are laid out
-//    once, zero-padded to multiples of 128 in every extent, by three elementwise passes; one
-//    GEMM kernel (128 x 128 tiles, three-part operands on v_mfma_f32_32x32x16_bf16, 16-deep slabs
+//    once, zero-padded to multiples of 128 in every extent: EA, X, EB, Y by an elementwise launch, H and
+//    H t by the epilogue of t; one GEMM kernel (128 x 128 tiles, three-part operands on v_mfma_f32_32x32x16_bf16, 16-deep slabs
 //    through two LDS buffers) then runs without any edge handling in its loop, sums up to two products into one
 //    accumulator and applies the epilogue of its role.  A batch item with a cell whose
 //    alpha + beta - out is beyond 40 ln 2 or not finite (a factor could underflow against a
@@ -261,7 +261,7 @@ struct BBWs {
   int* flags;      // (B): items to redo exactly
   float *ea, *x;   // (B, Mp, Kp): exp(a - alpha), ea * u_a
   float *eb, *y;   // (B, Kp, Np)
-  float *r, *h, *nht;  // (B, Mp, Np): exp(alpha + beta - out), g r, -h t
+  float *h, *nht;  // (B, Mp, Np): g exp(alpha + beta - out), -h t
 };
 inline size_t bb_ws_floats(int B, int M, int K, int N, BBWs* w, float* base) {
   size_t off = 0;
@@ -279,13 +279,13 @@ inline size_t bb_ws_floats(int B, int M, int K, int N, BBWs* w, float* base) {
     t.flags = reinterpret_cast<int*>(take(B));
     t.ea = take(B * Mp * Kp); t.x = take(B * Mp * Kp);
     t.eb = take(B * Kp * Np); t.y = take(B * Kp * Np);
-    t.r = take(B * Mp * Np); t.h = take(B * Mp * Np); t.nht = take(B * Mp * Np);
+    t.h = take(B * Mp * Np); t.nht = take(B * Mp * Np);
   }
   if (w) *w = t;
   return off;
 }
 
-// The three passes move four cells per lane and instruction (the padded extents are multiples of
+// The passes move four cells per lane and instruction (the padded extents are multiples of
 // 128; rows of the caller's tensors start at any element, which the loads take).
 __device__ __forceinline__ float4 exp4_st(float4 v, float m) {
   return make_float4(exp_st(v.x - m), exp_st(v.y - m), exp_st(v.z - m), exp_st(v.w - m));
@@ -329,15 +329,15 @@ __device__ __forceinline__ void bb_prep_a(unsigned blk, const elem_t* __restrict
   bool bad = false;
   for (int k = lane * 4; k < Kp; k += step) {
     // (the fill -inf gives exp = 0 in the padding; a row of -inf has mx = -inf and NaN here, and is
-    //  flagged by the pass that forms H)
+    //  flagged where H is formed)
     const float4 e = k < K ? exp4_st(ld4m(ar + k, K - k, -INFINITY), mx) : zero;
     const float4 xv = (ur && k < K) ? mul4(e, ld4m(ur + k, K - k, 0.f)) : zero;
     bad = bad || !splits4(xv);
     st4(er + k, e);
     st4(xr + k, xv);
   }
-  // (the flags are being cleared here: a row that does not split has no maximum, and the pass that
-  //  forms H flags its item)
+  // (the flags are being cleared here: a row that does not split has no maximum, and its item
+  //  is flagged where H is formed)
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     if (off < lpr) bad = bad | (bool)__shfl_xor((int)bad, off, 64);
@@ -403,45 +403,6 @@ __global__ __launch_bounds__(256) void k_bb_prep_ab(const elem_t* __restrict__ a
   else bb_prep_a(blockIdx.x - split, a, ua, w.alpha, w.ea, w.x, w.flags, M, K, Mp, Kp, rows);
 }
 
-// R = exp(alpha + beta - out), H = g R over the padded (Mp, Np) grid (zeros in the padding), four
-// cells of a row per lane; an item with a cell beyond the guard is flagged.
-__global__ __launch_bounds__(256) void k_bb_prep_h(const elem_t* __restrict__ out, const elem_t* __restrict__ g,
-                                                   const float* __restrict__ alpha, const float* __restrict__ beta,
-                                                   float* __restrict__ r, float* __restrict__ h,
-                                                   int* __restrict__ flags, int M, int N, int Mp, int Np,
-                                                   long quads) {
-  const long q = (long)blockIdx.x * 256 + threadIdx.x;
-  if (q >= quads) return;
-  const int nq = Np / 4;
-  const int n = (int)(q % nq) * 4;
-  const long bm = q / nq;
-  const long batch = bm / Mp;
-  const int m = (int)(bm - batch * Mp);
-  float rv[4] = {0.f, 0.f, 0.f, 0.f}, hv[4] = {0.f, 0.f, 0.f, 0.f};
-  const int cnt = N - n;
-  if (m < M && cnt > 0) {
-    const long src = (batch * M + m) * N + n;
-    const float al = alpha[bm];
-    const float4 be4 = ld4(beta + batch * Np + n), o4 = ld4m(out + src, cnt, 0.f), g4 = ld4m(g + src, cnt, 0.f);
-    const float be[4] = {be4.x, be4.y, be4.z, be4.w}, o[4] = {o4.x, o4.y, o4.z, o4.w}, gv[4] = {g4.x, g4.y, g4.z, g4.w};
-    const float lim = kMfmaGuardBits * kLn2 + 1e-3f;
-    bool bad = !(al > -INFINITY);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < cnt) {
-        const float ex = al + be[i] - o[i];
-        // (a negated comparison: NaN and +inf fail it; alpha, beta not finite make ex not finite or NaN)
-        bad = bad || !(ex <= lim) || !(be[i] > -INFINITY);
-        rv[i] = exp_st(ex);
-        hv[i] = gv[i] * rv[i];
-        bad = bad || !splits(hv[i]);
-      }
-    if (bad) flags[batch] = 1;
-  }
-  st4(r + bm * Np + n, make_float4(rv[0], rv[1], rv[2], rv[3]));
-  st4(h + bm * Np + n, make_float4(hv[0], hv[1], hv[2], hv[3]));
-}
-
 // One tile of C = P1 Q1 (+ P2 Q2) and its epilogue; for a gradient also of C0 = P3 Q3.  Operands are padded workspace arrays:
 //   RT: the rows operand is stored [row][red] (staged transposed), else [red][row];
 //   CT: the columns operand is stored [col][red], else [red][col].
@@ -454,11 +415,15 @@ struct BBMM {
   const float* cols0;
   int Rp, Cp, Qp;       // padded extents: output rows, output columns, reduction
   // epilogue
-  const float* f_acc;   // kEpiT: R; kEpiGrad: EA / EB - the factor of the accumulator
+  const float* f_acc;   // kEpiGrad: EA / EB, the factor of the accumulator
   const float* f0;      // kEpiGrad: X / Y, the factor of C0
-  const float* h;       // kEpiT: H
+  const elem_t* out;    // kEpiT: what R and H are formed from
+  const elem_t* g;
+  const float* alpha;
+  const float* beta;
+  float* h;             // kEpiT: H
   float* nht;           // kEpiT: -H t
-  int* flags;           // kEpiT: per item, set where -H t does not split
+  int* flags;           // kEpiT: per item, set beyond the guard and where H or -H t does not split
   float* tt;            // kEpiT: t unrounded, (B, R, C) unpadded
   elem_t* dst;          // kEpiT: grad_g; kEpiGrad: grad_a / grad_b; (B, R, C) unpadded
   int R, C;             // true extents of the output
@@ -578,18 +543,55 @@ void k_bb_mm(const BBMM p) {
   const int cc = clamp4(p.C - col);                              // columns of the piece that exist
   float* strip = reinterpret_cast<float*>(smem) + wave * kStripFloats;
   if constexpr (EPI == kEpiT) {
+    // R = exp(alpha + beta - out), H = g R (zeros in the padding): formed here, where R is used and H first is.
+    // (512, 128^3): a pass of its own that wrote both took 25 us, this launch 56 with R and H read and 56 so.
     bool bad = false;
-    acc_rows(acc, strip, lane, [](int) {},
+    const float lim = kMfmaGuardBits * kLn2 + 1e-3f;
+    const int pc = min(col, p.C - 4), shift = col - pc;  // a piece over the right edge reads the last four columns
+    const float4 be4 = ld4(p.beta + (long)batch * p.Cp + col);
+    const float be[4] = {be4.x, be4.y, be4.z, be4.w};
+    auto columns = [&](float4 v, float (&x)[4]) __attribute__((always_inline)) {
+      if (shift & 1) v = make_float4(v.y, v.z, v.w, 0.f);
+      if (shift & 2) v = make_float4(v.z, v.w, 0.f, 0.f);
+      x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    };
+    float4 o4[4], g4[4];
+    float al[4];
+    acc_rows(acc, strip, lane,
+             [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+               for (int t = 0; t < 4; ++t) {
+                 const int row = row0 + 16 * q + 4 * t;
+                 const long src = ((long)batch * p.R + min(row, p.R - 1)) * p.C + pc;
+                 o4[t] = ld4(p.out + src);
+                 g4[t] = ld4(p.g + src);
+                 al[t] = p.alpha[(long)batch * p.Rp + row];
+               }
+             },
              [&](int q, int t, float4 v) __attribute__((always_inline)) {
                const int ru = 16 * q + 4 * t;
                const long pu = pbase + (long)ru * p.Cp;
                const long du = ((long)batch * p.R + row0 + ru) * p.C + col;  // unpadded arrays
-               const float4 rv = ld4a(p.f_acc + pu), hv = ld4a(p.h + pu);
-               const float4 tv = make_float4(rv.x * v.x, rv.y * v.y, rv.z * v.z, rv.w * v.w);
-               const float4 nv = make_float4(-hv.x * tv.x, -hv.y * tv.y, -hv.z * tv.z, -hv.w * tv.w);
+               const int live = row0 + ru < p.R ? cc : 0;
+               float o[4], gv[4], rv[4], hv[4];
+               columns(o4[t], o);
+               columns(g4[t], gv);
+               bad = bad || (live > 0 && !(al[t] > -INFINITY));
+#pragma unroll
+               for (int i = 0; i < 4; ++i) {
+                 const float ex = al[t] + be[i] - o[i], r = exp_st(ex), h = gv[i] * r;
+                 const bool in = i < live;
+                 // (a negated comparison: NaN and +inf fail it; alpha, beta not finite make ex not finite or NaN)
+                 bad = bad || (in && (!(ex <= lim) || !(be[i] > -INFINITY) || !splits(h)));
+                 rv[i] = in ? r : 0.f;
+                 hv[i] = in ? h : 0.f;
+               }
+               const float4 tv = make_float4(rv[0] * v.x, rv[1] * v.y, rv[2] * v.z, rv[3] * v.w);
+               const float4 nv = make_float4(-hv[0] * tv.x, -hv[1] * tv.y, -hv[2] * tv.z, -hv[3] * tv.w);
                bad = bad || !splits4(nv);
+               st4a(p.h + pu, make_float4(hv[0], hv[1], hv[2], hv[3]));
                st4a(p.nht + pu, nv);
-               if (row0 + ru < p.R && cc > 0) {
+               if (live > 0) {
                  st4m(p.tt + du, cc, tv);
                  if constexpr (!kElemF32) st4m(p.dst + du, cc, tv);
                }
@@ -634,9 +636,6 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
                 [&](dim3 grid, unsigned split) {
       hipLaunchKernelGGL(k_bb_prep_ab, grid, dim3(256), 0, s, p.a, p.ua, p.b, p.ub, w, split, M, K, N, Mp, Kp, Np, rows);
     });
-    const long quads = (long)B * Mp * (Np / 4);
-    hipLaunchKernelGGL(k_bb_prep_h, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, p.out, p.g, w.alpha,
-                       w.beta, w.r, w.h, w.flags, M, N, Mp, Np, quads);
     if (int e = launch_status()) return e;
   }
   const bool has_a = p.ua != nullptr, has_b = p.ub != nullptr;
@@ -646,7 +645,7 @@ int bwdbwd_factored(const BB& p, const BBWs& w, int B, hipStream_t s) {
     if (has_a) { q.rows[n] = w.x; q.cols[n] = w.eb; ++n; }
     if (has_b) { q.rows[n] = w.ea; q.cols[n] = w.y; ++n; }
     q.pairs = n; q.Rp = Mp; q.Cp = Np; q.Qp = Kp; q.R = M; q.C = N;
-    q.f_acc = w.r; q.h = w.h; q.nht = w.nht; q.flags = w.flags; q.tt = p.tt; q.dst = p.gg;
+    q.out = p.out; q.g = p.g; q.alpha = w.alpha; q.beta = w.beta; q.h = w.h; q.nht = w.nht; q.flags = w.flags; q.tt = p.tt; q.dst = p.gg;
     if (int e = launch_mm<true, false, kEpiT>(q, B, s)) return e;
   }
   {  // grad_a = X (H EB^T) + EA (H Y^T - (H t) EB^T)
