@@ -59,6 +59,14 @@ at::TensorOptions workspace(const Tensor& t) { return t.options().dtype(at::kFlo
 // `g` as the kernels read it
 Tensor incoming(const Tensor& g, at::ScalarType type) { return g.to(type).contiguous(); }
 
+// A saved-tensor hook may hand back something else than it was given: a tensor on the host or of another type, size or
+// order is refused here, before its address reaches a kernel.
+void require(const Tensor& t, const char* name, const Tensor& like, at::ScalarType type, at::IntArrayRef sizes) {
+  TORCH_CHECK(t.is_cuda() && t.device() == like.device(), name, " is on ", t.device(), ", expected ", like.device());
+  TORCH_CHECK(t.scalar_type() == type, name, " must be ", type, ", got ", t.scalar_type());
+  TORCH_CHECK(t.is_contiguous() && t.sizes() == sizes, name, " must be contiguous, of sizes ", sizes, ", got ", t.sizes());
+}
+
 // -------------------------------------------------------------------- logbmm
 // The gradients where none of their own will be asked for (see LogBmm::backward).  A node all the same: it is what
 // refuses an incoming gradient with a tangent.
@@ -89,14 +97,24 @@ struct LogBmm : torch::autograd::Function<LogBmm> {
           "genbmm_logbmm_fwd_path");
     ctx->save_for_backward({a, b, out, stats});
     ctx->saved_data["path"] = path;
+    ctx->saved_data["type"] = a.scalar_type();
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list saved = ctx->get_saved_variables();
     const Tensor &a = saved[0], &b = saved[1];
     // `out` as a value: what it owes to a and b is part of the gradients' own derivative
-    const Tensor g = incoming(grads[0], a.scalar_type()), out = saved[2].detach();
+    const Tensor g = incoming(grads[0], ctx->saved_data["type"].toScalarType()), out = saved[2].detach();
     const int64_t path = ctx->saved_data["path"].toInt();
+    TORCH_CHECK(a.dim() == 3 && b.dim() == 3, "a and b must have 3 dimensions");
+    const Dims d = dims_of(a, b);
+    const at::ScalarType type = g.scalar_type();
+    require(g, "the incoming gradient", g, type, {d.B, d.M, d.N});
+    require(a, "a", g, type, {d.B, d.M, d.K});
+    require(b, "b", g, type, {d.B, d.K, d.N});
+    require(out, "the result", g, type, {d.B, d.M, d.N});
+    require(saved[3], "the forward's workspace", g, at::kFloat,
+            {(int64_t)genbmm_logbmm_stats_size_path(d.B, d.M, d.K, d.N, (int)path)});
     if (at::GradMode::is_enabled()) {  // differentiated again: the Python node has the formula
       const py::gil_scoped_acquire gil;
       const py::tuple r = py::module_::import("genbmm_amd.genmul").attr("_LogBmmGrad").attr("apply")(a, b, g, out, saved[3], path);
@@ -113,8 +131,11 @@ variable_list argmax_backward(AutogradContext* ctx, const Tensor& grad, bool pro
   const variable_list saved = ctx->get_saved_variables();
   const Tensor& idx = saved[0];
   const at::ScalarType type = ctx->saved_data["type"].toScalarType();
-  const int B = idx.size(0), M = idx.size(1), K = ctx->saved_data["K"].toInt(), N = idx.size(2);
+  const int B = grad.size(0), M = grad.size(1), K = ctx->saved_data["K"].toInt(), N = grad.size(2);
   const Tensor g = incoming(grad, type);
+  require(g, "the incoming gradient", g, type, {B, M, N});
+  require(idx, "the indices", g, at::kInt, {B, M, N});
+  if (prod) require(saved[1], "the factors", g, at::kFloat, {2, B, M, N});
   const c10::DeviceGuard guard(g.device());
   Tensor ga = at::empty({B, M, K}, g.options()), gb = at::empty({B, K, N}, g.options());
   if (prod)

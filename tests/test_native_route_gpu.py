@@ -143,3 +143,15 @@ def test_hooks_traces_streams_threads(gpu, op):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert all(torch.equal(got[i], want) for i in range(4))
+
+
+@pytest.mark.parametrize("op", list(PAIRS))
+@pytest.mark.parametrize("unpack", [lambda t: t.cpu(), lambda t: t.double(), lambda t: t[..., :1],
+                                    lambda t: torch.stack([t, t], -1)[..., 0]])
+def test_what_a_saved_tensor_hook_may_not_return(gpu, op, unpack):
+    a, b, g = operands(gpu, 2, 6, 5, 7, torch.float32)
+    x = a.clone().requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        out = PAIRS[op][0](x, b)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(out, x, g)
