@@ -432,7 +432,7 @@ struct BBMM {
 // The products run on the bf16 matrix instruction, every operand cut into three parts while it is staged
 // (split_bf16.h; logbmm_split.h has the staging and the inner loop): on the fp32 instruction, which does a
 // sixteenth of the reduction steps in the same time, the five launches of (512, 128^3) took 245 us; three-part
-// 240, and 205 with H EB^T and EA^T H formed in the launches that use them (a second set of accumulators)
+// 240, and 205 (178 with steps of one line staged) with H EB^T and EA^T H formed in the launches that use them (a second set of accumulators)
 // instead of written out and read back.
 // Bound by what the workspace arrays move (two or four in, one to three more in the epilogue).
 using BBTile = MTile<128, 128, 2>;
