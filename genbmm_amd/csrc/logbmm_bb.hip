@@ -213,11 +213,18 @@ __device__ __forceinline__ void bb_grad_b(const BB& p, unsigned blk, unsigned nb
   });
 }
 
-// Both gradients in one launch, which need t and not each other: workgroups [0, split) take grad_a.
-template <bool ONLY>
+// Both gradients need t and not each other.  Over flagged items, of which there are hardly ever any, they are one
+// launch, workgroups [0, split) grad_a's; over all items a launch each, which has each pass's own registers
+// (a whole (512, 128^3): 1.86 ms, in one launch 1.99).
 __global__ __launch_bounds__(256) void k_log_bwdbwd_ab(const BB p, unsigned split, long rows, long total) {
-  if (blockIdx.x < split) bb_grad_a<ONLY>(p, blockIdx.x, split, rows);
-  else bb_grad_b<ONLY>(p, blockIdx.x - split, gridDim.x - split, total);
+  if (blockIdx.x < split) bb_grad_a<true>(p, blockIdx.x, split, rows);
+  else bb_grad_b<true>(p, blockIdx.x - split, gridDim.x - split, total);
+}
+__global__ __launch_bounds__(256) void k_log_bwdbwd_a(const BB p, long rows) {
+  bb_grad_a<false>(p, blockIdx.x, gridDim.x, rows);
+}
+__global__ __launch_bounds__(256) void k_log_bwdbwd_b(const BB p, long total) {
+  bb_grad_b<false>(p, blockIdx.x, gridDim.x, total);
 }
 
 // Two passes' workgroups in one launch of go(grid, split), the first pass's in front; in two launches where the
@@ -240,9 +247,17 @@ int launch_exact(const BB& p, int B, hipStream_t s) {
     if (int e = launch_status()) return e;
   }
   const long rows = tmk > 0 ? (long)B * p.M : 0;  // four rows per workgroup
-  launch_pair(bb_grid(p, (rows + 3) / 4), blocks(tkn), [&](dim3 grid, unsigned split) {
-    hipLaunchKernelGGL(p.only ? k_log_bwdbwd_ab<true> : k_log_bwdbwd_ab<false>, grid, dim3(256), 0, s, p, split, rows, tkn);
-  });
+  const dim3 grid_a = bb_grid(p, (rows + 3) / 4), grid_b = blocks(tkn);
+  if (p.only) {
+    if (grid_a.x + grid_b.x > 0)
+      hipLaunchKernelGGL(k_log_bwdbwd_ab, dim3(grid_a.x + grid_b.x), dim3(256), 0, s, p, grid_a.x, rows, tkn);
+    return launch_status();
+  }
+  if (grid_a.x > 0) {
+    hipLaunchKernelGGL(k_log_bwdbwd_a, grid_a, dim3(256), 0, s, p, rows);
+    if (int e = launch_status()) return e;
+  }
+  if (grid_b.x > 0) hipLaunchKernelGGL(k_log_bwdbwd_b, grid_b, dim3(256), 0, s, p, tkn);
   return launch_status();
 }
 
