@@ -157,13 +157,25 @@ def stream_of(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
+def dense(t):
+    """t as the kernels read it, by differentiable torch operations: contiguous, and written out if it carries
+    torch's lazy negative bit (`z.conj().imag`), which `contiguous` keeps where the strides already fit."""
+    t = t.contiguous()
+    return t.resolve_neg() if t.is_neg() else t
+
+
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return ctypes.c_void_p(addr(t))
 
 
 def addr(t):
-    """`ptr` as a plain integer (None: NULL), which the declared argument types take as well."""
-    return t.data_ptr() if t is not None else None
+    """The address of t's memory as a plain integer (None: NULL), which the declared argument types take as well as
+    a pointer (`ptr`).  Refused where the memory holds the values with the other sign."""
+    if t is None:
+        return None
+    if t.is_neg():
+        raise RuntimeError("genbmm_amd: a tensor with the lazy negative bit has no memory that holds its values")
+    return t.data_ptr()
 
 
 def call(name, t, *args):

@@ -56,14 +56,15 @@ Dims dims_of(const Tensor& a, const Tensor& b) { return {(int)a.size(0), (int)a.
 
 at::TensorOptions workspace(const Tensor& t) { return t.options().dtype(at::kFloat); }
 
-// `g` as the kernels read it
-Tensor incoming(const Tensor& g, at::ScalarType type) { return g.to(type).contiguous(); }
+// `g` as the kernels read it: contiguous() keeps the lazy negative bit of a tensor whose strides already fit
+Tensor incoming(const Tensor& g, at::ScalarType type) { return g.to(type).contiguous().resolve_neg(); }
 
-// A saved-tensor hook may hand back something else than it was given: a tensor on the host or of another type, size or
-// order is refused here, before its address reaches a kernel.
+// A saved-tensor hook may hand back something else than it was given: a tensor on the host, of another type, size or
+// order or with the lazy negative bit is refused here, before its address reaches a kernel.
 void require(const Tensor& t, const char* name, const Tensor& like, at::ScalarType type, at::IntArrayRef sizes) {
   TORCH_CHECK(t.is_cuda() && t.device() == like.device(), name, " is on ", t.device(), ", expected ", like.device());
   TORCH_CHECK(t.scalar_type() == type, name, " must be ", type, ", got ", t.scalar_type());
+  TORCH_CHECK(!t.is_neg(), name, " has the lazy negative bit: no memory holds its values");
   TORCH_CHECK(t.is_contiguous() && t.sizes() == sizes, name, " must be contiguous, of sizes ", sizes, ", got ", t.sizes());
 }
 

@@ -94,7 +94,7 @@ def _canonical(a, b):
             raise RuntimeError("shape mismatch: a is %s, b is %s" % (tuple(a.shape), tuple(b.shape)))
         a = a.expand(batch + a.shape[-2:]).reshape((-1,) + a.shape[-2:])
         b = b.expand(batch + b.shape[-2:]).reshape((-1,) + b.shape[-2:])
-    a, b = a.contiguous(), b.contiguous()
+    a, b = _lib.dense(a), _lib.dense(b)
 
     def restore(out):
         if batch is not None:
@@ -147,8 +147,8 @@ class _LogBmmGrad(torch.autograd.Function):
             return None, None, None, None, None, None
         a, b, g, out = ctx.saved_tensors
         B, M, K, N = _lib.dense_dims(a, b)
-        u_a = None if u_a is None else u_a.to(a.dtype).contiguous()
-        u_b = None if u_b is None else u_b.to(a.dtype).contiguous()
+        u_a = None if u_a is None else _lib.dense(u_a.to(a.dtype))
+        u_b = None if u_b is None else _lib.dense(u_b.to(a.dtype))
         ga = torch.empty_like(a)
         gb = torch.empty_like(b)
         gg = torch.empty_like(g)
@@ -190,7 +190,7 @@ class LogMatMul(torch.autograd.Function):
         a, b, out, stats = ctx.saved_tensors
         # `out` as a value: what it owes to a and b is part of _LogBmmGrad's own derivative.  With its history
         # a second-order pass came through here once more, on a gradient of zeros: (512, 128^3) 527 -> 432 us
-        grad_a, grad_b = _LogBmmGrad.apply(a, b, grad_output.to(a.dtype).contiguous(), out.detach(), stats, ctx.path)
+        grad_a, grad_b = _LogBmmGrad.apply(a, b, _lib.dense(grad_output.to(a.dtype)), out.detach(), stats, ctx.path)
         return grad_a, grad_b, None
 
 
@@ -202,7 +202,7 @@ def _argmax_backward(ctx, grad_output, prod):
     else:
         (idx,) = ctx.saved_tensors
     B, M, K, N = ctx.dims
-    g = grad_output.to(ct).contiguous()
+    g = _lib.dense(grad_output.to(ct))
     grad_a = torch.empty(B, M, K, dtype=ct, device=g.device)
     grad_b = torch.empty(B, K, N, dtype=ct, device=g.device)
     if ct == torch.float64:

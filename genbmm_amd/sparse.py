@@ -54,7 +54,7 @@ class _BandShift(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, data, w_out, dcol, dband, fill):
-        data = data.contiguous()
+        data = _lib.dense(data)
         B, n, w_in = data.shape
         out = torch.empty(B, n, w_out, dtype=data.dtype, device=data.device)
         _call("genbmm_band_shift", data, _lib.addr(data), _lib.addr(out), B, n, w_in, w_out,
@@ -74,7 +74,7 @@ class _BandTranspose(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, data, lu, ld):
-        data = data.contiguous()
+        data = _lib.dense(data)
         B, n, _ = data.shape
         out = torch.empty_like(data)
         _call("genbmm_band_transpose", data, _lib.addr(data), _lib.addr(out), B, n, lu, ld)
@@ -90,7 +90,7 @@ class _BandTranspose(torch.autograd.Function):
 class _BandToDense(torch.autograd.Function):
     @staticmethod
     def forward(ctx, data, lu, ld, fill):
-        data = data.contiguous()
+        data = _lib.dense(data)
         B, n, _ = data.shape
         out = torch.empty(B, n, n, dtype=data.dtype, device=data.device)
         _call("genbmm_band_to_dense", data, _lib.addr(data), _lib.addr(out), B, n, lu, ld,
@@ -109,7 +109,7 @@ class _BandFromDense(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, dense, lu, ld):
-        dense = dense.contiguous()
+        dense = _lib.dense(dense)
         B, n_rows, n = dense.shape
         out = torch.empty(B, n, lu + ld + 1, dtype=dense.dtype, device=dense.device)
         _call("genbmm_band_from_dense", dense, _lib.addr(dense), _lib.addr(out), B, n_rows, n,
@@ -283,7 +283,7 @@ class BandedMatrix:
         needs_grad = torch.is_grad_enabled() and (self.data.requires_grad or other.data.requires_grad)
         if (code is not None and not needs_grad and _native(self.data) and _native(other.data)
                 and self.data.shape[:2] == other.data.shape[:2]):
-            a, b = self.data.contiguous(), other.data.contiguous()
+            a, b = _lib.dense(self.data), _lib.dense(other.data)
             batch, n, _ = a.shape
             data = torch.empty(batch, n, lu + ld + 1, dtype=a.dtype, device=a.device)
             _call("genbmm_band_op", a, _lib.addr(a), self.lu, self.ld, _lib.addr(b), other.lu,
@@ -350,7 +350,7 @@ class BandedMatrix:
         # Functions save (and differentiate with respect to) what they were given
         # (float16 / bfloat16 bands go to the `_f16` / `_bf16` entry points as they are)
         a, b = self.data, other.data
-        out = fn(a.contiguous(), self.lu, self.ld, b.contiguous(), other.lu, other.ld, lu, ld)
+        out = fn(_lib.dense(a), self.lu, self.ld, _lib.dense(b), other.lu, other.ld, lu, ld)
         return BandedMatrix(out, lu, ld, self.fill)
 
     def multiply(self, other):
@@ -377,7 +377,7 @@ class BandedMatrix:
     def multiply_back(self, other, out, grad_out):
         """Gradient of `self.multiply(other)` with respect to self, given the gradient of
         the product's band tensor (reference sparse.py:363-379; `out` is not needed)."""
-        a, b = self.data.detach().contiguous(), other.data.detach().contiguous()
+        a, b = _lib.dense(self.data.detach()), _lib.dense(other.data.detach())
         g = grad_out.data if isinstance(grad_out, BandedMatrix) else grad_out
         grad_a, _ = _backward(a, b, (self.lu, self.ld, other.lu, other.ld), None, None, g, MODE_MUL)
         return BandedMatrix(grad_a, self.lu, self.ld, self.fill)
@@ -405,8 +405,8 @@ def _check_pair(a, b):
 
 
 def _forward(a, a_lu, a_ld, b, b_lu, b_ld, mode):
-    a = a.contiguous()
-    b = b.contiguous()
+    a = _lib.dense(a)
+    b = _lib.dense(b)
     B, n = _check_pair(a, b)
     if a.shape[2] != a_lu + a_ld + 1 or b.shape[2] != b_lu + b_ld + 1:
         raise RuntimeError("band widths do not match lu + ld + 1")
@@ -431,7 +431,7 @@ def _forward(a, a_lu, a_ld, b, b_lu, b_ld, mode):
 def _backward(a, b, bands, out, idx, g, mode, ws=None):
     a_lu, a_ld, b_lu, b_ld = bands
     B, n = a.shape[0], a.shape[1]
-    g = g.to(a.dtype).contiguous()
+    g = _lib.dense(g.to(a.dtype))
     grad_a = torch.empty_like(a)
     grad_b = torch.empty_like(b)
     if _f64(a):
@@ -466,7 +466,7 @@ class BandedMul(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        a, b = (t.contiguous() for t in ctx.saved_tensors)
+        a, b = (_lib.dense(t) for t in ctx.saved_tensors)
         grad_a, grad_b = _backward(a, b, ctx.bands, None, None, grad_output, MODE_MUL)
         return (grad_a, None, None, grad_b) + (None,) * 4
 
@@ -491,8 +491,8 @@ class _BandedLogGrad(torch.autograd.Function):
             return (None,) * 6
         a, b, g, out = ctx.saved_tensors
         a_lu, a_ld, b_lu, b_ld = ctx.bands
-        u_a = None if u_a is None else u_a.contiguous()
-        u_b = None if u_b is None else u_b.contiguous()
+        u_a = None if u_a is None else _lib.dense(u_a)
+        u_b = None if u_b is None else _lib.dense(u_b)
         ga, gb, gg = torch.empty_like(a), torch.empty_like(b), torch.empty_like(g)
         if a.dtype in _lib.HALF_SUFFIX:
             # the gradient with respect to g is read back by the other two: a float copy of it
@@ -523,8 +523,8 @@ class BandedLogMul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         a, b, out, ws = ctx.saved_tensors
-        a, b = a.contiguous(), b.contiguous()
-        g = grad_output.to(a.dtype).contiguous()
+        a, b = _lib.dense(a), _lib.dense(b)
+        g = _lib.dense(grad_output.to(a.dtype))
         # (`out` as a value, as in LogMatMul.backward)
         grad_a, grad_b = _BandedLogGrad.apply(a, b, g, out.detach(), ws, ctx.bands)
         return (grad_a, None, None, grad_b) + (None,) * 4
@@ -545,7 +545,7 @@ class BandedMaxMul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         a, b, idx = ctx.saved_tensors
-        a, b = a.contiguous(), b.contiguous()
+        a, b = _lib.dense(a), _lib.dense(b)
         grad_a, grad_b = _backward(a, b, ctx.bands, None, idx, grad_output, MODE_MAX)
         return (grad_a, None, None, grad_b) + (None,) * 4
 
@@ -559,7 +559,7 @@ class BandedSampleMul(torch.autograd.Function):
     def forward(ctx, a, a_lu, a_ld, b, b_lu, b_ld, o_lu, o_ld, stream=None):
         from .genmul import _next_stream
 
-        a, b = a.contiguous(), b.contiguous()
+        a, b = _lib.dense(a), _lib.dense(b)
         B, n = _check_pair(a, b)
         if a.shape[2] != a_lu + a_ld + 1 or b.shape[2] != b_lu + b_ld + 1:
             raise RuntimeError("band widths do not match lu + ld + 1")
