@@ -122,11 +122,12 @@ __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk
       sl[q] = (k >= 0 && k < kc ? k : kKC) * 64 + lane;  // [kKC]: the spare cells
       tv[q] = __fmul_rn(x.fv(q), x.gv(q));
     } else {
-      // the lane's cell, or its spare one: an index below the part wraps around, and none is K or beyond
-      const unsigned k = min((unsigned)(x.iv(q) - c0), (unsigned)kKC);
+      // the lane's cell, or its spare one: an index below the part wraps around, one of K or beyond (none that the
+      // library writes) may fall to a cell of the last part that is not written out.  Its factor does not exist.
+      const unsigned k = min((unsigned)x.iv(q) - (unsigned)c0, (unsigned)kKC);
       sl[q] = k * 64 + lane;
       tv[q] = x.gv(q);
-      if (PROD == 1 && k < kKC) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
+      if (PROD == 1 && (int)k < kc) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
     }
   }
 #pragma unroll

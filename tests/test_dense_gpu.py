@@ -741,6 +741,42 @@ def test_prodmax_factors_workspace(gpu, B, M, K, N):
     assert rc != 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("prod", [False, True])
+@pytest.mark.parametrize("B,M,K,N", [(2, 37, 5, 41), (1, 33, 130, 70), (3, 20, 128, 16), (1, 5, 9000, 6)])
+def test_argmax_backward_of_an_index_that_names_no_cell(gpu, dtype, prod, B, M, K, N):
+    """[k == idx] holds for no k where a caller's index is negative or K and beyond - just beyond, to the end of its
+    128 cells and on: such a term adds nothing, and its factor is not looked for (K of one part, of several, of
+    several workgroups)."""
+    torch.manual_seed(K)
+    a, b = (torch.randint(-4, 5, s).to(gpu, dtype) for s in ((B, M, K), (B, K, N)))
+    g = torch.randint(-2, 3, (B, M, N)).to(gpu, dtype)
+    idx = torch.randint(0, K, (B, M, N), dtype=torch.int32)
+    none = torch.tensor([-2 ** 31, -129, -1, K, K + 1, K + 100, K + 127, K + 128, 2 ** 31 - 1], dtype=torch.int32)
+    lost = torch.rand(B, M, N) < 0.5
+    idx[lost] = none[torch.randint(0, len(none), (int(lost.sum()),))]
+    lib, idxd = _lib.load(), idx.to(gpu)
+    ga, gb = torch.full_like(a, float("nan")), torch.full_like(b, float("nan"))
+    ends = [_lib.ptr(ga), _lib.ptr(gb), B, M, K, N, _lib.stream_of(a)]
+    suffix = "_f64" if dtype == torch.float64 else _lib.HALF_SUFFIX.get(dtype, "")
+    if prod:
+        factors = [] if dtype == torch.float64 else [_lib.ptr(None)]
+        rc = getattr(lib, "genbmm_prodmax_bwd" + suffix)(_lib.ptr(a), _lib.ptr(b), _lib.ptr(idxd), *factors, _lib.ptr(g), *ends)
+    else:
+        rc = getattr(lib, "genbmm_argmax_bwd" + suffix)(_lib.ptr(idxd), _lib.ptr(g), *ends)
+    assert rc == 0
+    # whole numbers of at most 8 * 70: exact in every type and order (bfloat16: a sum of terms up to 256 is, and
+    # one rounding of a larger one is the same)
+    keep = torch.where(lost, torch.zeros(()).double(), g.cpu().double())
+    li = torch.where(lost, torch.zeros((), dtype=torch.int64), idx.long())
+    ac, bc = a.cpu().double(), b.cpu().double()
+    ta = keep * torch.gather(bc, 1, li) if prod else keep
+    tb = keep * torch.gather(ac, 2, li) if prod else keep
+    wa = torch.zeros(B, M, K, dtype=torch.float64).scatter_add_(2, li, ta)
+    wb = torch.zeros(B, K, N, dtype=torch.float64).scatter_add_(1, li, tb)
+    assert torch.equal(ga.cpu(), wa.to(dtype)) and torch.equal(gb.cpu(), wb.to(dtype))
+
+
 @pytest.mark.parametrize("prod", [False, True])
 def test_max_index_through_c_abi(gpu, prod):
     torch.manual_seed(3)
