@@ -12,6 +12,7 @@ raises.
 import ctypes
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -125,22 +126,28 @@ def load():
     return lib
 
 
-_host = None
+_host = None    # the extension; False: it does not load
 
 
 def host():
-    """The extension with the eager products' autograd nodes (once). Raises RuntimeError if it has not been built."""
+    """The extension with the eager products' autograd nodes (csrc/host.cpp), loaded once; None where none was built for
+    this torch and this Python, or where it does not load.  genmul's Functions then carry every call, with the same
+    results and more host time."""
     global _host
     if _host is None:
         load()      # the library it is linked to
-        path = os.path.join(_HERE, "lib", "_host.so")
-        if not os.path.exists(path):
-            raise RuntimeError("genbmm_amd: %s is missing; build it with `python -m genbmm_amd.build`" % path)
-        spec = importlib.util.spec_from_file_location("genbmm_amd.lib._host", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        _host = module
-    return _host
+        from . import build
+
+        spec = importlib.util.spec_from_file_location("genbmm_amd.lib._host", build.host_path())
+        try:
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            _host = module
+        except ImportError as e:
+            _host = False
+            warnings.warn("genbmm_amd: small products take longer than they need to, without their native autograd nodes "
+                          "(%s); build them with `python -m genbmm_amd.build`" % e, RuntimeWarning, stacklevel=2)
+    return _host or None
 
 
 def version():

@@ -5,7 +5,7 @@
 This takes the place of the reference's setup.py (setup.py:1-27, a
 torch CUDAExtension named `_genbmm`): the kernels are a plain shared library with a C ABI
 (include/genbmm_gfx950.h) that genbmm_amd/_lib.py loads with ctypes; beside it a small
-torch extension (csrc/host.cpp, lib/_host.so) holds the eager products' autograd nodes.  hipcc cross-compiles for gfx950 without
+torch extension (csrc/host.cpp, lib/_host.*.so) holds the eager products' autograd nodes.  hipcc cross-compiles for gfx950 without
 a GPU being present.
 """
 import os
@@ -47,17 +47,19 @@ HIPCC_FLAGS = [
 EXTRA_FLAGS = {"banded.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
-# The eager route's autograd nodes (csrc/host.cpp): a Python extension linked to the library above, built by the
-# host compiler against torch's own headers.
-HOST_NAME = "_host.so"
-
-
 def lib_path():
     return os.path.join(LIBDIR, LIBNAME)
 
 
 def host_path():
-    return os.path.join(LIBDIR, HOST_NAME)
+    """The eager route's autograd nodes (csrc/host.cpp): a Python extension linked to the library above, built by the
+    host compiler against torch's own headers.  It uses torch's C++ interface, which is no stable one: the torch
+    and the Python it was built for are in its name, so that one built for others is not found."""
+    import sysconfig
+
+    import torch
+
+    return os.path.join(LIBDIR, "_host.torch-%s%s" % (torch.__version__, sysconfig.get_config_var("EXT_SUFFIX")))
 
 
 def _host_commands(obj):

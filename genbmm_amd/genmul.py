@@ -40,6 +40,7 @@ from . import _lib
 
 _COMPUTE = torch.float32   # every workspace, whatever the tensors' element type
 _DTYPES = (torch.float32, torch.float64, torch.float16, torch.bfloat16)
+_NATIVE = (torch.float32, torch.float16, torch.bfloat16)    # what the native route takes
 
 
 def _f64(t):
@@ -110,12 +111,14 @@ _call = _lib.call
 def _native(name, a, b, *args):
     """The eager route of csrc/host.cpp: the function `name` of it on operands that need no conversion
     (3-D contiguous float32 / float16 / bfloat16 tensors of one GPU, no trace or transform around the call); None
-    for any other, which the Functions below take or refuse.  Same library calls, same results bit for bit, without
-    the Python nodes' share of a small step: (16, 64^3) logbmm forward and both gradients 107 -> 54 us (torch's
-    own multiplication with its gradients: 49)."""
-    if not (isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor) and a.is_cuda and b.is_cuda):
+    for any other, and where the extension is not there, which the Functions below take or refuse.  Same library
+    calls, same results bit for bit, without the Python nodes' share of a small step: (16, 64^3) logbmm forward and
+    both gradients 107 -> 54 us (torch's own multiplication with its gradients: 49)."""
+    if not (isinstance(a, torch.Tensor) and isinstance(b, torch.Tensor) and a.is_cuda and b.is_cuda
+            and a.dtype == b.dtype and a.dtype in _NATIVE and a.dim() == 3 and b.dim() == 3):
         return None
-    return getattr(_lib.host(), name)(a, b, *args)
+    host = _lib.host()
+    return getattr(host, name)(a, b, *args) if host is not None else None
 
 
 # --------------------------------------------------------------------- logbmm

@@ -4,6 +4,7 @@ and the no-CPU-fallback rule."""
 import ctypes
 import os
 import re
+import warnings
 
 import pytest
 import torch
@@ -263,6 +264,34 @@ def test_no_host_pointer_reaches_the_library(monkeypatch):
         with pytest.raises(ValueError, match="cuda device"):
             attempt()
     assert not calls
+
+
+@pytest.mark.parametrize("there", [False, True])
+def test_without_the_host_extension_the_functions_carry_the_call(monkeypatch, tmp_path, there):
+    """No extension for this Python and torch, or one that does not load: said once, and a plain pair of operands goes
+    on to the Python Functions.  Operands that it never takes do not ask for it."""
+    from genbmm_amd import build, genmul
+
+    assert torch.__version__ in os.path.basename(build.host_path())
+    path = tmp_path / "_host.so"
+    if there:
+        path.write_text("no library")
+    monkeypatch.setattr(build, "host_path", lambda: str(path))
+    monkeypatch.setattr(_lib, "_host", None)
+    a = torch.empty(2, 3, 4)
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+
+    cuda = lambda t: t.as_subclass(OnGpu)
+    for x, y in ((cuda(a.double()), cuda(a.double())), (cuda(a[0]), cuda(a[0])), (cuda(a), cuda(a.half())), (a, a), (a, 1)):
+        assert genmul._native("plain", x, y) is None
+    assert _lib._host is None
+    with pytest.warns(RuntimeWarning, match="genbmm_amd.build"):
+        assert genmul._native("plain", cuda(a), cuda(a.transpose(1, 2).contiguous())) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host() is None and genmul._native("logbmm", cuda(a), cuda(a), 0, 5) is None
 
 
 def test_product_does_not_import_the_oracle():

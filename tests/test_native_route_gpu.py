@@ -68,6 +68,24 @@ def test_second_order(gpu, dtype, part, B, M, K, N):
     assert all(torch.equal(p, q) for p, q in zip(*got))
 
 
+@pytest.mark.parametrize("op", list(PAIRS))
+def test_without_the_extension(gpu, op, monkeypatch):
+    """Where it was not built for this torch the Python Functions carry the call."""
+    a, b, g = operands(gpu, 2, 40, 33, 50, torch.float32)
+
+    def run():
+        x, y = a.clone().requires_grad_(), b.clone().requires_grad_()
+        out = PAIRS[op][0](x, y)
+        return type(out.grad_fn).__name__, [out.detach()] + list(torch.autograd.grad(out, (x, y), g))
+
+    name, want = run()
+    monkeypatch.setattr(_lib, "_host", False)
+    python, got = run()
+    assert "MatMulBackward" not in name
+    assert "MatMulBackward" in python
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
+
+
 def test_what_takes_the_route(gpu):
     a, b, _ = operands(gpu, 2, 6, 5, 7, torch.float32)
     assert native(a, b) and native(torch.nn.Parameter(a), b)
