@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -91,43 +92,58 @@ def hipcc():
 
 
 def build(verbose=True):
-    """Compile every source for gfx950 and link the shared library. Always recompiles."""
+    """Compile every source for gfx950 and link the shared library; then, with torch and a host compiler there, the host
+    extension, without which the package only takes longer (a RuntimeWarning says why it was not built).
+    Always recompiles."""
     os.makedirs(LIBDIR, exist_ok=True)
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     cc = hipcc()
+
+    def start(cmd):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+
+    def failure(what, proc):
+        """The compiler's output if it failed, else None; waits for it."""
+        out = proc.communicate()[0].decode()
+        return "compiler failed on %s:\n%s" % (what, out) if proc.returncode != 0 else None
+
+    host, host_trouble = None, None
+    try:
+        host_compile, host_link = _host_commands(os.path.join(objdir, "host.o"))
+        host = start(host_compile)
+    except (ImportError, OSError) as e:  # no torch, no compiler
+        host_trouble = str(e)
     procs = []
     for src in SOURCES:
         for suffix, elem in PER_ELEMENT.get(src, (("", 0),)):
             obj = os.path.join(objdir, src.replace(".hip", suffix + ".o"))
             cmd = ([cc] + HIPCC_FLAGS + EXTRA_FLAGS.get(src, []) + ["-DGENBMM_ELEM=%d" % elem, "-c",
                    os.path.join(CSRC, src), "-o", obj])
-            if verbose:
-                print(" ".join(cmd), flush=True)
-            procs.append((src + suffix, obj,
-                          subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
-    host_obj = os.path.join(objdir, "host.o")
-    host_compile, host_link = _host_commands(host_obj)
-    if verbose:
-        print(" ".join(host_compile), flush=True)
-    procs.append(("host.cpp", host_obj, subprocess.Popen(host_compile, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
-    objs = []
-    for src, obj, proc in procs:
-        out = proc.communicate()[0].decode()
-        if proc.returncode != 0:
-            raise RuntimeError("compiler failed on %s:\n%s" % (src, out))
-        if obj != host_obj:
-            objs.append(obj)
+            procs.append((src + suffix, obj, start(cmd)))
+    troubles = [failure(what, proc) for what, _, proc in procs]
+    if host is not None:
+        host_trouble = failure("host.cpp", host)
+    for trouble in troubles:
+        if trouble:
+            raise RuntimeError(trouble)
     tmp = lib_path() + ".tmp"
-    cmd = [cc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc"] + objs + ["-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    cmd = [cc, "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-rdc"] + [obj for _, obj, _ in procs] + ["-o", tmp]
+    trouble = failure(LIBNAME, start(cmd))
+    if trouble:
+        raise RuntimeError(trouble)
     os.replace(tmp, lib_path())
-    if verbose:
-        print(" ".join(host_link), flush=True)
-    subprocess.run(host_link, check=True)
-    os.replace(host_path() + ".tmp", host_path())
+    if not host_trouble:
+        host_trouble = failure("the link of host.cpp", start(host_link))
+    if host_trouble:
+        if host is not None and os.path.exists(host_path()):
+            os.remove(host_path())          # an earlier build's
+        warnings.warn("genbmm_amd: %s is built, the host extension is not: %s" % (LIBNAME, host_trouble), RuntimeWarning,
+                      stacklevel=2)
+    else:
+        os.replace(host_path() + ".tmp", host_path())
     return lib_path()
 
 

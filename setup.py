@@ -22,8 +22,8 @@ class build_py(_build_py):
 
         spec = importlib.util.spec_from_file_location("genbmm_amd_build", os.path.join(ROOT, "genbmm_amd", "build.py"))
         mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)   # torch is not needed to compile
-        mod.build(verbose=False)
+        spec.loader.exec_module(mod)
+        mod.build(verbose=False)       # without torch: the library, not the extension
         inc = os.path.join(ROOT, "genbmm_amd", "include")
         os.makedirs(inc, exist_ok=True)
         shutil.copy(os.path.join(ROOT, "include", "genbmm_gfx950.h"), inc)

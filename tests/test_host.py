@@ -294,6 +294,29 @@ def test_without_the_host_extension_the_functions_carry_the_call(monkeypatch, tm
         assert _lib.host() is None and genmul._native("logbmm", cuda(a), cuda(a), 0, 5) is None
 
 
+@pytest.mark.parametrize("trouble", ["no torch", "no compiler", "no headers"])
+def test_the_library_is_built_whether_or_not_the_host_extension_can_be(monkeypatch, tmp_path, trouble):
+    """The C library needs hipcc alone (here a stand-in that writes what it is asked for)."""
+    import shutil
+    import sys
+
+    from genbmm_amd import build
+
+    cc = tmp_path / "hipcc"
+    cc.write_text('#!/bin/sh\nwhile [ $# -gt 1 ]; do [ "$1" = -o ] && echo x > "$2"; shift; done\n')
+    cc.chmod(0o755)
+    monkeypatch.setattr(build, "hipcc", lambda: str(cc))
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build, "LIBDIR", str(tmp_path / "lib"))
+    if trouble == "no torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    else:
+        monkeypatch.setattr(shutil, "which", lambda name: str(tmp_path / "none") if trouble == "no compiler" else shutil.os.path.join("/bin", "false"))
+    with pytest.warns(RuntimeWarning, match="host extension"):
+        path = build.build(verbose=False)
+    assert os.listdir(tmp_path / "lib") == [build.LIBNAME] and path == str(tmp_path / "lib" / build.LIBNAME)
+
+
 def test_product_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "genbmm_amd")
     for fn in os.listdir(pkg):
