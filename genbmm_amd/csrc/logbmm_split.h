@@ -15,10 +15,12 @@
 // the staged form and the inner loop.  Ragged edges are a second instantiation of each
 // kernel (RAGGED), handled as in logbmm_mfma.h: lines of a tile beyond the matrix re-read
 // the last line (under a shift that makes the factor vanish where the line feeds stored
-// results), stores are masked.  Any sizes: pieces that straddle the right edge are read element
-// by element and the reduction tail is filled by the loader of the last slab in the forward; the
-// backward reads a straddling piece from the last lines and moves its values down when they are
-// staged, and its partial last slab is a step of its own behind the loop.  (Backward of
+// results), stores are masked.  Any sizes: where the reduction is contiguous a thread reads four
+// steps of a line, where the lines are, some steps of one line - lines beyond the matrix are the
+// last one again -, so nothing is astride an edge, and the partial last slab of the forward and the
+// backward is a step of its own behind the loop, with a loader of its own.  The sampling sweep reads
+// its last slab whole and zeroes what lies beyond K; its targets alone come in pieces of four
+// columns, of which one astride the right edge is moved down (shift_down).  (Backward of
 // (64, 511, 509, 510): 368 us on the fp32 instruction, 256 here.)
 //
 // LDS layouts, three planes (h, m, l) per operand, words of two bf16:
@@ -26,14 +28,14 @@
 //    words]; a lane stages four consecutive reduction steps of a line (one 8-byte store
 //    per plane) and reads the eight steps of its line that the instruction wants from it
 //    as one 16-byte load.
-//  * an operand whose source is [reduction][line]: plane[8 step pairs][lines + 8]; a lane
-//    stages a pair of reduction steps for LW consecutive lines (the pair shares a word;
-//    one store of LW words per plane) and reads its eight steps as four words a row apart.
-//  * the same, staged by a line's own threads (SplitL, what forward, backward and sweep use): plane[half of the
-//    slab][line][4 words], an operand one 16-byte read.  The form above takes four reads an operand, which the
-//    compiler pairs across operands and then moves apart (24 moves and a wait for each pair per slab, ahead of the
-//    products): (64, 512^3) forward 108 -> 102 us, both gradients 229 -> 210; (48, 251, 173, 301) 33.8 -> 28.8
-//    and 49.8 -> 46.6, results bit for bit.
+//  * an operand whose source is [reduction][line], staged by a line's own threads (SplitL): plane[half of the
+//    slab][line][4 words], an operand one 16-byte read.
+//  * the same for the one-tile kernels of logbmm_self.h, whose threads hold four lines (SplitS): plane[8 step
+//    pairs][lines + 8]; a thread stages a pair of reduction steps of its four lines (the pair shares a word; one
+//    16-byte store per plane) and the instruction's eight steps are four words a row apart.  The compiler pairs
+//    these four reads across operands and then moves them apart (24 moves and a wait for each pair per slab, ahead
+//    of the products): (64, 512^3) forward 108 us and both gradients 229 in this form, 102 and 210 by SplitL;
+//    (48, 251, 173, 301) 33.8 -> 28.8 and 49.8 -> 46.6, results bit for bit.
 #pragma once
 
 #include "logbmm_mfma.h"
@@ -67,39 +69,25 @@ struct SplitT {
   }
 };
 
-// source [reduction][line]
+// source [reduction][line], a thread stages a pair of reduction steps of four lines
 template <int OUT, int NT>
 struct SplitS {
   static constexpr int LD = OUT + 8;         // words per step pair (lanes 32.. read four rows on: other banks)
   static constexpr int PLANE = 8 * LD;
   static constexpr int BUF = 3 * PLANE;
-  static constexpr int LW = OUT * 8 / NT;    // lines per piece (a pair of reduction steps, LW lines); one piece per thread
-  static_assert(LW == 2 || LW == 4, "");
-  static constexpr int Q = OUT / LW;         // pieces per step pair
-  static __device__ __forceinline__ int pair(int tid) { return tid / Q; }          // reduction steps 2 pair, 2 pair + 1
-  static __device__ __forceinline__ int line0(int tid) { return (tid % Q) * LW; }
-  static __device__ __forceinline__ void put(unsigned* __restrict__ buf, int tid, const float (&even)[LW],
-                                             const float (&odd)[LW]) {
-    unsigned h[LW], m[LW], l[LW];
-#pragma unroll
-    for (int j = 0; j < LW; ++j) split2(even[j], odd[j], h[j], m[j], l[j]);
-    unsigned* p = buf + pair(tid) * LD + line0(tid);
-    if constexpr (LW == 4) {
-      uintx4 w;
-      w.x = h[0]; w.y = h[1]; w.z = h[2]; w.w = h[3]; *reinterpret_cast<uintx4*>(p) = w;
-      w.x = m[0]; w.y = m[1]; w.z = m[2]; w.w = m[3]; *reinterpret_cast<uintx4*>(p + PLANE) = w;
-      w.x = l[0]; w.y = l[1]; w.z = l[2]; w.w = l[3]; *reinterpret_cast<uintx4*>(p + 2 * PLANE) = w;
-    } else {
-      uintx2 w;
-      w.x = h[0]; w.y = h[1]; *reinterpret_cast<uintx2*>(p) = w;
-      w.x = m[0]; w.y = m[1]; *reinterpret_cast<uintx2*>(p + PLANE) = w;
-      w.x = l[0]; w.y = l[1]; *reinterpret_cast<uintx2*>(p + 2 * PLANE) = w;
-    }
-  }
+  static_assert(OUT * 2 == NT, "one piece of a pair and four lines per thread");
+  static __device__ __forceinline__ int pair(int tid) { return tid / (OUT / 4); }  // reduction steps 2 pair, 2 pair + 1
+  static __device__ __forceinline__ int line0(int tid) { return (tid % (OUT / 4)) * 4; }
   static __device__ __forceinline__ void put(unsigned* __restrict__ buf, int tid, float4 even, float4 odd) {
-    static_assert(LW == 4, "");
     const float e[4] = {even.x, even.y, even.z, even.w}, o[4] = {odd.x, odd.y, odd.z, odd.w};
-    put(buf, tid, e, o);
+    unsigned h[4], m[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split2(e[j], o[j], h[j], m[j], l[j]);
+    unsigned* p = buf + pair(tid) * LD + line0(tid);
+    uintx4 w;
+    w.x = h[0]; w.y = h[1]; w.z = h[2]; w.w = h[3]; *reinterpret_cast<uintx4*>(p) = w;
+    w.x = m[0]; w.y = m[1]; w.z = m[2]; w.w = m[3]; *reinterpret_cast<uintx4*>(p + PLANE) = w;
+    w.x = l[0]; w.y = l[1]; w.z = l[2]; w.w = l[3]; *reinterpret_cast<uintx4*>(p + 2 * PLANE) = w;
   }
   static __device__ __forceinline__ bf16x8 frag(const unsigned* __restrict__ buf, int plane, int line0, int lane) {
     const unsigned* p = buf + plane * PLANE + (lane >> 5) * 4 * LD + line0 + (lane & 31);
