@@ -7,10 +7,9 @@
 // 107 us by the Python Functions, 54 here, 49 for one multiplication of torch's own with its gradients.
 //
 // Which calls it takes (`plain`): tensors of the exact types Tensor / Parameter, float32 / float16 / bfloat16, 3-D,
-// contiguous, of one batch size, on one GPU, under no trace, dispatch mode or functorch transform, whose reduction
-// is not cut in Python.  For any other the functions return None and genmul.py goes on as it does without them -
-// conversions, double precision, the messages of what is refused.  A node of this file refuses
-// forward-mode tangents and batched gradients as the Python ones do (neither has a derivative formula for them).
+// contiguous, of one batch size, on one GPU, without a forward-mode tangent, under no trace, dispatch mode or functorch
+// transform, whose reduction is not cut in Python.  For any other the functions return None and genmul.py goes on as
+// it does without them - conversions, double precision, the messages of what is refused.
 #include <ATen/core/TorchDispatchUtils.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
@@ -68,25 +67,10 @@ void require(const Tensor& t, const char* name, const Tensor& like, at::ScalarTy
   TORCH_CHECK(t.is_contiguous() && t.sizes() == sizes, name, " must be contiguous, of sizes ", sizes, ", got ", t.sizes());
 }
 
-// -------------------------------------------------------------------- logbmm
-// The gradients where none of their own will be asked for (see LogBmm::backward).  A node all the same: it is what
-// refuses an incoming gradient with a tangent.
-struct LogGrad : torch::autograd::Function<LogGrad> {
-  static variable_list forward(AutogradContext*, const Tensor& a, const Tensor& b, const Tensor& g, const Tensor& out,
-                               const Tensor& stats, int64_t path) {
-    const c10::DeviceGuard guard(a.device());
-    const Dims d = dims_of(a, b);
-    Tensor ga = at::empty_like(a), gb = at::empty_like(b);
-    check(GENBMM_BY_TYPE(a, genbmm_logbmm_bwd_path, at_<E>(a), at_<E>(b), at_<E>(out), at_<E>(g), at_<float>(stats),
-                         at_<E>(ga), at_<E>(gb), d.B, d.M, d.K, d.N, (int)path, stream_of(a)),
-          "genbmm_logbmm_bwd_path");
-    return {ga, gb};
-  }
-  static variable_list backward(AutogradContext*, variable_list) {
-    TORCH_CHECK(false, "genbmm_amd: not reached, the second order is genmul._LogBmmGrad's");
-  }
-};
+// a forward-mode tangent: a C++ node refuses it as a RuntimeError, the Python nodes as its NotImplementedError
+bool has_tangent(const Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
 
+// -------------------------------------------------------------------- logbmm
 struct LogBmm : torch::autograd::Function<LogBmm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& a, const Tensor& b, int64_t path) {
     const c10::DeviceGuard guard(a.device());
@@ -116,13 +100,18 @@ struct LogBmm : torch::autograd::Function<LogBmm> {
     require(out, "the result", g, type, {d.B, d.M, d.N});
     require(saved[3], "the forward's workspace", g, at::kFloat,
             {(int64_t)genbmm_logbmm_stats_size_path(d.B, d.M, d.K, d.N, (int)path)});
-    if (at::GradMode::is_enabled()) {  // differentiated again: the Python node has the formula
+    // differentiated again, where the Python node has the formula, or along a tangent, which it refuses
+    if (at::GradMode::is_enabled() || has_tangent(g) || has_tangent(a) || has_tangent(b)) {
       const py::gil_scoped_acquire gil;
       const py::tuple r = py::module_::import("genbmm_amd.genmul").attr("_LogBmmGrad").attr("apply")(a, b, g, out, saved[3], path);
       return {r[0].cast<Tensor>(), r[1].cast<Tensor>(), Variable()};
     }
-    const variable_list r = LogGrad::apply(a, b, g, out, saved[3], path);
-    return {r[0], r[1], Variable()};
+    const c10::DeviceGuard guard(a.device());
+    Tensor ga = at::empty_like(a), gb = at::empty_like(b);
+    check(GENBMM_BY_TYPE(a, genbmm_logbmm_bwd_path, at_<E>(a), at_<E>(b), at_<E>(out), at_<E>(g), at_<float>(saved[3]),
+                         at_<E>(ga), at_<E>(gb), d.B, d.M, d.K, d.N, (int)path, stream_of(a)),
+          "genbmm_logbmm_bwd_path");
+    return {ga, gb, Variable()};
   }
 };
 
@@ -224,6 +213,7 @@ bool plain(const py::handle& pa, const py::handle& pb) {
   if (type != at::kFloat && type != at::kHalf && type != at::kBFloat16) return false;
   const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(2);
   if (b.size(0) != B || b.size(1) != K || !a.is_contiguous() || !b.is_contiguous()) return false;
+  if (has_tangent(a) || has_tangent(b)) return false;
   constexpr int64_t most = 0x7fffffff;
   if (B > most || M > most || N > most) return false;
   if (K >= 4096) return false;  // genmul._reduction_splits may cut it

@@ -100,37 +100,62 @@ def test_what_takes_the_route(gpu):
         assert not native(x, y)
 
 
+def refusal(f, *args):
+    """(type, message) of what f raises."""
+    with pytest.raises(Exception) as e:
+        f(*args)
+    return e.type, str(e.value)
+
+
+def same_refusal(attempt, fs, kind, words):
+    """Every f of fs refused by `attempt`, with one type and one message that says `words`."""
+    got = [refusal(attempt, f) for f in fs]
+    assert got[0][0] is kind and words in got[0][1] and all(x == got[0] for x in got), got
+
+
 @pytest.mark.parametrize("op", list(PAIRS))
 def test_refused_as_before(gpu, op):
     a, b, g = operands(gpu, 2, 6, 5, 7, torch.float32)
-    for f in PAIRS[op]:
+
+    def forward_mode(f, which=0):
+        with forward_ad.dual_level():
+            x = [a, b]
+            x[which] = forward_ad.make_dual(x[which], x[which])
+            f(*x)
+
+    def batched(f):
         x = a.clone().requires_grad_()
-        with forward_ad.dual_level(), pytest.raises(Exception):       # no forward-mode formula
-            f(forward_ad.make_dual(a, a), b)
+        torch.autograd.grad(f(x, b), x, torch.stack([g, g]), is_grads_batched=True)
+
+    def twice(f):
+        x = a.clone().requires_grad_()
+        out = f(x * 1, b)
+        torch.autograd.grad(out, x, g)
+        torch.autograd.grad(out, x, g)
+
+    def changed(f):
+        x = (a * 1).requires_grad_()
         out = f(x, b)
-        with pytest.raises(RuntimeError):                             # no batching rule
-            torch.autograd.grad(out, x, torch.stack([g, g]), is_grads_batched=True)
-        with pytest.raises(Exception):
-            torch.func.vmap(f)(torch.stack([a, a]), torch.stack([b, b]))
-        with pytest.raises(Exception):
-            torch.func.grad(lambda t: f(t, b).sum())(a)
-        y = a.clone().requires_grad_()
-        out = f(y * 1, b)
-        torch.autograd.grad(out, y, g)
-        with pytest.raises(RuntimeError):                             # the graph is gone
-            torch.autograd.grad(out, y, g)
+        with torch.no_grad():
+            x.add_(1)
+        torch.autograd.grad(out, x, g)
+
+    def tangent(f):
+        x = a.clone().requires_grad_()
+        out = f(x, b)
+        with forward_ad.dual_level():
+            torch.autograd.grad(out, x, forward_ad.make_dual(g, g))
+
+    fs = PAIRS[op]
+    same_refusal(forward_mode, fs, NotImplementedError, "jvp")
+    same_refusal(lambda f: forward_mode(f, 1), fs, NotImplementedError, "jvp")
+    same_refusal(batched, fs, RuntimeError, "doesn't have storage")
+    same_refusal(lambda f: torch.func.vmap(f)(torch.stack([a, a]), torch.stack([b, b])), fs, RuntimeError, "setup_context")
+    same_refusal(lambda f: torch.func.grad(lambda t: f(t, b).sum())(a), fs, RuntimeError, "setup_context")
+    same_refusal(twice, fs, RuntimeError, "a second time")
     if op == "log":
-        for f in PAIRS[op]:
-            x = (a * 1).requires_grad_()
-            out = f(x, b)
-            with torch.no_grad():
-                x.add_(1)
-            with pytest.raises(RuntimeError):                         # saved for the backward, then changed
-                torch.autograd.grad(out, x, g)
-            x = a.clone().requires_grad_()
-            out = f(x, b)
-            with forward_ad.dual_level(), pytest.raises(Exception):   # a tangent on the incoming gradient
-                torch.autograd.grad(out, x, forward_ad.make_dual(g, g))
+        same_refusal(changed, fs, RuntimeError, "modified by an inplace operation")    # saved for the backward
+        same_refusal(tangent, fs, NotImplementedError, "jvp")
 
 
 @pytest.mark.parametrize("op", list(PAIRS))
