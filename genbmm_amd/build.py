@@ -8,6 +8,7 @@ torch CUDAExtension named `_genbmm`): the kernels are a plain shared library wit
 torch extension (csrc/host.cpp, lib/_host.*.so) holds the eager products' autograd nodes.  hipcc cross-compiles for gfx950 without
 a GPU being present.
 """
+import glob
 import os
 import shutil
 import subprocess
@@ -135,11 +136,11 @@ def build(verbose=True):
     if trouble:
         raise RuntimeError(trouble)
     os.replace(tmp, lib_path())
+    for old in glob.glob(os.path.join(glob.escape(LIBDIR), "_host.*")):
+        os.remove(old)                      # an earlier build's: linked to the library that has just been replaced
     if not host_trouble:
         host_trouble = failure("the link of host.cpp", start(host_link))
     if host_trouble:
-        if host is not None and os.path.exists(host_path()):
-            os.remove(host_path())          # an earlier build's
         warnings.warn("genbmm_amd: %s is built, the host extension is not: %s" % (LIBNAME, host_trouble), RuntimeWarning,
                       stacklevel=2)
     else:

@@ -296,7 +296,8 @@ def test_without_the_host_extension_the_functions_carry_the_call(monkeypatch, tm
 
 @pytest.mark.parametrize("trouble", ["no torch", "no compiler", "no headers"])
 def test_the_library_is_built_whether_or_not_the_host_extension_can_be(monkeypatch, tmp_path, trouble):
-    """The C library needs hipcc alone (here a stand-in that writes what it is asked for)."""
+    """The C library needs hipcc alone (here a stand-in that writes what it is asked for).  An extension that was built
+    against the library before it does not stay beside the new one, whichever torch it was for."""
     import shutil
     import sys
 
@@ -308,6 +309,9 @@ def test_the_library_is_built_whether_or_not_the_host_extension_can_be(monkeypat
     monkeypatch.setattr(build, "hipcc", lambda: str(cc))
     monkeypatch.setattr(build, "HERE", str(tmp_path))
     monkeypatch.setattr(build, "LIBDIR", str(tmp_path / "lib"))
+    (tmp_path / "lib").mkdir()
+    for earlier in (os.path.basename(build.host_path()), "_host.torch-0.so"):
+        (tmp_path / "lib" / earlier).write_text("linked to the library before")
     if trouble == "no torch":
         monkeypatch.setitem(sys.modules, "torch", None)
     else:
