@@ -1,5 +1,4 @@
-"""Timing of every benchmark configuration on one MI355X (bench.py covers only the
-headline line the driver reads).
+"""Timing of every benchmark configuration on one MI355X (bench.py covers only the headline).
 
     python bench_configs.py [--reps 20] [--cpu]
 

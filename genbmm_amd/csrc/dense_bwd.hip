@@ -38,8 +38,10 @@ constexpr int kKC = 128;  // cells of the reduction axis per lane
 // prodmaxbmm (814, 76, 51, 83) 165 -> 153; clamped addresses in the place of the uniform tests: 5 % slower).
 // One wave on a SIMD issues everything itself, so instructions count: a slot by one unsigned minimum and a column's
 // addresses carried along (two chunks of a column 687 -> 482 instructions, of a row 950 -> 760): max and
-// sample (256, 256^3) 75 -> 66 us, (64, 512^3) 123 -> 99, (40, 251, 173, 301) 21.5 -> 17.8, (100, 500, 300, 510)
-// 197 -> 159, (512, 128^3) 34 either way (memory).  With the product semiring's factors the same took more registers
+// sample, again and again on one set of buffers, which the Infinity Cache holds in part, and (in brackets) on other
+// buffers each time, as behind a forward: (256, 256^3) 74 -> 65 us (85 -> 78), (64, 512^3) 124 -> 99 (133 -> 111),
+// (40, 251, 173, 301) 21.6 -> 17.9 (22.5 -> 20.7), (100, 500, 300, 510) 198 -> 160 (200 -> 163), (512, 128^3) 34
+// (43) either way (memory).  With the product semiring's factors the same took more registers
 // than a wave's 256 ((512, 128^3) 47 -> 51, (64, 512^3) 158 -> 139): it keeps the longer form.
 static_assert(kKC == 128, "the shifts of the write-out");
 constexpr int kArgAcc = 64 * kKC + 64;  // floats of LDS: the cells, one spare cell per lane

@@ -43,14 +43,16 @@ def test_results(gpu, op, dtype, B, M, K, N):
     for needs in ("ab", "a", "b"):
         x, y = a.clone().requires_grad_("a" in needs), b.clone().requires_grad_("b" in needs)
         wrt = [t for t in (x, y) if t.requires_grad]
-        for grad in (g, g.float(), g.transpose(1, 2).contiguous().transpose(1, 2), g[:1, :1, :1].expand_as(g) if g.numel() else g):
+        # (a gradient of another type: values that the result's type does not hold)
+        for grad in (g, torch.randn_like(g, dtype=torch.float64), g.transpose(1, 2).contiguous().transpose(1, 2),
+                     g[:1, :1, :1].expand_as(g) if g.numel() else g):
             if op == "prodmax" and M == 0:      # no factors to read the gradient from: refused
                 for f in (new, old):
-                    with pytest.raises(RuntimeError):
-                        torch.autograd.grad(f(x, y), wrt, grad.to(dtype))
+                    with pytest.raises(RuntimeError, match="genbmm_prodmax_bwd"):
+                        torch.autograd.grad(f(x, y), wrt, grad)
                 continue
-            got = torch.autograd.grad(new(x, y), wrt, grad.to(dtype))
-            want = torch.autograd.grad(old(x, y), wrt, grad.to(dtype))
+            got = torch.autograd.grad(new(x, y), wrt, grad)
+            want = torch.autograd.grad(old(x, y), wrt, grad)
             assert all(torch.equal(p, q) for p, q in zip(got, want))
 
 
@@ -196,5 +198,5 @@ def test_what_a_saved_tensor_hook_may_not_return(gpu, op, unpack):
     x = a.clone().requires_grad_()
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
         out = PAIRS[op][0](x, b)
-    with pytest.raises(RuntimeError):
+    with pytest.raises(RuntimeError, match="expected|must be"):
         torch.autograd.grad(out, x, g)
