@@ -123,6 +123,7 @@ def load():
         fn.argtypes = argtypes
         fn.restype = ctypes.c_size_t
     _lib = lib
+    host()
     return lib
 
 
@@ -134,8 +135,8 @@ def host():
     this torch and this Python, or where it does not load.  genmul's Functions then carry every call, with the same
     results and more host time."""
     global _host
+    load()      # the library it is linked to; the first call of it comes here itself
     if _host is None:
-        load()      # the library it is linked to
         from . import build
 
         spec = importlib.util.spec_from_file_location("genbmm_amd.lib._host", build.host_path())
@@ -145,8 +146,8 @@ def host():
             _host = module
         except ImportError as e:
             _host = False
-            warnings.warn("genbmm_amd: small products take longer than they need to, without their native autograd nodes "
-                          "(%s); build them with `python -m genbmm_amd.build`" % e, RuntimeWarning, stacklevel=2)
+            warnings.warn("genbmm_amd: small products take longer than they need to, without the host extension "
+                          "(%s); build it with `python -m genbmm_amd.build`" % e, RuntimeWarning, stacklevel=2)
     return _host or None
 
 
@@ -167,6 +168,8 @@ def stream_of(t):
 def dense(t):
     """t as the kernels read it, by differentiable torch operations: contiguous, and written out if it carries
     torch's lazy negative bit (`z.conj().imag`), which `contiguous` keeps where the strides already fit."""
+    if _host and _host.is_dense(t):
+        return t
     t = t.contiguous()
     return t.resolve_neg() if t.is_neg() else t
 
@@ -180,6 +183,8 @@ def addr(t):
     a pointer (`ptr`).  Refused where the memory holds the values with the other sign."""
     if t is None:
         return None
+    if _host:
+        return _host.address(t)
     if t.is_neg():
         raise RuntimeError("genbmm_amd: a tensor with the lazy negative bit has no memory that holds its values")
     return t.data_ptr()

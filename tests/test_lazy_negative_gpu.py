@@ -11,6 +11,14 @@ pytestmark = pytest.mark.gpu
 STREAM = (11, 4)
 
 
+@pytest.fixture(autouse=True, params=[True, False], ids=["extension", "python"])
+def extension(request, monkeypatch):
+    """With the host extension, whose checks look at the bit as well, and without it."""
+    assert _lib.host() is not None
+    if not request.param:
+        monkeypatch.setattr(_lib, "_host", False)
+
+
 def lazy(t):
     """t's values, contiguous, with the negative bit set: the storage holds -t."""
     x = torch._neg_view((-t).contiguous())
