@@ -142,6 +142,18 @@ __device__ __forceinline__ void st4m(E* p, int cnt, float4 v) {
   if (cnt > 1) p[1] = to_elem<E>(v.y);
   if (cnt > 2) p[2] = to_elem<E>(v.z);
 }
+// The bytes [x, x + bytes) as a buffer, and an element of it at `at` (per lane) + `base` (uniform) bytes: the uniform
+// part costs no address arithmetic in the lanes.  Reads beyond the end give 0 (at must not be negative).
+typedef __amdgpu_buffer_rsrc_t buf_t;
+template <class E>
+__device__ __forceinline__ buf_t buf_of(const E* x, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<E*>(x), 0, bytes, 0x00020000);
+}
+template <class E>
+__device__ __forceinline__ E buf_ld(buf_t x, int at, int base) {
+  if constexpr (sizeof(E) == 4) return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(x, at, base, 0));
+  else return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b16(x, at, base, 0));
+}
 __device__ __forceinline__ int clamp4(int x) { return min(max(x, 0), 4); }
 
 // ---------------------------------------------------------------- tile loaders

@@ -657,15 +657,15 @@ inline int64_t header_offset(int B, int M, int N) {
   const int64_t o = (int64_t)B * (M + N) + tiles32(B, M, N);
   return (o + 3) & ~(int64_t)3;
 }
-// Small matrices: a whole batch item per workgroup (logbmm_item.h).
+// Small matrices: a whole batch item per workgroup (logbmm_item.h), wherever its LDS suffices.
 inline bool item_shape(int M, int K, int N) {
-  return M >= 1 && K >= 1 && N >= 1 && M <= 64 && K <= 64 && N <= 64;
+  return M >= 1 && K >= 1 && N >= 1 && max(max(M, K), N) <= kItemMax && 4 * item_bwd_floats(M, K, N, 8, 2) <= kItemLds;
 }
 
-// Items of one 128 x 128 tile, each extent large enough for the tile to pay: forward
-// and backward form everything they need themselves (logbmm_self.h).
+// Items of one 128 x 128 tile that are too large for that: forward and backward form
+// everything they need themselves (logbmm_self.h).
 inline bool self_shape(int M, int K, int N) {
-  return max(max(M, K), N) <= kSelfMax && min(min(M, K), N) >= 64 && !item_shape(M, K, N);
+  return max(max(M, K), N) <= kSelfMax && min(min(M, K), N) >= 32 && !item_shape(M, K, N);
 }
 
 // Shapes whose forward runs on the matrix cores (given alignment and path).
@@ -682,6 +682,25 @@ inline bool fwd_mfma_shape(int B, int M, int K, int N) {
   if (!mfma_extents(M, N, K)) return false;
   const int64_t t128 = tiles128(B, M, N);
   return t128 <= 0x7fffffff;
+}
+// Narrower extents, as far as the three-part kernels' 128 x 128 tiles still beat the factored vector-ALU kernels (whose
+// tiles are 64 wide): by the cells computed, padding included, of the latter and of the former.
+// Forward: half as many or more ((305,90,131,93) 57 -> 43 us; 0.38 of them, (1000,60,60,160): 57 -> 72), or tiles so few that
+// the chip is not full and a reduction worth their prologue ((40,33,512,40) 53 -> 43; (64,400,33,64) 16 -> 19).
+// Both gradients: 0.7 of one tile's share in sum ((2000,33,200,33) 204 -> 158, (1000,48,140,64) 101 -> 88;
+// 0.63, (1000,60,60,160): 108 -> 120), or few tiles ((64,400,33,64) 62 -> 42).
+inline double tile_share(int out_r, int out_c) {  // vector-ALU kernels' cells over 128 x 128 tiles' cells
+  return (double)(ceil_div(out_r, 64) * (int64_t)ceil_div(out_c, 64)) / (4.0 * ceil_div(out_r, 128) * ceil_div(out_c, 128));
+}
+inline bool fwd_narrow_shape(int B, int M, int K, int N) {
+  if (min(M, N) <= 32 || K < kMS || mfma_extents(M, N, K)) return false;
+  const int64_t t128 = tiles128(B, M, N);
+  return t128 <= 0x7fffffff && (tile_share(M, N) >= 0.5 || (t128 <= 512 && K >= 96));
+}
+inline bool bwd_narrow_shape(int B, int M, int K, int N) {
+  if (min(min(M, K), N) <= 32) return false;
+  const int64_t ta = tiles128(B, M, K), tb = tiles128(B, K, N);
+  return ta + tb <= 0x7fffffff && (tile_share(M, K) + tile_share(K, N) >= 0.7 || ta + tb <= 512);
 }
 inline LogPrepared prepared_of(const float* stats, int B, int M, int K, int N) {
   float* base = const_cast<float*>(stats) + header_offset(B, M, N);
@@ -978,31 +997,40 @@ int launch_bwd_split_both(LogBwdArgs pa, LogBwdArgs pb, const float* stats, int 
 // padding and there are tiles enough to give every compute unit two workgroups of
 // eight waves), 1 for 128x128, 0 for none (path, or extents too small).  `long_cols`:
 // the 256 side is the column side of the output.
-inline int mfma_kind(int path, int B, int out_r, int out_c, int red, bool long_cols) {
-  if (!auto_path(path) || !mfma_extents(out_r, out_c, red)) return 0;
+inline int tile_kind(int B, int out_r, int out_c, bool long_cols) {
   const int64_t t128 = tiles128(B, out_r, out_c);
   if (t128 > 0x7fffffff) return 0;
   const int L = long_cols ? out_c : out_r;
   if (ceil_div(L, 256) * 2 == ceil_div(L, 128) && t128 >= 512) return 2;
   return 1;
 }
+inline int mfma_kind(int path, int B, int out_r, int out_c, int red, bool long_cols) {
+  return auto_path(path) && mfma_extents(out_r, out_c, red) ? tile_kind(B, out_r, out_c, long_cols) : 0;
+}
+// The forward's tiling: the three-part kernels take narrower extents.
+inline int fwd_kind(int path, int B, int M, int K, int N) {
+  if (split_path(path) && fwd_narrow_shape(B, M, K, N)) return tile_kind(B, M, N, false);
+  return fwd_mfma_shape(B, M, K, N) ? mfma_kind(path, B, M, N, K, false) : 0;
+}
 
 // The tiling of both gradients of a matrix-core shape in one launch of the three-part kernels: 2 or 1 as
 // above, 0 where the gradients are too narrow for tiles (K) or an item too large.  The two gradients count
 // their tiles apart and may land on either side of the 512: both then run on 128 x 128 tiles.
 inline int bwd_split_kind(int B, int M, int K, int N) {
-  if (!fwd_mfma_shape(B, M, K, N) || !bwd_split_sizes(M, K, N)) return 0;
-  const int ka = mfma_kind(GENBMM_PATH_AUTO, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_AUTO, B, K, N, M, false);
+  if (!bwd_split_sizes(M, K, N)) return 0;
+  if (!(mfma_extents(M, K, N) && mfma_extents(K, N, M)) && !bwd_narrow_shape(B, M, K, N)) return 0;
+  const int ka = tile_kind(B, M, K, true), kb = tile_kind(B, K, N, false);
   return ka == 0 || kb == 0 ? 0 : min(ka, kb);
 }
 
 // What the forward keeps under GENBMM_PATH_RECIP: 1 / S alone where both gradients run on the three-part
 // kernels, which form EA and EB again; all three factors where they run on the fp32 instruction (an item too
-// large for the former), as under GENBMM_PATH_FACTORS; nothing where no gradient is tiled (K below 96): the
-// vector-ALU kernels read maxima and `out` ((64, 300, 60, 300): 32 MB that the forward wrote and nothing read).
+// large for the former), as under GENBMM_PATH_FACTORS; nothing where the forward or every gradient runs on the
+// vector ALU or an item in a workgroup: those read maxima and `out`.
 inline int recip_keeps(int B, int M, int K, int N) {
-  if (!fwd_mfma_shape(B, M, K, N) || self_shape(M, K, N)) return kKeepNone;
+  if (item_shape(M, K, N) || self_shape(M, K, N) || fwd_kind(GENBMM_PATH_AUTO, B, M, K, N) == 0) return kKeepNone;
   if (bwd_split_kind(B, M, K, N) != 0) return kKeepRecip;
+  if (!fwd_mfma_shape(B, M, K, N)) return kKeepNone;
   const int ka = mfma_kind(GENBMM_PATH_AUTO, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_AUTO, B, K, N, M, false);
   return ka != 0 || kb != 0 ? kKeepFactors : kKeepNone;
 }
@@ -1038,10 +1066,19 @@ int run_bwd(const LogBwdArgs& p, const float* stats, int path, int B, hipStream_
   return launch_bwd_exact<BCfgMid, GRAD_A>(p, B, s);
 }
 
-template <int G, int TB, bool FULL>
+template <int W, int U, int H>
 void launch_item_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int* hdr, int B, int M,
                      int K, int N, hipStream_t s) {
-  hipLaunchKernelGGL((k_log_item_fwd<G, TB, FULL>), dim3(B), dim3(G * G), 0, s, a, b, out, stats, hdr, M, K, N);
+  const int lds = 4 * item_fwd_floats(M, K, N, W, H);
+  if (H > 1) allow_lds(k_log_item_fwd<W, U, H>, lds);
+  hipLaunchKernelGGL((k_log_item_fwd<W, U, H>), dim3(B), dim3(64 * W), lds, s, a, b, out, stats, hdr, M, K, N);
+}
+template <int W, int U, int H>
+void launch_item_bwd(const elem_t* a, const elem_t* b, const elem_t* out, const elem_t* g, elem_t* grad_a, elem_t* grad_b,
+                     int B, int M, int K, int N, hipStream_t s) {
+  const int lds = 4 * item_bwd_floats(M, K, N, W, H);
+  if (H > 1) allow_lds(k_log_item_bwd<W, U, H>, lds);
+  hipLaunchKernelGGL((k_log_item_bwd<W, U, H>), dim3(B), dim3(64 * W), lds, s, a, b, out, g, grad_a, grad_b, M, K, N);
 }
 
 // keep: the workspace is as large as genbmm_logbmm_stats_size says and receives what a
@@ -1108,13 +1145,18 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
   if (missing(a, mk) || missing(b, kn) || missing(out, mn)) return GENBMM_E_NULLPTR;
   int keep = keep_factors && (path == GENBMM_PATH_FACTORS || factors) ? kKeepFactors : kKeepNone;
   if (path == GENBMM_PATH_RECIP) keep = recip_keeps(B, M, K, N);
-  if (stats && B > 0 && item_shape(M, K, N) && auto_path(path)) {  // whole items per workgroup
+  if (keep == kKeepFactors && (!fwd_mfma_shape(B, M, K, N) || (!factors && item_shape(M, K, N))))
+    keep = kKeepNone;  // (the workspace has no room for them)
+  if (stats && B > 0 && item_shape(M, K, N) && auto_path(path) && !(factors && keep == kKeepFactors)) {  // whole items per workgroup
     int* hdr = prepared_of(stats, B, M, K, N).hdr;
+    const int most = max(max(M, K), N);
     if (M == 32 && K == 32 && N == 32)  // one wave per item on the matrix cores
       hipLaunchKernelGGL(k_log_item32_fwd, dim3((B + 3) / 4), dim3(256), 0, s, a, b, out, stats, hdr, B);
-    else if (M == 64 && K == 64 && N == 64) launch_item_fwd<16, 4, true>(a, b, out, stats, hdr, B, M, K, N, s);
-    else if (max(max(M, K), N) <= 32) launch_item_fwd<16, 2, false>(a, b, out, stats, hdr, B, M, K, N, s);
-    else launch_item_fwd<16, 4, false>(a, b, out, stats, hdr, B, M, K, N, s);
+    else if (most <= 32) launch_item_fwd<4, 2, 1>(a, b, out, stats, hdr, B, M, K, N, s);
+    else if (most <= 48) launch_item_fwd<4, 3, 1>(a, b, out, stats, hdr, B, M, K, N, s);
+    else if (most <= 64) launch_item_fwd<4, 4, 1>(a, b, out, stats, hdr, B, M, K, N, s);
+    else if (most <= 96) launch_item_fwd<8, 3, 2>(a, b, out, stats, hdr, B, M, K, N, s);
+    else launch_item_fwd<8, 4, 2>(a, b, out, stats, hdr, B, M, K, N, s);
     return launch_status();
   }
   DenseArgs p{};
@@ -1131,7 +1173,7 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
   }
   if (stats && K > 0 && path != GENBMM_PATH_EXACT) {
     const int64_t big_tiles = (int64_t)B * ceil_div(M, 128) * ceil_div(N, 128);
-    switch (fwd_mfma_shape(B, M, K, N) ? mfma_kind(path, B, M, N, K, false) : 0) {
+    switch (fwd_kind(path, B, M, K, N)) {
       case 2:
         if (split_path(path)) {
           if (split_big_fits(B, M, N)) return launch_fwd_split<MTBig>(p, stats, B, M, K, N, keep, s);
@@ -1171,14 +1213,19 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
   p.vec_n = (N % 4 == 0) && aligned16(b) && aligned16(out) && aligned16(g) && aligned16(grad_b);
   const float* st = (path == GENBMM_PATH_EXACT || mn == 0) ? nullptr : stats;
   if (st && B > 0 && item_shape(M, K, N) && auto_path(path)) {
+    const int most = max(max(M, K), N);
     if (M == 32 && K == 32 && N == 32)
       hipLaunchKernelGGL(k_log_item32_bwd, dim3((B + 3) / 4), dim3(256), 0, s, a, b, out, g, grad_a, grad_b, B);
-    else if (M == 64 && K == 64 && N == 64)
-      hipLaunchKernelGGL((k_log_item_bwd<16, 4, true>), dim3(B), dim3(256), 0, s, a, b, out, g, grad_a, grad_b, M, K, N);
-    else if (max(max(M, K), N) <= 32)
-      hipLaunchKernelGGL((k_log_item_bwd<16, 2>), dim3(B), dim3(256), 0, s, a, b, out, g, grad_a, grad_b, M, K, N);
+    else if (most <= 32)
+      launch_item_bwd<4, 2, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
+    else if (most <= 48)
+      launch_item_bwd<4, 3, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
+    else if (most <= 64)
+      launch_item_bwd<4, 4, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
+    else if (most <= 96)
+      launch_item_bwd<8, 3, 2>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
     else
-      hipLaunchKernelGGL((k_log_item_bwd<16, 4>), dim3(B), dim3(256), 0, s, a, b, out, g, grad_a, grad_b, M, K, N);
+      launch_item_bwd<8, 4, 2>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
     return launch_status();
   }
   if (st && B > 0 && self_shape(M, K, N) && auto_path(path)) {
@@ -1198,8 +1245,11 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
     }
     return launch_status();
   }
-  if (path == GENBMM_PATH_RECIP && recip_keeps(B, M, K, N) != kKeepRecip) path = GENBMM_PATH_FACTORS;
-  if (st && grad_a && grad_b && mk > 0 && kn > 0 && fwd_mfma_shape(B, M, K, N)) {
+  if (path == GENBMM_PATH_RECIP) {
+    const int keeps = recip_keeps(B, M, K, N);
+    if (keeps != kKeepRecip) path = keeps == kKeepFactors ? GENBMM_PATH_FACTORS : GENBMM_PATH_AUTO;
+  }
+  if (st && grad_a && grad_b && mk > 0 && kn > 0) {
     LogBwdArgs pa = p, pb = p;
     pa.grad = grad_a;
     pb.grad = grad_b;
@@ -1212,7 +1262,7 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
     }
     const int ka = mfma_kind(path, B, M, K, N, true), kb = mfma_kind(path, B, K, N, M, false);
     const bool lean = path != GENBMM_PATH_FACTORS;
-    if (ka == kb && ka != 0)
+    if (ka == kb && ka != 0 && fwd_mfma_shape(B, M, K, N))
       return ka == 2 ? launch_bwd_mfma_both<MTWide, MTTall>(pa, pb, st, B, s, lean)
                      : launch_bwd_mfma_both<MT128, MT128>(pa, pb, st, B, s, lean);
   }
@@ -1264,7 +1314,6 @@ int static_workspace(float** ws) {
 // matrix-core kernels only.
 bool log_fwd_writes_factors(const float* stats, int B, int M, int K, int N, LogFactors* f) {
   if (!stats || K <= 0 || (int64_t)B * M * N == 0) return false;
-  if (B > 0 && item_shape(M, K, N)) return false;   // whole-item kernels
   if (!fwd_mfma_shape(B, M, K, N)) return false;
   if (mfma_kind(GENBMM_PATH_AUTO, B, M, N, K, false) == 0) return false;
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
@@ -1424,7 +1473,8 @@ size_t genbmm_logbmm_stats_size_path(int B, int M, int K, int N, int path) {
   // the by-products of the matrix-core forward (the one-tile kernels keep the maxima only)
   int keep = kKeepNone;
   if (path == GENBMM_PATH_RECIP) keep = recip_keeps(B, M, K, N);
-  else if (path == GENBMM_PATH_FACTORS && fwd_mfma_shape(B, M, K, N) && !self_shape(M, K, N)) keep = kKeepFactors;
+  else if (path == GENBMM_PATH_FACTORS && fwd_mfma_shape(B, M, K, N) && !item_shape(M, K, N) && !self_shape(M, K, N))
+    keep = kKeepFactors;
   if (keep == kKeepRecip) n += (int64_t)B * M * N;
   else if (keep == kKeepFactors)
     n += (int64_t)B * ((int64_t)M * K + (int64_t)K * N + (int64_t)M * N);

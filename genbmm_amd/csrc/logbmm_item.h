@@ -1,8 +1,6 @@
-// logbmm for small matrices (M, K, N <= 64): one workgroup per batch item, the
-// whole item in LDS, one launch for the forward and one for both gradients.
-// At these sizes the problem is launch- and HBM-bound (a 32^3 item is 12 KB of
-// operands and 0.2 M products), so the kernels read every operand exactly once
-// and write every result exactly once, in contiguous runs.
+// logbmm for small matrices (extents of at most 128, and their LDS below): one workgroup per batch item, the
+// whole item in LDS, one launch for the forward and one for both gradients, the
+// contractions on v_mfma_f32_16x16x4_f32.
 //
 // Same factored form as the large kernels: alpha[m] = max_k a, beta[n] = max_k b
 // are taken inside the workgroup, EA = exp(a - alpha), EB = exp(b - beta),
@@ -11,6 +9,23 @@
 // item (backward) for which the factoring is not exact to fp32 - S < 2^-40, a
 // shift at the reference's -1e9 floor, anything non-finite - is recomputed inside
 // the same kernel from global memory with the reference's own two-pass form.
+//
+// Staging: a wave takes groups of four neighbouring rows of an array, its lanes the columns (a row is
+// contiguous in memory; all loads of the item are issued before the first is waited for).  A row's
+// maximum is then one wave's reduction and a scalar, a column's is joined through LDS, and a lane's
+// four rows are four neighbouring steps of an operand whose lines are the columns: one 16-byte store.
+// Arrays are padded to multiples of 16 with zeros, lines are 16 j + 4 words apart: the 16-byte reads of
+// a matrix operand (16 lines x 4 steps each) and the stores across lines meet every bank evenly.
+//
+// Why 16 x 16 tiles of the fp32 instruction: padding to 16 instead of 32 or 64 is what sizes in between
+// cost ((8192,39^3): 2.4 times fewer products than with 32), and at these extents an item's products take no longer
+// than its memory traffic, so the three-part form of the larger kernels would pay its cuts for nothing.
+//
+// Measured, forward + both gradients (before: the item on the vector ALU up to 64^3, the factored vector-ALU kernels or one
+// 128 x 128 tile beyond): (2048,64^3) 44 + 73 -> 33 + 53 us, (8192,39^3) 99 + 158 -> 55 + 83 (bfloat16 112 + 220 -> 51 + 77),
+// (5163,57^3) float16 113 + 245 -> 65 + 104, (1806,69,53,54) 76 + 151 -> 35 + 58, (512,64,128,64) 27 + 47 -> 18 + 38,
+// (948,88^3) 46 + 109 -> 41 + 84, (500,96^3) 26 + 61 -> 25 + 49, (16,64^3) 9.6 + 14.1 -> 8.1 + 10.3.  (2048,64^3) moves 302 MB:
+// 3.5 TB/s; what it spends beside memory is issue slots, some 700 of them a wave and direction on staging.
 #pragma once
 
 #include "common.h"
@@ -19,6 +34,10 @@
 namespace GENBMM_NS {
 
 constexpr float kItemGuardBits = 40.f;
+constexpr int kItemMax = 128;  // largest extent these kernels take
+// Of the backward's workgroup, at most; beyond, one 128 x 128 tile per item (two workgroups of three-part products: (500,100^3)
+// 29 + 70 us against 36 + 63 in one workgroup of 160 KB).
+constexpr int kItemLds = 136 * 1024;
 
 // log-sum-exp of a[m,:] + b[:,n] the way the reference's kernel does it
 // (matmul_cuda_kernel.cu:27-41): running maximum from -1e9, then the sum.
@@ -33,237 +52,360 @@ __device__ __forceinline__ float item_exact_out(const elem_t* __restrict__ arow,
   return logf(s) + mx;
 }
 
-// (row, column) of elements tid, tid + nt, tid + 2 nt, ... of a row-major array
-// with C columns, without a division per element.
-struct RowMajorWalk {
-  int r, c, dr, dc, C;
-  __device__ __forceinline__ RowMajorWalk(int tid, int nt, int cols) : C(cols) {
-    r = tid / C;
-    c = tid - r * C;
-    dr = nt / C;
-    dc = nt - dr * C;
-  }
-  __device__ __forceinline__ void next() {
-    r += dr;
-    c += dc;
-    if (c >= C) {
-      c -= C;
-      ++r;
-    }
-  }
-};
-
 // exp(x - shift), with the all -inf row / column (shift = -inf) giving zeros
 __device__ __forceinline__ float item_exp(float x, float shift) {
   return fast_exp2((x - (shift == -INFINITY ? 0.f : shift)) * kLog2e);
 }
 
-// TB x TB outputs per thread on a G x G thread grid.  Used with G = 16: TB = 2
-// covers items up to 32 x 32, TB = 4 up to 64 x 64.  (One wave per item, G = 8 and
-// TB = 4, measured slower at 8192 items of 32^3: the chain of dependent phases of
-// an item gets longer than the extra items in flight make up for.)
-// FULL: M = K = N = G * TB, known to the compiler - the index arithmetic that is most of
-// the general kernel's instructions (it is issue-bound, not memory-bound) folds away.
-template <int G, int TB, bool FULL = false>
-__global__ __launch_bounds__(G * G, TB == 2 ? 8 : 1) void k_log_item_fwd(const elem_t* __restrict__ a,
-                                                      const elem_t* __restrict__ b,
-                                                      elem_t* __restrict__ out,
-                                                      float* __restrict__ stats,
-                                                      int* __restrict__ hdr, int M_, int K_,
-                                                      int N_) {
-  constexpr int NT = G * G, S = G * TB, LD = S + 1;
-  const int M = FULL ? S : M_, K = FULL ? S : K_, N = FULL ? S : N_;
-  static_assert(2 * S <= NT, "row and column scans use 2*S threads");
-  if (hdr && blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = kWsNone;  // no per-tile flags in this workspace
-  __shared__ float At[S * LD];  // [k][m]: a, then EA; finally the output tile [m][n]
-  __shared__ float Bs[S * LD];  // [k][n]: b, then EB
-  __shared__ float al[S], be[S];
-  const int tid = threadIdx.x, batch = blockIdx.x;
-  const elem_t* ab = a + (long)batch * M * K;
-  const elem_t* bb = b + (long)batch * K * N;
-  // All reads of the item are issued before the first one is waited for (a thread owns
-  // elements tid, tid + NT, ... of each operand): one trip to memory, not one per element.
-  constexpr int PER = TB * TB;  // S * S / NT
-  float ra[PER], rb[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int e = tid + u * NT;
-    ra[u] = e < M * K ? ab[e] : 0.f;
-    rb[u] = e < K * N ? bb[e] : 0.f;
-  }
-  {
-    RowMajorWalk w(tid, NT, K);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if (w.r < M) At[w.c * LD + w.r] = ra[u];
-      w.next();
-    }
-  }
-  {
-    RowMajorWalk w(tid, NT, N);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if (w.r < K) Bs[w.r * LD + w.c] = rb[u];
-      w.next();
-    }
-  }
-  __syncthreads();
-  // row / column maxima: one thread per row, one per column (LDS atomics on the
-  // shared maximum while loading measured slower: 32 lanes on one address)
-  if (tid < M) {
-    float mx = -INFINITY;
-    for (int k = 0; k < K; ++k) mx = fmaxf(mx, At[k * LD + tid]);
-    al[tid] = mx;
-  } else if (tid >= S && tid - S < N) {
-    float mx = -INFINITY;
-    for (int k = 0; k < K; ++k) mx = fmaxf(mx, Bs[k * LD + tid - S]);
-    be[tid - S] = mx;
-  }
-  __syncthreads();
-  for (RowMajorWalk w(tid, NT, K); w.r < M; w.next()) {
-    const int m = w.r, k = w.c;
-    At[k * LD + m] = item_exp(At[k * LD + m], al[m]);
-  }
-  for (RowMajorWalk w(tid, NT, N); w.r < K; w.next()) {
-    const int k = w.r, n = w.c, e = w.r * N + w.c;
-    Bs[k * LD + n] = item_exp(Bs[k * LD + n], be[n]);
-  }
-  if (stats) {
-    float* st = stats + (long)batch * (M + N);
-    if (tid < M) st[tid] = al[tid];
-    else if (tid >= S && tid - S < N) st[M + tid - S] = be[tid - S];
-  }
-  __syncthreads();
+// The larger of two values that are no numbers of a computation yet (fmaxf would quiet each of them in an instruction
+// of its own first); of a NaN and a number the number.
+__device__ __forceinline__ float item_max(float x, float y) { return __builtin_amdgcn_fmed3f(x, y, INFINITY); }
 
-  const int ty = tid / G, tx = tid % G;
-  float acc[TB][TB];
+// Maxima over the wave of four registers, as scalars: two registers become one at each exchange between the halves
+// and quarters of the wave, then four rotations within a quarter serve all four (18 instructions; a reduction
+// of each takes 50).
+__device__ __forceinline__ void item_wave_max4(float (&v)[4], float (&m)[4]) {
+  auto u = [](float x) { return __float_as_uint(x); };
+  auto f = [](unsigned x) { return __uint_as_float(x); };
+  const auto p = __builtin_amdgcn_permlane32_swap(u(v[0]), u(v[1]), false, false);  // halves: of v0, of v1
+  const auto q = __builtin_amdgcn_permlane32_swap(u(v[2]), u(v[3]), false, false);
+  const float x = item_max(f(p[0]), f(p[1])), y = item_max(f(q[0]), f(q[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(u(x), u(y), false, false);  // quarters: of v0, v2, v1, v3
+  float z = item_max(f(r[0]), f(r[1]));
+  auto turn = [&](auto ctrl) __attribute__((always_inline)) {
+    z = item_max(z, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(z), decltype(ctrl)::value, 0xf, 0xf, true)));
+  };
+  turn(std::integral_constant<int, 0x128>{});  // row_ror:8
+  turn(std::integral_constant<int, 0x124>{});
+  turn(std::integral_constant<int, 0x122>{});
+  turn(std::integral_constant<int, 0x121>{});
+  const int at[4] = {0, 32, 16, 48};
 #pragma unroll
-  for (int i = 0; i < TB; ++i)
+  for (int t = 0; t < 4; ++t) m[t] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), at[t]));
+}
+
+// Of an R x C array, the rows 4 (wave + W u) + t and the columns lane + 64 h that a wave stages.  `raw` is as
+// loaded: always the same loads (rows and columns beyond the matrix read its last ones), none waited for
+// before it is used.  Rows beyond the matrix may stay its last one's copies: what they meet is zero.
+template <int W, int U, int H>
+struct ItemRows {
+  elem_t raw[U][4][H];
+  float v[U][4][H];
+  __device__ __forceinline__ void load(const elem_t* __restrict__ x, int R, int C, int wave, int lane) {
+    constexpr int kSize = sizeof(elem_t);
+    const buf_t src = buf_of(x, (unsigned)(R * C * kSize));
+    const int pitch = C * kSize, last = (R - 1) * pitch;
 #pragma unroll
-    for (int j = 0; j < TB; ++j) acc[i][j] = 0.f;
-#pragma unroll 4
-  for (int k = 0; k < K; ++k) {
-    float av[TB], bv[TB];
+    for (int h = 0; h < H; ++h) {
+      const int at = min(lane + 64 * h, C - 1) * kSize;
 #pragma unroll
-    for (int i = 0; i < TB; ++i) av[i] = At[k * LD + ty * TB + i];
+      for (int u = 0; u < U; ++u) {
+        const int first = 4 * (wave + W * u) * pitch;  // uniform
 #pragma unroll
-    for (int j = 0; j < TB; ++j) bv[j] = Bs[k * LD + tx * TB + j];
-#pragma unroll
-    for (int i = 0; i < TB; ++i)
-#pragma unroll
-      for (int j = 0; j < TB; ++j) acc[i][j] = __builtin_fmaf(av[i], bv[j], acc[i][j]);
-  }
-  __syncthreads();  // At becomes the output tile
-  const float thr = fast_exp2(-kItemGuardBits);
-#pragma unroll
-  for (int i = 0; i < TB; ++i)
-#pragma unroll
-    for (int j = 0; j < TB; ++j) {
-      const int m = ty * TB + i, n = tx * TB + j;
-      if (m < M && n < N) {
-        const float shift = al[m] + be[n], s = acc[i][j];
-        const bool ok = (s >= thr) && (s < INFINITY) && (shift >= kFloor) && (shift < INFINITY);
-        At[m * LD + n] = ok ? __builtin_fmaf(fast_log2(s), kLn2, shift)
-                            : item_exact_out(ab + (long)m * K, bb + n, K, N);
+        for (int t = 0; t < 4; ++t) raw[u][t][h] = buf_ld<elem_t>(src, at, min(first + t * pitch, last));
       }
     }
-  __syncthreads();
-  elem_t* ob = out + (long)batch * M * N;
-  for (RowMajorWalk w(tid, NT, N); w.r < M; w.next()) {
-    const int m = w.r, n = w.c, e = w.r * N + w.c;
-    ob[e] = to_elem<elem_t>(At[m * LD + n]);
+  }
+  // v: the loaded cells, -infinity in columns beyond the matrix
+  __device__ __forceinline__ void settle(int C, int lane) {
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[u][t][h] = lane + 64 * h < C ? (float)raw[u][t][h] : -INFINITY;
+  }
+  // f(u, first row, column chunk) for every group within Rp rows, in the lanes inside Cp columns
+  template <class F>
+  static __device__ __forceinline__ void each(int Rp, int Cp, int wave, int lane, F&& f) {
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      if (lane + 64 * h < Cp) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int r0 = 4 * (wave + W * u);
+          if (r0 < Rp) f(u, r0, h);  // uniform
+        }
+      }
+  }
+  __device__ __forceinline__ void put_rows(float* __restrict__ dst, int ld, int Rp, int Cp, int wave, int lane) const {
+    each(Rp, Cp, wave, lane, [&](int u, int r0, int h) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) dst[(r0 + t) * ld + lane + 64 * h] = v[u][t][h];
+    });
+  }
+  // transposed: [column][row]
+  __device__ __forceinline__ void put_cols(float* __restrict__ dst, int ld, int Rp, int Cp, int wave, int lane) const {
+    each(Rp, Cp, wave, lane, [&](int u, int r0, int h) __attribute__((always_inline)) {
+      *reinterpret_cast<float4*>(dst + (lane + 64 * h) * ld + r0) =
+          make_float4(v[u][0][h], v[u][1][h], v[u][2][h], v[u][3][h]);
+    });
+  }
+};
+
+// The maxima of a's rows (left in al[u][t], scalars) and a becomes exp(a - alpha).
+template <int W, int U, int H>
+__device__ __forceinline__ void item_rows_exp(ItemRows<W, U, H>& x, float (&al)[U][4]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float m[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      m[t] = x.v[u][t][0];
+#pragma unroll
+      for (int h = 1; h < H; ++h) m[t] = item_max(m[t], x.v[u][t][h]);
+    }
+    item_wave_max4(m, al[u]);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float sh = al[u][t] == -INFINITY ? 0.f : al[u][t];
+#pragma unroll
+      for (int h = 0; h < H; ++h) x.v[u][t][h] = fast_exp2((x.v[u][t][h] - sh) * kLog2e);
+    }
+  }
+}
+// A wave's part of the maxima of b's columns into part[wave][64 H]; after a barrier item_cols_join has them.
+template <int W, int U, int H>
+__device__ __forceinline__ void item_cols_part(const ItemRows<W, U, H>& x, float* __restrict__ part, int wave, int lane) {
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    float m = x.v[0][0][h];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) m = item_max(m, x.v[u][t][h]);
+    part[(wave * H + h) * 64 + lane] = m;
+  }
+}
+template <int W, int H>
+__device__ __forceinline__ void item_cols_join(const float* __restrict__ part, int lane, float (&be)[H]) {
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    be[h] = part[h * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < W; ++w) be[h] = item_max(be[h], part[(w * H + h) * 64 + lane]);
+  }
+}
+template <int W, int U, int H>
+__device__ __forceinline__ void item_cols_exp(ItemRows<W, U, H>& x, const float (&be)[H]) {
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const float sh = be[h] == -INFINITY ? 0.f : be[h];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x.v[u][t][h] = fast_exp2((x.v[u][t][h] - sh) * kLog2e);
   }
 }
 
-template <int G, int TB, bool FULL = false>
-__global__ __launch_bounds__(G * G, TB == 2 ? 6 : 1) void k_log_item_bwd(const elem_t* __restrict__ a,
-                                                      const elem_t* __restrict__ b,
-                                                      const elem_t* __restrict__ outp,
-                                                      const elem_t* __restrict__ g,
-                                                      elem_t* __restrict__ grad_a,
-                                                      elem_t* __restrict__ grad_b, int M_, int K_,
-                                                      int N_) {
-  constexpr int NT = G * G, S = G * TB, LD = S + 1;
-  const int M = FULL ? S : M_, K = FULL ? S : K_, N = FULL ? S : N_;
-  static_assert(2 * S <= NT, "row and column scans use 2*S threads");
-  __shared__ float Ea[S * LD];  // [m][k]: a, EA, finally grad_a
-  __shared__ float Eb[S * LD];  // [k][n]: b, EB, finally grad_b
-  __shared__ float Hs[S * LD];  // [m][n]: H
-  __shared__ float al[S], be[S];
-  const int tid = threadIdx.x, batch = blockIdx.x;
+typedef float item_f4 __attribute__((ext_vector_type(4)));
+// Four steps of a line: neighbours in LDS, or ld words apart.
+__device__ __forceinline__ item_f4 item_frag(const float* p) { return *reinterpret_cast<const item_f4*>(p); }
+__device__ __forceinline__ item_f4 item_frag(const float* p, int ld) {
+  item_f4 r;
+  r[0] = p[0]; r[1] = p[ld]; r[2] = p[2 * ld]; r[3] = p[3 * ld];
+  return r;
+}
+// A 16 x 16 tile over `chunks` times 16 steps: result element r of lane (l15, q) is line 4 q + r of x,
+// line l15 of y.  x(c), y(c): the lane's four steps 16 c + 4 q ... of its line l15 of either operand.
+// (Which four steps an instruction sums is free as long as both operands agree.)
+template <class X, class Y>
+__device__ __forceinline__ item_f4 item_tile(int chunks, X&& x, Y&& y) {
+  item_f4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
+  item_f4 xv = x(0), yv = y(0);
+  for (int c = 1; c <= chunks; ++c) {
+    const int nx = c < chunks ? c : c - 1;
+    const item_f4 xn = x(nx), yn = y(nx);
+    c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[0], yv[0], c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[1], yv[1], c1, 0, 0, 0);
+    c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[2], yv[2], c0, 0, 0, 0);
+    c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[3], yv[3], c1, 0, 0, 0);
+    xv = xn; yv = yn;
+  }
+  return c0 + c1;
+}
+
+// Tile `at`, at + step, ... of a list of rows of C tiles.
+struct ItemTiles {
+  int r, c, C;
+  __device__ __forceinline__ ItemTiles(int at, int C_) : r(0), c(at), C(C_) { wrap(); }
+  __device__ __forceinline__ void wrap() {
+    while (c >= C) {
+      c -= C;
+      ++r;
+    }
+  }
+  __device__ __forceinline__ void next(int step) {
+    c += step;
+    wrap();
+  }
+};
+
+// The padded extents and LDS (floats) of an item.
+struct ItemPad {
+  int M, K, N;
+};
+__host__ __device__ inline ItemPad item_pad(int M, int K, int N) {
+  return ItemPad{(M + 15) & ~15, (K + 15) & ~15, (N + 15) & ~15};
+}
+__host__ __device__ inline int item_bwd_arrays(int M, int K, int N) {
+  const ItemPad p = item_pad(M, K, N);
+  return p.K * (p.M + 4) + p.K * (p.N + 4) + p.M * (p.N + 4);
+}
+inline int item_fwd_floats(int M, int K, int N, int W, int H) {
+  const ItemPad p = item_pad(M, K, N);
+  return (p.M + p.N) * (p.K + 4) + W * H * 64 + p.M + p.N;
+}
+inline int item_bwd_floats(int M, int K, int N, int W, int H) {
+  return item_bwd_arrays(M, K, N) + W * H * 64;
+}
+
+// W waves; U groups of four rows per wave (4 W U >= every extent), H column chunks of 64.
+template <int W, int U, int H>
+__global__ __launch_bounds__(64 * W) void k_log_item_fwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+                                                         elem_t* __restrict__ out, float* __restrict__ stats,
+                                                         int* __restrict__ hdr, int M, int K, int N) {
+  extern __shared__ __attribute__((aligned(16))) float item_smem[];
+  const ItemPad pad = item_pad(M, K, N);
+  const int ldk = pad.K + 4;
+  float* const Ea = item_smem;             // [m][k]
+  float* const Eb = Ea + pad.M * ldk;      // [n][k]
+  float* const part = Eb + pad.N * ldk;    // [wave][column]
+  float* const s_al = part + W * H * 64;
+  float* const s_be = s_al + pad.M;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int batch = blockIdx.x;
+  if (hdr && batch == 0 && tid == 0) hdr[0] = kWsNone;  // no per-tile flags in this workspace
+  const elem_t* ab = a + (long)batch * M * K;
+  const elem_t* bb = b + (long)batch * K * N;
+  ItemRows<W, U, H> xa, xb;
+  xa.load(ab, M, K, wave, lane);
+  xb.load(bb, K, N, wave, lane);
+
+  float al[U][4], be[H];
+  xa.settle(K, lane);
+  item_rows_exp(xa, al);
+  xa.put_rows(Ea, ldk, pad.M, pad.K, wave, lane);
+  xb.settle(N, lane);
+  item_cols_part(xb, part, wave, lane);
+  float* st = stats ? stats + (long)batch * (M + N) : nullptr;
+  if (lane == 0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int m = 4 * (wave + W * u) + t;
+        if (m < pad.M) s_al[m] = al[u][t];
+        if (st && m < M) st[m] = al[u][t];
+      }
+  }
+  __syncthreads();
+  item_cols_join<W, H>(part, lane, be);
+  item_cols_exp(xb, be);
+  xb.put_cols(Eb, ldk, pad.K, pad.N, wave, lane);
+  if (wave == 0) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int n = lane + 64 * h;
+      if (n < pad.N) s_be[n] = be[h];
+      if (st && n < N) st[M + n] = be[h];
+    }
+  }
+  __syncthreads();
+
+  const int l15 = lane & 15, q4 = 4 * (lane >> 4);
+  const int tm = pad.M >> 4, tn = pad.N >> 4, chunks = pad.K >> 4;
+  const float thr = fast_exp2(-kItemGuardBits);
+  elem_t* ob = out + (long)batch * M * N;
+  ItemTiles w(wave, tn);
+  for (; w.r < tm; w.next(W)) {  // uniform
+    const int m0 = w.r * 16, n0 = w.c * 16;
+    const float* xl = Eb + (n0 + l15) * ldk + q4;
+    const float* yl = Ea + (m0 + l15) * ldk + q4;
+    const item_f4 s = item_tile(chunks, [&](int c) { return item_frag(xl + 16 * c); },
+                                [&](int c) { return item_frag(yl + 16 * c); });
+    const int m = m0 + l15, n = n0 + q4;
+    const float am = s_al[m];
+    const item_f4 bn = item_frag(s_be + n);
+    float o[4];
+    int redo = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float shift = am + bn[r];
+      const bool ok = (s[r] >= thr) && (s[r] < INFINITY) && (shift >= kFloor) && (shift < INFINITY);
+      if (!ok && m < M && n + r < N) redo |= 1 << r;
+      o[r] = __builtin_fmaf(fast_log2(s[r]), kLn2, shift);
+    }
+    if (__builtin_amdgcn_ballot_w64(redo != 0) != 0) {  // rare
+#pragma unroll 1
+      for (int r = 0; r < 4; ++r)
+        if (redo >> r & 1) {
+          const float e = item_exact_out(ab + (long)m * K, bb + n + r, K, N);
+          o[0] = r == 0 ? e : o[0]; o[1] = r == 1 ? e : o[1]; o[2] = r == 2 ? e : o[2]; o[3] = r == 3 ? e : o[3];
+        }
+    }
+    if (m < M) st4m(ob + m * N + n, N - n, make_float4(o[0], o[1], o[2], o[3]));
+  }
+}
+
+template <int W, int U, int H>
+__global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+                                                         const elem_t* __restrict__ outp, const elem_t* __restrict__ g,
+                                                         elem_t* __restrict__ grad_a, elem_t* __restrict__ grad_b,
+                                                         int M, int K, int N) {
+  extern __shared__ __attribute__((aligned(16))) float item_smem[];
+  const ItemPad pad = item_pad(M, K, N);
+  const int ldm = pad.M + 4, ldn = pad.N + 4;
+  float* const EaT = item_smem;           // [k][m]
+  float* const Eb = EaT + pad.K * ldm;    // [k][n]
+  float* const Hs = Eb + pad.K * ldn;     // [m][n]
+  float* const part = Hs + pad.M * ldn;   // [wave][column]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int batch = blockIdx.x;
   const elem_t* ab = a + (long)batch * M * K;
   const elem_t* bb = b + (long)batch * K * N;
   const elem_t* ob = outp + (long)batch * M * N;
   const elem_t* gb = g + (long)batch * M * N;
   elem_t* gab = grad_a ? grad_a + (long)batch * M * K : nullptr;
   elem_t* gbb = grad_b ? grad_b + (long)batch * K * N : nullptr;
-  // all reads of the item in flight together (see the forward)
-  constexpr int PER = TB * TB;
-  float ra[PER], rb[PER], ro[PER], rg[PER];
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int e = tid + u * NT;
-    ra[u] = e < M * K ? ab[e] : 0.f;
-    rb[u] = e < K * N ? bb[e] : 0.f;
-    ro[u] = e < M * N ? ob[e] : 0.f;
-    rg[u] = e < M * N ? gb[e] : 0.f;
-  }
-  {
-    RowMajorWalk w(tid, NT, K);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if (w.r < M) Ea[w.r * LD + w.c] = ra[u];
-      w.next();
-    }
-  }
-  {
-    RowMajorWalk w(tid, NT, N);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if (w.r < K) Eb[w.r * LD + w.c] = rb[u];
-      w.next();
-    }
-  }
+  ItemRows<W, U, H> xa, xb, xo, xg;
+  xb.load(bb, K, N, wave, lane);
+  xa.load(ab, M, K, wave, lane);
+  xo.load(ob, M, N, wave, lane);
+  xg.load(gb, M, N, wave, lane);
+
+  float al[U][4], be[H];
+  xb.settle(N, lane);
+  item_cols_part(xb, part, wave, lane);
+  xa.settle(K, lane);
+  item_rows_exp(xa, al);
+  xa.put_cols(EaT, ldm, pad.M, pad.K, wave, lane);
   __syncthreads();
-  if (tid < M) {
-    float mx = -INFINITY;
-    for (int k = 0; k < K; ++k) mx = fmaxf(mx, Ea[tid * LD + k]);
-    al[tid] = mx;
-  } else if (tid >= S && tid - S < N) {
-    float mx = -INFINITY;
-    for (int k = 0; k < K; ++k) mx = fmaxf(mx, Eb[k * LD + tid - S]);
-    be[tid - S] = mx;
-  }
-  __syncthreads();
+  item_cols_join<W, H>(part, lane, be);
+  item_cols_exp(xb, be);
+  xb.put_rows(Eb, ldn, pad.K, pad.N, wave, lane);
+  // H, and whether the factoring is exact for this item: S < 2^-40, NaN or infinities anywhere are not
   const float lim = kItemGuardBits * kLn2 + 1e-3f;
-  int bad = 0;
-  for (RowMajorWalk w(tid, NT, K); w.r < M; w.next()) {
-    const int m = w.r, k = w.c, e = w.r * K + w.c;
-    Ea[m * LD + k] = item_exp(Ea[m * LD + k], al[m]);
-  }
-  for (RowMajorWalk w(tid, NT, N); w.r < K; w.next()) {
-    const int k = w.r, n = w.c, e = w.r * N + w.c;
-    Eb[k * LD + n] = item_exp(Eb[k * LD + n], be[n]);
-  }
-  {
-    RowMajorWalk w(tid, NT, N);
+  float most = 0.f, worst = 0.f;  // worst stays 0 while every exponent is finite
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      if (w.r < M) {
-        const int m = w.r, n = w.c;
-        const float ex = al[m] + be[n] - ro[u];
-        if (!(ex <= lim) || !(ex > -INFINITY)) bad = 1;  // S < 2^-40, NaN or infinities: not exact
-        Hs[m * LD + n] = rg[u] * fast_exp2(ex * kLog2e);
+  for (int h = 0; h < H; ++h)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bool in = 4 * (wave + W * u) + t < M && lane + 64 * h < N;
+        const float ex = in ? al[u][t] + be[h] - (float)xo.raw[u][t][h] : 0.f;
+        most = fmaxf(most, ex);
+        worst = __builtin_fmaf(ex, 0.f, worst);
+        xg.v[u][t][h] = (in ? (float)xg.raw[u][t][h] : 0.f) * fast_exp2(ex * kLog2e);
       }
-      w.next();
-    }
-  }
-  bad = __syncthreads_or(bad);
-  if (bad) {
+  const int bad = !(most <= lim) || !(worst == 0.f);
+  xg.put_rows(Hs, ldn, pad.M, pad.N, wave, lane);
+  if (__syncthreads_or(bad)) {
     // the reference's form for the whole item (matmul_cuda_kernel.cu:159-184):
     // exp(a + b - out) * g summed over n (grad_a) / m (grad_b), from global memory
     if (gab)
-      for (int e = tid; e < M * K; e += NT) {
+      for (int e = tid; e < M * K; e += 64 * W) {
         const int m = e / K, k = e - m * K;
         const float av = ab[e];
         float s = 0.f;
@@ -272,7 +414,7 @@ __global__ __launch_bounds__(G * G, TB == 2 ? 6 : 1) void k_log_item_bwd(const e
         gab[e] = to_elem<elem_t>(s);
       }
     if (gbb)
-      for (int e = tid; e < K * N; e += NT) {
+      for (int e = tid; e < K * N; e += 64 * W) {
         const int k = e / N, n = e - k * N;
         const float bv = bb[e];
         float s = 0.f;
@@ -283,54 +425,37 @@ __global__ __launch_bounds__(G * G, TB == 2 ? 6 : 1) void k_log_item_bwd(const e
     return;
   }
 
-  const int ty = tid / G, tx = tid % G;
-  float ga[TB][TB], gw[TB][TB];
-#pragma unroll
-  for (int i = 0; i < TB; ++i)
-#pragma unroll
-    for (int j = 0; j < TB; ++j) ga[i][j] = gw[i][j] = 0.f;
-  if (gab) {  // rows m = ty*TB+i, columns k = tx*TB+j, sum over n
-#pragma unroll 4
-    for (int n = 0; n < N; ++n) {
-      float hv[TB], ev[TB];
-#pragma unroll
-      for (int i = 0; i < TB; ++i) hv[i] = Hs[(ty * TB + i) * LD + n];
-#pragma unroll
-      for (int j = 0; j < TB; ++j) ev[j] = Eb[(tx * TB + j) * LD + n];
-#pragma unroll
-      for (int i = 0; i < TB; ++i)
-#pragma unroll
-        for (int j = 0; j < TB; ++j) ga[i][j] = __builtin_fmaf(hv[i], ev[j], ga[i][j]);
+  const int l15 = lane & 15, q4 = 4 * (lane >> 4);
+  const int tk = pad.K >> 4, tn = pad.N >> 4, tm = pad.M >> 4;
+  // grad_a's tiles, then grad_b's: a wave that is done with the former goes on in the latter's list
+  ItemTiles w(wave, tk);
+  if (gab) {
+    for (; w.r < tm; w.next(W)) {  // uniform; four k of a row m: sum over n
+      const int m0 = w.r * 16, k0 = w.c * 16;
+      const float* xl = Eb + (k0 + l15) * ldn + q4;
+      const float* yl = Hs + (m0 + l15) * ldn + q4;
+      const item_f4 s = item_tile(tn, [&](int c) { return item_frag(xl + 16 * c); },
+                                  [&](int c) { return item_frag(yl + 16 * c); });
+      const int m = m0 + l15, k = k0 + q4;
+      const item_f4 e = item_frag(EaT + k * ldm + m, ldm);
+      if (m < M) st4m(gab + m * K + k, K - k, make_float4(e[0] * s[0], e[1] * s[1], e[2] * s[2], e[3] * s[3]));
+    }
+    w = ItemTiles((w.r - tm) * tk + w.c, tn);
+  } else {
+    w = ItemTiles(wave, tn);
+  }
+  if (gbb) {
+    for (; w.r < tk; w.next(W)) {  // uniform; four n of a row k: sum over m
+      const int k0 = w.r * 16, n0 = w.c * 16;
+      const float* xl = Hs + q4 * ldn + n0 + l15;
+      const float* yl = EaT + (k0 + l15) * ldm + q4;
+      const item_f4 s = item_tile(tm, [&](int c) { return item_frag(xl + 16 * c * ldn, ldn); },
+                                  [&](int c) { return item_frag(yl + 16 * c); });
+      const int k = k0 + l15, n = n0 + q4;
+      const item_f4 e = item_frag(Eb + k * ldn + n);
+      if (k < K) st4m(gbb + k * N + n, N - n, make_float4(e[0] * s[0], e[1] * s[1], e[2] * s[2], e[3] * s[3]));
     }
   }
-  if (gbb) {  // rows k = ty*TB+i, columns n = tx*TB+j, sum over m
-#pragma unroll 4
-    for (int m = 0; m < M; ++m) {
-      float ev[TB], hv[TB];
-#pragma unroll
-      for (int i = 0; i < TB; ++i) ev[i] = Ea[m * LD + ty * TB + i];
-#pragma unroll
-      for (int j = 0; j < TB; ++j) hv[j] = Hs[m * LD + tx * TB + j];
-#pragma unroll
-      for (int i = 0; i < TB; ++i)
-#pragma unroll
-        for (int j = 0; j < TB; ++j) gw[i][j] = __builtin_fmaf(ev[i], hv[j], gw[i][j]);
-    }
-  }
-  __syncthreads();  // all sums taken: scale in place, each thread its own cells
-#pragma unroll
-  for (int i = 0; i < TB; ++i)
-#pragma unroll
-    for (int j = 0; j < TB; ++j) {
-      const int r = ty * TB + i, c = tx * TB + j;
-      Ea[r * LD + c] *= ga[i][j];
-      Eb[r * LD + c] *= gw[i][j];
-    }
-  __syncthreads();
-  if (gab)
-    for (RowMajorWalk w(tid, NT, K); w.r < M; w.next()) gab[w.r * K + w.c] = to_elem<elem_t>(Ea[w.r * LD + w.c]);
-  if (gbb)
-    for (RowMajorWalk w(tid, NT, N); w.r < K; w.next()) gbb[w.r * N + w.c] = to_elem<elem_t>(Eb[w.r * LD + w.c]);
 }
 
 }  // namespace GENBMM_NS

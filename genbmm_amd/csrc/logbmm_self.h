@@ -1,5 +1,5 @@
-// logbmm for batch items whose three extents are all at most 128: the whole
-// item is one 128 x 128 tile, so a workgroup can do everything the larger
+// logbmm for batch items whose three extents are all at most 128 (and too large for
+// logbmm_item.h): the whole item is one 128 x 128 tile, so a workgroup can do everything the larger
 // problems need separate launches and a large workspace for.
 //
 // Forward (one workgroup of four waves per item): every thread requests its

@@ -124,10 +124,13 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
 /*
  * The same two functions with the kernel family named per call (tests and
  * measurements; the plain functions are GENBMM_PATH_AUTO).
- *   GENBMM_PATH_AUTO   whole-item kernels for matrices up to 64^3, the matrix
- *                      cores where the shape allows (every extent at least
- *                      96, or items of one 128 x 128 tile), else the factored
- *                      kernels on the vector ALU;
+ *   GENBMM_PATH_AUTO   an item per workgroup for small matrices (no extent
+ *                      above 128, the item's LDS below 136 KB: 96^3, or
+ *                      128 x 100 x 64), one 128 x 128 tile per item up to
+ *                      128^3, larger problems in tiles of 128 and more, all
+ *                      on the matrix cores; extents of 32 or less beside
+ *                      larger ones, and many narrow results whose tiles would
+ *                      be mostly padding, on the factored vector-ALU kernels;
  *   GENBMM_PATH_EXACT  the online / exp-per-term kernels only (what a NULL
  *                      `stats` gives; a non-NULL one still receives the maxima);
  *   GENBMM_PATH_VALU   the factored kernels contracting with v_fma_f32 on the
@@ -157,8 +160,9 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *                      float16 / bfloat16 tensors want, whose `out` is stored
  *                      rounded (4 bytes per result cell).  Items too large for
  *                      the bf16 instruction's backward keep all three factors
- *                      and take FACTORS's; problems with an extent below 96 or
- *                      none above 128 keep nothing and weigh by exp(max - out).
+ *                      and take FACTORS's; items of one workgroup and gradients
+ *                      on the vector ALU keep nothing and weigh by
+ *                      exp(max - out).
  *                      One gradient alone (the other pointer NULL) is formed
  *                      from `out`.
  * Any other value: GENBMM_E_MODE.  Forward and backward of one problem need not

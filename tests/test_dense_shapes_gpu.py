@@ -148,3 +148,66 @@ def test_sample_on_flat_and_peaked_distributions(gpu, scale, shape):
     # a sampled term always has mass (never a masked one)
     picked = torch.gather(a.unsqueeze(-1) + b.unsqueeze(-3), 2, got.unsqueeze(2)).squeeze(2)
     assert bool((picked[live] > -1e8).all())
+
+# Edges of the whole-item log kernels (tiles of 16, groups of four rows per wave, 64 columns per chunk, the sizes at
+# which another instantiation takes over, the largest items) and of the 128-wide tiles on narrower extents behind them.
+_LOG_EDGES = [(3, 1, 1, 1), (3, 15, 16, 17), (2, 17, 33, 31), (2, 32, 33, 48), (2, 49, 48, 47), (2, 64, 63, 64), (2, 65, 64, 1),
+              (2, 16, 65, 64), (1, 95, 96, 97), (2, 97, 16, 95), (1, 128, 100, 64), (1, 5, 128, 127), (1, 128, 1, 128),
+              (1, 100, 80, 100), (1, 96, 97, 96), (1, 104, 100, 97), (2, 33, 130, 35), (2, 130, 33, 40), (600, 33, 129, 64),
+              (2, 70, 200, 90), (1, 40, 512, 33)]
+
+
+@pytest.mark.parametrize("B,M,K,N", _LOG_EDGES)
+def test_log_products_at_the_edges_of_their_kernels(gpu, B, M, K, N):
+    """Against float64 (a few roundings of values around 10: 1e-5), and the half types against the float kernels
+    on the same widened values, rounded once."""
+    torch.manual_seed(M + K + N)
+    a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
+    want = oracle.logbmm_grads64(a, b, g)
+    ad, bd = a.to(gpu).requires_grad_(True), b.to(gpu).requires_grad_(True)
+    out = genbmm.logbmm(ad, bd)
+    for got, ref in zip((out.detach(),) + torch.autograd.grad(out, (ad, bd), g.to(gpu)), want):
+        assert torch.allclose(got.cpu().double(), ref, rtol=1e-5, atol=1e-5), (B, M, K, N)
+    lib = _lib.load()
+    for dt, sfx in ((torch.float16, "_f16"), (torch.bfloat16, "_bf16")):
+        half = [x.to(gpu, dt) for x in (a, b, g)]
+        wide = [x.float() for x in half]
+        res = []
+        for sfx_, (x, y, gg) in ((sfx, half), ("", wide)):
+            o, gx, gy = torch.empty_like(gg), torch.empty_like(x), torch.empty_like(y)
+            ws = torch.empty(lib.genbmm_logbmm_stats_size(B, M, K, N), device=gpu)
+            assert getattr(lib, "genbmm_logbmm_fwd" + sfx_)(*map(_lib.ptr, (x, y, o, ws)), B, M, K, N, _lib.stream_of(x)) == 0
+            if sfx_ == "":
+                o_float, o = o, res[0].float()      # the half backward reads `out` as stored
+            assert getattr(lib, "genbmm_logbmm_bwd" + sfx_)(*map(_lib.ptr, (x, y, o, gg, ws, gx, gy)), B, M, K, N,
+                                                            _lib.stream_of(x)) == 0
+            if sfx_ == "":
+                assert torch.equal(res[0], o_float.to(dt)), (dt, B, M, K, N)
+                assert torch.equal(res[1], gx.to(dt)) and torch.equal(res[2], gy.to(dt)), (dt, B, M, K, N)
+            res += [o, gx, gy]
+
+
+@pytest.mark.parametrize("B,M,K,N", [(3, 17, 20, 33), (2, 65, 70, 50), (2, 100, 100, 60), (2, 120, 128, 40)])
+def test_log_items_that_cannot_be_factored(gpu, B, M, K, N):
+    """Rows 200 apart, a masked row and a masked column (-inf), a row at the floor: cells (forward) and items (backward)
+    that the factored form does not carry.  The other items keep their bits."""
+    torch.manual_seed(7)
+    a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
+    clean = [x.to(gpu) for x in (a, b, g)]
+    a[0, 3, : K // 2] -= 200
+    b[0, K // 2 :] -= 200
+    a[0, 5], b[0, :, 7], a[0, 6] = -float("inf"), -float("inf"), -1e9
+    g[0, 5], g[0, :, 7], g[0, 6] = 0, 0, 0
+    outs = []
+    for x, y, z in (clean, [t.to(gpu) for t in (a, b, g)]):
+        x, y = x.requires_grad_(True), y.requires_grad_(True)
+        o = genbmm.logbmm(x, y)
+        outs.append((o.detach(),) + torch.autograd.grad(o, (x, y), z))
+    for u, v in zip(*outs):
+        assert torch.equal(u[1:], v[1:])
+    want = torch.logsumexp(a[0].double().unsqueeze(2) + b[0].double().unsqueeze(0), 1)
+    got = outs[1][0][0].cpu().double()
+    live = torch.ones(M, N, dtype=torch.bool)
+    live[5], live[6], live[:, 7] = False, False, False
+    assert torch.allclose(got[live], want[live], rtol=1e-5, atol=1e-5)
+    assert bool((got[5] == -float("inf")).all()) and bool((got[:, 7][live[:, 0]] == -float("inf")).all())
