@@ -23,6 +23,7 @@
 #include "banded_argmax.h"
 #include "banded_block.h"
 #include "banded_direct.h"
+#include "banded_grads.h"
 #include "banded_flat.h"
 #include "banded_max.h"
 #include "banded_sample.h"
@@ -175,6 +176,23 @@ inline void launch_dir(const BandArgs& p, int B, hipStream_t s) {
   };
   if (plan.steps <= kDirStepsSmall) go(k_band_dir<KIND, PREP, DirPlanSmall>, dir_plan_small(plan));
   else go(k_band_dir<KIND, PREP, DirPlan>, plan);
+}
+
+// Both gradients on 32 x 32 blocks (banded_grads.h).
+inline bool blk_grads_ok(const BandArgs& p, int B) {
+  GradSide ga, gb;
+  return grad_plan(ga, gb, p, B) && grad_pays(ga, gb, p, B);
+}
+template <bool PREP>
+inline void launch_blk_grads(const BandArgs& p, int B, hipStream_t s) {
+  GradSide ga, gb;
+  grad_plan(ga, gb, p, B);
+  const int waves = max(grad_waves(ga), grad_waves(gb)), na = B * ga.chunks, nb = B * gb.chunks;
+  const int lds = (int)max(grad_lds_bytes(ga), grad_lds_bytes(gb));
+  auto kern = k_band_blk_grads<PREP>;
+  if (lds > (int)kStripLdsLimit)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(na + nb)), dim3((unsigned)(64 * waves)), lds, s, p, ga, gb, na, nb);
 }
 
 // grad_a and grad_b in one launch where both plans travel in the small form, else one launch each.
@@ -368,11 +386,14 @@ static int banded_bwd(const elem_t* a, int a_lu, int a_ld, const elem_t* b, int 
   if (ta == 0) return GENBMM_OK;
   hipStream_t s = (hipStream_t)stream;
   if (mode != GENBMM_BAND_MAX && (mode == GENBMM_BAND_MUL || (workspace && workspace_used(p))) && dir_bwd_ok(p)) {
+    const bool blk = blk_grads_ok(p, B);
     if (mode == GENBMM_BAND_MUL) {
-      launch_dir_grads<false>(p, B, s);
+      if (blk) launch_blk_grads<false>(p, B, s);
+      else launch_dir_grads<false>(p, B, s);
     } else {  // H = g / S is formed by both kernels as they read g: the workspace is only read
       set_workspace(p, workspace, B);
-      launch_dir_grads<true>(p, B, s);
+      if (blk) launch_blk_grads<true>(p, B, s);
+      else launch_dir_grads<true>(p, B, s);
     }
     return launch_status();
   }

@@ -154,6 +154,12 @@ __device__ __forceinline__ E buf_ld(buf_t x, int at, int base) {
   if constexpr (sizeof(E) == 4) return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(x, at, base, 0));
   else return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b16(x, at, base, 0));
 }
+// (writes beyond the end are dropped)
+template <class E>
+__device__ __forceinline__ void buf_st(buf_t x, int at, E v) {
+  if constexpr (sizeof(E) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), x, at, 0, 0);
+  else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), x, at, 0, 0);
+}
 __device__ __forceinline__ int clamp4(int x) { return min(max(x, 0), 4); }
 
 // ---------------------------------------------------------------- tile loaders
