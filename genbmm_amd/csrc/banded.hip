@@ -109,17 +109,23 @@ inline void launch_max_fwd(const BandArgs& p, int B, hipStream_t s) {
   const MaxDims d = max_dims(p.Wa, p.Wb, Wseg);
   const int strips = ceil_div(p.n, kMaxRows);
   const long rows = (long)B * p.n;
-  auto go = [&](auto kernel) {
+  const bool wide = d.bytes > 40 * 1024 || (long)B * strips * nseg <= 512;  // eight waves (k_band_max_fwd)
+  auto go = [&](auto kernel, int waves) {
     if (d.bytes > kStripLdsLimit)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)d.bytes);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((long)B * strips * nseg)), dim3(256), d.bytes, s, p, strips, d,
-                       rows * p.Wa, rows * p.Wb, nseg, Wseg);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((long)B * strips * nseg)), dim3((unsigned)(64 * waves)), d.bytes, s, p,
+                       strips, d, rows * p.Wa, rows * p.Wb, nseg, Wseg);
   };
   // The pairs' end costs a cell about eleven instructions: 33 diagonals each (64 x 4096) 87.4 -> 83-85.5 us in
   // pairs, 17 diagonals each 45.1 -> 46.0
-  if (min(p.Wa, p.Wb) >= 24) go(k_band_max_fwd<true>);
-  else go(k_band_max_fwd<false>);
+  if (min(p.Wa, p.Wb) >= 24) {
+    if (wide) go(k_band_max_fwd<true, 8>, 8);
+    else go(k_band_max_fwd<true, 4>, 4);
+  } else {
+    if (wide) go(k_band_max_fwd<false, 8>, 8);
+    else go(k_band_max_fwd<false, 4>, 4);
+  }
 }
 
 inline void launch_prep(const BandArgs& p, const elem_t* a, int a_lu, const elem_t* b, int b_lu, int B,

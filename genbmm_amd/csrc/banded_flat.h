@@ -16,9 +16,9 @@ typedef float mm_f4 __attribute__((ext_vector_type(4)));
 // elements (16 bytes of floats, 8 of a half type) from the aligned address below and laid
 // down as floats with row stride `pitch`: tensor[first + r * W + k] lands at
 // L[origin() + r * pitch + k].
-// load() only issues the reads of one batch of 256 * U pieces, store() consumes them.
+// load() only issues the reads of one batch of NT * U pieces (NT: threads), store() consumes them.
 // E: float (a workspace) or the element type of the caller's tensors (widened by the load).
-template <int U, class E = float>
+template <int U, class E = float, int NT = 256>
 struct MmFlat {
   mm_f4 v[U];
   int nvec, lead, W, gap;
@@ -39,12 +39,12 @@ struct MmFlat {
     inside = abeg >= tensor && abeg + 4 * (long)nvec <= tensor_end;
   }
   __device__ __forceinline__ int origin() const { return lead + gap; }
-  __device__ __forceinline__ bool more(int batch) const { return batch * 256 * U < nvec; }
+  __device__ __forceinline__ bool more(int batch) const { return batch * NT * U < nvec; }
   __device__ __forceinline__ void load(const E* lo, const E* hi, int batch, int tid) {
     if (inside) {  // uniform
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int vi = tid + 256 * (u + batch * U);
+        const int vi = tid + NT * (u + batch * U);
         v[u] = mm_f4{0.f, 0.f, 0.f, 0.f};
         if (vi < nvec) {
           const float4 x = ld4a(abeg + 4 * vi);
@@ -55,7 +55,7 @@ struct MmFlat {
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int vi = tid + 256 * (u + batch * U);
+      const int vi = tid + NT * (u + batch * U);
       mm_f4 x = mm_f4{0.f, 0.f, 0.f, 0.f};
       if (vi < nvec) {
         const E* q = abeg + 4 * vi;
@@ -73,7 +73,7 @@ struct MmFlat {
     bool bad = false;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int vi = tid + 256 * (u + batch * U);
+      const int vi = tid + NT * (u + batch * U);
       if (vi < nvec) {
         const mm_f4 x = v[u];
         bad |= !(fabsf(x[0]) <= FLT_MAX) || !(fabsf(x[1]) <= FLT_MAX) || !(fabsf(x[2]) <= FLT_MAX) ||

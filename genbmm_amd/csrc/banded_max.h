@@ -5,13 +5,13 @@
 // A workgroup owns 64 rows i.  Their rows of a and the 64 + Wo - 1 rows of b that they
 // meet are copied to LDS once, as they lie in memory (16-byte pieces, odd row strides: the
 // 64 lanes of a wave are 64 consecutive rows and fall in different banks).  A lane owns
-// one row; a wave walks blocks of 8 adjacent result diagonals j (blocks w, w + 4, ...
-// - their sum lengths pair up, so the four waves get equal work), reading one value of
+// one row; a wave walks blocks of 8 adjacent result diagonals j (blocks w, w + WAVES, ...
+// - their sum lengths pair up, so the waves get equal work), reading one value of
 // its own row per k and 8 values of b on an anti-diagonal.  The 8 cells walk the union of
 // their k ranges without predicates: the rows of b lie at least 7 cells apart in LDS, with
-// -inf between them.  Strips that touch the matrix edge take a loop with the per-cell k
-// range of the reference instead.  Values and indices go
-// through LDS so that the strip's rows are written as one contiguous run.
+// -inf between them, and a strip at the matrix's edge has -inf in the cells of a and the rows
+// of b that lie outside it.  Values and indices go through LDS so that the strip's rows are
+// written as one contiguous run.
 //
 // Compared with the chunked strip kernel (banded_strip.h) the sliding operand is staged
 // once instead of once per 32 diagonals, and the result leaves in 16-byte stores.
@@ -51,15 +51,18 @@ inline MaxDims max_dims(int Wa, int Wb, int Wo) {
 // maximum, and one compare and one select keep the pair that raised it last: 2.5 instructions per term
 // instead of 4 - and which k of its pair it was is found behind the walk, by forming the first one's sum
 // again.  The first pair that attains the maximum and the first k inside it are what the walk with a
-// strict comparison keeps.  64 x 4096, 65 diagonals each 281 -> 273 us, 16 x 4096, 129 diagonals each
-// 536 -> 497.  What is left has no single bound (counters, 64 x 4096): 1.8 waves per SIMD issue vector
-// instructions in 63 % of a busy compute unit's cycles (85 M of them) and keep its LDS reading in 50 %
-// (nine values per eight terms; a quarter of that are bank conflicts), and compute units have no wave for a
-// fifth of the launch.
-template <bool PAIRS>
-__global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int strips, const MaxDims d,
+// strict comparison keeps (16 x 4096, 129 diagonals each 536 -> 497 us).
+//
+// Eight waves where LDS leaves a compute unit three workgroups or fewer (four waves each kept 1.8 on a SIMD, which
+// issued in 63 % of its cycles), and for grids of one round.  With that, and strips at the matrix's edge on the same
+// walk as the others instead of a loop of predicated single terms that the launch's end waited for:
+// 64 x 4096, 65 diagonals each 272 -> 177 us, bfloat16 291 -> 165, 49 diagonals 153 -> 125; 2 x 500, 65 diagonals
+// 72 -> 16; 57 x 366, 20 and 22 diagonals 17.3 -> 11.5.  (Eight waves on narrow bands: 17 diagonals 47 -> 60.)
+template <bool PAIRS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : 2) void k_band_max_fwd(const BandArgs p, int strips, const MaxDims d,
                                                          long cells_a, long cells_b, int nseg, int Wseg) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
+  constexpr int NT = 64 * WAVES, BLOCKS = (160 / 8 + WAVES - 1) / WAVES;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int wg = xcd_strip_id();
@@ -76,51 +79,63 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
   const int q0 = x0 - r_lu + j_lo;  // first row of b that the segment's cells meet
   const int qr0 = max(q0, 0), qr1 = min(q0 + d.q_rows, n);
   const int pr1 = min(x0 + kMaxRows, n);
-  MmFlat<14, elem_t> sq;
-  MmFlat<6, elem_t> sp;
+  MmFlat<14 * 256 / NT, elem_t, NT> sq;
+  MmFlat<6 * 256 / NT, elem_t, NT> sp;
   sq.init(p.b, p.b + cells_b, (bn + qr0) * Wb, (qr1 - qr0) * Wb, Wb, d.qp);
   sq.load(p.b, p.b + cells_b, 0, tid);
   sp.init(p.a, p.a + cells_a, (bn + x0) * Wa, (pr1 - x0) * Wa, Wa, d.pp);
   sp.load(p.a, p.a + cells_a, 0, tid);
-  sq.store(QL, 0, tid);
+  const int qp = d.qp, pp = d.pp;
+  float* QR = QL + (qr0 - q0) * qp;  // (row q0 of b, inside the matrix or not, lies at QL)
+  sq.store(QR, 0, tid);
   for (int b = 1; sq.more(b); ++b) {
     sq.load(p.b, p.b + cells_b, b, tid);
-    sq.store(QL, b, tid);
+    sq.store(QR, b, tid);
   }
   sp.store(PL, 0, tid);
   for (int b = 1; sp.more(b); ++b) {
     sp.load(p.a, p.a + cells_a, b, tid);
     sp.store(PL, b, tid);
   }
+  float* Pt = PL + sp.origin();  // a[x0 + r][k] = Pt[r * pp + k]
+  float* Qt = QL + sq.origin();  // b[q0 + r][k2] = Qt[r * qp + k2]
   {  // -inf between the rows of b (and before the first): cells that are no k of a cell
-    const int gap = d.qp - Wb, first = sq.origin() - (qr0 - q0) * d.qp;
-    for (int e = tid; e < (d.q_rows + 1) * gap; e += 256) {
-      const int r = e / gap, c = e - r * gap;
-      const int at = first + (r - 1) * d.qp + Wb + c;
+    const int gap = qp - Wb;
+    for (int e = tid; e < (d.q_rows + 1) * gap; e += NT) {
+      const int r = e / gap, c = e - r * gap, at = sq.origin() + (r - 1) * qp + Wb + c;
       if (at >= 0) QL[at] = -INFINITY;
     }
   }
+  // A strip at the matrix's edge: rows of b outside it, and cells of a in rows outside it, are no terms either.
+  const bool interior = x0 >= max(p.a_lu, r_lu) && x0 + kMaxRows - 1 <= n - 1 - max(Wa - 1 - p.a_lu, Wo - 1 - r_lu);
+  if (!interior) {  // uniform
+    __syncthreads();  // the operands' cells are staged (and, in the first and last piece, cells beyond them)
+    const int above = min(qr0 - q0, d.q_rows), below = min(max(q0 + d.q_rows - qr1, 0), d.q_rows - above);
+    for (int e = tid; e < (above + below) * Wb; e += NT) {
+      const int r = e / Wb, c = e - r * Wb;
+      Qt[(r < above ? r : d.q_rows - below + r - above) * qp + c] = -INFINITY;
+    }
+    for (int e = tid; e < kMaxRows * Wa; e += NT) {
+      const int r = e / Wa, k = e - r * Wa;
+      if ((unsigned)(x0 + r + k - p.a_lu) >= (unsigned)n) Pt[r * pp + k] = -INFINITY;
+    }
+  }
   __syncthreads();
-  const int pp = d.pp, qp = d.qp;
-  const float* Pt = PL + sp.origin();                        // a[x0 + r][k] = Pt[r * pp + k]
-  const float* Qt = QL + sq.origin() - (qr0 - q0) * qp;      // b[q0 + r][k2] = Qt[r * qp + k2]
 
   // ---- products
   const int x = x0 + lane;
-  // every row of the strip is inside the matrix with its whole band, and so is every b row
-  const bool interior = x0 >= max(p.a_lu, r_lu) && x0 + kMaxRows - 1 <= n - 1 - max(Wa - 1 - p.a_lu, Wo - 1 - r_lu);
   const float* ap = Pt + lane * pp;
   const int nblocks = (Ws + 7) >> 3;
-  float val[5][8];  // blocks wave, wave + 4, ...: at most 5 of them (Ws <= 160)
-  int ind[5][8];
+  float val[BLOCKS][8];  // blocks wave, wave + WAVES, ... (Ws <= 160)
+  int ind[BLOCKS][8];
 #pragma unroll
-  for (int s = 0; s < 5; ++s) {
+  for (int s = 0; s < BLOCKS; ++s) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       val[s][t] = kFloor;
       ind[s][t] = -1;
     }
-    const int jb = wave + 4 * s;
+    const int jb = wave + WAVES * s;
     if (jb < nblocks) {
       const int j0 = j_lo + 8 * jb;
       // b[o][k2] of cell t at step k: Qt[(lane + j0 - j_lo + t) * qp + k - j0 - t + Wb - 1]
@@ -133,7 +148,7 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
           ind[s][t] = k;
         }
       };
-      if (interior) {
+      {
         // all 8 cells walk the union of their k ranges: where a cell has no such k it reads
         // -inf from between the rows
         const int klo = max(0, j0 - (Wb - 1)), khi = min(Wa - 1, j0 + 7);
@@ -183,16 +198,6 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
               if (val[s][t] == 0.f) val[s][t] = ap[ind[s][t]] + bp[t * dt + ind[s][t]];
           }
         }
-      } else if (x < n) {
-        // the reference's k range per cell (k2 in [0, Wb), dense row i + k - lu_a in [0, n))
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const int j = j0 + t, o = x + j - r_lu;
-          if (j < j_lo + Ws && o >= 0 && o < n) {
-            const int klo = max(max(0, j - (Wb - 1)), p.a_lu - x), khi = min(min(Wa - 1, j), n - 1 + p.a_lu - x);
-            for (int k = klo; k <= khi; ++k) fold(t, ap[k], bp[t * dt + k], k);
-          }
-        }
       }
     }
   }
@@ -201,8 +206,8 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
   float* Sv = smem;
   int* Si = reinterpret_cast<int*>(smem + ((kMaxRows * Ws + 3) & ~3));
 #pragma unroll
-  for (int s = 0; s < 5; ++s) {
-    const int jb = wave + 4 * s;
+  for (int s = 0; s < BLOCKS; ++s) {
+    const int jb = wave + WAVES * s;
     if (jb < nblocks) {
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
@@ -223,12 +228,12 @@ __global__ __launch_bounds__(256, 2) void k_band_max_fwd(const BandArgs p, int s
   typedef int mm_i4 __attribute__((ext_vector_type(4)));
   if (Ws == Wo && (cells & 3) == 0 &&
       ((reinterpret_cast<uintptr_t>(ob) | reinterpret_cast<uintptr_t>(ib)) & 15) == 0) {
-    for (int e = 4 * tid; e < cells; e += 1024) {  // the strip's rows are one contiguous run
+    for (int e = 4 * tid; e < cells; e += 4 * NT) {  // the strip's rows are one contiguous run
       st4a(ob + e, *reinterpret_cast<const float4*>(Sv + e));
       *reinterpret_cast<mm_i4*>(ib + e) = *reinterpret_cast<const mm_i4*>(Si + e);
     }
   } else {
-    for (int e = tid; e < cells; e += 256) {  // runs of Ws cells, one per row
+    for (int e = tid; e < cells; e += NT) {  // runs of Ws cells, one per row
       const int r = e / Ws, c = e - r * Ws;
       ob[(long)r * Wo + c] = to_elem<elem_t>(Sv[e]);
       ib[(long)r * Wo + c] = Si[e];
