@@ -1,15 +1,18 @@
-// The eager route of logbmm, maxbmm, prodmaxbmm and samplebmm in native code: checks, allocations, the library
-// calls and the autograd nodes of genmul.py's Functions, for operands that need no conversion.
+// The eager route of logbmm, maxbmm, prodmaxbmm, samplebmm and of the banded products (+,x), log and max in native
+// code: checks, allocations, the library calls and the autograd nodes of genmul.py's and sparse.py's Functions, for
+// operands that need no conversion.
 //
 // What it is for: a small product's forward and gradients wait for the host.  A Python node costs its own
 // construction, a hand-over of the interpreter lock to the autograd engine's thread and back, and a nested node
 // for logbmm's first backward; (16, 64^3) forward and both gradients, 25 us of kernels:
-// 107 us by the Python Functions, 54 here, 49 for one multiplication of torch's own with its gradients.
+// 107 us by the Python Functions, 54 here, 49 for one multiplication of torch's own with its gradients.  Narrow bands
+// likewise: 129 x 247, 6 and 12 diagonals, multiply with both gradients 91 -> 53 us, 98 x 641, 30 and 17, multiply_max 91 -> 53.
 //
 // Which calls it takes (`plain`): tensors of the exact types Tensor / Parameter, float32 / float16 / bfloat16, 3-D,
 // contiguous, of one batch size, on one GPU, without a forward-mode tangent, under no trace, dispatch mode or functorch
-// transform, whose reduction is not cut in Python.  For any other the functions return None and genmul.py goes on as
-// it does without them - conversions, double precision, the messages of what is refused.
+// transform, whose reduction is not cut in Python; band tensors (`plain_bands`) likewise, of one size, whose widths are
+// those of their bands and which no dense product takes the place of.  For any other the functions return None and
+// the Python side goes on as it does without them - conversions, double precision, the messages of what is refused.
 #include <ATen/core/TorchDispatchUtils.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
@@ -18,6 +21,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
+
+#include <algorithm>
 
 #include "genbmm_gfx950.h"
 
@@ -195,6 +200,79 @@ struct SampleBmm : torch::autograd::Function<SampleBmm> {
   }
 };
 
+// ------------------------------------------------------------ banded products
+struct Bands {
+  int a_lu, a_ld, b_lu, b_ld;
+};
+Bands bands_of(AutogradContext* ctx) {
+  const auto v = ctx->saved_data["bands"].toIntVector();
+  return {(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+}
+
+// saved: the operands and what the forward left beside the result - the index of every cell (max), the result and the
+// workspace (log), nothing ((+,x))
+template <int MODE>
+struct BandProduct : torch::autograd::Function<BandProduct<MODE>> {
+  static constexpr bool kLog = MODE == GENBMM_BAND_LOG, kMax = MODE == GENBMM_BAND_MAX;
+  static Tensor forward(AutogradContext* ctx, const Tensor& a, const Tensor& b, int64_t a_lu, int64_t a_ld, int64_t b_lu,
+                        int64_t b_ld) {
+    const c10::DeviceGuard guard(a.device());
+    const Bands w{(int)a_lu, (int)a_ld, (int)b_lu, (int)b_ld};
+    const int B = a.size(0), n = a.size(1);
+    Tensor out = at::empty({B, n, a.size(2) + b.size(2) - 1}, a.options()), idx, ws;
+    if (kMax) idx = at::empty(out.sizes(), a.options().dtype(at::kInt));
+    if (kLog) ws = at::empty({(int64_t)genbmm_banded_workspace_size(w.a_lu, w.a_ld, w.b_lu, w.b_ld, B, n)}, workspace(a));
+    check(GENBMM_BY_TYPE(a, genbmm_banded_fwd, at_<E>(a), w.a_lu, w.a_ld, at_<E>(b), w.b_lu, w.b_ld, at_<E>(out),
+                         kMax ? at_<int32_t>(idx) : nullptr, kLog ? at_<float>(ws) : nullptr, B, n, MODE, stream_of(a)),
+          "genbmm_banded_fwd");
+    if (kLog) ctx->save_for_backward({a, b, out, ws});
+    else if (kMax) ctx->save_for_backward({a, b, idx});
+    else ctx->save_for_backward({a, b});
+    ctx->saved_data["bands"] = std::vector<int64_t>{a_lu, a_ld, b_lu, b_ld};
+    ctx->saved_data["type"] = a.scalar_type();
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &a = saved[0], &b = saved[1];
+    const Tensor g = incoming(grads[0], ctx->saved_data["type"].toScalarType());
+    const Bands w = bands_of(ctx);
+    const at::ScalarType type = g.scalar_type();
+    const int64_t B = g.size(0), n = g.size(1), wa = w.a_lu + w.a_ld + 1, wb = w.b_lu + w.b_ld + 1;
+    require(g, "the incoming gradient", g, type, {B, n, wa + wb - 1});
+    require(a, "a", g, type, {B, n, wa});
+    require(b, "b", g, type, {B, n, wb});
+    Tensor out, ws, scratch;
+    if (kMax) require(saved[2], "the indices", g, at::kInt, g.sizes());
+    if (kLog) {
+      out = saved[2].detach();  // as a value (LogBmm)
+      ws = saved[3];
+      require(out, "the result", g, type, g.sizes());
+      require(ws, "the forward's workspace", g, at::kFloat,
+              {(int64_t)genbmm_banded_workspace_size(w.a_lu, w.a_ld, w.b_lu, w.b_ld, (int)B, (int)n)});
+      if (at::GradMode::is_enabled() || has_tangent(g) || has_tangent(a) || has_tangent(b)) {
+        const py::gil_scoped_acquire gil;
+        const py::tuple r = py::module_::import("genbmm_amd.sparse")
+                                .attr("_BandedLogGrad")
+                                .attr("apply")(a, b, g, out, ws, py::make_tuple(w.a_lu, w.a_ld, w.b_lu, w.b_ld));
+        return {r[0].cast<Tensor>(), r[1].cast<Tensor>(), Variable(), Variable(), Variable(), Variable()};
+      }
+    }
+    const c10::DeviceGuard guard(g.device());
+    Tensor ga = at::empty_like(a), gb = at::empty_like(b);
+    if (kLog) {  // (a buffer of this call's own: see sparse._backward)
+      const int64_t need = genbmm_banded_scratch_size(w.a_lu, w.a_ld, w.b_lu, w.b_ld, (int)B, (int)n);
+      if (need > 0) scratch = at::empty({need}, workspace(g));
+    }
+    check(GENBMM_BY_TYPE(g, genbmm_banded_bwd_scratch, at_<E>(a), w.a_lu, w.a_ld, at_<E>(b), w.b_lu, w.b_ld,
+                         kLog ? at_<E>(out) : nullptr, kMax ? at_<int32_t>(saved[2]) : nullptr,
+                         kLog ? at_<float>(ws) : nullptr, scratch.defined() ? at_<float>(scratch) : nullptr, at_<E>(g),
+                         at_<E>(ga), at_<E>(gb), (int)B, (int)n, MODE, stream_of(g)),
+          "genbmm_banded_bwd_scratch");
+    return {ga, gb, Variable(), Variable(), Variable(), Variable()};
+  }
+};
+
 // ------------------------------------------------------------------ entry
 // A GPU tensor with storage of its own and nothing in front of it: what is not one of these keys is a wrapper
 // (functorch, a fake or proxy tensor, a Python subclass), a lazy conjugate or negative, or another layout.
@@ -211,25 +289,42 @@ bool eager() {
          !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 
-bool plain(const py::handle& pa, const py::handle& pb) {
+constexpr int64_t kMost = 0x7fffffff;
+
+// two 3-D contiguous tensors of one type and one GPU, with nothing around them
+bool plain_pair(const py::handle& pa, const py::handle& pb) {
   if (!THPVariable_CheckExact(pa.ptr()) || !THPVariable_CheckExact(pb.ptr())) return false;
   const Tensor &a = THPVariable_Unpack(pa.ptr()), &b = THPVariable_Unpack(pb.ptr());
   if (!bare(a) || !bare(b) || a.dim() != 3 || b.dim() != 3 || a.scalar_type() != b.scalar_type() || a.device() != b.device())
     return false;
   const at::ScalarType type = a.scalar_type();
   if (type != at::kFloat && type != at::kHalf && type != at::kBFloat16) return false;
+  return a.is_contiguous() && b.is_contiguous() && !has_tangent(a) && !has_tangent(b);
+}
+
+bool plain(const py::handle& pa, const py::handle& pb) {
+  if (!plain_pair(pa, pb)) return false;
+  const Tensor &a = THPVariable_Unpack(pa.ptr()), &b = THPVariable_Unpack(pb.ptr());
   const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(2);
-  if (b.size(0) != B || b.size(1) != K || !a.is_contiguous() || !b.is_contiguous()) return false;
-  if (has_tangent(a) || has_tangent(b)) return false;
-  constexpr int64_t most = 0x7fffffff;
-  if (B > most || M > most || N > most) return false;
+  if (b.size(0) != B || b.size(1) != K || B > kMost || M > kMost || N > kMost) return false;
   if (K >= 4096) return false;  // genmul._reduction_splits may cut it
   return eager();
 }
 
+// `dense`: a product that sparse._dense_pays may send through dense matrices where both bands are wide
+bool plain_bands(const py::handle& pa, int64_t a_lu, int64_t a_ld, const py::handle& pb, int64_t b_lu, int64_t b_ld, bool dense) {
+  if (!plain_pair(pa, pb)) return false;
+  const Tensor &a = THPVariable_Unpack(pa.ptr()), &b = THPVariable_Unpack(pb.ptr());
+  const int64_t B = a.size(0), n = a.size(1), wa = a.size(2), wb = b.size(2);
+  if (b.size(0) != B || b.size(1) != n || std::min({a_lu, a_ld, b_lu, b_ld}) < 0) return false;
+  if (B > kMost || n > kMost || wa > kMost || wb > kMost || wa != a_lu + a_ld + 1 || wb != b_lu + b_ld + 1) return false;
+  if (dense && std::min(wa, wb) > 128) return false;
+  return eager();
+}
+
 template <class F>
-py::object on(const py::handle& pa, const py::handle& pb, F&& f) {
-  if (!plain(pa, pb)) return py::none();
+py::object on(const py::handle& pa, const py::handle& pb, bool takes, F&& f) {
+  if (!takes) return py::none();
   const Tensor a = THPVariable_Unpack(pa.ptr()), b = THPVariable_Unpack(pb.ptr());
   Tensor out;
   {
@@ -268,17 +363,26 @@ PYBIND11_MODULE(_host, m) {
   if (PyModule_AddFunctions(m.ptr(), kMethods) != 0) throw py::error_already_set();
   m.def("plain", &plain);
   m.def("logbmm", [](const py::handle& a, const py::handle& b, int64_t path, int64_t half_path) {
-    return on(a, b, [&](const Tensor& x, const Tensor& y) {
+    return on(a, b, plain(a, b), [&](const Tensor& x, const Tensor& y) {
       return LogBmm::apply(x, y, x.scalar_type() == at::kFloat ? path : half_path);
     });
   });
   m.def("maxbmm", [](const py::handle& a, const py::handle& b) {
-    return on(a, b, [](const Tensor& x, const Tensor& y) { return MaxBmm::apply(x, y); });
+    return on(a, b, plain(a, b), [](const Tensor& x, const Tensor& y) { return MaxBmm::apply(x, y); });
   });
   m.def("prodmaxbmm", [](const py::handle& a, const py::handle& b) {
-    return on(a, b, [](const Tensor& x, const Tensor& y) { return ProdMaxBmm::apply(x, y); });
+    return on(a, b, plain(a, b), [](const Tensor& x, const Tensor& y) { return ProdMaxBmm::apply(x, y); });
   });
+#define GENBMM_BAND(name, mode, dense)                                                                             \
+  m.def(name, [](const py::handle& a, int64_t a_lu, int64_t a_ld, const py::handle& b, int64_t b_lu, int64_t b_ld) { \
+    return on(a, b, plain_bands(a, a_lu, a_ld, b, b_lu, b_ld, dense), [&](const Tensor& x, const Tensor& y) {        \
+      return BandProduct<mode>::apply(x, y, a_lu, a_ld, b_lu, b_ld);                                                 \
+    });                                                                                                              \
+  })
+  GENBMM_BAND("band_mul", GENBMM_BAND_MUL, true);
+  GENBMM_BAND("band_log", GENBMM_BAND_LOG, true);
+  GENBMM_BAND("band_max", GENBMM_BAND_MAX, false);
   m.def("samplebmm", [](const py::handle& a, const py::handle& b, uint64_t seed, uint64_t offset) {
-    return on(a, b, [&](const Tensor& x, const Tensor& y) { return SampleBmm::apply(x, y, (int64_t)seed, (int64_t)offset); });
+    return on(a, b, plain(a, b), [&](const Tensor& x, const Tensor& y) { return SampleBmm::apply(x, y, (int64_t)seed, (int64_t)offset); });
   });
 }

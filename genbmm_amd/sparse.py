@@ -339,11 +339,14 @@ class BandedMatrix:
         lu, ld = self.lu + other.ld, self.ld + other.lu
         return BandedMatrix(banddiag(d, lu, ld)[0], lu, ld, self.fill)
 
-    def _product(self, other, fn):
+    def _product(self, other, fn, eager=None):
         batch, n, _ = self.data.shape
         assert other.data.shape[1] == n
         lu = self.lu + other.ld
         ld = self.ld + other.lu
+        out = eager and _eager(eager, self.data, self.lu, self.ld, other.data, other.lu, other.ld)
+        if out is not None:
+            return BandedMatrix(out, lu, ld, self.fill)
         if (fn is bandedbmm or fn is bandedlogbmm) and self._dense_pays(other, fn is bandedlogbmm):
             return self._product_dense(other, fn is bandedlogbmm)
         # views are copied here, by a differentiable torch operation, so that the
@@ -355,15 +358,15 @@ class BandedMatrix:
 
     def multiply(self, other):
         """Dense(other)^T @ Dense(self) in band form (reference sparse.py:229-240)."""
-        return self._product(other, bandedbmm)
+        return self._product(other, bandedbmm, "band_mul")
 
     def multiply_log(self, other):
         """The same product in the (logsumexp, +) semiring (reference sparse.py:242-253)."""
-        return self._product(other, bandedlogbmm)
+        return self._product(other, bandedlogbmm, "band_log")
 
     def multiply_max(self, other):
         """The same product in the (max, +) semiring (reference sparse.py:255-266)."""
-        return self._product(other, bandedmaxbmm)
+        return self._product(other, bandedmaxbmm, "band_max")
 
     def multiply_sample(self, other, stream=None):
         """The log product whose gradient is a one-hot sample: every result cell draws one of
@@ -384,6 +387,16 @@ class BandedMatrix:
 
 
 # ------------------------------------------------------------------ autograd
+def _eager(name, a, a_lu, a_ld, b, b_lu, b_ld):
+    """The product `name` by csrc/host.cpp's nodes on band tensors that need no conversion, as genmul._native takes the
+    dense products' calls; None for any other.  Same library calls, same results bit for bit."""
+    if not (type(a_lu) is type(a_ld) is type(b_lu) is type(b_ld) is int and isinstance(a, torch.Tensor)
+            and isinstance(b, torch.Tensor) and a.is_cuda and b.is_cuda):
+        return None
+    host = _lib.host()
+    return getattr(host, name)(a, a_lu, a_ld, b, b_lu, b_ld) if host is not None else None
+
+
 def _f64(t):
     return t.dtype == torch.float64
 
