@@ -1,4 +1,6 @@
 // Dense semiring batched matmul: the arg-max backward kernels (gfx950).
+#include <type_traits>
+
 #include "common.h"
 
 namespace GENBMM_NS {
@@ -17,7 +19,7 @@ namespace {
 // therefore happen in the reference's order, so the result is bit-identical, in
 // O(M*N) work.  Products are rounded before the add (the build uses
 // -ffp-contract=on: no fusion across statements).
-constexpr int kKC = 128;  // cells of the reduction axis per lane
+constexpr int kKC = 128;  // cells of the reduction axis per lane, at most (KC: those of an instantiation)
 
 // The 64 lanes of a workgroup are (line, part): 64 >> ps lines (rows m of grad_a,
 // columns n of grad_b) times 2^ps parts of kKC consecutive k, so that one workgroup
@@ -43,10 +45,18 @@ constexpr int kKC = 128;  // cells of the reduction axis per lane
 // (40, 251, 173, 301) 21.6 -> 17.9 (22.5 -> 20.7), (100, 500, 300, 510) 198 -> 160 (200 -> 163), (512, 128^3) 34
 // (43) either way (memory).  With the product semiring's factors the same took more registers
 // than a wave's 256 ((512, 128^3) 47 -> 51, (64, 512^3) 158 -> 139): it keeps the longer form.
+//
+// A K of 96, 64 or 32 and less takes as many cells per lane: what bounds the waves of a compute unit is their LDS,
+// and six, nine or nineteen waves hide each other's chains (chunks are shorter then, for the registers).  On other
+// buffers each time, max and (in brackets) product semiring, from 128 cells: (5753, 54^3) 95 -> 85 us (138 -> 132),
+// (2048, 48^3) 33.5 -> 23.6 (39.6 -> 33.6), (814, 76, 51, 83) 45 -> 34 (68 -> 64), (1000, 90^3) 58 -> 52 (100 -> 88),
+// (8192, 32^3) 60 -> 49 (75 -> 72).
 static_assert(kKC == 128, "the shifts of the write-out");
-constexpr int kArgAcc = 64 * kKC + 64;  // floats of LDS: the cells, one spare cell per lane
-constexpr int kChA = 32, kChB = 16;     // cells per chunk (a column's cells are single loads, and at most
-                                        // 63 loads can be in flight)
+constexpr int kChB = 16;  // cells of a column per chunk (single loads, and at most 63 loads can be in flight)
+template <int KC>
+constexpr int kArgAcc = 64 * KC + 64;  // floats of LDS: the cells, one spare cell per lane
+template <int KC>
+constexpr int kChA = KC == kKC ? 32 : 16;  // cells of a row per chunk
 
 // Chunks of a line as they come from memory - indices, gradients and for PROD == 2 the other factor;
 // nothing is converted before it is added, which would wait for the load - of a row (pieces of four
@@ -58,9 +68,9 @@ typedef elem_t argmax_e4 __attribute__((ext_vector_type(4), aligned(sizeof(elem_
 // loads are flat and drain all others)
 template <class E>
 using argmax_global = const __attribute__((address_space(1))) E*;
-template <int PROD>
+template <int PROD, int KC>
 struct ArgRow {
-  static constexpr int CH = kChA;
+  static constexpr int CH = kChA<KC>;
   argmax_i4 i4[CH / 4];
   argmax_e4 g4[CH / 4];
   argmax_f4 f4[PROD == 2 ? CH / 4 : 1];
@@ -88,14 +98,14 @@ __device__ __forceinline__ void wave_lds_sync() {
 // (the cells of a partial last chunk, index -1 behind them) and add(chunk, number).  No load stands
 // under a branch in the loop - the last chunk is asked for again instead -: behind a branch the compiler
 // can no longer tell which loads are younger than the chunk it waits for, and waits for all of them.
-template <class Chunk, class Load, class Tail, class Add>
+template <int KC, class Chunk, class Load, class Tail, class Add>
 __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int cells, int kcap, Load load, Tail tail, Add add) {
   const int lane = threadIdx.x, full = cells / Chunk::CH;
   Chunk x, y;
   if (full > 0) load(x, 0);
 #pragma unroll 16
   for (int kk = 0; kk < kcap; ++kk) accs[kk * 64 + lane] = 0.f;
-  accs[kKC * 64 + lane] = 0.f;
+  accs[KC * 64 + lane] = 0.f;
   int c = 0;
   for (; c + 1 < full; c += 2) {
     load(y, c + 1);
@@ -111,7 +121,7 @@ __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int cells,
 }
 // The chunk's terms (g, times the other factor for the product semiring) in order.  other(cell, k):
 // that factor read from its matrix (PROD == 1), only when the index falls into the lane's part.
-template <int PROD, class Chunk, class Other>
+template <int PROD, int KC, class Chunk, class Other>
 __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk& x, int c0, int kc, Other other) {
   constexpr int CH = Chunk::CH;
   const int lane = threadIdx.x;
@@ -121,12 +131,12 @@ __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk
   for (int q = 0; q < CH; ++q) {
     if constexpr (PROD == 2) {
       const int k = x.iv(q) - c0;
-      sl[q] = (k >= 0 && k < kc ? k : kKC) * 64 + lane;  // [kKC]: the spare cells
+      sl[q] = (k >= 0 && k < kc ? k : KC) * 64 + lane;  // [KC]: the spare cells
       tv[q] = __fmul_rn(x.fv(q), x.gv(q));
     } else {
       // the lane's cell, or its spare one: an index below the part wraps around, one of K or beyond (none that the
       // library writes) may fall to a cell of the last part that is not written out.  Its factor does not exist.
-      const unsigned k = min((unsigned)x.iv(q) - (unsigned)c0, (unsigned)kKC);
+      const unsigned k = min((unsigned)x.iv(q) - (unsigned)c0, (unsigned)KC);
       sl[q] = k * 64 + lane;
       tv[q] = x.gv(q);
       if (PROD == 1 && (int)k < kc) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
@@ -141,8 +151,8 @@ __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk
 }
 
 // grad_a: line = row m, read in pieces of four cells (any alignment).
-// (blk: the workgroup's number among those of grad_a; accs: kArgAcc floats of LDS)
-template <int PROD>
+// (blk: the workgroup's number among those of grad_a; accs: kArgAcc<KC> floats of LDS)
+template <int PROD, int KC>
 __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int blk,
                                                    const elem_t* __restrict__ bmat,
                                                    const float* __restrict__ fac,
@@ -155,28 +165,28 @@ __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int
   const int kc_id = blk % k_chunks, rt = blk / k_chunks;
   const int batch = rt / row_tiles;
   const int m = (rt - batch * row_tiles) * lines + line;
-  const int c0 = kc_id * (parts * kKC) + part * kKC;  // first k of this lane
-  const int kc = min(kKC, K - c0);                    // <= 0: the part lies beyond K
+  const int c0 = kc_id * (parts * KC) + part * KC;  // first k of this lane
+  const int kc = min(KC, K - c0);                    // <= 0: the part lies beyond K
   const long row = (long)batch * M + min(m, M - 1);   // lanes beyond the matrix walk the last row
   const int32_t* irow = idx + row * N;
   const elem_t* grow = g + row * N;
   const elem_t* bb = PROD == 1 ? bmat + (long)batch * K * N : nullptr;
   const float* frow = PROD == 2 ? fac + row * N : nullptr;
-  const int kcap = min(kKC, K);  // no lane has more cells
-  using Chunk = ArgRow<PROD>;
+  const int kcap = min(KC, K);  // no lane has more cells
+  using Chunk = ArgRow<PROD, KC>;
   auto load = [&](Chunk& x, int c) __attribute__((always_inline)) {
-    const int n0 = c * kChA;
+    const int n0 = c * Chunk::CH;
 #pragma unroll
-    for (int q = 0; q < kChA / 4; ++q) {
+    for (int q = 0; q < Chunk::CH / 4; ++q) {
       x.i4[q] = *reinterpret_cast<const argmax_i4*>(irow + n0 + 4 * q);
       x.g4[q] = *reinterpret_cast<const argmax_e4*>(grow + n0 + 4 * q);
       if constexpr (PROD == 2) x.f4[q] = *reinterpret_cast<const argmax_f4*>(frow + n0 + 4 * q);
     }
   };
   auto tail = [&](Chunk& x, int c) __attribute__((always_inline)) {
-    const int n0 = c * kChA;
+    const int n0 = c * Chunk::CH;
 #pragma unroll
-    for (int q = 0; q < kChA / 4; ++q) {
+    for (int q = 0; q < Chunk::CH / 4; ++q) {
       const int nq = n0 + 4 * q;
       if (nq + 4 <= N) {  // uniform
         x.i4[q] = *reinterpret_cast<const argmax_i4*>(irow + nq);
@@ -193,45 +203,45 @@ __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int
       }
     }
   };
-  argmax_walk<Chunk>(accs, N, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
-    argmax_add<PROD>(accs, x, c0, kc, [&](int q, int k) { return (float)bb[(long)k * N + c * kChA + q]; });
+  argmax_walk<KC, Chunk>(accs, N, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
+    argmax_add<PROD, KC>(accs, x, c0, kc, [&](int q, int k) { return (float)bb[(long)k * N + c * Chunk::CH + q]; });
   });
-  // The cells change places, through registers, to [lane][kKC + 1] - a row's parts one after the other -
+  // The cells change places, through registers, to [lane][KC + 1] - a row's parts one after the other -
   // so that the rows leave in runs (a lane storing its own cells, 16 bytes at a time and 512 apart, took
   // longer than the walk).
   wave_lds_sync();
   {
-    float cell[kKC];
+    float cell[KC];
 #pragma unroll
-    for (int k0 = 0; k0 < kKC; k0 += 32)
+    for (int k0 = 0; k0 < KC; k0 += 32)
       if (k0 < kcap) {  // uniform
 #pragma unroll
         for (int kk = k0; kk < k0 + 32; ++kk) cell[kk] = accs[kk * 64 + lane];
       }
     wave_lds_sync();
 #pragma unroll
-    for (int k0 = 0; k0 < kKC; k0 += 32)
+    for (int k0 = 0; k0 < KC; k0 += 32)
       if (k0 < kcap) {
 #pragma unroll
-        for (int kk = k0; kk < k0 + 32; ++kk) accs[lane * (kKC + 1) + kk] = cell[kk];
+        for (int kk = k0; kk < k0 + 32; ++kk) accs[lane * (KC + 1) + kk] = cell[kk];
       }
   }
   wave_lds_sync();
-  const int kw = parts * kKC, w0 = kc_id * kw, kn = min(kw, K - w0);
+  const int kw = parts * KC, w0 = kc_id * kw, kn = min(kw, K - w0);
   const int m0 = (rt - batch * row_tiles) * lines, rows = min(lines, M - m0);
   elem_t* dst = grad_a + ((long)batch * M + m0) * K + w0;
-  auto cell_of = [&](int kk) { return accs + (kk >> 7) * (kKC + 1) + (kk & (kKC - 1)); };
+  auto cell_of = [&](int kk) { return KC < kKC ? accs + kk : accs + (kk >> 7) * (kKC + 1) + (kk & (kKC - 1)); };
   if (lines >= 8) {
     for (int kk = lane; kk < kn; kk += 64) {
       const float* src = cell_of(kk);
 #pragma unroll 8
-      for (int r = 0; r < rows; ++r) dst[(long)r * K + kk] = to_elem<elem_t>(src[r * parts * (kKC + 1)]);
+      for (int r = 0; r < rows; ++r) dst[(long)r * K + kk] = to_elem<elem_t>(src[r * parts * (KC + 1)]);
     }
   } else {
     // K beyond 1024, a few long rows: the loads of a row overlap, not those of a column of four rows or fewer
     // (maxbmm forward and backward (1, 16, 4096, 16) 92 -> 83.5 us, (1, 8, 8192, 8) 98 -> 86)
     for (int r = 0; r < rows; ++r) {
-      const int off = r * parts * (kKC + 1), whole = kn >> 6;
+      const int off = r * parts * (KC + 1), whole = kn >> 6;
       elem_t* row = dst + (long)r * K;
 #pragma unroll 8
       for (int i = 0; i < whole; ++i) row[64 * i + lane] = to_elem<elem_t>(cell_of(64 * i + lane)[off]);
@@ -241,8 +251,8 @@ __device__ __forceinline__ void argmax_bwd_a_block(float* __restrict__ accs, int
 }
 
 // grad_b: line = column n.
-// (blk: the workgroup's number among those of grad_b; accs: kArgAcc floats of LDS)
-template <int PROD>
+// (blk: the workgroup's number among those of grad_b; accs: kArgAcc<KC> floats of LDS)
+template <int PROD, int KC>
 __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int blk,
                                                    const elem_t* __restrict__ amat,
                                                    const float* __restrict__ fac,
@@ -255,13 +265,13 @@ __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int
   const int kc_id = blk % k_chunks, ct = blk / k_chunks;
   const int batch = ct / col_tiles;
   const int n = (ct - batch * col_tiles) * lines + line, nn = min(n, N - 1);
-  const int c0 = kc_id * (parts * kKC) + part * kKC;
-  const int kc = min(kKC, K - c0);
+  const int c0 = kc_id * (parts * KC) + part * KC;
+  const int kc = min(KC, K - c0);
   const int32_t* icol = idx + (long)batch * M * N + nn;
   const elem_t* gcol = g + (long)batch * M * N + nn;
   const elem_t* ab = PROD == 1 ? amat + (long)batch * M * K : nullptr;
   const float* fcol = PROD == 2 ? fac + (long)batch * M * N + nn : nullptr;
-  const int kcap = min(kKC, K);  // no lane has more cells
+  const int kcap = min(KC, K);  // no lane has more cells
   using Chunk = ArgCol<PROD>;
   // HOLD: where a lane's cells of a chunk lie, one address each, a chunk on at a time.  Formed anew from the row's
   // number they take three scalar instructions a load, which a lone wave issues in the place of everything else.
@@ -302,8 +312,8 @@ __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int
       if constexpr (PROD == 2) x.f[q] = in ? fcol[(long)(m0 + q) * N] : 0.f;
     }
   };
-  argmax_walk<Chunk>(accs, M, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
-    argmax_add<PROD>(accs, x, c0, kc, [&](int q, int k) { return (float)ab[(long)(c * kChB + q) * K + k]; });
+  argmax_walk<KC, Chunk>(accs, M, kcap, load, tail, [&](const Chunk& x, int c) __attribute__((always_inline)) {
+    argmax_add<PROD, KC>(accs, x, c0, kc, [&](int q, int k) { return (float)ab[(long)(c * kChB + q) * K + k]; });
   });
   if (n < N)
 #pragma unroll 16
@@ -314,8 +324,9 @@ __device__ __forceinline__ void argmax_bwd_b_block(float* __restrict__ accs, int
 // Both gradients in one launch, batch item by batch item (ta workgroups of grad_a, then tb of
 // grad_b, per item; XCD-aware numbering): both read the item's idx and g, which then come from
 // memory once.
-template <int PROD>
-__global__ __launch_bounds__(64) void k_argmax_bwd_both(const elem_t* __restrict__ amat,
+// KC: below kKC where K is no larger (one part per line).
+template <int PROD, int KC>
+__global__ __launch_bounds__(64, KC == 32 ? 3 : KC < kKC ? 2 : 1) void k_argmax_bwd_both(const elem_t* __restrict__ amat,
                                                        const elem_t* __restrict__ bmat,
                                                        const float* __restrict__ fac_a,
                                                        const float* __restrict__ fac_b,
@@ -325,14 +336,14 @@ __global__ __launch_bounds__(64) void k_argmax_bwd_both(const elem_t* __restrict
                                                        elem_t* __restrict__ grad_b, int M, int K, int N,
                                                        int row_tiles, int kc_a, int ps_a,
                                                        int col_tiles, int kc_b, int ps_b) {
-  __shared__ float accs[kArgAcc];
+  __shared__ float accs[kArgAcc<KC>];
   const int ta = row_tiles * kc_a, tb = col_tiles * kc_b;
   const int v = xcd_renumber(blockIdx.x, gridDim.x);
   const int item = v / (ta + tb), r = v - item * (ta + tb);
   if (r < ta)
-    argmax_bwd_a_block<PROD>(accs, item * ta + r, bmat, fac_a, idx, g, grad_a, M, K, N, row_tiles, kc_a, ps_a);
+    argmax_bwd_a_block<PROD, KC>(accs, item * ta + r, bmat, fac_a, idx, g, grad_a, M, K, N, row_tiles, kc_a, ps_a);
   else
-    argmax_bwd_b_block<PROD>(accs, item * tb + r - ta, amat, fac_b, idx, g, grad_b, M, K, N, col_tiles, kc_b, ps_b);
+    argmax_bwd_b_block<PROD, KC>(accs, item * tb + r - ta, amat, fac_b, idx, g, grad_b, M, K, N, col_tiles, kc_b, ps_b);
 }
 
 // Parts per workgroup for a reduction axis of K cells: the smallest power of two that
@@ -365,14 +376,19 @@ int run_argmax_bwd(const elem_t* a, const elem_t* b, const int32_t* idx, const f
   const int col_tiles = ceil_div(N, 64 >> ps_b), kc_b = ceil_div(K, kKC << ps_b);
   const int64_t total = (int64_t)B * ((int64_t)row_tiles * kc_a + (int64_t)col_tiles * kc_b);
   if (total > 0x7fffffffLL) return GENBMM_E_SHAPE;
-  if (PROD && factors)
-    hipLaunchKernelGGL((k_argmax_bwd_both<2>), dim3((unsigned)total), dim3(64), 0, s, a, b, factors + mn, factors,
-                       idx, g, grad_a, grad_b, M, K, N, row_tiles, kc_a, ps_a,
-                       col_tiles, kc_b, ps_b);
-  else
-    hipLaunchKernelGGL((k_argmax_bwd_both<kGather>), dim3((unsigned)total), dim3(64), 0, s, a, b,
-                       (const float*)nullptr, (const float*)nullptr, idx, g, grad_a, grad_b, M, K, N, row_tiles,
+  auto go = [&](auto kern, const float* fa, const float* fb) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64), 0, s, a, b, fa, fb, idx, g, grad_a, grad_b, M, K, N, row_tiles,
                        kc_a, ps_a, col_tiles, kc_b, ps_b);
+  };
+  auto pick = [&](auto kc) {
+    constexpr int KC = decltype(kc)::value;
+    if (PROD && factors) go(k_argmax_bwd_both<2, KC>, factors + mn, factors);
+    else go(k_argmax_bwd_both<kGather, KC>, (const float*)nullptr, (const float*)nullptr);
+  };
+  if (K <= 32) pick(std::integral_constant<int, 32>{});
+  else if (K <= 64) pick(std::integral_constant<int, 64>{});
+  else if (K <= 96) pick(std::integral_constant<int, 96>{});
+  else pick(std::integral_constant<int, kKC>{});
   if (int e = launch_status()) return e;
   return GENBMM_OK;
 }
