@@ -135,7 +135,7 @@ __global__ __launch_bounds__(C::NT) void k_max_fwd(const DenseArgs p) {
 // software-pipelined: the codes two steps ahead and the first operand's values one step
 // ahead are requested before the current rows are finished and stored.
 //
-// Op supplies what differs: Extra load(e) (read together with the code of cell e),
+// Op supplies what differs: code(c) (the code of what idx holds), Extra load(e, c) (read together with it),
 // none(e) (a cell whose code is -1) and cell<TAIL>(e, kb, av, br, stride, low, valid, extra) with
 // av[j] = first operand at k = kb + j, br[j * stride] = second operand; the group's terms are
 // low <= j < valid.
@@ -189,8 +189,8 @@ __device__ __forceinline__ void resolve_walk(const E* __restrict__ first, const 
       const int m = row_of(mb, r);
       const long e = (long)min(m, M - 1) * N + nc;
       const int c = ib[e];
-      ex[r] = op.load(cell0 + e);
-      code[r] = (live && m < m_end) ? c : 0;
+      ex[r] = op.load(cell0 + e, c);
+      code[r] = (live && m < m_end) ? op.code(c) : 0;
     }
   };
   // first k of each row's group (-1: not a group of the staged rows kc..) and the
@@ -294,7 +294,8 @@ struct MaxResolve {
   int32_t* idx;
   float* fa;  // optional: the two factors of the winning term per cell (product semiring)
   float* fb;
-  __device__ __forceinline__ Extra load(long) const { return Extra{}; }
+  __device__ __forceinline__ int code(int c) const { return c; }
+  __device__ __forceinline__ Extra load(long, int) const { return Extra{}; }
   __device__ __forceinline__ void none(long e) const {
     out[e] = to_elem<elem_t>(kFloor);
     if (fa) {
@@ -578,13 +579,20 @@ __global__ __launch_bounds__(C::NT, 2) void k_sample_sweep(const DenseArgs p,
 // Second level of the sampling sweep: rem at the start of the group (G terms) goes
 // through multiply-adds term by term; the index is the group's first term plus the
 // number of terms after which rem is still >= 0 (rem only falls).
-template <int G>
+// PACKED (the matrix-core sweep): idx holds -rem with the number of its slab in the low bits (`tmask` of them; tmask
+// minus that number), and rem is read nowhere else - sweep and resolve
+// move 134 MB less at (64, 512^3): forward, draw and both gradients 508 -> 495 us.
+template <int G, bool PACKED>
 struct SampleResolve {
   typedef float Extra;
   const float* rem;
   int32_t* idx;
-  int K;
-  __device__ __forceinline__ float load(long e) const { return rem[e]; }
+  int K, tmask;
+  __device__ __forceinline__ int code(int c) const { return PACKED && c < 0 ? -2 - (tmask - (c & tmask)) : c; }
+  __device__ __forceinline__ float load(long e, int c) const {
+    if constexpr (PACKED) return -__int_as_float(c & ~tmask);
+    else return rem[e];
+  }
   __device__ __forceinline__ void none(long) const {}
   template <ResTail TAIL>
   __device__ __forceinline__ void cell(long e, int kb, const float (&av)[G], const float* br, int stride,
@@ -601,14 +609,14 @@ struct SampleResolve {
   }
 };
 
-template <int COLS, ResTail TAIL, int G>
+template <int COLS, ResTail TAIL, int G, bool PACKED>
 __global__ __launch_bounds__(kResWaves * 64, 4) void k_sample_resolve(
     const float* __restrict__ ea, const float* __restrict__ eb, const float* __restrict__ remw,
     int32_t* __restrict__ idx, int* __restrict__ valid, int M, int K, int N, int panels,
-    int row_chunks, int rows_per) {
+    int row_chunks, int rows_per, int tmask) {
   __shared__ float Bs[kResFloats];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *valid = 0;  // the 1/S array of the workspace is gone
-  SampleResolve<G> op{remw, idx, K};
+  if (blockIdx.x == 0 && threadIdx.x == 0) *valid = 0;  // the 1/S array of the workspace is the caller's to overwrite
+  SampleResolve<G, PACKED> op{remw, idx, K, tmask};
   // 16-term groups: two rows per step keep the pipelined values within the registers
   resolve_walk<COLS, TAIL, G, (G > 8 ? 2 : kResRows)>(ea, eb, idx, op, M, K, N, panels, row_chunks,
                                                      rows_per, Bs);
@@ -859,9 +867,9 @@ int launch_sweep(DenseArgs p, const float* stats, int B, int M, int K, int N, hi
   return launch_status();
 }
 
-// Second level of a sweep that left group codes (groups of `group` terms) in idx and
-// rem in the workspace's scratch array.
-template <int G>
+// Second level of a sweep that left group codes (groups of G terms) in idx and
+// rem in the workspace's scratch array, or both in idx (tmask != 0).
+template <int G, bool PACKED>
 int launch_sample_resolve(DenseArgs p, const LogFactors& f, int B, int M, int K, int N, hipStream_t s) {
   const int cols = K > 256 ? 32 : 64;
   int panels, row_chunks, rows_per;
@@ -870,16 +878,16 @@ int launch_sample_resolve(DenseArgs p, const LogFactors& f, int B, int M, int K,
     return e;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(rgrid), dim3(kResWaves * 64), 0, s, f.ea, f.eb, f.scratch, p.idx,
-                       f.valid, M, K, N, panels, row_chunks, rows_per);
+                       f.valid, M, K, N, panels, row_chunks, rows_per, PACKED ? log_sample_tag_mask(K) : 0);
   };
   const ResTail tail = resolve_tail(K, G);
   if (cols == 64) {
-    if (tail == kWhole) go(k_sample_resolve<64, kWhole, G>);
-    else if (tail == kRagged) go(k_sample_resolve<64, kRagged, G>);
-    else go(k_sample_resolve<64, kShort, G>);
+    if (tail == kWhole) go(k_sample_resolve<64, kWhole, G, PACKED>);
+    else if (tail == kRagged) go(k_sample_resolve<64, kRagged, G, PACKED>);
+    else go(k_sample_resolve<64, kShort, G, PACKED>);
   } else {
-    if (tail == kWhole) go(k_sample_resolve<32, kWhole, G>);
-    else go(k_sample_resolve<32, kRagged, G>);  // K > 256
+    if (tail == kWhole) go(k_sample_resolve<32, kWhole, G, PACKED>);
+    else go(k_sample_resolve<32, kRagged, G, PACKED>);  // K > 256
   }
   return launch_status();
 }
@@ -894,7 +902,7 @@ int launch_sweep_two(DenseArgs p, const float* stats, const LogFactors& f, int B
   hipLaunchKernelGGL((k_sample_sweep<C, true>), grid, dim3(C::NT), 0, s, p, stats, f.ea, f.eb,
                      f.scratch);
   if (int e = launch_status()) return e;
-  return launch_sample_resolve<kSampleGroup>(p, f, B, M, K, N, s);
+  return launch_sample_resolve<kSampleGroup, false>(p, f, B, M, K, N, s);
 }
 
 int run_sample(const elem_t* a, const elem_t* b, elem_t* out, int32_t* idx, float* stats,
@@ -921,7 +929,7 @@ int run_sample(const elem_t* a, const elem_t* b, elem_t* out, int32_t* idx, floa
     if (log_fwd_writes_factors(stats, B, M, K, N, &f)) {
       if (log_sample_mfma_ok(K)) {  // sweep on the matrix cores, groups of 16 terms
         if (int e = log_sample_sweep_mfma(a, b, out, idx, stats, seed, offset, B, M, K, N, s)) return e;
-        return launch_sample_resolve<16>(p, f, B, M, K, N, s);
+        return launch_sample_resolve<16, true>(p, f, B, M, K, N, s);
       }
       switch (pick_shape(B, M, N, false)) {
         case kWide: return launch_sweep_two<CfgWide>(p, stats, f, B, M, K, N, s);

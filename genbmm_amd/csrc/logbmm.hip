@@ -787,7 +787,7 @@ int launch_sample_sweep_mfma(DenseArgs p, const float* stats, int* flags, int B,
   const LogPrepared ws = prepared_of(stats, B, M, K, N);
   hipLaunchKernelGGL(k_sample_sweep_split<T>, dim3((unsigned)total), dim3(T::NT), 0, s, ws.ea, ws.eb,
                      p.out, stats, flags, ws.r, p.idx, p.seed, p.offset, M, K, N, tiles_m, tiles_n,
-                     TF::TR, TF::TC, p.tiles_m, p.tiles_n, ceil_div(K, kMS) <= 62 ? 63 : 127);
+                     TF::TR, TF::TC, p.tiles_m, p.tiles_n, log_sample_tag_mask(K));
   if (int e = launch_status()) return e;
   const int ftotal = B * p.tiles_m * p.tiles_n;
   hipLaunchKernelGGL((k_sample_fixup<CfgWide, TF::TR, TF::TC>), dim3(min(ftotal, kFixupGrid)),
@@ -1329,6 +1329,7 @@ int log_fwd_with_factors(const elem_t* a, const elem_t* b, elem_t* out, float* s
   return run_fwd(a, b, out, stats, B, M, K, N, GENBMM_PATH_AUTO, true, s, true);
 }
 
+int log_sample_tag_mask(int K) { return ceil_div(K, kMS) <= 62 ? 63 : 127; }
 bool log_sample_mfma_ok(int K) { return ceil_div(K, kMS) <= kSampleSlabs; }
 
 int log_sample_sweep_mfma(const elem_t* a, const elem_t* b, elem_t* out, int32_t* idx,

@@ -571,7 +571,7 @@ __device__ __forceinline__ void split_slab_rows(const unsigned* __restrict__ R, 
 // register per cell keeps, by a signed-integer minimum over (value with its low six bits
 // replaced by 62 - slab; seven bits and 126 - slab for more than 62 slabs: `tmask` = 63 or 127),
 // the slab in which the prefix sum passes t and -rem at the start of that slab.  S is the reciprocal of the forward's 1 / S, the targets are shrunk by 2^-22;
-// results: the code -2 - slab in idx, rem in `remw`.  The partial products are added in the
+// results: that register in idx (negative; its bits of rem and its tag are all that the resolve needs).  The partial products are added in the
 // forward's order, so the sums the sweep compares with its targets are the forward's.  A tile
 // with a cell whose S is below 2^-40 or not finite, or that lies in a tile the forward
 // flagged, sets that flag and leaves: the forward's tile is redone exactly.  128 x 128 tiles of
@@ -589,7 +589,7 @@ template <class T>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restrict__ ws_eb,
                           const elem_t* __restrict__ out, const float* __restrict__ stats,
-                          int* __restrict__ flags, float* __restrict__ remw, int32_t* __restrict__ idx,
+                          int* __restrict__ flags, const float* __restrict__ ws_r, int32_t* __restrict__ idx,
                           uint64_t seed, uint64_t offset, int M, int K, int N, int tiles_m, int tiles_n, int ftr,
                           int ftc, int ftiles_m, int ftiles_n, int tmask) {
   constexpr int NT = T::NT;
@@ -654,7 +654,7 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
     const bool blocks = (N & 3) == 0;
     float4 r4[16];
 #pragma unroll
-    for (int t = 0; t < 16; ++t) r4[t] = ld4(remw + cell0 + (long)min(m0 + wm0 + lr + 4 * t, M - 1) * N + nc);
+    for (int t = 0; t < 16; ++t) r4[t] = ld4(ws_r + cell0 + (long)min(m0 + wm0 + lr + 4 * t, M - 1) * N + nc);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -745,27 +745,21 @@ void k_sample_sweep_split(const float* __restrict__ ws_ea, const float* __restri
   multiply(slabs - 1);
   __syncthreads();  // every wave is done with the staged slabs
 
-  // ---- slab in which the prefix passes t, and rem at its start, row by row
+  // ---- the slab in which the prefix passes t, and rem at its start, row by row
   const int cc = clamp4(N - (n0 + wn0 + lc)), rows_left = M - (m0 + wm0) - lr;
-  const long ubase = cell0 + (long)(m0 + wm0) * N + n0 + wn0 + lr * N + lc;
-  floatx16 code[2][2];
+  float* dst = reinterpret_cast<float*>(idx) + cell0 + (long)(m0 + wm0) * N + n0 + wn0 + lr * N + lc;  // bit patterns
 #pragma unroll
   for (int x = 0; x < 4; ++x)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int v = low[x >> 1][x & 1][i], below = tmask - (v & tmask);
       // a target that the sums never reach lies within their rounding of the total: the last term
-      code[x >> 1][x & 1][i] = __int_as_float(below >= slabs ? K - 1 : -2 - below);
-      acc[x >> 1][x & 1][i] = -__int_as_float(v & ~tmask);
+      acc[x >> 1][x & 1][i] = __int_as_float(below >= slabs ? K - 1 : v);
     }
-  auto rows_to = [&](const floatx16 (&src)[2][2], float* dst) __attribute__((always_inline)) {
-    acc_rows(src, strip, lane, [](int) {}, [&](int q, int t, float4 v) __attribute__((always_inline)) {
-      const int ru = 16 * q + 4 * t;
-      if (cc > 0 && ru < rows_left) st4m(dst + ubase + (long)ru * N, cc, v);
-    });
-  };
-  rows_to(code, reinterpret_cast<float*>(idx));  // bit patterns
-  rows_to(acc, remw);
+  acc_rows(acc, strip, lane, [](int) {}, [&](int q, int t, float4 v) __attribute__((always_inline)) {
+    const int ru = 16 * q + 4 * t;
+    if (cc > 0 && ru < rows_left) st4m(dst + (long)ru * N, cc, v);
+  });
 }
 
 // ---------------------------------------------------------------- backward

@@ -33,10 +33,11 @@ int log_fwd_with_factors(const elem_t* a, const elem_t* b, elem_t* out, float* s
 bool log_fwd_writes_factors(const float* stats, int B, int M, int K, int N, LogFactors* f);
 
 // For a workspace that log_fwd_writes_factors() accepts: the sampling sweep on the
-// matrix cores.  Leaves in idx the code -2 - group (groups of 16 terms; K - 1, final: the
-// prefix sums never reach the target) and in the scratch array rem at the start of that
-// group; tiles that the forward or the sweep flagged are redone exactly (out and the
-// final index).  The caller resolves the codes.
+// matrix cores.  Leaves in idx -rem at the start of a group of 16 terms, its low bits (log_sample_tag_mask())
+// replaced by that mask minus the group's number - a negative integer - or K - 1, final: the
+// prefix sums never reach the target; tiles that the forward or the sweep flagged are redone exactly (out and the
+// final index).  The caller resolves what is negative.
+int log_sample_tag_mask(int K);
 bool log_sample_mfma_ok(int K);  // the sweep below takes reductions up to 126 slabs of 16 terms
 int log_sample_sweep_mfma(const elem_t* a, const elem_t* b, elem_t* out, int32_t* idx,
                           const float* stats, uint64_t seed, uint64_t offset, int B, int M, int K,
