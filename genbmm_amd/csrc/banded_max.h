@@ -152,10 +152,26 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : 2) void k_band_max_fwd
         // all 8 cells walk the union of their k ranges: where a cell has no such k it reads
         // -inf from between the rows
         const int klo = max(0, j0 - (Wb - 1)), khi = min(Wa - 1, j0 + 7);
-        auto fold2 = [&](int t, float a0, float a1, float b0, float b1, int k) __attribute__((always_inline)) {
-          const float m = __builtin_fmaxf(__builtin_fmaxf(val[s][t], a0 + b0), a1 + b1);
-          if (m > val[s][t]) ind[s][t] = k;
-          val[s][t] = m;
+        // four cells at a time: their compares, then their selects
+        auto fold4 = [&](int t, float a0, const float (&b0)[8], int k) __attribute__((always_inline)) {
+          const float v[4] = {a0 + b0[t], a0 + b0[t + 1], a0 + b0[t + 2], a0 + b0[t + 3]};
+          const Mask4 up(v[0] > val[s][t], v[1] > val[s][t + 1], v[2] > val[s][t + 2], v[3] > val[s][t + 3]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            val[s][t + q] = up[q] ? v[q] : val[s][t + q];
+            ind[s][t + q] = up[q] ? k : ind[s][t + q];
+          }
+        };
+        auto pairs4 = [&](int t, float a0, float a1, const float (&b0)[8], const float (&b1)[8], int k) __attribute__((always_inline)) {
+          float m[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) m[q] = __builtin_fmaxf(__builtin_fmaxf(val[s][t + q], a0 + b0[t + q]), a1 + b1[t + q]);
+          const Mask4 up(m[0] > val[s][t], m[1] > val[s][t + 1], m[2] > val[s][t + 2], m[3] > val[s][t + 3]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            ind[s][t + q] = up[q] ? k : ind[s][t + q];
+            val[s][t + q] = m[q];
+          }
         };
         int k = klo;
         for (; k + 3 <= khi; k += 4) {
@@ -169,12 +185,12 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : 2) void k_band_max_fwd
 #pragma unroll
           for (int u = 0; u < 4; u += 2)
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
+            for (int t = 0; t < 8; t += 4) {
               if (PAIRS) {
-                fold2(t, av[u], av[u + 1], bv[u][t], bv[u + 1][t], k + u);
+                pairs4(t, av[u], av[u + 1], bv[u], bv[u + 1], k + u);
               } else {
-                fold(t, av[u], bv[u][t], k + u);
-                fold(t, av[u + 1], bv[u + 1][t], k + u + 1);
+                fold4(t, av[u], bv[u], k + u);
+                fold4(t, av[u + 1], bv[u + 1], k + u + 1);
               }
             }
         }

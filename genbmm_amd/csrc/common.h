@@ -382,6 +382,19 @@ __device__ __forceinline__ void add4_ordered(float* __restrict__ accs, const int
   accs[s[3]] = v3;
 }
 
+// Four conditions for selects.  A compare writes its mask two wait states before a select may read it; left to
+// itself the compiler pairs the two on one mask register and idles between them - an issue slot per cell of a
+// walk that issue bounds.  Here the four compares come first, on masks of their own.
+struct Mask4 {
+  unsigned long long m[4];
+  __device__ __forceinline__ Mask4(bool c0, bool c1, bool c2, bool c3)
+      : m{__builtin_amdgcn_ballot_w64(c0), __builtin_amdgcn_ballot_w64(c1), __builtin_amdgcn_ballot_w64(c2),
+          __builtin_amdgcn_ballot_w64(c3)} {
+    asm("" : "+s"(m[0]), "+s"(m[1]), "+s"(m[2]), "+s"(m[3]));
+  }
+  __device__ __forceinline__ bool operator[](int i) const { return __builtin_amdgcn_inverse_ballot_w64(m[i]); }
+};
+
 // ------------------------------------------------------------- host helpers
 inline int check_dense_dims(int B, int M, int K, int N) {
   if (B < 0 || M < 0 || K < 0 || N < 0) return GENBMM_E_SHAPE;

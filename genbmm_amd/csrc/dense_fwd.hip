@@ -116,8 +116,12 @@ __global__ __launch_bounds__(C::NT) void k_max_fwd(const DenseArgs p) {
 #pragma unroll
       for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j)
-          if (mx[i][j] > before[i][j]) ind[i][j] = code;
+        for (int j = 0; j < C::TN; j += 4) {
+          const Mask4 up(mx[i][j] > before[i][j], mx[i][j + 1] > before[i][j + 1], mx[i][j + 2] > before[i][j + 2],
+                         mx[i][j + 3] > before[i][j + 3]);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) ind[i][j + q] = up[q] ? code : ind[i][j + q];
+        }
     }
   }
   // the values come with the indices from k_max_resolve; without terms there is none
