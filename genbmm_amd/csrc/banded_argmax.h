@@ -16,14 +16,16 @@
 // its cells in that order, accumulating in LDS at [k][lane]: whatever k each lane adds to, the 64 lanes
 // stay in 64 different banks, and no cell is shared, so there is no barrier.  grad_b's lanes, at one i,
 // take 64 adjacent cells of row i straight from memory; grad_a's cells pass through a tile of LDS (lanes
-// that read their own rows fetch a cache line for every 16 bytes: 220 us).  The next chunk is in flight
+// that read their own rows fetch a cache line for every 16 bytes: 220 us).  The next three chunks are in flight
 // while one is added, and no load stands under a branch: behind one the compiler waits for every load.
 // Both gradients are one launch, strip by strip, so that the second use of g and idx comes from a cache.
 //
-// Bound by the loads in flight and the ordered additions (add4_ordered: one LDS round trip per four
-// cells); g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each.  Measured there:
-// 255 us as two launches of four-wave workgroups that passed g and idx through LDS tiles behind two
-// barriers each, 175 us now (bfloat16 335 -> 137; 512 x 512, 17 diagonals 92 -> 45).
+// g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each: 180 -> 152 us there, 2.7 TB/s (behind a
+// forward, other buffers each time).  Of the 28, 7 are addresses and slots that no longer follow clamped rows (grad_b), the rest
+// pieces of four cells a load and a store (grad_a) and results that leave as one run instead of 32 diagonals at a time.
+// What it waits for now: timed in parts, 55 us are the walk over LDS without loads, additions and results; the ordered
+// additions (add4_ordered: one LDS round trip per four cells) and the loads then share two waves a SIMD, which LDS
+// bounds.  More loads in flight change nothing (the forward's lines are still being written back meanwhile).
 #pragma once
 
 #include "banded_cells.h"
@@ -32,9 +34,8 @@ namespace GENBMM_NS {
 
 constexpr int kArgRows = 64;  // rows per workgroup: the lanes
 constexpr int kArgKC = 128;   // diagonals per workgroup
-constexpr int kArgCh = 16;    // cells of a row (grad_a), rows (grad_b) per chunk
-constexpr int kArgTile = kArgCh + 1;   // grad_a's tile: floats per row
-constexpr int kArgSlots = kArgCh + 4;  // and bytes per row (odd strides in banks)
+constexpr int kArgCh = 16;    // cells of a row per chunk (grad_a)
+constexpr int kArgChB = 8;    // rows per chunk (grad_b)
 
 // diagonals of a gradient per workgroup, and the workgroups that all W of them take
 inline int argmax_kw(int W) { return min(W, kArgKC); }
@@ -42,12 +43,18 @@ inline int argmax_parts(int W) { return (W + kArgKC - 1) / kArgKC; }
 // the cells and one spare cell per lane (terms that are not the lane's); grad_a: the tile
 __host__ __device__ inline int argmax_cells(int kw) { return kArgRows * (kw + 1); }
 inline size_t argmax_bwd_bytes(int Wa, int Wb) {
-  return max(sizeof(float) * (argmax_cells(argmax_kw(Wa)) + kArgRows * kArgTile) + kArgRows * kArgSlots,
+  return max(sizeof(float) * (argmax_cells(argmax_kw(Wa)) + kArgRows * kArgCh) + kArgRows * kArgCh,
              sizeof(float) * (size_t)argmax_cells(argmax_kw(Wb)));
 }
 
+typedef int arg_i4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef elem_t arg_e4 __attribute__((ext_vector_type(4), aligned(sizeof(elem_t))));
+struct ArgRowChunk {  // four cells of each of four rows
+  arg_i4 i[4];
+  arg_e4 g[4];
+};
 struct ArgColChunk {  // one cell of each of CH rows
-  static constexpr int CH = kArgCh;
+  static constexpr int CH = kArgChB;
   int i[CH];
   elem_t g[CH];
 };
@@ -58,164 +65,234 @@ __device__ __forceinline__ void argmax_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// The lane's cells cleared, then `chunks` chunks: load(chunk, number), slots(chunk, number, slot, value)
+// The lane's cells cleared, then `chunks` chunks: load(chunk, number), slots(chunk, number, cells' numbers, values)
 template <class Chunk, class Load, class Slots>
 __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int kw, int chunks, Load load, Slots slots) {
   constexpr int CH = Chunk::CH;
   const int lane = threadIdx.x;
-  Chunk x, y;
+  Chunk v0, v1, v2, v3;  // loads three chunks ahead (48 of the 63 that a wave can wait for)
   auto add = [&](const Chunk& ch, int c) __attribute__((always_inline)) {
-    int sl[CH];
+    if (c >= chunks) return;  // uniform
+    unsigned kr[CH];
     float tv[CH];
-    slots(ch, c, sl, tv);
+    slots(ch, c, kr, tv);
 #pragma unroll
     for (int q = 0; q < CH; q += 4) {
-      const int s4[4] = {sl[q], sl[q + 1], sl[q + 2], sl[q + 3]};
+      const unsigned k4[4] = {kr[q], kr[q + 1], kr[q + 2], kr[q + 3]};
       const float t4[4] = {tv[q], tv[q + 1], tv[q + 2], tv[q + 3]};
-      add4_ordered(accs, s4, t4);
+      add4_ordered(accs + lane, k4, t4);
     }
   };
-  if (chunks > 0) load(x, 0);
+  const int last = chunks - 1;
+  if (chunks > 0) {
+    load(v0, 0);
+    load(v1, min(1, last));
+    load(v2, min(2, last));
+  }
 #pragma unroll 16
   for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
-  int c = 0;
-  for (; c + 1 < chunks; c += 2) {
-    load(y, c + 1);
-    add(x, c);
-    load(x, min(c + 2, chunks - 1));
-    add(y, c + 1);
+  for (int c = 0; c < chunks; c += 4) {
+    load(v3, min(c + 3, last));
+    add(v0, c);
+    load(v0, min(c + 4, last));
+    add(v1, c + 1);
+    load(v1, min(c + 5, last));
+    add(v2, c + 2);
+    load(v2, min(c + 6, last));
+    add(v3, c + 3);
   }
-  if (c < chunks) add(x, c);
 }
 
-// The sums leave as rows, 32 diagonals at a time: they change places in LDS, through registers, from
-// [k][lane] to [row][k] (32 whole diagonals: the k of a row permuted by its row number, which keeps both
-// sides clear of bank conflicts), and go to memory in runs along the band.
+// The sums leave as rows: they change places in LDS, through registers, from [k][lane] to [row][k], rows an odd number
+// of cells apart, and where a row has no other diagonals go to memory as the one run that they are there, 16 bytes a
+// lane.  (Runs of 32 diagonals, each in its own pass over the rows: a third of the kernel's time.)
 __device__ __forceinline__ void argmax_write_out(float* __restrict__ accs, int kw, elem_t* __restrict__ out, int W,
                                                  int rows) {
-  const int lane = threadIdx.x;
-  for (int k0 = 0; k0 < kw; k0 += 32) {
-    const int cw = min(32, kw - k0);
-    float* t = accs + k0 * kArgRows;
-    float v[32];
-    argmax_lds_sync();
+  const int lane = threadIdx.x, pitch = kw | 1;
+  float v[kArgKC];
+  argmax_lds_sync();
 #pragma unroll
-    for (int q = 0; q < 32; ++q) v[q] = t[min(q, cw) * kArgRows + lane];  // (row kw: the spare cells)
-    argmax_lds_sync();
-    if (cw == 32) {  // uniform
+  for (int k0 = 0; k0 < kArgKC; k0 += 32)
+    if (k0 < kw) {  // uniform
 #pragma unroll
-      for (int q = 0; q < 32; ++q) t[lane * 32 + (q ^ (lane & 31))] = v[q];
-      argmax_lds_sync();
-      const int c = lane & 31;
-#pragma unroll 8
-      for (int r = lane >> 5; r < rows; r += 2) out[(long)r * W + k0 + c] = to_elem<elem_t>(t[r * 32 + (c ^ (r & 31))]);
-    } else {
+      for (int q = k0; q < k0 + 32; ++q) v[q] = accs[min(q, kw - 1) * kArgRows + lane];
+    }
+  argmax_lds_sync();
 #pragma unroll
-      for (int q = 0; q < 32; ++q)
-        if (q < cw) t[lane * cw + q] = v[q];
-      argmax_lds_sync();
-      for (int e = lane; e < rows * cw; e += 64) {
-        const int r = e / cw, c = e - r * cw;
-        out[(long)r * W + k0 + c] = to_elem<elem_t>(t[e]);
+  for (int k0 = 0; k0 < kArgKC; k0 += 32)
+    if (k0 < kw) {
+#pragma unroll
+      for (int q = k0; q < k0 + 32; ++q) accs[lane * pitch + min(q, kw - 1)] = v[q];  // (beyond kw: the last again)
+    }
+  argmax_lds_sync();
+  const int cells = rows * kw;
+  // e < 2^13: e / kw = e inv / 2^32 (kw > 1).  Rows of even length have a gap behind each.
+  const unsigned inv = 0xffffffffu / (unsigned)kw + 1, gaps = (kw & 1) ? 0u : inv;
+  if (W == kw) {  // uniform
+    int e = 4 * lane;
+#pragma unroll 4
+    for (; e + 3 < cells; e += 256) {
+      float4 x;
+      if (kw & 1) {  // uniform
+        x = *reinterpret_cast<const float4*>(accs + e);
+      } else {
+        const int r = (int)__umulhi(e, gaps), c = e - r * kw;
+        const float* s = accs + e + r;
+        x = make_float4(s[0], s[1 + (c + 1 >= kw)], s[2 + (c + 2 >= kw)], s[3 + (c + 3 >= kw)]);
       }
+      arg_e4 y;
+      y[0] = to_elem<elem_t>(x.x); y[1] = to_elem<elem_t>(x.y); y[2] = to_elem<elem_t>(x.z); y[3] = to_elem<elem_t>(x.w);
+      *reinterpret_cast<arg_e4*>(out + e) = y;
+    }
+    for (int t = (cells & ~3) + lane; t < cells; t += 64) out[t] = to_elem<elem_t>(accs[t + (int)__umulhi(t, gaps)]);
+  } else {
+    for (int e = lane; e < cells; e += 64) {
+      const int r = kw == 1 ? e : (int)__umulhi(e, inv);
+      out[(long)r * W + e - r * kw] = to_elem<elem_t>(accs[r * pitch + e - r * kw]);
     }
   }
 }
 
-// grad_a, rows [i0, i0 + 64), diagonals [w0, w0 + kw).  Sixteen cells of four rows per load; their terms
-// and the slots they go to (a byte: kw <= 128 marks the spare) change places to the lane of their row
-// through a tile of LDS.
+// grad_a, rows [i0, i0 + 64), diagonals [w0, w0 + kw).  A lane loads four cells of a row, four lanes the sixteen
+// of a chunk; their terms and the cells they go to (a byte: kw <= 128 marks the spare) change places to the
+// lane of their row through a tile of LDS (pieces of four turned by their row: sixteen lanes meet all banks either
+// way).  Loads three chunks ahead.  NARROW: rows shorter than a chunk, read cell by cell.
+template <bool NARROW>
 __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const BandArgs& p, int batch, int i0, int w0) {
   const int n = p.n, Wa = p.Wa, Wb = p.Wb, Wo = p.Wo, lane = threadIdx.x;
   const int kw = min(kArgKC, Wa - w0);
-  float* gt = accs + argmax_cells(kw);
-  unsigned char* st = reinterpret_cast<unsigned char*>(gt + kArgRows * kArgTile);
+  float* const gt = accs + argmax_cells(kw);
+  unsigned* const st = reinterpret_cast<unsigned*>(gt + kArgRows * kArgCh);
   const int jlo = w0, jhi = min(w0 + kw - 1 + Wb - 1, Wo - 1);  // cells with a term on these diagonals
-  const int lr = lane >> 4, lj = lane & 15;
+  const int lr = lane >> 2, lq = lane & 3;
   const long base = ((long)batch * n + i0) * Wo;
   const elem_t* gb = p.g + base;
   const int32_t* ib = p.idx + base;
   const int last = n - 1 - i0;  // rows behind the matrix re-read its last row (nothing of them is stored)
-  elem_t gv[kArgCh];
-  int iv[kArgCh];
-  unsigned ro[kArgCh];
+  // every cell of the strip inside the matrix: o = i + j - r_lu in [0, n)
+  const bool inner = i0 >= p.r_lu && (long)i0 + kArgRows - 1 + Wo - 1 - p.r_lu < n;
+  ArgRowChunk x, y, z;
+  long row[4];
 #pragma unroll
-  for (int u = 0; u < kArgCh; ++u) ro[u] = (unsigned)(min(4 * u + lr, last) * Wo + min(lj, Wo - 1));
+  for (int u = 0; u < 4; ++u) row[u] = (long)min(16 * u + lr, last) * Wo + (NARROW ? 0 : 4 * lq);
   // the last chunk of a row starts inside the row, the cells that the chunk before it held are masked
   auto start = [&](int j0) __attribute__((always_inline)) { return max(min(j0, Wo - kArgCh), 0); };
-  auto load = [&](int j0) __attribute__((always_inline)) {
+  auto load = [&](ArgRowChunk& v, int j0) __attribute__((always_inline)) {
     const elem_t* gs = gb + start(j0);
     const int32_t* is = ib + start(j0);
 #pragma unroll
-    for (int u = 0; u < kArgCh; ++u) {
-      gv[u] = gs[ro[u]];
-      iv[u] = is[ro[u]];
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (NARROW) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = min(4 * lq + e, Wo - 1);
+          v.g[u][e] = gs[row[u] + j];
+          v.i[u][e] = is[row[u] + j];
+        }
+      } else {
+        v.g[u] = *reinterpret_cast<const arg_e4*>(gs + row[u]);
+        v.i[u] = *reinterpret_cast<const arg_i4*>(is + row[u]);
+      }
     }
   };
-  load(jlo);
-#pragma unroll 16
-  for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
-  for (int j0 = jlo; j0 <= jhi; j0 += kArgCh) {
+  float4* const gput = reinterpret_cast<float4*>(gt) + lr * 4 + (lq ^ (lr & 3));  // (16 u keeps the turn)
+  const float4* const gget = reinterpret_cast<const float4*>(gt) + lane * 4;
+  auto stage = [&](const ArgRowChunk& v, int j0) __attribute__((always_inline)) {
     argmax_lds_sync();  // the tile has been read
-    const int j = start(j0) + lj, o = i0 + lr + j - p.r_lu;
-    const unsigned lim = j >= j0 && j <= jhi ? n : 0;  // inside the matrix: o = i + j - r_lu in [0, n)
+    const bool whole = inner && j0 + kArgCh <= Wo && j0 + kArgCh - 1 <= jhi;  // uniform: sixteen new cells of every row
+    const int j = start(j0) + 4 * lq, o = i0 + lr + j - p.r_lu;
 #pragma unroll
-    for (int u = 0; u < kArgCh; ++u) {
-      const unsigned kr = (unsigned)(iv[u] - w0);
-      const bool ok = kr < (unsigned)kw && (unsigned)(o + 4 * u) < lim;
-      gt[(4 * u + lr) * kArgTile + lj] = (float)gv[u];
-      st[(4 * u + lr) * kArgSlots + lj] = (unsigned char)(ok ? kr : kw);
+    for (int u = 0; u < 4; ++u) {
+      gput[64 * u] = make_float4((float)v.g[u][0], (float)v.g[u][1], (float)v.g[u][2], (float)v.g[u][3]);
+      unsigned k[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) k[e] = min((unsigned)(v.i[u][e] - w0), (unsigned)kw);
+      if (!whole) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned lim = j + e >= j0 && j + e <= jhi ? n : 0;
+          k[e] = (unsigned)(o + 16 * u + e) < lim ? k[e] : kw;
+        }
+      }
+      st[64 * u + lane] = k[0] | k[1] << 8 | k[2] << 16 | k[3] << 24;
     }
     argmax_lds_sync();
-    load(j0 + kArgCh);  // (past the band: the row's last cells again)
-    float tv[kArgCh];
-    unsigned sw[kArgCh / 4];
+  };
+  auto add = [&]() __attribute__((always_inline)) {
+    float4 t[4];
 #pragma unroll
-    for (int q = 0; q < kArgCh; ++q) tv[q] = gt[lane * kArgTile + q];
+    for (int q = 0; q < 4; ++q) t[q] = gget[q ^ (lane & 3)];
+    const uint4 w4 = reinterpret_cast<const uint4*>(st)[lane];
+    const unsigned w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
-    for (int q = 0; q < kArgCh / 4; ++q) sw[q] = *reinterpret_cast<const unsigned*>(st + lane * kArgSlots + 4 * q);
-#pragma unroll
-    for (int q = 0; q < kArgCh; q += 4) {
-      const unsigned w = sw[q >> 2];
-      const int s4[4] = {(int)(w & 255) * kArgRows + lane, (int)(w >> 8 & 255) * kArgRows + lane,
-                         (int)(w >> 16 & 255) * kArgRows + lane, (int)(w >> 24) * kArgRows + lane};
-      const float t4[4] = {tv[q], tv[q + 1], tv[q + 2], tv[q + 3]};
-      add4_ordered(accs, s4, t4);
+    for (int q = 0; q < 4; ++q) {
+      const unsigned k4[4] = {w[q] & 255, w[q] >> 8 & 255, w[q] >> 16 & 255, w[q] >> 24};
+      const float t4[4] = {t[q].x, t[q].y, t[q].z, t[q].w};
+      add4_ordered(accs + lane, k4, t4);
     }
+  };
+  // (a chunk past the band asks for its row's last cells again)
+  auto turn = [&](ArgRowChunk& v, int j0) __attribute__((always_inline)) {
+    if (j0 <= jhi) stage(v, j0);  // uniform
+    load(v, j0 + 3 * kArgCh);
+    if (j0 <= jhi) add();
+  };
+  // (in this order, as the loop's: the waits for x in its first turn are those of every turn)
+  load(x, jlo);
+  __builtin_amdgcn_sched_barrier(0);
+  load(y, jlo + kArgCh);
+  __builtin_amdgcn_sched_barrier(0);
+  load(z, jlo + 2 * kArgCh);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 16
+  for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
+  for (int j0 = jlo; j0 <= jhi; j0 += 3 * kArgCh) {
+    turn(x, j0);
+    turn(y, j0 + kArgCh);
+    turn(z, j0 + 2 * kArgCh);
   }
   argmax_write_out(accs, kw, p.o0 + ((long)batch * n + i0) * Wa + w0, Wa, min(kArgRows, n - i0));
 }
 
-// grad_b, rows [o0, o0 + 64), diagonals [w0, w0 + kw)
+// grad_b, rows [o0, o0 + 64), diagonals [w0, w0 + kw).  A lane's cell of row i is j = o - i + r_lu, one less a row
+// further down: in memory row i + 1's lies Wo - 1 cells behind row i's for every lane, so a chunk's addresses are
+// a base and offsets that never change.  A lane whose j lies outside the row reads a cell of a row t before or
+// behind; k2 of that cell, in [0, Wb) or none, is t Wo away from what its index says for this lane, and Wo >= Wb.
+// (Formed from clamped j and row numbers, addresses and slots took 25 of a cell's 34 instructions, now 8 of 17.)
 __device__ __forceinline__ void argmax_band_b(float* __restrict__ accs, const BandArgs& p, int batch, int o0, int w0) {
+  constexpr int ES = sizeof(elem_t);
   const int n = p.n, Wa = p.Wa, Wb = p.Wb, Wo = p.Wo, lane = threadIdx.x;
-  const int kw = min(kArgKC, Wb - w0), spare = kw * kArgRows + lane;
+  const int kw = min(kArgKC, Wb - w0);
   const elem_t* gb = p.g + (long)batch * n * Wo;
   const int32_t* ib = p.idx + (long)batch * n * Wo;
   // cells with a term on these diagonals, and the rows i that hold them for some lane
   const int jlo = max(0, Wb - w0 - kw), jhi = min(Wo - 1, Wa + Wb - 2 - w0);
   const int ilo = max(0, o0 + p.r_lu - jhi), ihi = min(n - 1, o0 + kArgRows - 1 + p.r_lu - jlo);
   const int jof = o0 + lane + p.r_lu;  // j = jof - i
-  argmax_walk<ArgColChunk>(
-      accs, kw, ihi < ilo ? 0 : (ihi - ilo + kArgCh) / kArgCh,
-      [&](ArgColChunk& x, int c) __attribute__((always_inline)) {
+  const int rows = Wo < (1 << 25) ? kArgChB : 1;  // of a chunk: its offsets fit 32 bits (cells behind them read as 0)
+  int off[kArgChB];
 #pragma unroll
-        for (int q = 0; q < kArgCh; ++q) {
-          const int i = min(ilo + c * kArgCh + q, ihi);  // uniform
-          const unsigned j = (unsigned)min(max(jof - i, 0), Wo - 1);
-          x.i[q] = (ib + (long)i * Wo)[j];
-          x.g[q] = (gb + (long)i * Wo)[j];
+  for (int q = 0; q < kArgChB; ++q) off[q] = q < rows ? lane + q * (Wo - 1) : -16;
+  argmax_walk<ArgColChunk>(
+      accs, kw, ihi < ilo ? 0 : (ihi - ilo + rows) / rows,
+      [&](ArgColChunk& x, int c) __attribute__((always_inline)) {
+        // lane 0's cell of the chunk's first row; the buffers end with the item
+        const long first = (long)(ilo + c * rows) * (Wo - 1) + (o0 + p.r_lu);
+        const unsigned left = (unsigned)min((long)n * Wo - first, 1L << 29);
+        const buf_t bi = buf_of(ib + first, left * 4), bg = buf_of(gb + first, left * ES);
+#pragma unroll
+        for (int q = 0; q < kArgChB; ++q) {
+          x.i[q] = buf_ld<int32_t>(bi, off[q] * 4, 0);
+          x.g[q] = buf_ld<elem_t>(bg, off[q] * ES, 0);
         }
       },
-      [&](const ArgColChunk& x, int c, int (&sl)[kArgCh], float (&tv)[kArgCh]) __attribute__((always_inline)) {
+      [&](const ArgColChunk& x, int c, unsigned (&kr)[kArgChB], float (&tv)[kArgChB]) __attribute__((always_inline)) {
+        const unsigned at = (unsigned)(Wb - 1 - w0 + ilo + c * rows) - (unsigned)jof;
 #pragma unroll
-        for (int q = 0; q < kArgCh; ++q) {
+        for (int q = 0; q < kArgChB; ++q) {
           // An index is a k of its cell, 0 (a cell outside the matrix) or -1 (no term; becomes far too
-          // large).  Where j was clamped it is 0 or at most Wa - 1, and k2 falls outside [0, Wb) by itself.
-          const int i = ilo + c * kArgCh + q;
-          const unsigned kr = ((unsigned)x.i[q] & 0x7fffffffu) + (unsigned)(Wb - 1 - w0 + i) - (unsigned)jof;
-          const unsigned lim = i <= ihi ? kw : 0;  // uniform
-          sl[q] = kr < lim ? (int)kr * kArgRows + lane : spare;
+          // large).  What lies behind the item reads as 0, a term of 0 wherever it falls.
+          kr[q] = min(((unsigned)x.i[q] & 0x7fffffffu) + (at + q), (unsigned)kw);  // kw: the spare cells
           tv[q] = (float)x.g[q];
         }
       });
@@ -227,7 +304,8 @@ __global__ __launch_bounds__(64) void k_band_argmax_bwd(const BandArgs p, int st
   const int parts = parts_a + parts_b, wg = xcd_renumber(blockIdx.x, gridDim.x);
   const int strip = wg / parts, part = wg - strip * parts;
   const int batch = strip / strips, r0 = (strip - batch * strips) * kArgRows;
-  if (part < parts_a) argmax_band_a(accs, p, batch, r0, part * kArgKC);
+  if (part < parts_a && p.Wo >= kArgCh) argmax_band_a<false>(accs, p, batch, r0, part * kArgKC);
+  else if (part < parts_a) argmax_band_a<true>(accs, p, batch, r0, part * kArgKC);
   else argmax_band_b(accs, p, batch, r0, (part - parts_a) * kArgKC);
 }
 

@@ -368,18 +368,19 @@ __device__ __forceinline__ int xcd_renumber(int w, int n) {
 // Four ordered additions with one LDS round trip: the four cells are read together,
 // the sums are chained in registers (a cell that was already hit earlier in the group
 // takes that sum instead of what it read), and written back in order.  A term whose k
-// is not this lane's goes to the lane's spare cell.
-__device__ __forceinline__ void add4_ordered(float* __restrict__ accs, const int (&s)[4],
-                                             const float (&v)[4]) {
-  const float r0 = accs[s[0]], r1 = accs[s[1]], r2 = accs[s[2]], r3 = accs[s[3]];
+// is not this lane's goes to the lane's spare cell.  Cell k lies at cells[64 k] (the numbers are compared, not the
+// addresses, which would each be formed twice).
+__device__ __forceinline__ void add4_ordered(float* cells, const unsigned (&k)[4], const float (&v)[4]) {
+  float *const p0 = cells + 64 * k[0], *const p1 = cells + 64 * k[1], *const p2 = cells + 64 * k[2], *const p3 = cells + 64 * k[3];
+  const float r0 = *p0, r1 = *p1, r2 = *p2, r3 = *p3;
   const float v0 = __fadd_rn(r0, v[0]);
-  const float v1 = __fadd_rn(s[1] == s[0] ? v0 : r1, v[1]);
-  const float v2 = __fadd_rn(s[2] == s[1] ? v1 : (s[2] == s[0] ? v0 : r2), v[2]);
-  const float v3 = __fadd_rn(s[3] == s[2] ? v2 : (s[3] == s[1] ? v1 : (s[3] == s[0] ? v0 : r3)), v[3]);
-  accs[s[0]] = v0;
-  accs[s[1]] = v1;
-  accs[s[2]] = v2;
-  accs[s[3]] = v3;
+  const float v1 = __fadd_rn(k[1] == k[0] ? v0 : r1, v[1]);
+  const float v2 = __fadd_rn(k[2] == k[1] ? v1 : (k[2] == k[0] ? v0 : r2), v[2]);
+  const float v3 = __fadd_rn(k[3] == k[2] ? v2 : (k[3] == k[1] ? v1 : (k[3] == k[0] ? v0 : r3)), v[3]);
+  *p0 = v0;
+  *p1 = v1;
+  *p2 = v2;
+  *p3 = v3;
 }
 
 // Four conditions for selects.  A compare writes its mask two wait states before a select may read it; left to

@@ -125,28 +125,28 @@ template <int PROD, int KC, class Chunk, class Other>
 __device__ __forceinline__ void argmax_add(float* __restrict__ accs, const Chunk& x, int c0, int kc, Other other) {
   constexpr int CH = Chunk::CH;
   const int lane = threadIdx.x;
-  int sl[CH];
+  unsigned kr[CH];
   float tv[CH];
 #pragma unroll
   for (int q = 0; q < CH; ++q) {
     if constexpr (PROD == 2) {
       const int k = x.iv(q) - c0;
-      sl[q] = (k >= 0 && k < kc ? k : KC) * 64 + lane;  // [KC]: the spare cells
+      kr[q] = k >= 0 && k < kc ? k : KC;  // [KC]: the spare cells
       tv[q] = __fmul_rn(x.fv(q), x.gv(q));
     } else {
       // the lane's cell, or its spare one: an index below the part wraps around, one of K or beyond (none that the
       // library writes) may fall to a cell of the last part that is not written out.  Its factor does not exist.
       const unsigned k = min((unsigned)x.iv(q) - (unsigned)c0, (unsigned)KC);
-      sl[q] = k * 64 + lane;
+      kr[q] = k;
       tv[q] = x.gv(q);
       if (PROD == 1 && (int)k < kc) tv[q] = __fmul_rn(other(q, x.iv(q)), tv[q]);
     }
   }
 #pragma unroll
   for (int q = 0; q < CH; q += 4) {
-    const int s4[4] = {sl[q], sl[q + 1], sl[q + 2], sl[q + 3]};
+    const unsigned k4[4] = {kr[q], kr[q + 1], kr[q + 2], kr[q + 3]};
     const float t4[4] = {tv[q], tv[q + 1], tv[q + 2], tv[q + 3]};
-    add4_ordered(accs, s4, t4);
+    add4_ordered(accs + lane, k4, t4);
   }
 }
 
