@@ -16,16 +16,17 @@
 // its cells in that order, accumulating in LDS at [k][lane]: whatever k each lane adds to, the 64 lanes
 // stay in 64 different banks, and no cell is shared, so there is no barrier.  grad_b's lanes, at one i,
 // take 64 adjacent cells of row i straight from memory; grad_a's cells pass through a tile of LDS (lanes
-// that read their own rows fetch a cache line for every 16 bytes: 220 us).  The next three chunks are in flight
+// that read their own rows fetch a cache line for every 16 bytes: 220 us).  The next chunks are in flight
 // while one is added, and no load stands under a branch: behind one the compiler waits for every load.
 // Both gradients are one launch, strip by strip, so that the second use of g and idx comes from a cache.
 //
-// g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each: 180 -> 152 us there, 2.7 TB/s (behind a
-// forward, other buffers each time).  Of the 28, 7 are addresses and slots that no longer follow clamped rows (grad_b), the rest
+// g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each: 180 -> 149 us there, 2.7 TB/s (behind a
+// forward, as a step runs them).  Of the 31, 7 are addresses and slots that no longer follow clamped rows (grad_b), the rest
 // pieces of four cells a load and a store (grad_a) and results that leave as one run instead of 32 diagonals at a time.
 // What it waits for now: timed in parts, 55 us are the walk over LDS without loads, additions and results; the ordered
 // additions (add4_ordered: one LDS round trip per four cells) and the loads then share two waves a SIMD, which LDS
-// bounds.  More loads in flight change nothing (the forward's lines are still being written back meanwhile).
+// bounds.  More loads in flight change nothing; chunks of 8 cells in grad_a, whose tile would leave room for an eighth wave on
+// a compute unit, 172 us, of 32 185 (five waves); of 8 rows in grad_b 153, of 4 about 10 more.
 #pragma once
 
 #include "banded_cells.h"
@@ -35,7 +36,7 @@ namespace GENBMM_NS {
 constexpr int kArgRows = 64;  // rows per workgroup: the lanes
 constexpr int kArgKC = 128;   // diagonals per workgroup
 constexpr int kArgCh = 16;    // cells of a row per chunk (grad_a)
-constexpr int kArgChB = 8;    // rows per chunk (grad_b)
+constexpr int kArgChB = 16;   // rows per chunk (grad_b)
 
 // diagonals of a gradient per workgroup, and the workgroups that all W of them take
 inline int argmax_kw(int W) { return min(W, kArgKC); }
@@ -70,7 +71,7 @@ template <class Chunk, class Load, class Slots>
 __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int kw, int chunks, Load load, Slots slots) {
   constexpr int CH = Chunk::CH;
   const int lane = threadIdx.x;
-  Chunk v0, v1, v2, v3;  // loads three chunks ahead (48 of the 63 that a wave can wait for)
+  Chunk v0, v1, v2, v3;  // loads ahead as far as the 63 that a wave can wait for reach
   auto add = [&](const Chunk& ch, int c) __attribute__((always_inline)) {
     if (c >= chunks) return;  // uniform
     unsigned kr[CH];
@@ -195,7 +196,7 @@ __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const Ba
       }
     }
   };
-  float4* const gput = reinterpret_cast<float4*>(gt) + lr * 4 + (lq ^ (lr & 3));  // (16 u keeps the turn)
+  float4* const gput = reinterpret_cast<float4*>(gt) + lr * 4 + (lq ^ (lr >> 2 & 3));  // (16 u keeps the turn)
   const float4* const gget = reinterpret_cast<const float4*>(gt) + lane * 4;
   auto stage = [&](const ArgRowChunk& v, int j0) __attribute__((always_inline)) {
     argmax_lds_sync();  // the tile has been read
@@ -221,7 +222,7 @@ __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const Ba
   auto add = [&]() __attribute__((always_inline)) {
     float4 t[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) t[q] = gget[q ^ (lane & 3)];
+    for (int q = 0; q < 4; ++q) t[q] = gget[q ^ (lane >> 2 & 3)];
     const uint4 w4 = reinterpret_cast<const uint4*>(st)[lane];
     const unsigned w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
