@@ -1029,7 +1029,9 @@ inline int bwd_split_kind(int B, int M, int K, int N) {
 // vector ALU or an item in a workgroup: those read maxima and `out`.
 inline int recip_keeps(int B, int M, int K, int N) {
   if (item_shape(M, K, N) || self_shape(M, K, N) || fwd_kind(GENBMM_PATH_AUTO, B, M, K, N) == 0) return kKeepNone;
-  if (bwd_split_kind(B, M, K, N) != 0) return kKeepRecip;
+  // (gradients on narrow extents read maxima and `out` too: a forward of such a shape has no room for 1 / S)
+  if (bwd_split_kind(B, M, K, N) != 0)
+    return fwd_mfma_shape(B, M, K, N) && mfma_extents(M, K, N) && mfma_extents(K, N, M) ? kKeepRecip : kKeepNone;
   if (!fwd_mfma_shape(B, M, K, N)) return kKeepNone;
   const int ka = mfma_kind(GENBMM_PATH_AUTO, B, M, K, N, true), kb = mfma_kind(GENBMM_PATH_AUTO, B, K, N, M, false);
   return ka != 0 || kb != 0 ? kKeepFactors : kKeepNone;

@@ -160,9 +160,9 @@ size_t genbmm_samplebmm_stats_size(int B, int M, int K, int N);
  *                      float16 / bfloat16 tensors want, whose `out` is stored
  *                      rounded (4 bytes per result cell).  Items too large for
  *                      the bf16 instruction's backward keep all three factors
- *                      and take FACTORS's; items of one workgroup and gradients
- *                      on the vector ALU keep nothing and weigh by
- *                      exp(max - out).
+ *                      and take FACTORS's; items of one workgroup, extents below 96
+ *                      and gradients on the vector ALU keep nothing and weigh
+ *                      by exp(max - out).
  *                      One gradient alone (the other pointer NULL) is formed
  *                      from `out`.
  * Any other value: GENBMM_E_MODE.  Forward and backward of one problem need not
