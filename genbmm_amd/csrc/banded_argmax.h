@@ -238,6 +238,15 @@ __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const Ba
     load(v, j0 + 3 * kArgCh);
     if (j0 <= jhi) add();
   };
+  if constexpr (NARROW) {  // one chunk
+    load(x, 0);
+#pragma unroll 16
+    for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
+    stage(x, 0);
+    add();
+    argmax_write_out(accs, kw, p.o0 + ((long)batch * n + i0) * Wa + w0, Wa, min(kArgRows, n - i0));
+    return;
+  }
   // (in this order, as the loop's: the waits for x in its first turn are those of every turn)
   load(x, jlo);
   __builtin_amdgcn_sched_barrier(0);
