@@ -1075,6 +1075,16 @@ void launch_item_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats
   if (H > 1) allow_lds(k_log_item_fwd<W, U, H>, lds);
   hipLaunchKernelGGL((k_log_item_fwd<W, U, H>), dim3(B), dim3(64 * W), lds, s, a, b, out, stats, hdr, M, K, N);
 }
+// (half types sweep only on the factors of larger extents)
+inline void launch_item_seq(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int* hdr, int B, int M, int K,
+                            int N, hipStream_t s) {
+  if constexpr (kElemF32) {
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(B), dim3(256), 0, s, a, b, out, stats, hdr, M, K, N); };
+    if (M == 64 && K == 64 && N == 64) go(k_log_item_seq<16, 4, true>);
+    else if (max(max(M, K), N) <= 32) go(k_log_item_seq<16, 2, false>);
+    else go(k_log_item_seq<16, 4, false>);
+  }
+}
 template <int W, int U, int H>
 void launch_item_bwd(const elem_t* a, const elem_t* b, const elem_t* out, const elem_t* g, elem_t* grad_a, elem_t* grad_b,
                      int B, int M, int K, int N, hipStream_t s) {
@@ -1149,11 +1159,13 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
   if (path == GENBMM_PATH_RECIP) keep = recip_keeps(B, M, K, N);
   if (keep == kKeepFactors && (!fwd_mfma_shape(B, M, K, N) || (!factors && item_shape(M, K, N))))
     keep = kKeepNone;  // (the workspace has no room for them)
-  if (stats && B > 0 && item_shape(M, K, N) && auto_path(path) && !(factors && keep == kKeepFactors)) {  // whole items per workgroup
+  const int most = max(max(M, K), N);
+  // whole items per workgroup; beyond 64 the sampling sweep's forward is one of the tiled ones
+  if (stats && B > 0 && item_shape(M, K, N) && auto_path(path) && !(factors && most > 64)) {
     int* hdr = prepared_of(stats, B, M, K, N).hdr;
-    const int most = max(max(M, K), N);
     if (M == 32 && K == 32 && N == 32)  // one wave per item on the matrix cores
       hipLaunchKernelGGL(k_log_item32_fwd, dim3((B + 3) / 4), dim3(256), 0, s, a, b, out, stats, hdr, B);
+    else if (kElemF32 && factors) launch_item_seq(a, b, out, stats, hdr, B, M, K, N, s);
     else if (most <= 32) launch_item_fwd<4, 2, 1>(a, b, out, stats, hdr, B, M, K, N, s);
     else if (most <= 48) launch_item_fwd<4, 3, 1>(a, b, out, stats, hdr, B, M, K, N, s);
     else if (most <= 64) launch_item_fwd<4, 4, 1>(a, b, out, stats, hdr, B, M, K, N, s);
@@ -1175,7 +1187,9 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
   }
   if (stats && K > 0 && path != GENBMM_PATH_EXACT) {
     const int64_t big_tiles = (int64_t)B * ceil_div(M, 128) * ceil_div(N, 128);
-    switch (fwd_kind(path, B, M, K, N)) {
+    // (the sampling sweep on narrow extents: the vector ALU's sums in the order of k, see k_log_item_seq)
+    const bool tiled = !factors || fwd_mfma_shape(B, M, K, N);
+    switch (tiled ? fwd_kind(path, B, M, K, N) : 0) {
       case 2:
         if (split_path(path)) {
           if (split_big_fits(B, M, N)) return launch_fwd_split<MTBig>(p, stats, B, M, K, N, keep, s);

@@ -458,4 +458,141 @@ __global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restric
   }
 }
 
+// ---------------------------------------------------------------- samplebmm's forward, extents of at most 64
+// The vector-ALU sweep forms its targets from S = exp(out - alpha - beta), so the draws of a pinned (seed, offset)
+// follow the last bit of `out`.  The sums of this forward are taken in the order of k, the one that those draws are
+// defined by (in k_log_item_fwd's order one draw in some 10^5 moves to a neighbouring term); (2048,64^3) 44 us against
+// 33 there.  TB x TB outputs per thread on a G x G thread grid, G = 16: TB = 2 covers items up to 32 x 32, TB = 4 up
+// to 64 x 64.  FULL: M = K = N = G * TB, known to the compiler, whose index arithmetic is most of the instructions.
+// (row, column) of elements tid, tid + nt, tid + 2 nt, ... of a row-major array
+// with C columns, without a division per element.
+struct RowMajorWalk {
+  int r, c, dr, dc, C;
+  __device__ __forceinline__ RowMajorWalk(int tid, int nt, int cols) : C(cols) {
+    r = tid / C;
+    c = tid - r * C;
+    dr = nt / C;
+    dc = nt - dr * C;
+  }
+  __device__ __forceinline__ void next() {
+    r += dr;
+    c += dc;
+    if (c >= C) {
+      c -= C;
+      ++r;
+    }
+  }
+};
+
+template <int G, int TB, bool FULL = false>
+__global__ __launch_bounds__(G * G, TB == 2 ? 8 : 1) void k_log_item_seq(const elem_t* __restrict__ a,
+                                                      const elem_t* __restrict__ b,
+                                                      elem_t* __restrict__ out,
+                                                      float* __restrict__ stats,
+                                                      int* __restrict__ hdr, int M_, int K_,
+                                                      int N_) {
+  constexpr int NT = G * G, S = G * TB, LD = S + 1;
+  const int M = FULL ? S : M_, K = FULL ? S : K_, N = FULL ? S : N_;
+  static_assert(2 * S <= NT, "row and column scans use 2*S threads");
+  if (hdr && blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = kWsNone;  // no per-tile flags in this workspace
+  __shared__ float At[S * LD];  // [k][m]: a, then EA; finally the output tile [m][n]
+  __shared__ float Bs[S * LD];  // [k][n]: b, then EB
+  __shared__ float al[S], be[S];
+  const int tid = threadIdx.x, batch = blockIdx.x;
+  const elem_t* ab = a + (long)batch * M * K;
+  const elem_t* bb = b + (long)batch * K * N;
+  // All reads of the item are issued before the first one is waited for (a thread owns
+  // elements tid, tid + NT, ... of each operand): one trip to memory, not one per element.
+  constexpr int PER = TB * TB;  // S * S / NT
+  float ra[PER], rb[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = tid + u * NT;
+    ra[u] = e < M * K ? ab[e] : 0.f;
+    rb[u] = e < K * N ? bb[e] : 0.f;
+  }
+  {
+    RowMajorWalk w(tid, NT, K);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if (w.r < M) At[w.c * LD + w.r] = ra[u];
+      w.next();
+    }
+  }
+  {
+    RowMajorWalk w(tid, NT, N);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if (w.r < K) Bs[w.r * LD + w.c] = rb[u];
+      w.next();
+    }
+  }
+  __syncthreads();
+  // row / column maxima: one thread per row, one per column (LDS atomics on the
+  // shared maximum while loading measured slower: 32 lanes on one address)
+  if (tid < M) {
+    float mx = -INFINITY;
+    for (int k = 0; k < K; ++k) mx = fmaxf(mx, At[k * LD + tid]);
+    al[tid] = mx;
+  } else if (tid >= S && tid - S < N) {
+    float mx = -INFINITY;
+    for (int k = 0; k < K; ++k) mx = fmaxf(mx, Bs[k * LD + tid - S]);
+    be[tid - S] = mx;
+  }
+  __syncthreads();
+  for (RowMajorWalk w(tid, NT, K); w.r < M; w.next()) {
+    const int m = w.r, k = w.c;
+    At[k * LD + m] = item_exp(At[k * LD + m], al[m]);
+  }
+  for (RowMajorWalk w(tid, NT, N); w.r < K; w.next()) {
+    const int k = w.r, n = w.c, e = w.r * N + w.c;
+    Bs[k * LD + n] = item_exp(Bs[k * LD + n], be[n]);
+  }
+  if (stats) {
+    float* st = stats + (long)batch * (M + N);
+    if (tid < M) st[tid] = al[tid];
+    else if (tid >= S && tid - S < N) st[M + tid - S] = be[tid - S];
+  }
+  __syncthreads();
+
+  const int ty = tid / G, tx = tid % G;
+  float acc[TB][TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) acc[i][j] = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < K; ++k) {
+    float av[TB], bv[TB];
+#pragma unroll
+    for (int i = 0; i < TB; ++i) av[i] = At[k * LD + ty * TB + i];
+#pragma unroll
+    for (int j = 0; j < TB; ++j) bv[j] = Bs[k * LD + tx * TB + j];
+#pragma unroll
+    for (int i = 0; i < TB; ++i)
+#pragma unroll
+      for (int j = 0; j < TB; ++j) acc[i][j] = __builtin_fmaf(av[i], bv[j], acc[i][j]);
+  }
+  __syncthreads();  // At becomes the output tile
+  const float thr = fast_exp2(-kItemGuardBits);
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) {
+      const int m = ty * TB + i, n = tx * TB + j;
+      if (m < M && n < N) {
+        const float shift = al[m] + be[n], s = acc[i][j];
+        const bool ok = (s >= thr) && (s < INFINITY) && (shift >= kFloor) && (shift < INFINITY);
+        At[m * LD + n] = ok ? __builtin_fmaf(fast_log2(s), kLn2, shift)
+                            : item_exact_out(ab + (long)m * K, bb + n, K, N);
+      }
+    }
+  __syncthreads();
+  elem_t* ob = out + (long)batch * M * N;
+  for (RowMajorWalk w(tid, NT, N); w.r < M; w.next()) {
+    const int m = w.r, n = w.c, e = w.r * N + w.c;
+    ob[e] = to_elem<elem_t>(At[m * LD + n]);
+  }
+}
+
 }  // namespace GENBMM_NS
