@@ -5,10 +5,10 @@
 // Same factored form as the large kernels: alpha[m] = max_k a, beta[n] = max_k b
 // are taken inside the workgroup, EA = exp(a - alpha), EB = exp(b - beta),
 // S = EA * EB, out = log S + alpha + beta, H = g * exp(alpha + beta - out),
-// grad_a = EA .* (H * EB^T), grad_b = EB .* (EA^T * H).  A cell (forward) or an
-// item (backward) for which the factoring is not exact to fp32 - S < 2^-40, a
-// shift at the reference's -1e9 floor, anything non-finite - is recomputed inside
-// the same kernel from global memory with the reference's own two-pass form.
+// grad_a = EA .* (H * EB^T), grad_b = EB .* (EA^T * H).  Rows of the result, rows of grad_a
+// and columns of grad_b with a cell for which the factoring is not exact to fp32 - S < 2^-40, a
+// shift below the reference's -1e9 floor, anything non-finite - are formed again at the end of
+// the same kernel in the reference's own two-pass form (item_fwd_rows, item_bwd_exact).
 //
 // Staging: a wave takes groups of four neighbouring rows of an array, its lanes the columns (a row is
 // contiguous in memory; all loads of the item are issued before the first is waited for).  A row's
@@ -51,6 +51,9 @@ __device__ __forceinline__ float item_exact_out(const elem_t* __restrict__ arow,
     s += fast_exp2(__builtin_fmaf((float)arow[k] + (float)bcol[(long)k * N], kLog2e, nm));
   return logf(s) + mx;
 }
+
+// Sums of shifts from which on every term lies so far below the reference's floor that its exponential is 0.
+constexpr float kItemDead = kFloor - 1024.f;
 
 // exp(x - shift), with the all -inf row / column (shift = -inf) giving zeros
 __device__ __forceinline__ float item_exp(float x, float shift) {
@@ -260,9 +263,76 @@ inline int item_bwd_floats(int M, int K, int N, int W, int H) {
   return item_bwd_arrays(M, K, N) + W * H * 64;
 }
 
+typedef elem_t item_e4 __attribute__((ext_vector_type(4), aligned(sizeof(elem_t))));
+
+// R rows (row: their numbers; the last ones may repeat) of a 16-column tile the way the reference's kernel forms them
+// (matmul_cuda_kernel.cu:27-41): running maximum from -1e9, then the sum.  The wave's lanes are the columns times
+// quarters of 16 terms: of a row they read four neighbours at a time.  The reads and one exponential a term bound it.
+// (500,96^3), 24 us where every cell factors: one such cell an item 26, nearly all cells 156 (each in the lane that found
+// it, from memory: 52 and 1325); (512,128,100,64) 29, 33 and 214.  Nearly all cells of thin products cost more than
+// tiles staged in LDS did ((512,100,40,100) 135 us, 93), the gradients then less (128, 135).
+template <int R>
+__device__ __forceinline__ void item_fwd_rows(const elem_t* __restrict__ ab, const elem_t* __restrict__ bb,
+                                              elem_t* __restrict__ ob, const int (&row)[R], int n0, int M, int K, int N,
+                                              int lane) {
+  const int n = n0 + (lane & 15), q = lane >> 4;
+  const elem_t* const bq = bb + min(n, N - 1);
+  float mx[R], nm[R], s[R];
+  auto walk = [&](auto add) __attribute__((always_inline)) {
+    float t[R];
+    int k0 = 0;
+    for (; k0 + 16 <= K; k0 += 16) {
+      item_e4 av[R];
+      float bv[4];
+#pragma unroll
+      for (int r = 0; r < R; ++r) av[r] = *reinterpret_cast<const item_e4*>(ab + row[r] * K + k0 + 4 * q);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bv[i] = (float)bq[(k0 + 4 * q + i) * N];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) t[r] = (float)av[r][i] + bv[i];
+        add(t);
+      }
+    }
+    for (; k0 < K; k0 += 4) {
+      const int k = min(k0 + q, K - 1);
+      const float bv = (float)bq[k * N];
+#pragma unroll
+      for (int r = 0; r < R; ++r) t[r] = k0 + q < K ? (float)ab[row[r] * K + k] + bv : -INFINITY;
+      add(t);
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    mx[r] = kFloor;
+    s[r] = 0.f;
+  }
+  walk([&](const float (&t)[R]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) mx[r] = fmaxf(mx[r], t[r]);
+  });
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], 16, 64));
+    mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], 32, 64));
+    nm[r] = -mx[r] * kLog2e;
+  }
+  walk([&](const float (&t)[R]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] += fast_exp2(__builtin_fmaf(t[r], kLog2e, nm[r]));
+  });
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    s[r] += __shfl_xor(s[r], 16, 64);
+    s[r] += __shfl_xor(s[r], 32, 64);
+    if (q == 0 && n < N) ob[row[r] * N + n] = to_elem<elem_t>(logf(s[r]) + mx[r]);
+  }
+}
+
 // W waves; U groups of four rows per wave (4 W U >= every extent), H column chunks of 64.
 template <int W, int U, int H>
-__global__ __launch_bounds__(64 * W) void k_log_item_fwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+__global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void k_log_item_fwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
                                                          elem_t* __restrict__ out, float* __restrict__ stats,
                                                          int* __restrict__ hdr, int M, int K, int N) {
   extern __shared__ __attribute__((aligned(16))) float item_smem[];
@@ -273,7 +343,9 @@ __global__ __launch_bounds__(64 * W) void k_log_item_fwd(const elem_t* __restric
   float* const part = Eb + pad.N * ldk;    // [wave][column]
   float* const s_al = part + W * H * 64;
   float* const s_be = s_al + pad.M;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x;
+  int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int batch = blockIdx.x;
   if (hdr && batch == 0 && tid == 0) hdr[0] = kWsNone;  // no per-tile flags in this workspace
   const elem_t* ab = a + (long)batch * M * K;
@@ -317,8 +389,10 @@ __global__ __launch_bounds__(64 * W) void k_log_item_fwd(const elem_t* __restric
   const int tm = pad.M >> 4, tn = pad.N >> 4, chunks = pad.K >> 4;
   const float thr = fast_exp2(-kItemGuardBits);
   elem_t* ob = out + (long)batch * M * N;
+  int* const marks = reinterpret_cast<int*>(part) + 64 * H * wave;  // of this wave's tiles: rows to be formed again
+  unsigned flagged = 0;                                             // tiles with such rows
   ItemTiles w(wave, tn);
-  for (; w.r < tm; w.next(W)) {  // uniform
+  for (int at = 0; w.r < tm; w.next(W), ++at) {  // uniform; at most 8 tiles
     const int m0 = w.r * 16, n0 = w.c * 16;
     const float* xl = Eb + (n0 + l15) * ldk + q4;
     const float* yl = Ea + (m0 + l15) * ldk + q4;
@@ -336,20 +410,148 @@ __global__ __launch_bounds__(64 * W) void k_log_item_fwd(const elem_t* __restric
       if (!ok && m < M && n + r < N) redo |= 1 << r;
       o[r] = __builtin_fmaf(fast_log2(s[r]), kLn2, shift);
     }
+    bool store = m < M;
     if (__builtin_amdgcn_ballot_w64(redo != 0) != 0) {  // rare
-#pragma unroll 1
-      for (int r = 0; r < 4; ++r)
-        if (redo >> r & 1) {
-          const float e = item_exact_out(ab + (long)m * K, bb + n + r, K, N);
-          o[0] = r == 0 ? e : o[0]; o[1] = r == 1 ? e : o[1]; o[2] = r == 2 ? e : o[2]; o[3] = r == 3 ? e : o[3];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)  // no term reaches the floor (a masked row or column), so none has mass beside it
+        if (am + bn[r] <= kItemDead && s[r] >= 0.f) {
+          o[r] = -INFINITY;
+          redo &= ~(1 << r);
         }
+      const unsigned long long cells = __builtin_amdgcn_ballot_w64(redo != 0);
+      const int again = (int)((cells | cells >> 16 | cells >> 32 | cells >> 48) & 0xffff);
+      marks[at] = again;
+      flagged |= again != 0 ? 1u << at : 0u;
+      store = store && !(again >> l15 & 1);
     }
-    if (m < M) st4m(ob + m * N + n, N - n, make_float4(o[0], o[1], o[2], o[3]));
+    if (store) st4m(ob + m * N + n, N - n, make_float4(o[0], o[1], o[2], o[3]));
+  }
+  if (flagged) {  // uniform
+    // (values of their own: nothing of this block is formed ahead of it)
+    asm volatile("" : "+s"(M), "+s"(K), "+s"(N), "+v"(lane));
+    for (; flagged; flagged &= flagged - 1) {
+      const int i = __builtin_ctz(flagged), tile = wave + W * i, m0 = tile / tn * 16, n0 = (tile - tile / tn * tn) * 16;
+      unsigned again = __builtin_amdgcn_readfirstlane(marks[i]);
+      while (again) {  // uniform
+        constexpr int R = U == 2 ? 2 : 4;  // (registers of eight waves a SIMD)
+        if (__builtin_popcount(again) < R / 2 + 1) {
+          const int row[1] = {m0 + __builtin_ctz(again)};
+          again &= again - 1;
+          item_fwd_rows<1>(ab, bb, ob, row, n0, M, K, N, lane);
+        } else {
+          int row[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            row[r] = again ? m0 + __builtin_ctz(again) : row[r > 0 ? r - 1 : 0];
+            again &= again - 1;
+          }
+          item_fwd_rows<R>(ab, bb, ob, row, n0, M, K, N, lane);
+        }
+      }
+    }
   }
 }
 
+// What marks a row or column to be formed again.  (Nothing clears the marks' place in LDS first: should what was there
+// look like one, a row more is formed so.)
+constexpr int kItemMark = 0x7fa5c3e1;
+
+// The marks of `count` rows (columns) become the list of their numbers, in place; by one wave.  Returns how many.
+__device__ __forceinline__ int item_list(int* __restrict__ marks, int count, int lane) {
+  unsigned long long set[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    set[h] = __builtin_amdgcn_ballot_w64(lane + 64 * h < count && marks[min(lane + 64 * h, count - 1)] == kItemMark);
+  const unsigned long long below = (1ULL << lane) - 1;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    if (set[h] >> lane & 1) marks[(h ? __builtin_popcountll(set[0]) : 0) + __builtin_popcountll(set[h] & below)] = lane + 64 * h;
+  return __builtin_popcountll(set[0]) + __builtin_popcountll(set[1]);
+}
+
+// Gradients of listed rows (grad_a) and columns (grad_b) in the reference's form (matmul_cuda_kernel.cu:159-184),
+// exp(a + b - out) * g summed over n and over m; Al [k][m], Bl [k][n] and Ol [m][n]: the operands and out in LDS.  A
+// lane takes four rows m of a k, or four rows k of a column, over the whole list: 16 terms for every ten reads.
+// One exponential a term bounds it.  Both gradients of (500,96^3), 48 us where every cell factors: one such cell an item
+// 91, one masked row 162, nearly all cells 221 (the whole item again, every cell in a thread of its own that read all
+// it needed from memory: 1480 each; by tiles staged in LDS 265 each); (2048,64^3) 53, then 116, 191 and 298 (1836).
+template <int W>
+__device__ __forceinline__ void item_bwd_exact(const elem_t* __restrict__ gb, const float* __restrict__ Al, int ldm,
+                                               const float* __restrict__ Bl, int ldn, const float* __restrict__ Ol,
+                                               const int* __restrict__ rows, int nr, const int* __restrict__ cols, int nc,
+                                               elem_t* __restrict__ gab, elem_t* __restrict__ gbb, int M, int K, int N,
+                                               int tid) {
+  constexpr int R = 4;
+  if (gab)
+    for (int e = tid; e < (nr + R - 1) / R * K; e += 64 * W) {
+      const int group = e / K, k = e - group * K;
+      const float* bl = Bl + k * ldn;
+      float av[R], s[R];
+      int m[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        m[r] = rows[min(R * group + r, nr - 1)];
+        av[r] = Al[k * ldm + m[r]];
+        s[r] = 0.f;
+      }
+      int n = 0;
+      for (; n + 3 < N; n += 4) {
+        const item_f4 b4 = item_frag(bl + n);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const item_f4 o4 = item_frag(Ol + m[r] * ldn + n);
+          const item_e4 g4 = *reinterpret_cast<const item_e4*>(gb + m[r] * N + n);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[r] = __builtin_fmaf(fast_exp(av[r] + b4[q] - o4[q]), (float)g4[q], s[r]);
+        }
+      }
+      for (; n < N; ++n)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          s[r] = __builtin_fmaf(fast_exp(av[r] + bl[n] - Ol[m[r] * ldn + n]), (float)gb[m[r] * N + n], s[r]);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (R * group + r < nr) gab[m[r] * K + k] = to_elem<elem_t>(s[r]);
+    }
+  if (gbb)
+    for (int e = tid; e < (K + R - 1) / R * nc; e += 64 * W) {
+      const int group = e / nc, n = cols[e - group * nc];
+      float bv[R], s[R];
+      const float* al[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int k = min(R * group + r, K - 1);
+        al[r] = Al + k * ldm;
+        bv[r] = Bl[k * ldn + n];
+        s[r] = 0.f;
+      }
+      int m = 0;
+      for (; m + 3 < M; m += 4) {
+        float ov[4], gv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          ov[q] = Ol[(m + q) * ldn + n];
+          gv[q] = (float)gb[(m + q) * N + n];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const item_f4 a4 = item_frag(al[r] + m);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[r] = __builtin_fmaf(fast_exp(a4[q] + bv[r] - ov[q]), gv[q], s[r]);
+        }
+      }
+      for (; m < M; ++m)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          s[r] = __builtin_fmaf(fast_exp(al[r][m] + bv[r] - Ol[m * ldn + n]), (float)gb[m * N + n], s[r]);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (R * group + r < K) gbb[(R * group + r) * N + n] = to_elem<elem_t>(s[r]);
+    }
+}
+
 template <int W, int U, int H>
-__global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+__global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 8 && U == 3 ? 4 : 1) void k_log_item_bwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
                                                          const elem_t* __restrict__ outp, const elem_t* __restrict__ g,
                                                          elem_t* __restrict__ grad_a, elem_t* __restrict__ grad_b,
                                                          int M, int K, int N) {
@@ -360,7 +562,8 @@ __global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restric
   float* const Eb = EaT + pad.K * ldm;    // [k][n]
   float* const Hs = Eb + pad.K * ldn;     // [m][n]
   float* const part = Hs + pad.M * ldn;   // [wave][column]
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x;
+  int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int batch = blockIdx.x;
   const elem_t* ab = a + (long)batch * M * K;
   const elem_t* bb = b + (long)batch * K * N;
@@ -384,7 +587,7 @@ __global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restric
   item_cols_join<W, H>(part, lane, be);
   item_cols_exp(xb, be);
   xb.put_rows(Eb, ldn, pad.K, pad.N, wave, lane);
-  // H, and whether the factoring is exact for this item: S < 2^-40, NaN or infinities anywhere are not
+  // H, and whether the factoring is exact for every cell: S < 2^-40, NaN or infinities anywhere are not
   const float lim = kItemGuardBits * kLn2 + 1e-3f;
   float most = 0.f, worst = 0.f;  // worst stays 0 while every exponent is finite
 #pragma unroll
@@ -401,28 +604,17 @@ __global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restric
       }
   const int bad = !(most <= lim) || !(worst == 0.f);
   xg.put_rows(Hs, ldn, pad.M, pad.N, wave, lane);
-  if (__syncthreads_or(bad)) {
-    // the reference's form for the whole item (matmul_cuda_kernel.cu:159-184):
-    // exp(a + b - out) * g summed over n (grad_a) / m (grad_b), from global memory
-    if (gab)
-      for (int e = tid; e < M * K; e += 64 * W) {
-        const int m = e / K, k = e - m * K;
-        const float av = ab[e];
-        float s = 0.f;
-        for (int n = 0; n < N; ++n)
-          s = __builtin_fmaf(fast_exp(av + (float)bb[(long)k * N + n] - (float)ob[(long)m * N + n]), (float)gb[(long)m * N + n], s);
-        gab[e] = to_elem<elem_t>(s);
-      }
-    if (gbb)
-      for (int e = tid; e < K * N; e += 64 * W) {
-        const int k = e / N, n = e - k * N;
-        const float bv = bb[e];
-        float s = 0.f;
-        for (int m = 0; m < M; ++m)
-          s = __builtin_fmaf(fast_exp((float)ab[(long)m * K + k] + bv - (float)ob[(long)m * N + n]), (float)gb[(long)m * N + n], s);
-        gbb[e] = to_elem<elem_t>(s);
-      }
-    return;
+  // Rows of grad_a and columns of grad_b that such a cell takes part in are formed again below, the rows together with
+  // those of its wave; the others need none of its H.
+  int* const rows = reinterpret_cast<int*>(part);  // marks, then lists (every wave has joined the columns' maxima)
+  int* const cols = rows + 64 * H;
+  const int redo = __syncthreads_or(bad);
+  if (redo) {  // rare
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      if (bad && lane + 64 * h < N) cols[lane + 64 * h] = kItemMark;
+    const int m = 4 * (wave + W * (lane >> 2)) + (lane & 3);
+    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane < 4 * U && m < M) rows[m] = kItemMark;
   }
 
   const int l15 = lane & 15, q4 = 4 * (lane >> 4);
@@ -455,6 +647,27 @@ __global__ __launch_bounds__(64 * W) void k_log_item_bwd(const elem_t* __restric
       const item_f4 e = item_frag(Eb + k * ldn + n);
       if (k < K) st4m(gbb + k * N + n, N - n, make_float4(e[0] * s[0], e[1] * s[1], e[2] * s[2], e[3] * s[3]));
     }
+  }
+  if (redo) {
+    // (values of their own: nothing of this block is formed ahead of it)
+    asm volatile("" : "+s"(M), "+s"(K), "+s"(N), "+v"(lane), "+s"(wave));
+    int* const counts = rows + 128 * H;
+    __syncthreads();  // the tiles' results are on their way, LDS is free
+    if (wave < 2) {
+      const int c = wave == 0 ? item_list(rows, M, lane) : item_list(cols, N, lane);
+      if (lane == 0) counts[wave] = c;
+    }
+    xa.load(ab, M, K, wave, lane);
+    xb.load(bb, K, N, wave, lane);
+    xo.load(ob, M, N, wave, lane);
+    xa.settle(K, lane);
+    xa.put_cols(EaT, ldm, pad.M, pad.K, wave, lane);
+    xb.settle(N, lane);
+    xb.put_rows(Eb, ldn, pad.K, pad.N, wave, lane);
+    xo.settle(N, lane);
+    xo.put_rows(Hs, ldn, pad.M, pad.N, wave, lane);
+    __syncthreads();
+    item_bwd_exact<W>(gb, EaT, ldm, Eb, ldn, Hs, rows, counts[0], cols, counts[1], gab, gbb, M, K, N, tid);
   }
 }
 

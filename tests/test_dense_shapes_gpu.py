@@ -213,6 +213,46 @@ def test_log_items_that_cannot_be_factored(gpu, B, M, K, N):
     assert bool((got[5] == -float("inf")).all()) and bool((got[:, 7][live[:, 0]] == -float("inf")).all())
 
 
+ITEMS = [(3, 20, 31, 17), (2, 3, 2, 5), (2, 48, 40, 33), (2, 64, 64, 64), (2, 65, 70, 50), (2, 96, 90, 72), (2, 128, 100, 64),
+         (2, 128, 16, 128), (2, 2, 128, 1), (3, 128, 4, 4)]
+
+
+def _log_grads(gpu, a, b, g, dt):
+    x, y = a.to(gpu, dt).requires_grad_(True), b.to(gpu, dt).requires_grad_(True)
+    o = genbmm.logbmm(x, y)
+    return [o.detach()] + list(torch.autograd.grad(o, (x, y), g.to(gpu, dt)))
+
+
+@pytest.mark.parametrize("dt, eps", [(torch.float32, 0.0), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("kind", ["one", "most"])
+@pytest.mark.parametrize("shape", ITEMS)
+def test_log_items_with_cells_that_cannot_be_factored(gpu, shape, kind, dt, eps):
+    """One such cell (its row and its column of the gradients are formed again, the others are not), and most of them.
+    A weight exp(a + b - out) is as good as its exponent: |a + b| and |out| stay below 256, so 3 x 2^-25 x 256 = 2.3e-5
+    and a few units of rounding; a gradient is off by at most that share of its sum over |g|.  Half types add
+    the rounding of `out`, which the weights are formed from (up to eps x |out|), and of the result."""
+    torch.manual_seed(11)
+    B, M, K, N = shape
+    a, b, g = torch.randn(B, M, K), torch.randn(B, K, N), torch.randn(B, M, N)
+    if kind == "most":
+        a, b = 20 * a, 20 * b
+    else:
+        a[0, 1, 0] += 60
+        b[0, 1, 0] += 60
+    a, b, g = (t.to(dt).float() for t in (a, b, g))
+    got = [t.double().cpu() for t in _log_grads(gpu, a, b, g, dt)]
+    x, y = a.double().requires_grad_(True), b.double().requires_grad_(True)
+    out = torch.logsumexp(x.unsqueeze(3) + y.unsqueeze(1), 2)
+    want = torch.autograd.grad(out, (x, y), g.double(), retain_graph=True)
+    size = torch.autograd.grad(out, (x, y), g.abs().double())
+    most = float(out.detach().abs().max())
+    assert most < 256
+    assert bool(((got[0] - out).abs() <= 2e-5 + (2.0 ** -23 + eps) * out.abs()).all())
+    share = 4e-5 + (0.0 if dt == torch.float32 else np.expm1(eps * most) + eps)
+    for p, q, s in zip(got[1:], want, size):
+        assert bool(((p - q).abs() <= share * s + 1e-6).all()), float(((p - q).abs() - share * s).max())
+
+
 # (shape, checksum of the indices, checksum of the results' bit patterns): what (77, 3) draws, taken on this GPU
 PINNED = [
     ((3, 32, 32, 32), 75771211, 5024752994044624),
