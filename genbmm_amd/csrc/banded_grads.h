@@ -348,9 +348,12 @@ __device__ __forceinline__ void grad_consume(const BandArgs& p, const GradSide& 
           v = z_in ? v : 0.f;  // outside the matrix: the reference's zero fill
           buf_st(dst, at(e) * ES, to_elem<elem_t>(v));
         }
-        if (!(worst == 0.f)) {  // rare; the stores above came from this lane: they stay in order
-#pragma unroll 1
-          for (int e = 0; e < 16; ++e) {
+        if (!(worst == 0.f)) {  // rare: those sums alone; the stores above came from this lane: they stay in order
+          unsigned bad = 0;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) bad |= acc[k][e] * kGradUnscale * 0.f == 0.f ? 0u : 1u << e;
+          for (; bad; bad &= bad - 1) {
+            const int e = __builtin_ctz(bad);
             const int ro = 8 * (e >> 2) + 4 * hi32 + (e & 3), line = l0 + ro, cell = Wr - 1 - 32 * d[k] + col - ro;
             if ((unsigned)line < (unsigned)n && (unsigned)cell < (unsigned)Wr) {
               constexpr int MODE = PREP ? GENBMM_BAND_LOG : GENBMM_BAND_MUL;
