@@ -20,7 +20,7 @@
 // while one is added, and no load stands under a branch: behind one the compiler waits for every load.
 // Both gradients are one launch, strip by strip, so that the second use of g and idx comes from a cache.
 //
-// g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each: 180 -> 149 us there, 2.7 TB/s (behind a
+// g and idx once and both gradients are 406 MB at 64 x 4096, 65 diagonals each: 180 -> 149 us there (behind a
 // forward, as a step runs them).  Of the 31, 7 are addresses and slots that no longer follow clamped rows (grad_b), the rest
 // pieces of four cells a load and a store (grad_a) and results that leave as one run instead of 32 diagonals at a time.
 // What it waits for now: timed in parts, 55 us are the walk over LDS without loads, additions and results; the ordered
@@ -84,22 +84,21 @@ __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int kw, in
       add4_ordered(accs + lane, k4, t4);
     }
   };
-  const int last = chunks - 1;
   if (chunks > 0) {
     load(v0, 0);
-    load(v1, min(1, last));
-    load(v2, min(2, last));
+    load(v1, 1);
+    load(v2, 2);
   }
 #pragma unroll 16
   for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
   for (int c = 0; c < chunks; c += 4) {
-    load(v3, min(c + 3, last));
+    load(v3, c + 3);
     add(v0, c);
-    load(v0, min(c + 4, last));
+    load(v0, c + 4);
     add(v1, c + 1);
-    load(v1, min(c + 5, last));
+    load(v1, c + 5);
     add(v2, c + 2);
-    load(v2, min(c + 6, last));
+    load(v2, c + 6);
     add(v3, c + 3);
   }
 }
@@ -191,8 +190,11 @@ __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const Ba
           v.i[u][e] = is[row[u] + j];
         }
       } else {
-        v.g[u] = *reinterpret_cast<const arg_e4*>(gs + row[u]);
-        v.i[u] = *reinterpret_cast<const arg_i4*>(is + row[u]);
+        // (a chunk past the band asks for one line: every row's last cells again cost 14 us of 83 with 33 diagonals an
+        // operand, 7 of 139 with 65)
+        const long at = j0 <= jhi ? row[u] : 0;
+        v.g[u] = *reinterpret_cast<const arg_e4*>(gs + at);
+        v.i[u] = *reinterpret_cast<const arg_i4*>(is + at);
       }
     }
   };
@@ -232,7 +234,6 @@ __device__ __forceinline__ void argmax_band_a(float* __restrict__ accs, const Ba
       add4_ordered(accs + lane, k4, t4);
     }
   };
-  // (a chunk past the band asks for its row's last cells again)
   auto turn = [&](ArgRowChunk& v, int j0) __attribute__((always_inline)) {
     if (j0 <= jhi) stage(v, j0);  // uniform
     load(v, j0 + 3 * kArgCh);
@@ -283,12 +284,13 @@ __device__ __forceinline__ void argmax_band_b(float* __restrict__ accs, const Ba
   int off[kArgChB];
 #pragma unroll
   for (int q = 0; q < kArgChB; ++q) off[q] = q < rows ? lane + q * (Wo - 1) : -16;
+  const int chunks = ihi < ilo ? 0 : (ihi - ilo + rows) / rows;
   argmax_walk<ArgColChunk>(
-      accs, kw, ihi < ilo ? 0 : (ihi - ilo + rows) / rows,
+      accs, kw, chunks,
       [&](ArgColChunk& x, int c) __attribute__((always_inline)) {
-        // lane 0's cell of the chunk's first row; the buffers end with the item
-        const long first = (long)(ilo + c * rows) * (Wo - 1) + (o0 + p.r_lu);
-        const unsigned left = (unsigned)min((long)n * Wo - first, 1L << 29);
+        // lane 0's cell of the chunk's first row; the buffers end with the item, a chunk past the rows has none
+        const long first = (long)(ilo + min(c, chunks - 1) * rows) * (Wo - 1) + (o0 + p.r_lu);
+        const unsigned left = c < chunks ? (unsigned)min((long)n * Wo - first, 1L << 29) : 0;
         const buf_t bi = buf_of(ib + first, left * 4), bg = buf_of(gb + first, left * ES);
 #pragma unroll
         for (int q = 0; q < kArgChB; ++q) {
