@@ -71,7 +71,10 @@ template <class Chunk, class Load, class Slots>
 __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int kw, int chunks, Load load, Slots slots) {
   constexpr int CH = Chunk::CH;
   const int lane = threadIdx.x;
-  Chunk v0, v1, v2, v3;  // loads ahead as far as the 63 that a wave can wait for reach
+  // Two chunks, 2 x 32 loads, ahead: about the 63 that a wave can leave in flight.  (A third's wait took part of the second
+  // with it, and its registers: 64 x 4096 with 5 diagonals an operand 29 us for 25, bfloat16 33 57 for 53, 65 the same;
+  // one ahead is slower from 17 on, 65 138 us for 131.)
+  Chunk v0, v1, v2;
   auto add = [&](const Chunk& ch, int c) __attribute__((always_inline)) {
     if (c >= chunks) return;  // uniform
     unsigned kr[CH];
@@ -87,19 +90,16 @@ __device__ __forceinline__ void argmax_walk(float* __restrict__ accs, int kw, in
   if (chunks > 0) {
     load(v0, 0);
     load(v1, 1);
-    load(v2, 2);
   }
 #pragma unroll 16
   for (int k = 0; k <= kw; ++k) accs[k * kArgRows + lane] = 0.f;
-  for (int c = 0; c < chunks; c += 4) {
-    load(v3, c + 3);
+  for (int c = 0; c < chunks; c += 3) {
+    load(v2, c + 2);
     add(v0, c);
-    load(v0, c + 4);
+    load(v0, c + 3);
     add(v1, c + 1);
-    load(v1, c + 5);
+    load(v1, c + 4);
     add(v2, c + 2);
-    load(v2, c + 6);
-    add(v3, c + 3);
   }
 }
 
