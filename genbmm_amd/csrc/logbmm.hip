@@ -1068,12 +1068,44 @@ int run_bwd(const LogBwdArgs& p, const float* stats, int path, int B, hipStream_
   return launch_bwd_exact<BCfgMid, GRAD_A>(p, B, s);
 }
 
-template <int W, int U, int H>
-void launch_item_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int* hdr, int B, int M,
-                     int K, int N, hipStream_t s) {
-  const int lds = 4 * item_fwd_floats(M, K, N, W, H);
-  if (H > 1) allow_lds(k_log_item_fwd<W, U, H>, lds);
-  hipLaunchKernelGGL((k_log_item_fwd<W, U, H>), dim3(B), dim3(64 * W), lds, s, a, b, out, stats, hdr, M, K, N);
+// What an item's arrays take of a workgroup of W waves (logbmm_item.h).
+template <int W, int UM, int UK, int HK, int HN>
+struct ItemCfg {
+  static int launch_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int* hdr, int B, int M, int K, int N,
+                        hipStream_t s) {
+    const int lds = 4 * item_fwd_floats(M, K, N, W, HN);
+    if (W > 4) allow_lds(k_log_item_fwd<W, UM, UK, HK, HN>, lds);
+    hipLaunchKernelGGL((k_log_item_fwd<W, UM, UK, HK, HN>), dim3(B), dim3(64 * W), lds, s, a, b, out, stats, hdr, M, K, N);
+    return launch_status();
+  }
+  static int launch_bwd(const elem_t* a, const elem_t* b, const elem_t* out, const elem_t* g, elem_t* grad_a, elem_t* grad_b,
+                        int B, int M, int K, int N, hipStream_t s) {
+    const int lds = 4 * item_bwd_floats(M, K, N, W, HN);
+    if (W > 4) allow_lds(k_log_item_bwd<W, UM, UK, HK, HN>, lds);
+    hipLaunchKernelGGL((k_log_item_bwd<W, UM, UK, HK, HN>), dim3(B), dim3(64 * W), lds, s, a, b, out, g, grad_a, grad_b, M, K,
+                       N);
+    return launch_status();
+  }
+};
+// Every extent up to 16, 32, 48, 64 has a case of its own, and of larger items so have those with two extents of at most 32
+// or such a K: the registers and the reads (rows and columns beyond a matrix are its last ones again) are what the extents
+// ask for, which leaves four workgroups of 8 waves a compute unit where the common case leaves one or two.  Forward and both
+// gradients (the common case; by tiles, before there were such items): (4096,1,128,1) 22 + 28 us (48 + 119; 39 + 82),
+// (4096,4,4,128) 20 + 29 (46 + 115; 45 + 76), (4096,128,4,4) 33 + 45 (55 + 121; 76 + 88), (4096,8,8,8) 9.0 + 10.1
+// (10.0 + 12.2).  The forward alone of (1..64,128,4,128), 10.5 us (11.2), was 8.7 by tiles, with the gradients 46.
+template <class F>
+int with_item_cfg(int M, int K, int N, F&& go) {
+  const int most = max(max(M, K), N);
+  if (most <= 16) return go(ItemCfg<4, 1, 1, 1, 1>{});
+  if (most <= 32) return go(ItemCfg<4, 2, 2, 1, 1>{});
+  if (most <= 48) return go(ItemCfg<4, 3, 3, 1, 1>{});
+  if (most <= 64) return go(ItemCfg<4, 4, 4, 1, 1>{});
+  if (M <= 32 && N <= 32) return go(ItemCfg<8, 1, 4, 2, 1>{});
+  if (K <= 32 && N <= 32) return go(ItemCfg<8, 4, 1, 1, 1>{});
+  if (M <= 32 && K <= 32) return go(ItemCfg<8, 1, 1, 1, 2>{});
+  if (K <= 32) return go(ItemCfg<8, 4, 1, 1, 2>{});
+  if (most <= 96) return go(ItemCfg<8, 3, 3, 2, 2>{});
+  return go(ItemCfg<8, 4, 4, 2, 2>{});
 }
 // (half types sweep only on the factors of larger extents)
 inline void launch_item_seq(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int* hdr, int B, int M, int K,
@@ -1085,14 +1117,6 @@ inline void launch_item_seq(const elem_t* a, const elem_t* b, elem_t* out, float
     else go(k_log_item_seq<16, 4, false>);
   }
 }
-template <int W, int U, int H>
-void launch_item_bwd(const elem_t* a, const elem_t* b, const elem_t* out, const elem_t* g, elem_t* grad_a, elem_t* grad_b,
-                     int B, int M, int K, int N, hipStream_t s) {
-  const int lds = 4 * item_bwd_floats(M, K, N, W, H);
-  if (H > 1) allow_lds(k_log_item_bwd<W, U, H>, lds);
-  hipLaunchKernelGGL((k_log_item_bwd<W, U, H>), dim3(B), dim3(64 * W), lds, s, a, b, out, g, grad_a, grad_b, M, K, N);
-}
-
 // keep: the workspace is as large as genbmm_logbmm_stats_size says and receives what a
 // backward wants beside the maxima; false: header_offset() + 4 floats of it are used.
 int launch_self_fwd(DenseArgs p, float* stats, int B, int M, int K, int N, bool split, hipStream_t s) {
@@ -1166,11 +1190,8 @@ int run_fwd(const elem_t* a, const elem_t* b, elem_t* out, float* stats, int B, 
     if (M == 32 && K == 32 && N == 32)  // one wave per item on the matrix cores
       hipLaunchKernelGGL(k_log_item32_fwd, dim3((B + 3) / 4), dim3(256), 0, s, a, b, out, stats, hdr, B);
     else if (kElemF32 && factors) launch_item_seq(a, b, out, stats, hdr, B, M, K, N, s);
-    else if (most <= 32) launch_item_fwd<4, 2, 1>(a, b, out, stats, hdr, B, M, K, N, s);
-    else if (most <= 48) launch_item_fwd<4, 3, 1>(a, b, out, stats, hdr, B, M, K, N, s);
-    else if (most <= 64) launch_item_fwd<4, 4, 1>(a, b, out, stats, hdr, B, M, K, N, s);
-    else if (most <= 96) launch_item_fwd<8, 3, 2>(a, b, out, stats, hdr, B, M, K, N, s);
-    else launch_item_fwd<8, 4, 2>(a, b, out, stats, hdr, B, M, K, N, s);
+    else
+      return with_item_cfg(M, K, N, [&](auto cfg) { return cfg.launch_fwd(a, b, out, stats, hdr, B, M, K, N, s); });
     return launch_status();
   }
   DenseArgs p{};
@@ -1229,19 +1250,10 @@ int run_bwd_both(const elem_t* a, const elem_t* b, const elem_t* out, const elem
   p.vec_n = (N % 4 == 0) && aligned16(b) && aligned16(out) && aligned16(g) && aligned16(grad_b);
   const float* st = (path == GENBMM_PATH_EXACT || mn == 0) ? nullptr : stats;
   if (st && B > 0 && item_shape(M, K, N) && auto_path(path)) {
-    const int most = max(max(M, K), N);
     if (M == 32 && K == 32 && N == 32)
       hipLaunchKernelGGL(k_log_item32_bwd, dim3((B + 3) / 4), dim3(256), 0, s, a, b, out, g, grad_a, grad_b, B);
-    else if (most <= 32)
-      launch_item_bwd<4, 2, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
-    else if (most <= 48)
-      launch_item_bwd<4, 3, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
-    else if (most <= 64)
-      launch_item_bwd<4, 4, 1>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
-    else if (most <= 96)
-      launch_item_bwd<8, 3, 2>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
     else
-      launch_item_bwd<8, 4, 2>(a, b, out, g, grad_a, grad_b, B, M, K, N, s);
+      return with_item_cfg(M, K, N, [&](auto cfg) { return cfg.launch_bwd(a, b, out, g, grad_a, grad_b, B, M, K, N, s); });
     return launch_status();
   }
   if (st && B > 0 && self_shape(M, K, N) && auto_path(path)) {

@@ -255,6 +255,7 @@ __host__ __device__ inline int item_bwd_arrays(int M, int K, int N) {
   const ItemPad p = item_pad(M, K, N);
   return p.K * (p.M + 4) + p.K * (p.N + 4) + p.M * (p.N + 4);
 }
+// (H: column chunks of N)
 inline int item_fwd_floats(int M, int K, int N, int W, int H) {
   const ItemPad p = item_pad(M, K, N);
   return (p.M + p.N) * (p.K + 4) + W * H * 64 + p.M + p.N;
@@ -330,9 +331,9 @@ __device__ __forceinline__ void item_fwd_rows(const elem_t* __restrict__ ab, con
   }
 }
 
-// W waves; U groups of four rows per wave (4 W U >= every extent), H column chunks of 64.
-template <int W, int U, int H>
-__global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void k_log_item_fwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+// W waves; UM, UK groups of four rows per wave (4 W UM >= M, 4 W UK >= K), HK, HN column chunks of 64 of K and N.
+template <int W, int UM, int UK, int HK, int HN>
+__global__ __launch_bounds__(64 * W, UM <= 2 && UK <= 2 ? 8 : W == 4 && UM == 3 ? 7 : 1) void k_log_item_fwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
                                                          elem_t* __restrict__ out, float* __restrict__ stats,
                                                          int* __restrict__ hdr, int M, int K, int N) {
   extern __shared__ __attribute__((aligned(16))) float item_smem[];
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
   float* const Ea = item_smem;             // [m][k]
   float* const Eb = Ea + pad.M * ldk;      // [n][k]
   float* const part = Eb + pad.N * ldk;    // [wave][column]
-  float* const s_al = part + W * H * 64;
+  float* const s_al = part + W * HN * 64;
   float* const s_be = s_al + pad.M;
   const int tid = threadIdx.x;
   int lane = tid & 63;
@@ -350,11 +351,12 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
   if (hdr && batch == 0 && tid == 0) hdr[0] = kWsNone;  // no per-tile flags in this workspace
   const elem_t* ab = a + (long)batch * M * K;
   const elem_t* bb = b + (long)batch * K * N;
-  ItemRows<W, U, H> xa, xb;
+  ItemRows<W, UM, HK> xa;
+  ItemRows<W, UK, HN> xb;
   xa.load(ab, M, K, wave, lane);
   xb.load(bb, K, N, wave, lane);
 
-  float al[U][4], be[H];
+  float al[UM][4], be[HN];
   xa.settle(K, lane);
   item_rows_exp(xa, al);
   xa.put_rows(Ea, ldk, pad.M, pad.K, wave, lane);
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
   float* st = stats ? stats + (long)batch * (M + N) : nullptr;
   if (lane == 0) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < UM; ++u)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int m = 4 * (wave + W * u) + t;
@@ -372,12 +374,12 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
       }
   }
   __syncthreads();
-  item_cols_join<W, H>(part, lane, be);
+  item_cols_join<W, HN>(part, lane, be);
   item_cols_exp(xb, be);
   xb.put_cols(Eb, ldk, pad.K, pad.N, wave, lane);
   if (wave == 0) {
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
+    for (int h = 0; h < HN; ++h) {
       const int n = lane + 64 * h;
       if (n < pad.N) s_be[n] = be[h];
       if (st && n < N) st[M + n] = be[h];
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
   const int tm = pad.M >> 4, tn = pad.N >> 4, chunks = pad.K >> 4;
   const float thr = fast_exp2(-kItemGuardBits);
   elem_t* ob = out + (long)batch * M * N;
-  int* const marks = reinterpret_cast<int*>(part) + 64 * H * wave;  // of this wave's tiles: rows to be formed again
+  int* const marks = reinterpret_cast<int*>(part) + 64 * HN * wave;  // of this wave's tiles: rows to be formed again
   unsigned flagged = 0;                                             // tiles with such rows
   ItemTiles w(wave, tn);
   for (int at = 0; w.r < tm; w.next(W), ++at) {  // uniform; at most 8 tiles
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 4 && U == 3 ? 7 : 1) void
       const int i = __builtin_ctz(flagged), tile = wave + W * i, m0 = tile / tn * 16, n0 = (tile - tile / tn * tn) * 16;
       unsigned again = __builtin_amdgcn_readfirstlane(marks[i]);
       while (again) {  // uniform
-        constexpr int R = U == 2 ? 2 : 4;  // (registers of eight waves a SIMD)
+        constexpr int R = UM <= 2 ? 2 : 4;  // (registers of eight waves a SIMD)
         if (__builtin_popcount(again) < R / 2 + 1) {
           const int row[1] = {m0 + __builtin_ctz(again)};
           again &= again - 1;
@@ -550,8 +552,8 @@ __device__ __forceinline__ void item_bwd_exact(const elem_t* __restrict__ gb, co
     }
 }
 
-template <int W, int U, int H>
-__global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 8 && U == 3 ? 4 : 1) void k_log_item_bwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
+template <int W, int UM, int UK, int HK, int HN>
+__global__ __launch_bounds__(64 * W, UM <= 2 && UK <= 2 ? 8 : W == 8 && (UM == 3 || UM != UK) ? 4 : 1) void k_log_item_bwd(const elem_t* __restrict__ a, const elem_t* __restrict__ b,
                                                          const elem_t* __restrict__ outp, const elem_t* __restrict__ g,
                                                          elem_t* __restrict__ grad_a, elem_t* __restrict__ grad_b,
                                                          int M, int K, int N) {
@@ -571,29 +573,31 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 8 && U == 3 ? 4 : 1) void
   const elem_t* gb = g + (long)batch * M * N;
   elem_t* gab = grad_a ? grad_a + (long)batch * M * K : nullptr;
   elem_t* gbb = grad_b ? grad_b + (long)batch * K * N : nullptr;
-  ItemRows<W, U, H> xa, xb, xo, xg;
+  ItemRows<W, UM, HK> xa;
+  ItemRows<W, UK, HN> xb;
+  ItemRows<W, UM, HN> xo, xg;
   xb.load(bb, K, N, wave, lane);
   xa.load(ab, M, K, wave, lane);
   xo.load(ob, M, N, wave, lane);
   xg.load(gb, M, N, wave, lane);
 
-  float al[U][4], be[H];
+  float al[UM][4], be[HN];
   xb.settle(N, lane);
   item_cols_part(xb, part, wave, lane);
   xa.settle(K, lane);
   item_rows_exp(xa, al);
   xa.put_cols(EaT, ldm, pad.M, pad.K, wave, lane);
   __syncthreads();
-  item_cols_join<W, H>(part, lane, be);
+  item_cols_join<W, HN>(part, lane, be);
   item_cols_exp(xb, be);
   xb.put_rows(Eb, ldn, pad.K, pad.N, wave, lane);
   // H, and whether the factoring is exact for every cell: S < 2^-40, NaN or infinities anywhere are not
   const float lim = kItemGuardBits * kLn2 + 1e-3f;
   float most = 0.f, worst = 0.f;  // worst stays 0 while every exponent is finite
 #pragma unroll
-  for (int h = 0; h < H; ++h)
+  for (int h = 0; h < HN; ++h)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < UM; ++u)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const bool in = 4 * (wave + W * u) + t < M && lane + 64 * h < N;
@@ -607,14 +611,14 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 8 && U == 3 ? 4 : 1) void
   // Rows of grad_a and columns of grad_b that such a cell takes part in are formed again below, the rows together with
   // those of its wave; the others need none of its H.
   int* const rows = reinterpret_cast<int*>(part);  // marks, then lists (every wave has joined the columns' maxima)
-  int* const cols = rows + 64 * H;
+  int* const cols = rows + 4 * W * UM;
   const int redo = __syncthreads_or(bad);
   if (redo) {  // rare
 #pragma unroll
-    for (int h = 0; h < H; ++h)
+    for (int h = 0; h < HN; ++h)
       if (bad && lane + 64 * h < N) cols[lane + 64 * h] = kItemMark;
     const int m = 4 * (wave + W * (lane >> 2)) + (lane & 3);
-    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane < 4 * U && m < M) rows[m] = kItemMark;
+    if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane < 4 * UM && m < M) rows[m] = kItemMark;
   }
 
   const int l15 = lane & 15, q4 = 4 * (lane >> 4);
@@ -651,7 +655,7 @@ __global__ __launch_bounds__(64 * W, U == 2 ? 8 : W == 8 && U == 3 ? 4 : 1) void
   if (redo) {
     // (values of their own: nothing of this block is formed ahead of it)
     asm volatile("" : "+s"(M), "+s"(K), "+s"(N), "+v"(lane), "+s"(wave));
-    int* const counts = rows + 128 * H;
+    int* const counts = cols + 64 * HN;
     __syncthreads();  // the tiles' results are on their way, LDS is free
     if (wave < 2) {
       const int c = wave == 0 ? item_list(rows, M, lane) : item_list(cols, N, lane);

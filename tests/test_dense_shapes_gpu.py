@@ -214,7 +214,8 @@ def test_log_items_that_cannot_be_factored(gpu, B, M, K, N):
 
 
 ITEMS = [(3, 20, 31, 17), (2, 3, 2, 5), (2, 48, 40, 33), (2, 64, 64, 64), (2, 65, 70, 50), (2, 96, 90, 72), (2, 128, 100, 64),
-         (2, 128, 16, 128), (2, 2, 128, 1), (3, 128, 4, 4)]
+         (2, 128, 16, 128), (2, 2, 128, 1), (3, 128, 4, 4), (3, 9, 5, 16), (2, 3, 4, 128), (2, 32, 128, 32), (2, 128, 32, 32),
+         (2, 32, 32, 128), (2, 128, 32, 128), (2, 66, 2, 67)]
 
 
 def _log_grads(gpu, a, b, g, dt):
