@@ -143,7 +143,8 @@ __device__ __forceinline__ void st4m(E* p, int cnt, float4 v) {
   if (cnt > 2) p[2] = to_elem<E>(v.z);
 }
 // The bytes [x, x + bytes) as a buffer, and an element of it at `at` (per lane) + `base` (uniform) bytes: the uniform
-// part costs no address arithmetic in the lanes.  Reads beyond the end give 0 (at must not be negative).
+// part costs no address arithmetic in the lanes.  Reads beyond the end give 0, and so does a negative `at` with base 0
+// (as an unsigned number it is beyond any end); with another base `at` must not be negative.
 typedef __amdgpu_buffer_rsrc_t buf_t;
 template <class E>
 __device__ __forceinline__ buf_t buf_of(const E* x, unsigned bytes) {
