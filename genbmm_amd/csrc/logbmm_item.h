@@ -6,9 +6,9 @@
 // are taken inside the workgroup, EA = exp(a - alpha), EB = exp(b - beta),
 // S = EA * EB, out = log S + alpha + beta, H = g * exp(alpha + beta - out),
 // grad_a = EA .* (H * EB^T), grad_b = EB .* (EA^T * H).  Rows of the result, rows of grad_a
-// and columns of grad_b with a cell for which the factoring is not exact to fp32 - S < 2^-40, a
-// shift below the reference's -1e9 floor, anything non-finite - are formed again at the end of
-// the same kernel in the reference's own two-pass form (item_fwd_rows, item_bwd_exact).
+// and columns of grad_b with a cell for which the factoring is not exact to fp32 - S < 2^-40,
+// anything non-finite, in the forward a shift below the reference's -1e9 floor - are formed again
+// at the end of the same kernel in the reference's own two-pass form (item_fwd_rows, item_bwd_exact).
 //
 // Staging: a wave takes groups of four neighbouring rows of an array, its lanes the columns (a row is
 // contiguous in memory; all loads of the item are issued before the first is waited for).  A row's

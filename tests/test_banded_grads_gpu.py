@@ -81,7 +81,8 @@ def test_gradients_at_both_ends_of_the_range(gpu, tiny, huge):
 def test_gradients_that_are_not_finite(gpu, mode):
     """An infinite or NaN gradient reaches the cells it is a term of and no other; the others of such a line (a row of the
     gradient's band) may be the exact way's, in which infinity meets no zero of a staged block, and lines without such
-    cells keep their bits.  Sums of the log product that its forward could not factor are the exact way's."""
+    cells keep their bits.  (Infinities within 31 cells of a row's end are left out: a staged block may hold them beside a
+    neighbouring line, times zero, and that line is then the exact way's as well.)  Sums of the log product that its forward could not factor are the exact way's."""
     torch.manual_seed(4)
     band = (32, 32, 32, 32)
     a, b, g = bands(2, 200, 65), bands(2, 200, 65), torch.randn(2, 200, 129)
